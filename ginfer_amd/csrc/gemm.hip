@@ -8,7 +8,7 @@
 // on the tile it falls in, on the rest of the batch, or on which of the three ran:
 //   gemm_nt_few_rows_kernel  up to 64 rows (a decode step, a small portion): the matrix cores' 32-bit instruction, a
 //                            wavefront per 16 columns and up to four blocks of 16 rows, operands straight from memory;
-//   gemm_nt_matrix_kernel    more rows: the matrix cores again, over tiles of up to 128 x 128 through LDS;
+//   gemm_nt_matrix_kernel    more rows: the matrix cores again, over tiles of 32 x 32 to 64 x 96 through LDS;
 //   gemm_nt_kernel           plain FMA, a tile of 64 x 64 per workgroup staged through LDS in steps of K: 33 to 64 rows
 //                            times 65,536 columns and more (a head), where it is the fastest of the three.
 // They are templated on storage, so that they also serve bfloat16 operands (the kernel tests' oracle and the
@@ -136,119 +136,173 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_kernel(TC* __restrict__ 
   }
 }
 
-// The same product on the matrix cores, for many rows.  v_mfma_f32_32x32x2_f32 takes 32-bit operands and adds the two
-// products of its step of K into the accumulator one after the other, each as a fused multiply-add: measured on the
-// device, its results over a K of 512 equal the chain of fmaf over ascending k bit for bit, for every element of the
-// tile.  So this kernel gives the bits of the kernel above at some three times its rate.  A workgroup of four
-// wavefronts, 2 x 2 over a tile of TM x TN; a wavefront owns (TM / 2) x (TN / 2) as blocks of 32 x 32.  Lane l supplies
-// row l % 32 of a block's A and W for k = step + l / 32 and receives, in register r, row 4 (l / 32) + 8 (r / 4) + r % 4
-// and column l % 32 of the block.  Staging as above (k-major in LDS, the next step of K on its way meanwhile); rows
-// are padded by two words so that the transposing stores of a wavefront fall into different banks.
-typedef __attribute__((ext_vector_type(16))) float f32x16;
+// The same product on the matrix cores, for many rows.  v_mfma_f32_16x16x4_f32 takes, from lane l, row l % 16 of A and of
+// W at k = step + l / 16 and adds its four products into the accumulator in ascending k as fused multiply-adds: measured
+// on the device, its results over a K of 512 equal the chain of fmaf over ascending k bit for bit, for every element of
+// the tile.  So this kernel gives the bits of the kernel above.  Register r of lane l receives row 4 (l / 16) + r, column
+// l % 16 of a block.
+//
+// A workgroup of four wavefronts, 2 x 2 over a tile of 32 BM x 32 BN; a wavefront owns BM x BN blocks of 16 x 16.  K must
+// not be split (one accumulator per element), so a block of 16 x 16 is a chain of K / 4 instructions of 32 cycles however
+// the chip is filled (30 us for a K of 8,960): small blocks, so that a few hundred rows make enough chains for all 1,024
+// SIMDs, and a chain that never waits.  DEPTH steps of TK elements are on their way from memory in registers while a step
+// is multiplied out of one of two buffers in LDS, one barrier a step; nothing in the loop is conditional (loads past the
+// end repeat the last step's), so that the compiler waits for just the step it stages.  A row of LDS holds every 16
+// elements of K with the four of a lane side by side (k = g, 4 + g, 8 + g, 12 + g): the operands of four instructions
+// come in one 16-byte read and need no exchange between lanes (with the row swaps of gfx950 after the read the chain of
+// a K of 8,960 took 91 us instead of 62), and with rows padded by four words neither side has bank conflicts.
+// Workgroups that share rows of W are neighbours on one XCD, whose L2 then reads W once.
+// Measured on MI355X, us, before (32 x 32 x 2 blocks in tiles of 64 x 64 to 128 x 128, two barriers a step) -> now, for
+// [rows] x 1,536 of a K of 8,960, x 2,048 of 1,536, and x 17,920 of 1,536: 65 rows 335 -> 62, 55 -> 13.6, 157 -> 62;
+// 256 rows 232 -> 99, 45 -> 21.6, 224 -> 124; 512 rows 232 -> 141, 47.5 -> 39, 327 -> 231; 2,048 rows 634 -> 433,
+// 136 -> 122, 905 -> 886 (127 of the 154 TFLOP/s that a large product reaches on this card).
+typedef __attribute__((ext_vector_type(4))) float f32x4;
 
-template <typename TA, typename TW, typename TC, int TM, int TN, int TK>
+template <typename TA, typename TW, typename TC, int BM, int BN, int TK, int DEPTH>
 __global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_matrix_kernel(TC* __restrict__ C, int64_t ldc,
-                                                                      const TA* __restrict__ A, int64_t lda,
-                                                                      const TW* __restrict__ W,
-                                                                      const TW* __restrict__ bias, int M, int N,
-                                                                      int K, int wide_a, int wide_w) {
-  constexpr int BM = TM / 64, BN = TN / 64;         // blocks of 32 x 32 per wavefront, down and across
+                                                                     const TA* __restrict__ A, int64_t lda,
+                                                                     const TW* __restrict__ W,
+                                                                     const TW* __restrict__ bias, int M, int N, int K,
+                                                                     int wide_a, int wide_w, int m_tiles, int n_tiles) {
+  constexpr int TM = 32 * BM, TN = 32 * BN, PAD = TK + 4;
   constexpr int GA = TM * TK / 4 / GEMM_THREADS, GW = TN * TK / 4 / GEMM_THREADS;
-  static_assert(GA >= 1 && GW >= 1 && TM % 64 == 0 && TN % 64 == 0 && TK % 2 == 0, "tile sizes");
-  __shared__ float a_s[TK][TM + 2];
-  __shared__ float w_s[TK][TN + 2];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
-  const int wm = (wave >> 1) * (TM / 2), wn = (wave & 1) * (TN / 2);     // the wavefront's corner in the tile
-  const int l32 = lane & 31, half = lane >> 5;
-  f32x16 acc[BM][BN];
+  static_assert(GA >= 1 && GW >= 1 && TK % 16 == 0 && DEPTH % 2 == 0, "tile sizes");
+  __shared__ float a_s[2][TM][PAD];
+  __shared__ float w_s[2][TN][PAD];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, i16 = lane & 15, kq = lane >> 4;
+  const int at = blockIdx.x >> 3;
+  const int mt = at % m_tiles, nt = (at / m_tiles) * 8 + (blockIdx.x & 7);
+  if (nt >= n_tiles) return;
+  const int m0 = mt * TM, n0 = nt * TN;
+  const int wm = (wave >> 1) * (TM / 2), wn = (wave & 1) * (TN / 2);
+  f32x4 acc[BM][BN];
 #pragma unroll
   for (int i = 0; i < BM; ++i)
 #pragma unroll
-    for (int j = 0; j < BN; ++j)
+    for (int j = 0; j < BN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float ra[DEPTH][GA][4], rw[DEPTH][GW][4];
+  // rows beyond the matrix are read as row 0's and dropped at the end: no branch in the loop
+  const TA* pa[GA];
+  const TW* pw[GW];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-  float ra[GA][4], rw[GW][4];
-  // a tile that lies inside C, with rows that allow 16-byte loads, asks nothing per load while its step lies inside K
-  const bool inside = wide_a && wide_w && m0 + TM <= M && n0 + TN <= N;
-  auto fetch = [&](int k0) {
-    if (inside && k0 + TK <= K) {
+  for (int i = 0; i < GA; ++i) {
+    const int gi = tid + i * GEMM_THREADS, m = m0 + gi / (TK / 4);
+    pa[i] = A + (int64_t)(m < M ? m : 0) * lda + (gi % (TK / 4)) * 4;
+  }
 #pragma unroll
-      for (int i = 0; i < GA; ++i) {
-        const int gi = tid + i * GEMM_THREADS, row = gi / (TK / 4), k = k0 + (gi % (TK / 4)) * 4;
-        load4<TA>(ra[i], A + (int64_t)(m0 + row) * lda + k, 4, true);
-      }
+  for (int i = 0; i < GW; ++i) {
+    const int gi = tid + i * GEMM_THREADS, n = n0 + gi / (TK / 4);
+    pw[i] = W + (int64_t)(n < N ? n : 0) * K + (gi % (TK / 4)) * 4;
+  }
+  auto fetch = [&](float (&xa)[GA][4], float (&xw)[GW][4], int k0) {
 #pragma unroll
-      for (int i = 0; i < GW; ++i) {
-        const int gi = tid + i * GEMM_THREADS, row = gi / (TK / 4), k = k0 + (gi % (TK / 4)) * 4;
-        load4<TW>(rw[i], W + (int64_t)(n0 + row) * K + k, 4, true);
-      }
-      return;
-    }
+    for (int i = 0; i < GA; ++i) load4<TA>(xa[i], pa[i] + k0, 4, true);
+#pragma unroll
+    for (int i = 0; i < GW; ++i) load4<TW>(xw[i], pw[i] + k0, 4, true);
+  };
+  auto fetch_carefully = [&](float (&xa)[GA][4], float (&xw)[GW][4], int k0) {
+    const int k = k0 + (tid % (TK / 4)) * 4, valid = k < K ? (K - k < 4 ? K - k : 4) : 0;
+#pragma unroll
+    for (int i = 0; i < GA; ++i) load4<TA>(xa[i], pa[i] + k0, valid, false);
+#pragma unroll
+    for (int i = 0; i < GW; ++i) load4<TW>(xw[i], pw[i] + k0, valid, false);
+  };
+  auto stage = [&](int b, float (&xa)[GA][4], float (&xw)[GW][4]) {
 #pragma unroll
     for (int i = 0; i < GA; ++i) {
-      const int gi = tid + i * GEMM_THREADS, row = gi / (TK / 4), k = k0 + (gi % (TK / 4)) * 4;
-      const int m = m0 + row;
-      const int valid = (m < M && k < K) ? (K - k < 4 ? K - k : 4) : 0;
-      if (valid) load4<TA>(ra[i], A + (int64_t)m * lda + k, valid, wide_a != 0);
-      else ra[i][0] = ra[i][1] = ra[i][2] = ra[i][3] = 0.f;
+      const int gi = tid + i * GEMM_THREADS;
+      float* to = &a_s[b][gi / (TK / 4)][(gi % (TK / 4)) / 4 * 16 + gi % 4];
+#pragma unroll
+      for (int g = 0; g < 4; ++g) to[4 * g] = xa[i][g];
     }
 #pragma unroll
     for (int i = 0; i < GW; ++i) {
-      const int gi = tid + i * GEMM_THREADS, row = gi / (TK / 4), k = k0 + (gi % (TK / 4)) * 4;
-      const int n = n0 + row;
-      const int valid = (n < N && k < K) ? (K - k < 4 ? K - k : 4) : 0;
-      if (valid) load4<TW>(rw[i], W + (int64_t)n * K + k, valid, wide_w != 0);
-      else rw[i][0] = rw[i][1] = rw[i][2] = rw[i][3] = 0.f;
+      const int gi = tid + i * GEMM_THREADS;
+      float* to = &w_s[b][gi / (TK / 4)][(gi % (TK / 4)) / 4 * 16 + gi % 4];
+#pragma unroll
+      for (int g = 0; g < 4; ++g) to[4 * g] = xw[i][g];
     }
   };
-  fetch(0);
-  for (int k0 = 0; k0 < K; k0 += TK) {
+  auto read = [&](int b, int kk, float (&x)[BM][4], float (&y)[BN][4]) {
 #pragma unroll
-    for (int i = 0; i < GA; ++i) {
-      const int gi = tid + i * GEMM_THREADS, row = gi / (TK / 4), kk = (gi % (TK / 4)) * 4;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) a_s[kk + j][row] = ra[i][j];
+    for (int i = 0; i < BM; ++i) {
+      const float4 v = *reinterpret_cast<const float4*>(&a_s[b][wm + i * 16 + i16][kk + 4 * kq]);
+      x[i][0] = v.x; x[i][1] = v.y; x[i][2] = v.z; x[i][3] = v.w;
     }
 #pragma unroll
-    for (int i = 0; i < GW; ++i) {
-      const int gi = tid + i * GEMM_THREADS, row = gi / (TK / 4), kk = (gi % (TK / 4)) * 4;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) w_s[kk + j][row] = rw[i][j];
+    for (int j = 0; j < BN; ++j) {
+      const float4 v = *reinterpret_cast<const float4*>(&w_s[b][wn + j * 16 + i16][kk + 4 * kq]);
+      y[j][0] = v.x; y[j][1] = v.y; y[j][2] = v.z; y[j][3] = v.w;
     }
+  };
+  // all operands of a step are asked for before the first is multiplied
+  auto multiply = [&](int b) {
+    float x[TK / 16][BM][4], y[TK / 16][BN][4];
+#pragma unroll
+    for (int c = 0; c < TK / 16; ++c) read(b, c * 16, x[c], y[c]);
+#pragma unroll
+    for (int c = 0; c < TK / 16; ++c) {
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int st = 0; st < 4; ++st)
+#pragma unroll
+        for (int i = 0; i < BM; ++i)
+#pragma unroll
+          for (int j = 0; j < BN; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[c][i][st], y[c][j][st], acc[i][j], 0, 0, 0);
+    }
+  };
+  const int steps = (wide_a && wide_w) ? K / TK : 0, last = (steps - 1) * TK;
+  if (steps > 0) {
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) fetch(ra[d], rw[d], d * TK < last ? d * TK : last);
+    stage(0, ra[0], rw[0]);
+    const int k1 = DEPTH * TK < last ? DEPTH * TK : last;
+    fetch(ra[0], rw[0], k1);
     __syncthreads();
-    if (k0 + TK < K) fetch(k0 + TK);        // on its way while this step is multiplied
+    int s0 = 0;
+    for (; s0 + DEPTH <= steps; s0 += DEPTH) {
 #pragma unroll
-    for (int k = 0; k < TK; k += 2) {
-      float a[BM], w[BN];
-#pragma unroll
-      for (int i = 0; i < BM; ++i) a[i] = a_s[k + half][wm + i * 32 + l32];
-#pragma unroll
-      for (int j = 0; j < BN; ++j) w[j] = w_s[k + half][wn + j * 32 + l32];
-#pragma unroll
-      for (int i = 0; i < BM; ++i)
-#pragma unroll
-        for (int j = 0; j < BN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], w[j], acc[i][j], 0, 0, 0);
+      for (int d = 0; d < DEPTH; ++d) {
+        multiply(d & 1);
+        stage((d & 1) ^ 1, ra[(d + 1) % DEPTH], rw[(d + 1) % DEPTH]);
+        const int k = (s0 + d + 1 + DEPTH) * TK;
+        fetch(ra[(d + 1) % DEPTH], rw[(d + 1) % DEPTH], k < last ? k : last);
+        __syncthreads();
+      }
     }
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+      if (s0 + d < steps) {
+        multiply(d & 1);
+        stage((d & 1) ^ 1, ra[(d + 1) % DEPTH], rw[(d + 1) % DEPTH]);
+        __syncthreads();
+      }
+    }
+  }
+  for (int k0 = steps * TK; k0 < K; k0 += TK) {
+    fetch_carefully(ra[0], rw[0], k0);
+    stage(0, ra[0], rw[0]);
+    __syncthreads();
+    multiply(0);
     __syncthreads();
   }
 #pragma unroll
-  for (int i = 0; i < BM; ++i)
+  for (int j = 0; j < BN; ++j) {
+    const int n = n0 + wn + j * 16 + i16;
+    if (n >= N) continue;
+    const float bv = bias ? Num<TW>::ld(bias + n) : 0.f;
 #pragma unroll
-    for (int j = 0; j < BN; ++j) {
-      const int n = n0 + wn + j * 32 + l32;
-      if (n >= N) continue;
-      const float b = bias ? Num<TW>::ld(bias + n) : 0.f;
+    for (int i = 0; i < BM; ++i)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int m = m0 + wm + i * 32 + half * 4 + 8 * (r / 4) + (r % 4);
+      for (int r = 0; r < 4; ++r) {
+        const int m = m0 + wm + i * 16 + 4 * kq + r;
         if (m >= M) continue;
         float v = acc[i][j][r];
-        if (bias) v += b;
+        if (bias) v += bv;
         Num<TC>::st(C + (int64_t)m * ldc + n, v);
       }
-    }
+  }
 }
 
 // Up to 16 rows (a decode step): one wavefront per 16 columns, no LDS.  v_mfma_f32_16x16x4_f32 takes, from lane l, row
@@ -259,7 +313,6 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_matrix_kernel(TC* __rest
 // lanes 16 and 32 apart).  Of FEW_SETS sets of FEW_DEPTH such loads of A and of W one is multiplied while the others
 // are under way.
 // Register r of lane l receives row 4 (l / 16) + r, column l % 16.
-typedef __attribute__((ext_vector_type(4))) float f32x4;
 #define FEW_DEPTH 8
 #define FEW_SETS 2
 #define FEW_DEPTH_BLOCKS 4     // ... with several blocks of rows (measured: 2, 4, 8)
@@ -400,12 +453,33 @@ extern "C" int ga_gemm_nt(void* C, int64_t ldc, const void* A, int64_t lda, cons
   // rows and very many columns, a head over a large vocabulary, the plain kernel is faster: measured at 151,936 columns)
   const bool few = M <= GEMM_MATRIX_FROM_ROWS && !(M > 32 && N >= 65536);
   const int row_blocks = (M + 15) / 16;
-  // many rows: the matrix cores, in the largest of the tiles 128 x 128, 128 x 64, 64 x 64 that still makes 256 workgroups
+  // many rows: the matrix cores, in tiles of 32 x 32, 64 x 64 or 64 x 96, whichever takes the least time by this sum.  A
+  // chip of 256 compute units works off `rounds` tiles each; the first costs a tile's whole chain, further ones overlap
+  // with it.  Measured in us at a K of 1,536 (alone / each further round): 13.2 / 8.5, 35.5 / 25.5, 47.5 / 39; the sums
+  // come within 6 % of what all the sizes above take in each tiling.
   const bool matrix = M > GEMM_MATRIX_FROM_ROWS;
-  const bool wide = matrix && (int64_t)((M + 127) / 128) * ((N + 127) / 128) >= 256;
-  const bool tall = matrix && !wide && (int64_t)((M + 127) / 128) * ((N + 63) / 64) >= 256;
-  const int tm = (wide || tall) ? 128 : 64, tn = few ? 16 : wide ? 128 : 64;
+  const int tile_m[3] = {32, 64, 64}, tile_n[3] = {32, 64, 96};
+  const float alone[3] = {13.2f, 35.5f, 47.5f}, further[3] = {8.5f, 25.5f, 39.f};
+  int tiling = 0, m_tiles = 0, n_tiles = 0;
+  float least = 0.f;
+  for (int t = 0; matrix && t < 3; ++t) {
+    const int64_t mt = (M + tile_m[t] - 1) / tile_m[t], nt = (N + tile_n[t] - 1) / tile_n[t];
+    const float us = alone[t] + further[t] * (float)((mt * nt + 255) / 256 - 1);
+    if (t == 0 || us < least) {
+      least = us;
+      tiling = t;
+      m_tiles = (int)mt;
+      n_tiles = (int)nt;
+    }
+  }
+  const int tm = 64, tn = few ? 16 : 64;
   dim3 grid((N + tn - 1) / tn, (M + tm - 1) / tm), block(GEMM_THREADS);
+  if (matrix) {
+    if ((M + 127) / 128 > 65535) return -2;
+    const int64_t groups = (int64_t)m_tiles * ((n_tiles + 7) / 8) * 8;     // one dimension: see the kernel's mapping
+    if (groups > 0x7fffffff / GEMM_THREADS) return -2;
+    grid = dim3((unsigned)groups);
+  }
   if (grid.y > 65535) return -2;
   // 16-byte loads (8 bytes for bfloat16) need rows that start at multiples of four elements
   const size_t unit = in_bf16 ? 8 : 16;
@@ -425,18 +499,18 @@ extern "C" int ga_gemm_nt(void* C, int64_t ldc, const void* A, int64_t lda, cons
     else if (few)                                                                                            \
       hipLaunchKernelGGL((gemm_nt_few_rows_kernel<TA, TW, TC, 4>), grid, dim3(64), 0, stream, (TC*)C, ldc,   \
                          (const TA*)A, lda, (const TW*)W, (const TW*)bias, M, N, K, wide_a, wide_w);         \
-    else if (matrix && wide)                                                                                 \
-      hipLaunchKernelGGL((gemm_nt_matrix_kernel<TA, TW, TC, 128, 128, 32>), grid, block, 0, stream,          \
+    else if (matrix && tiling == 0)                                                                          \
+      hipLaunchKernelGGL((gemm_nt_matrix_kernel<TA, TW, TC, 1, 1, 64, 2>), grid, block, 0, stream,           \
                          (TC*)C, ldc, (const TA*)A, lda, (const TW*)W, (const TW*)bias, M, N, K, wide_a,     \
-                         wide_w);                                                                            \
-    else if (matrix && tall)                                                                                 \
-      hipLaunchKernelGGL((gemm_nt_matrix_kernel<TA, TW, TC, 128, 64, 32>), grid, block, 0, stream,           \
+                         wide_w, m_tiles, n_tiles);                                                          \
+    else if (matrix && tiling == 1)                                                                          \
+      hipLaunchKernelGGL((gemm_nt_matrix_kernel<TA, TW, TC, 2, 2, 32, 2>), grid, block, 0, stream,           \
                          (TC*)C, ldc, (const TA*)A, lda, (const TW*)W, (const TW*)bias, M, N, K, wide_a,     \
-                         wide_w);                                                                            \
+                         wide_w, m_tiles, n_tiles);                                                          \
     else if (matrix)                                                                                         \
-      hipLaunchKernelGGL((gemm_nt_matrix_kernel<TA, TW, TC, 64, 64, 32>), grid, block, 0, stream,            \
+      hipLaunchKernelGGL((gemm_nt_matrix_kernel<TA, TW, TC, 2, 3, 32, 2>), grid, block, 0, stream,           \
                          (TC*)C, ldc, (const TA*)A, lda, (const TW*)W, (const TW*)bias, M, N, K, wide_a,     \
-                         wide_w);                                                                            \
+                         wide_w, m_tiles, n_tiles);                                                          \
     else                                                                                                     \
       hipLaunchKernelGGL((gemm_nt_kernel<TA, TW, TC, 64, 64, 32>), grid, block, 0, stream, (TC*)C, ldc,      \
                          (const TA*)A, lda, (const TW*)W, (const TW*)bias, M, N, K, wide_a, wide_w);         \

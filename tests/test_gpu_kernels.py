@@ -179,8 +179,8 @@ def test_gemm_nt_at_drawn_sizes(seed):
 def test_gemm_nt_32_bit_is_the_chain_of_fused_multiply_adds_over_ascending_k(M):
     """What the 32-bit product IS, stated without any kernel: every element starts at zero and takes its K terms in
     ascending order, each as one fused multiply-add (one rounding); the bias is added last.  3 rows run on the
-    16x16x4 matrix instruction, 40 on the same with three blocks of rows to a wavefront, 70 on the 32x32x2 matrix
-    instruction: all must give these bits (the plain-FMA kernel is held against them in the test below)."""
+    16x16x4 matrix instruction, 40 on the same with three blocks of rows to a wavefront, 70 on the same over tiles
+    through LDS: all must give these bits (the plain-FMA kernel is held against them in the test below)."""
     from ginfer_amd.kernels import ops
     N, K = 5, 37
     a, w, b = rnd((M, K), torch.float32, 31), rnd((N, K), torch.float32, 32), rnd((N,), torch.float32, 33)
@@ -213,6 +213,19 @@ def test_gemm_nt_on_the_matrix_cores_gives_the_bits_of_the_fma_kernel(dtype, M, 
         pieces = torch.cat([ops.gemm_nt(a[r:r + rows].contiguous(), w, b, out_dtype=torch.float32) for r in range(0, M, rows)])
         assert torch.equal(pieces, full), "rows %d at a time: %d elements differ" % (rows, int((pieces != full).sum()))
     assert torch.equal(ops.gemm_nt(a[M - 1:].contiguous(), w, b, out_dtype=torch.float32)[0], full[M - 1])
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 31, 64), (97, 33, 63), (96, 64, 65), (129, 100, 128), (70, 40, 193),       # 32 x 32
+                                   (2047, 1537, 31), (2049, 1500, 96), (2048, 1536, 100),                        # 64 x 64
+                                   (255, 4700, 32), (257, 4607, 95), (300, 4609, 224)])                          # 64 x 96
+def test_gemm_nt_tiles_at_their_edges(M, N, K):
+    """One row, column or element of K more or less than the three tilings of the kernel for many rows hold, and K of one
+    step, an odd and an even number of steps: the bits of 16 rows at a time, which another kernel multiplies."""
+    from ginfer_amd.kernels import ops
+    a, w, b = rnd((M, K), torch.float32, 21), rnd((N, K), torch.float32, 22), rnd((N,), torch.float32, 23)
+    full = ops.gemm_nt(a, w, b)
+    for r in sorted({0, M // 2, M - 16}):
+        assert torch.equal(ops.gemm_nt(a[r:r + 16].contiguous(), w, b), full[r:r + 16]), "rows from %d" % r
 
 
 @pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-4), (torch.bfloat16, 1e-2)])
