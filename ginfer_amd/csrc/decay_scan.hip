@@ -6,137 +6,99 @@
 // with i + rot_dims / 2; angle tables cos, sin float [positions, rot_dims / 2]) and are then multiplied by q_scale and
 // k_scale.  q, k and v are 32-bit rows of one projection (a common row stride).
 // The state is 32-bit, [slot][head][dim][vdim]; a request whose q_start is 0 starts from zeros.  A workgroup owns one
-// (entry, head, block of 16 value columns) and walks the entry's tokens in order, up to 16 at a time: the tile's q, k, a and v go
-// through LDS (asked for from memory a tile ahead), every thread keeps the state of one column and every 16th row in registers, and the rows' partial
-// outputs are added in a fixed order.  So a token's result does not depend on how the request's tokens were cut into
-// steps, nor on what else is in the batch.
+// (entry, head, block of 8 or 16 value columns) and walks the entry's tokens in order (decay_walk.h): a token's result does
+// not depend on how the request's tokens were cut into steps, nor on what else is in the batch.
 // gla_decay: a = sigmoid(z)^(1/tau), z = A2 (low) + b (A2 handed over transposed), `low` being the rows of a narrow projection (32-bit), as
 //   exp(-softplus(-z) / tau), all in 32-bit.
 // head_norm_gate (times out_scale; weight: shared by the heads, or every head its own): out[t, h, :] = o[t, h, :] / sqrt(mean(o[t, h, :]^2) + eps) (* weight[:]) (* silu(gate[t, h, :]), or * sigmoid of it).
 // silu_inputs: the recurrence reads silu(q), silu(k), silu(v) in place of the projection's numbers.
-#include "common.h"
+#include "decay_walk.h"
 #include "ginfer_amd.h"
 
 #define DS_THREADS 256
-#define DS_COLS 16        // value columns of a workgroup
-#define DS_SLICES 16      // a column's rows are dealt to this many threads
 
-template <int R, int TILE>   // R rows of the state per thread: dim <= 16 * R; TILE tokens per trip through LDS (<= 16)
-__global__ __launch_bounds__(DS_THREADS) void decay_scan_kernel(
+// q, k and v as the recurrence reads them: the projection's numbers or their silu, turned by position, scaled
+template <bool ROT>
+struct DecayRows {
+  struct Plain { float q, k, a; };
+  struct Turned { float q, k, a, q2, k2, c, s; };
+  typedef typename std::conditional<ROT, Turned, Plain>::type Raw;
+  const float *q, *k, *v;              // the entry's first token, the head's first channel or column
+  const float* decay;                  // the same of [tokens, heads * dim]; or one number, and both steps are 0
+  const float *cos_t, *sin_t;          // the first token's position
+  int64_t stride;
+  int decay_token, decay_channel, half;
+  float q_scale, k_scale;
+  bool acts;                           // whether finish and finish_v apply the silu: asked once a tile, not per element
+  template <bool ACT>
+  __device__ __forceinline__ float act(float z) const { return ACT ? z / (1.0f + expf(-z)) : z; }
+  __device__ __forceinline__ void load(Raw& x, int start, int t, int i) const {
+    const float *qp = q + start * stride, *kp = k + start * stride;
+    const uint32_t row = (uint32_t)t * (uint32_t)stride;
+    x.q = qp[row + i];
+    x.k = kp[row + i];
+    x.a = (decay + (int64_t)start * decay_token)[(uint32_t)(t * decay_token + i * decay_channel)];
+    if constexpr (ROT) {               // (a channel that is not turned reads what channel 0 reads, and drops it)
+      const int at = i < 2 * half ? i : 0, f = at < half ? at : at - half, other = at < half ? at + half : at - half;
+      x.c = (cos_t + (int64_t)start * half)[(uint32_t)(t * half + f)];
+      x.s = (sin_t + (int64_t)start * half)[(uint32_t)(t * half + f)];
+      x.q2 = qp[row + other];
+      x.k2 = kp[row + other];
+    }
+  }
+  template <bool ACT>
+  __device__ __forceinline__ void finish(const Raw& x, int i, float& qv, float& kv, float& a) const {
+    qv = act<ACT>(x.q);
+    kv = act<ACT>(x.k);
+    if constexpr (ROT) {
+      if (i < 2 * half) {              // the pair (lo, hi) becomes (lo c - hi s, hi c + lo s)
+        const float qo = act<ACT>(x.q2), ko = act<ACT>(x.k2);
+        qv = i < half ? qv * x.c - qo * x.s : qv * x.c + qo * x.s;
+        kv = i < half ? kv * x.c - ko * x.s : kv * x.c + ko * x.s;
+      }
+    }
+    qv *= q_scale;
+    kv *= k_scale;
+    a = x.a;
+  }
+  __device__ __forceinline__ float load_v(int start, int t, int c) const {
+    return (v + start * stride)[(uint32_t)t * (uint32_t)stride + c];
+  }
+  template <bool ACT>
+  __device__ __forceinline__ float finish_v(float x) const { return act<ACT>(x); }
+};
+
+// Measured on MI355X, 2,048 tokens of one request, 12 heads of 64 x 128, us, before (16 columns a workgroup whose every wavefront
+// brings, walks and adds up, operands in single reads, three barriers a tile) -> now: a decay per channel 412 -> 118, a
+// constant one with rotation 450 -> 143, with silu 463 -> 174; 28 heads 415 -> 167, 456 -> 286, 476 -> 236; five entries of 918
+// tokens 107 -> 52, 113 -> 73, 115 -> 68.  64 entries of one token: 18.7 -> 18.9 (reading and writing the state).
+template <int R, int COLS, int TILE, bool ROT>   // R rows of the state per thread: dim <= 16 * R
+__global__ __launch_bounds__(dw_threads(COLS)) void decay_scan_kernel(
     float* __restrict__ out, const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
     int64_t stride, const float* __restrict__ decay, const float* __restrict__ head_decay, const float* __restrict__ cos_t,
     const float* __restrict__ sin_t, int rot_dims, float q_scale, float k_scale, float* __restrict__ state,
     const int64_t* __restrict__ slots, const int32_t* __restrict__ cu, const int32_t* __restrict__ q_start, int heads,
     int dim, int vdim, int silu_inputs) {
-  constexpr int DP = DS_SLICES * R;
-  __shared__ float qs[TILE][DP], ks[TILE][DP], as[TILE][DP], vs[TILE][DS_COLS];
-  __shared__ float partial[TILE][DS_SLICES][DS_COLS];
-  const int e = blockIdx.x, h = blockIdx.y, v0 = blockIdx.z * DS_COLS;
+  const int e = blockIdx.x, h = blockIdx.y;
   const int first = cu[e], n = cu[e + 1] - first;
   if (n <= 0) return;
-  const int j = threadIdx.x % DS_COLS, s = threadIdx.x / DS_COLS;
-  const bool col_ok = v0 + j < vdim;
-  float* st = state + ((slots[e] * heads + h) * (int64_t)dim) * vdim + v0 + j;
-  float S[R];
   const int start = q_start[e];
-  const bool fresh = start == 0;
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const int i = s + DS_SLICES * r;
-    S[r] = (!fresh && col_ok && i < dim) ? st[(int64_t)i * vdim] : 0.f;
-  }
-  const int hd = heads * dim, half = rot_dims / 2;
-  const float hdec = head_decay ? head_decay[h] : 0.f;
-  // A thread's share of a tile's q, k and a (PER elements each) and one v: asked for a tile ahead, into registers, so
-  // that the way to memory runs beside the walk over the tile before.
-  constexpr int PER = TILE * DP / DS_THREADS;
-  float rq[PER], rk[PER], ra[PER], rv;
-  // q, k and v as the recurrence reads them: the projection's numbers, or their silu
-  auto act = [&](float z) { return silu_inputs ? z / (1.0f + expf(-z)) : z; };
-  // without a rotation, the activation (and the scales behind it) waits until a tile is stored to LDS: the fetch runs a tile
-  // ahead, and nothing in it should use what its loads bring
-  const bool late = silu_inputs && rot_dims == 0;
-  auto fetch = [&](int t0) {
-    const int nt = min(TILE, n - t0);
-#pragma unroll
-    for (int x = 0; x < PER; ++x) {
-      const int idx = threadIdx.x + x * DS_THREADS;
-      const int tt = idx / DP, i = idx % DP;
-      float qv = 0.f, kv = 0.f, a = 0.f;
-      if (tt < nt && i < dim) {
-        const int64_t row = first + t0 + tt;
-        const float* qp = q + row * stride + h * dim;
-        const float* kp = k + row * stride + h * dim;
-        qv = late ? qp[i] : act(qp[i]);
-        kv = late ? kp[i] : act(kp[i]);
-        if (i < rot_dims) {
-          const int f = i < half ? i : i - half, other = i < half ? i + half : i - half;
-          const int64_t at = (int64_t)(start + t0 + tt) * half + f;
-          const float c = cos_t[at], sn = sin_t[at];
-          const float qo = act(qp[other]), ko = act(kp[other]);
-          // the pair (lo, hi) becomes (lo c - hi s, hi c + lo s)
-          qv = i < half ? qv * c - qo * sn : qv * c + qo * sn;
-          kv = i < half ? kv * c - ko * sn : kv * c + ko * sn;
-        }
-        if (!late) {
-          qv *= q_scale;
-          kv *= k_scale;
-        }
-        a = decay ? decay[row * hd + h * dim + i] : hdec;
-      }
-      rq[x] = qv;
-      rk[x] = kv;
-      ra[x] = a;
-    }
-    const int tt = threadIdx.x / DS_COLS, jj = threadIdx.x % DS_COLS;      // 16 * DS_COLS == DS_THREADS
-    rv = (tt < nt && v0 + jj < vdim) ? v[(int64_t)(first + t0 + tt) * stride + h * vdim + v0 + jj] : 0.f;
-  };
-  fetch(0);
-  for (int t0 = 0; t0 < n; t0 += TILE) {
-    const int nt = min(TILE, n - t0);
-    __syncthreads();                                   // the tile before is read out
-#pragma unroll
-    for (int x = 0; x < PER; ++x) {
-      const int idx = threadIdx.x + x * DS_THREADS;
-      qs[idx / DP][idx % DP] = late ? act(rq[x]) * q_scale : rq[x];
-      ks[idx / DP][idx % DP] = late ? act(rk[x]) * k_scale : rk[x];
-      as[idx / DP][idx % DP] = ra[x];
-    }
-    {
-      const int tt = threadIdx.x / DS_COLS, jj = threadIdx.x % DS_COLS;
-      if (tt < TILE) vs[tt][jj] = act(rv);
-    }
-    __syncthreads();
-    if (t0 + TILE < n) fetch(t0 + TILE);
-    for (int tt = 0; tt < nt; ++tt) {
-      const float vv = vs[tt][j];
-      float acc = 0.f;
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const int i = s + DS_SLICES * r;
-        S[r] = as[tt][i] * S[r] + ks[tt][i] * vv;
-        acc += S[r] * qs[tt][i];
-      }
-      partial[tt][s][j] = acc;
-    }
-    __syncthreads();
-    {
-      const int tt = threadIdx.x / DS_COLS, jj = threadIdx.x % DS_COLS;
-      if (tt < nt && v0 + jj < vdim) {
-        float o = 0.f;
-#pragma unroll
-        for (int p = 0; p < DS_SLICES; ++p) o += partial[tt][p][jj];
-        out[((int64_t)(first + t0 + tt) * heads + h) * vdim + v0 + jj] = o;
-      }
-    }
-  }
-  if (col_ok) {
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int i = s + DS_SLICES * r;
-      if (i < dim) st[(int64_t)i * vdim] = S[r];
-    }
-  }
+  DecayRows<ROT> rows;
+  rows.q = q + first * stride + h * dim;
+  rows.k = k + first * stride + h * dim;
+  rows.v = v + first * stride + h * vdim;
+  rows.decay = decay ? decay + (int64_t)first * heads * dim + h * dim : head_decay + h;
+  rows.decay_token = decay ? heads * dim : 0;
+  rows.decay_channel = decay ? 1 : 0;
+  rows.half = rot_dims / 2;
+  rows.cos_t = ROT ? cos_t + (int64_t)start * rows.half : nullptr;
+  rows.sin_t = ROT ? sin_t + (int64_t)start * rows.half : nullptr;
+  rows.stride = stride;
+  rows.q_scale = q_scale;
+  rows.k_scale = k_scale;
+  rows.acts = silu_inputs != 0;
+  decay_walk<R, COLS, TILE>(out + ((int64_t)first * heads + h) * vdim, rows, state + ((slots[e] * heads + h) * (int64_t)dim) * vdim,
+                            start == 0, n, heads, dim, vdim, (int)blockIdx.z * COLS);
 }
 
 // decay[t, c] = exp(-softplus(-z) / tau), z = sum_r a2t[r, c] * low[t, r] + bias[c], the sum in ascending r.  a2t is the
@@ -344,27 +306,26 @@ __global__ __launch_bounds__(DS_THREADS) void wide_norm_gate_rows_kernel(T* __re
 
 extern "C" int ga_decay_scan(void* out, const void* q, const void* k, const void* v, int64_t stride, const void* decay,
                              const void* head_decay, const void* cos_t, const void* sin_t, int rot_dims, float q_scale,
-                             float k_scale, void* state, const void* slots, const void* cu, const void* q_start, int entries,
+                             float k_scale, void* state, const void* slots, const void* cu, const void* q_start, int tokens, int entries,
                              int heads, int dim, int vdim, int silu_inputs, hipStream_t stream) {
   if (entries <= 0) return 0;
-  if (heads <= 0 || dim <= 0 || vdim <= 0 || dim > 16 * DS_SLICES) return -1;
-  if (heads > 65535 || (vdim + DS_COLS - 1) / DS_COLS > 65535) return -2;
+  if (heads <= 0 || dim <= 0 || vdim <= 0 || dim > 16 * DW_SLICES) return -1;
+  if (heads > 65535 || (vdim + 15) / 16 > 65535 || stride >= (1ll << 27)) return -2;    // (a tile's offsets are 32-bit)
   if ((decay == nullptr) == (head_decay == nullptr)) return -3;
   if (rot_dims < 0 || rot_dims % 2 || rot_dims > dim || (rot_dims > 0 && (!cos_t || !sin_t))) return -4;
-  dim3 grid(entries, heads, (vdim + DS_COLS - 1) / DS_COLS), block(DS_THREADS);
-  const int rows = (dim + DS_SLICES - 1) / DS_SLICES;
-#define GO(R, T) hipLaunchKernelGGL((decay_scan_kernel<R, T>), grid, block, 0, stream, (float*)out, (const float*)q, (const float*)k, \
-                                 (const float*)v, stride, (const float*)decay, (const float*)head_decay, (const float*)cos_t,  \
-                                 (const float*)sin_t, rot_dims, q_scale, k_scale, (float*)state, (const int64_t*)slots,       \
-                                 (const int32_t*)cu, (const int32_t*)q_start, heads, dim, vdim, silu_inputs)
-  if (rows <= 1) GO(1, 16);
-  else if (rows <= 2) GO(2, 16);
-  else if (rows <= 3) GO(3, 16);
-  else if (rows <= 4) GO(4, 16);
-  else if (rows <= 6) GO(6, 16);
-  else if (rows <= 8) GO(8, 16);
-  else if (rows <= 12) GO(12, 16);
-  else GO(16, 8);      // the widest heads take half the tokens a trip: the tile's operands fill the LDS
+  const int rows = (dim + DW_SLICES - 1) / DW_SLICES;
+#define GO(R, C, T, ROT) hipLaunchKernelGGL((decay_scan_kernel<R, C, T, ROT>), dim3(entries, heads, (vdim + C - 1) / C), dim3(dw_threads(C)), 0,  \
+                                 stream, (float*)out, (const float*)q, (const float*)k, (const float*)v, stride, (const float*)decay,   \
+                                 (const float*)head_decay, (const float*)cos_t, (const float*)sin_t, rot_dims, q_scale, k_scale,        \
+                                 (float*)state, (const int64_t*)slots, (const int32_t*)cu, (const int32_t*)q_start, heads, dim, vdim,   \
+                                 silu_inputs)
+#define GR(R, C, T) do { if (rot_dims > 0) GO(R, C, T, true); else GO(R, C, T, false); } while (0)
+  if (decay_walk_narrow(tokens, entries, heads, vdim)) {
+    DW_ROWS(rows, 8, GR);
+  } else {
+    DW_ROWS(rows, 16, GR);
+  }
+#undef GR
 #undef GO
   return GA_CHECK_LAUNCH();
 }

@@ -112,8 +112,8 @@ int ga_short_conv_update(void* state, const void* x, const void* slots, const vo
 // ---- gated_recurrence.hip: the HGRN2 recurrence.  proj float [tokens, 2 heads dim + heads vdim] (row stride given) holds
 // (q before its SiLU | forget-gate logits | v); state float [slots, heads, dim, vdim]; out float [tokens, heads, vdim]
 int ga_hgrn2_scan(void* out, const void* proj, int64_t proj_stride, const void* f_bias, const void* lower, void* state,
-                  const void* slots, const void* cu, const void* q_start, int entries, int heads, int dim, int vdim,
-                  hipStream_t stream);
+                  const void* slots, const void* cu, const void* q_start, int tokens, int entries, int heads, int dim,
+                  int vdim, hipStream_t stream);
 // out [rows, vdim] (compute dtype) = x / sqrt(mean(x^2) + eps) * weight, x float [rows, vdim], weight float [vdim]
 int ga_headwise_rmsnorm(void* out, const void* x, const void* weight, int64_t rows, int vdim, float eps, int out_bf16,
                         hipStream_t stream);
@@ -300,8 +300,8 @@ int ga_layer_norm_add(void* residual, int num_tokens, const void* y1, int y1_f32
 // whose q_start is 0; out float [tokens, heads, vdim]
 int ga_decay_scan(void* out, const void* q, const void* k, const void* v, int64_t stride, const void* decay,
                   const void* head_decay, const void* cos_t, const void* sin_t, int rot_dims, float q_scale, float k_scale,
-                  void* state, const void* slots, const void* cu, const void* q_start, int entries, int heads, int dim,
-                  int vdim, int silu_inputs, hipStream_t stream);
+                  void* state, const void* slots, const void* cu, const void* q_start, int tokens, int entries, int heads,
+                  int dim, int vdim, int silu_inputs, hipStream_t stream);
 // decay float [tokens, channels] = sigmoid(a2 low + bias)^(1 / tau); low: 32-bit rows of `rank` numbers with a stride; a2t:
 // a2 transposed, float [rank, channels]
 int ga_gla_decay(void* decay, const void* low, int64_t low_stride, const void* a2t, const void* bias, int tokens,

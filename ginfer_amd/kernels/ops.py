@@ -956,7 +956,8 @@ def hgrn2_scan(proj, f_bias, lower, state, slots, step, heads, dim, vdim, update
     out = torch.empty((T, heads, vdim), dtype=torch.float32, device=proj.device)
     lib = build.load("gated_recurrence")
     _check(lib.ga_hgrn2_scan(_ptr(out), _ptr(proj), _i64(proj.stride(0)), _ptr(f_bias), _ptr(lower), _ptr(state), _ptr(slots),
-                             _ptr(step.cu_tokens), _ptr(step.q_start), _i(E), _i(heads), _i(dim), _i(vdim), _stream()), "hgrn2_scan")
+                             _ptr(step.cu_tokens), _ptr(step.q_start), _i(T), _i(E), _i(heads), _i(dim), _i(vdim), _stream()),
+           "hgrn2_scan")
     return out
 
 
@@ -1632,7 +1633,7 @@ def decay_scan(proj, q_start, k_start, v_start, state, slots, step, heads, dim, 
     lib = build.load("decay_scan")
     _check(lib.ga_decay_scan(_ptr(out), _ptr(q), _ptr(k), _ptr(v), _i64(proj.stride(0)), _ptr(decay), _ptr(head_decay),
                              _ptr(cos), _ptr(sin), _i(rot), _f(q_scale), _f(k_scale), _ptr(state), _ptr(slots),
-                             _ptr(step.cu_tokens), _ptr(step.q_start), _i(E), _i(heads), _i(dim), _i(vdim),
+                             _ptr(step.cu_tokens), _ptr(step.q_start), _i(T), _i(E), _i(heads), _i(dim), _i(vdim),
                              _i(1 if silu_inputs else 0), _stream()), "decay_scan")
     return out
 

@@ -264,6 +264,35 @@ def test_recurrence_across_cuts_and_a_slot_that_was_used(heads, dim, vdim):
         assert torch.equal(state[3], final), kind
 
 
+@pytest.mark.parametrize("dim", [16, 48, 64, 130, 250])
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 16, 17, 40])
+def test_recurrences_of_many_entries_give_the_bits_of_one_alone(dim, n):
+    """Many entries take workgroups of 16 value columns, a single one takes 8 and wavefronts that only bring and put: the
+    same bits, with tokens below, at and above what either walks at a time (4 to 16), and odd columns."""
+    from ginfer_amd.kernels import ops
+    E, heads, vdim = 33, 8, 17
+    g = torch.Generator().manual_seed(n)
+    proj = torch.randn((E * n, 2 * heads * dim + heads * vdim), generator=g).cuda()
+    decay = (torch.rand((E * n, heads * dim), generator=g) * 0.9 + 0.1).cuda()
+    bias, lower = torch.randn((heads * dim,), generator=g).cuda(), torch.rand((heads * dim,), generator=g).cuda()
+    state = torch.randn((E, heads, dim, vdim), generator=g).cuda()
+    ang = torch.outer(torch.arange(64.0), torch.linspace(1.0, 0.01, 5)).cuda()
+    tables = dict(cos=torch.cos(ang).contiguous(), sin=torch.sin(ang).contiguous())
+    runs = {
+        "channel": lambda p, d, st, sl, step: ops.decay_scan(p, 0, heads * dim, 2 * heads * dim, st, sl, step, heads, dim, vdim, decay=d),
+        "head": lambda p, d, st, sl, step: ops.decay_scan(p, 0, heads * dim, 2 * heads * dim, st, sl, step, heads, dim, vdim,
+                                                          head_decay=lower[:heads].contiguous(), silu_inputs=True, **tables),
+        "hgrn2": lambda p, d, st, sl, step: ops.hgrn2_scan(p, bias, lower, st, sl, step, heads, dim, vdim)}
+    for kind, run in runs.items():
+        many, one = state.clone(), state.clone()
+        got = run(proj, decay, many, torch.arange(E, device="cuda"), _Step([n] * E, [3] * E))
+        for e in (0, 17, E - 1):
+            rows = slice(e * n, (e + 1) * n)
+            alone = run(proj[rows], decay[rows].contiguous(), one, torch.tensor([e], device="cuda"), _Step([n], [3]))
+            assert torch.equal(alone, got[rows]), kind
+            assert torch.equal(one[e], many[e]), kind
+
+
 def test_heads_normed_and_gated():
     from ginfer_amd.kernels import ops
     g = torch.Generator().manual_seed(3)
