@@ -87,11 +87,12 @@ int ga_clamped_glu(void* out, const void* gu, int tokens, int inter, float limit
 
 // ---- scalar_norm.hip: RMS norm with ONE gain for all coordinates (gain: one float or bfloat16).  rows: out [num_rows,
 // hidden] = norm of the rows x[rows[r]] of the float stream (rows null: all rows in order).  add: residual float
-// [tokens, hidden] += norm(y); copy (or null): the new residual in y's dtype
+// [tokens, hidden] += norm(y); copy (or null): the new residual, in bfloat16 (copy_bf16; always for a bfloat16 y) or float.
+// parts > 1: y is float [parts, tokens, hidden], added up in order (hidden a multiple of 4 up to 4,096, 16-byte addresses)
 int ga_scalar_rmsnorm_rows(void* out, const void* x, const void* gain, const void* rows, int num_rows, int hidden, float eps,
                            int out_bf16, int gain_bf16, hipStream_t stream);
 int ga_add_scalar_rmsnorm(void* residual, const void* y, const void* gain, void* copy, int tokens, int hidden, float eps,
-                          int y_bf16, int gain_bf16, hipStream_t stream);
+                          int y_bf16, int gain_bf16, int parts, int copy_bf16, hipStream_t stream);
 
 // ---- embedding_sinusoid.hip: out float [tokens, hidden] = table_scale * table[ids] + (sin | cos)(position * freq[i / 2]), then the norm
 // with one gain (gain null: no norm); freq float [(hidden + 1) / 2]

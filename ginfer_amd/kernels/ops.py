@@ -864,20 +864,32 @@ def scalar_rmsnorm_rows(x, gain, eps, dtype, rows=None):
     return out
 
 
-def add_scalar_rmsnorm(residual, y, gain, eps, copy=False):
-    """residual float32 [T, H] += g * y / sqrt(mean(y^2) + eps), in place; y [T, H] float32 or bfloat16.  With copy the
-    new residual also comes back in y's dtype (what the next product reads); for a float32 y that is the residual itself."""
+ADD_SCALAR_NORM_PARTS_MAX = 4096     # columns up to which the kernel adds partial sums up itself
+
+
+def add_scalar_rmsnorm(residual, y, gain, eps, copy=False, copy_dtype=None):
+    """residual float32 [T, H] += g * y / sqrt(mean(y^2) + eps), in place; y [T, H] float32 or bfloat16, or float32 partial
+    sums [parts, T, H], added up in order.  With copy the new residual also comes back in y's dtype or `copy_dtype` (what the
+    next product reads); in float32 that is the residual itself."""
     _dev(residual, y, gain)
     _need(residual.dtype == torch.float32 and residual.dim() == 2 and residual.is_contiguous(),
           "residual must be contiguous float32 [T, H]")
-    _need(y.shape == residual.shape and y.is_contiguous(), "y must be contiguous %s, got %s", tuple(residual.shape), tuple(y.shape))
     T, H = residual.shape
-    out = None
-    if copy and y.dtype != torch.float32:
-        out = torch.empty((T, H), dtype=y.dtype, device=y.device)
+    parts = 1
+    if y.dim() == 3:
+        _need(y.dtype == torch.float32, "partial sums must be float32, got %s", y.dtype)
+        if H % 4 or H > ADD_SCALAR_NORM_PARTS_MAX:
+            y = y.sum(dim=0)
+        else:
+            parts = y.shape[0]
+    _need(tuple(y.shape[-2:]) == (T, H) and y.is_contiguous(), "y must be contiguous %s, got %s", (T, H), tuple(y.shape))
+    out, out_dtype = None, copy_dtype or y.dtype
+    _need(y.dtype == torch.float32 or out_dtype == y.dtype, "the copy of a bfloat16 y is bfloat16")
+    if copy and out_dtype != torch.float32:
+        out = torch.empty((T, H), dtype=out_dtype, device=y.device)
     lib = build.load("scalar_norm")
     _check(lib.ga_add_scalar_rmsnorm(_ptr(residual), _ptr(y), _ptr(gain), _ptr(out), _i(T), _i(H), _f(eps), _i(_is_bf16(y.dtype)),
-                                     _i(_scalar_gain(gain)), _stream()), "add_scalar_rmsnorm")
+                                     _i(_scalar_gain(gain)), _i(parts), _i(_is_bf16(out_dtype)), _stream()), "add_scalar_rmsnorm")
     if not copy:
         return None
     return out if out is not None else residual

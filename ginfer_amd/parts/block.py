@@ -102,6 +102,9 @@ class OutputNormBlock(Arrangement):
             if norm is not None and not hasattr(norm, "add_normed"):
                 raise ValueError("the norms of this block sit on the sublayers' outputs: %s has no add_normed"
                                  % type(norm).__name__)
+        # the feed-forward's last product may leave its partial sums to the norm behind it
+        self._parts_ok = (getattr(self.feed_forward, "makes_partial_sums", False)
+                          and getattr(self.feed_forward_norm, "adds_partial_sums", False))
 
     def cache_spec(self):
         conv = self.input_conv.cache_spec() if self.input_conv is not None else None
@@ -119,7 +122,8 @@ class OutputNormBlock(Arrangement):
         m = self.mixer.forward(h, step, mixer_cache)
         x = self.mixer_norm.add_normed(residual, m, copy=self.feed_forward is not None)
         if self.feed_forward is not None:
-            self.feed_forward_norm.add_normed(residual, self.feed_forward.forward(x))
+            y = self.feed_forward.forward(x, parts_ok=True) if self._parts_ok else self.feed_forward.forward(x)
+            self.feed_forward_norm.add_normed(residual, y)
         return None
 
 

@@ -54,6 +54,7 @@ class ClampedGLU(Part):
     The tensors are named gate, up and down."""
 
     capturable = True
+    makes_partial_sums = True      # forward takes parts_ok: the result may be float32 [parts, T, H] for the norm that follows
 
     def __init__(self, hidden_size, intermediate_size, limit, dtype, device, alpha=1.702, shift=1.0):
         self.hidden_size, self.intermediate_size = int(hidden_size), int(intermediate_size)
@@ -72,7 +73,7 @@ class ClampedGLU(Part):
     def kernel_modules(self):
         return ["activation", "gemm"] + (["gemm_skinny"] if self.dtype == torch.bfloat16 else [])
 
-    def forward(self, x):
+    def forward(self, x, parts_ok=False):
         # few rows (decode): the weight-streaming product with the activation in its epilogue, where the rules would
         # take that kernel for the SiLU gate too; else the product and the activation's own pass
         if (x.dtype == torch.bfloat16 and ops.gemm_skinny_supported(x, self.w_gate_up)
@@ -80,7 +81,7 @@ class ClampedGLU(Part):
             act = ops.gemm_skinny(x, self.w_gate_up, gated=True, gate_bounds=(self.limit, self.alpha, self.shift))
         else:
             act = ops.clamped_glu(linear(x, self.w_gate_up), self.limit, self.alpha, self.shift)
-        return linear(act, self.w_down)
+        return linear(act, self.w_down, parts_ok=parts_ok)
 
 
 @register_feed_forward("squared_relu")

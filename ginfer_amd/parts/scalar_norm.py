@@ -14,6 +14,7 @@ class ScalarRMSNorm(Part):
 
     capturable = True
     accepts_partial_sums = False
+    adds_partial_sums = True     # add_normed takes float32 [parts, T, H] and adds the parts up in order
     foldable = False         # the products around it cannot fold it: it does not sit before a product
 
     def __init__(self, size, eps, dtype, device):
@@ -40,4 +41,4 @@ class ScalarRMSNorm(Part):
     def add_normed(self, residual, y, copy=False):
         """residual += norm(y) in place.  With copy: the new residual in the compute dtype (for the product that reads it
         next); in 32-bit that is the residual itself."""
-        return ops.add_scalar_rmsnorm(residual, y, self.weight, self.eps, copy=copy)
+        return ops.add_scalar_rmsnorm(residual, y, self.weight, self.eps, copy=copy, copy_dtype=self.dtype)

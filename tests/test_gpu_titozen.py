@@ -152,6 +152,21 @@ def test_norm_with_one_gain():
         assert H.rel_err(copy.float().cpu(), ref) < 5e-3
 
 
+@pytest.mark.parametrize("width", [4, 1000, 1024, 1028, 2052, 4096, 4100, 1001])
+@pytest.mark.parametrize("parts", [1, 2, 5])
+def test_norm_with_one_gain_over_partial_sums(width, parts):
+    """Widths at the edges of what a thread holds, and beyond what the kernel takes in parts; a copy in either type."""
+    from ginfer_amd.kernels import ops
+    g = torch.Generator().manual_seed(width)
+    x, y, gain = torch.randn((3, width), generator=g) * 3, torch.randn((parts, 3, width), generator=g), torch.tensor([0.7])
+    ref = x.double() + pt.scalar_norm(y.double().sum(0), 0.7, 1e-5)
+    for dtype in (torch.bfloat16, torch.float32):
+        res = x.cuda().clone()
+        copy = ops.add_scalar_rmsnorm(res, (y if parts > 1 else y[0]).cuda(), gain.cuda(), 1e-5, copy=True, copy_dtype=dtype)
+        assert H.rel_err(res.cpu(), ref) < 1e-6 and copy.dtype == dtype
+        assert torch.equal(copy, res.to(dtype))
+
+
 def test_embedding_with_position_vectors_far_into_a_sequence():
     from ginfer_amd.kernels import ops
     g = torch.Generator().manual_seed(1)
