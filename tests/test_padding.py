@@ -78,3 +78,12 @@ def test_rows_go_to_records_and_tiles():
     assert rows == [0, 21] and pos == [5, 8] and entries == [0, 2]
     assert sorted(tiles) == [(1, 1, 16, 0), (1, 17, 4, 16), (3, 22, 3, 40)]
     assert tiles[0] == (3, 22, 3, 40)            # the tile with the most keys comes first
+
+
+def test_a_step_of_portions_alone_gets_no_records_of_single_tokens():
+    host = host_arrays([40, 7], [0, 16])
+    assert len(host["decode_info"]) == 0
+    p = pad_step(host, 64, 8, 16, pad_slot=99, n_single=0)
+    assert p["decode_info"].shape == (0, 4)
+    full = pad_step(host, 64, 8, 16, pad_slot=99)
+    assert all(np.array_equal(p[k], full[k]) for k in ("ids", "pos", "ent", "cu", "q_len", "rows", "tiles", "state_slots"))
