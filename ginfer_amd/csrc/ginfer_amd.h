@@ -94,6 +94,13 @@ int ga_scalar_rmsnorm_rows(void* out, const void* x, const void* gain, const voi
 int ga_add_scalar_rmsnorm(void* residual, const void* y, const void* gain, void* copy, int tokens, int hidden, float eps,
                           int y_bf16, int gain_bf16, int parts, int copy_bf16, hipStream_t stream);
 
+// ---- gemm_tiles.hip: bfloat16 products over tiles through LDS; A [M, K] (row stride lda), W [rows, K] contiguous, 16-byte
+// addresses, K a multiple of 64, cols of 8.  gated: W is [2 cols, K], C [M, cols] bfloat16 = activation(A.gate^T) * (A.up^T), kind 0
+// SiLU, 1 bounded sigmoid, 2 bounded step; parts: C float [parts, M, cols], partial sums over K
+int ga_gemm_tiles_gated(void* C, int64_t ldc, const void* A, int64_t lda, const void* W, int M, int cols, int K, int kind,
+                        float limit, float alpha, float shift, hipStream_t stream);
+int ga_gemm_tiles_parts(void* C, const void* A, int64_t lda, const void* W, int M, int cols, int K, int parts, hipStream_t stream);
+
 // ---- embedding_sinusoid.hip: out float [tokens, hidden] = table_scale * table[ids] + (sin | cos)(position * freq[i / 2]), then the norm
 // with one gain (gain null: no norm); freq float [(hidden + 1) / 2]
 int ga_embedding_sinusoid_norm(void* out, const void* table, const void* ids, const void* positions, const void* freq,

@@ -428,6 +428,48 @@ def gemm_skinny_supported(a, w):
             and w.is_contiguous() and w.data_ptr() % 16 == 0)
 
 
+def gemm_tiles_supported(a, w):
+    """Whether the kernels over tiles through LDS take these operands (any number of rows; offsets count in 32 bits)."""
+    return (a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and a.dim() == 2 and a.shape[0] > 0 and a.shape[1] > 0
+            and a.shape[1] % 64 == 0 and w.shape[0] % 16 == 0 and a.stride(1) == 1 and a.stride(0) >= a.shape[1]
+            and a.stride(0) % 8 == 0 and a.data_ptr() % 16 == 0 and w.is_contiguous() and w.data_ptr() % 16 == 0
+            and w.numel() < 1 << 31 and a.shape[0] * a.stride(0) < 1 << 31)
+
+
+def gemm_tiles_gated(a, w, bounds=None):
+    """a [M, K], w [2N, K] (gate over up) -> bfloat16 [M, N] = silu(a.gate^T) * (a.up^T), both sums in 32-bit and one
+    rounding; with bounds = (limit, alpha, shift) g * sigmoid(alpha g) * (u + shift), g = min(gate, limit), u = clamp(up,
+    -limit, limit) (alpha = infinity: the sigmoid's limit, relu(g))."""
+    _dev(a, w)
+    _need(gemm_tiles_supported(a, w) and a.shape[1] == w.shape[1], "the kernel over tiles does not take %s %s x %s %s", a.dtype,
+          tuple(a.shape), w.dtype, tuple(w.shape))
+    M, N = a.shape[0], w.shape[0] // 2
+    kind, (limit, alpha, shift) = 0, bounds or (0.0, 1.0, 0.0)
+    if bounds is not None:
+        _need(limit > 0, "the gate's bound must be positive, got %r", limit)
+        kind = 2 if alpha == float("inf") else 1
+    out = torch.empty((M, N), dtype=a.dtype, device=a.device)
+    lib = build.load("gemm_tiles")
+    _check(lib.ga_gemm_tiles_gated(_ptr(out), _i64(N), _ptr(a), _i64(a.stride(0)), _ptr(w), _i(M), _i(N), _i(a.shape[1]), _i(kind),
+                                   _f(limit), _f(alpha), _f(shift), _stream()), "gemm_tiles_gated")
+    return out
+
+
+def gemm_tiles_parts(a, w, parts):
+    """a [M, K] . w [N, K]^T as float32 partial sums [parts, M, N] over parts of K, for the consumer to add in order."""
+    _dev(a, w)
+    _need(gemm_tiles_supported(a, w) and a.shape[1] == w.shape[1], "the kernel over tiles does not take %s %s x %s %s", a.dtype,
+          tuple(a.shape), w.dtype, tuple(w.shape))
+    slabs = a.shape[1] // 64
+    _need(1 <= parts <= slabs and (parts - 1) * -(-slabs // parts) < slabs, "%d parts of %d slabs leave one empty", parts, slabs)
+    M, N = a.shape[0], w.shape[0]
+    out = torch.empty((parts, M, N), dtype=torch.float32, device=a.device)
+    lib = build.load("gemm_tiles")
+    _check(lib.ga_gemm_tiles_parts(_ptr(out), _ptr(a), _i64(a.stride(0)), _ptr(w), _i(M), _i(N), _i(a.shape[1]), _i(parts), _stream()),
+           "gemm_tiles_parts")
+    return out
+
+
 def gemm_skinny(a, w, bias=None, out=None, out_dtype=None, nt=0, ks=0, grid_splits=1, gated=False, into_norm=None,
                 pack=0, gate_bounds=None):
     """a [M <= 64, K] . w [N, K]^T (+ bias) -> [M, N] in bfloat16 (or float32): the decode step's products,

@@ -78,6 +78,31 @@ class Tuning:
     # The gate-up product lies transposed (weights as the library's first operand) for row counts from this on that
     # are a multiple of it: the library's tiles then fit the rows.
     transposed_gate_up_row_multiple: int = 256
+    # ---- the package's products over tiles through LDS (csrc/gemm_tiles.hip, with its measurements).  The gated product of at
+    # least so many rows of weights and elements of K: beyond `library_from_rows` rows up to `tiles_gated_few_rows` always,
+    # up to `tiles_gated_some_rows` while tiles of 128 rows of W make one round of the chip (7B shape, 256 rows: the library's 87 us
+    # against 115), up to `tiles_gated_odd_rows` again always (row counts the library's tiles do not fit: 300 rows 35 -> 30 and
+    # 125 -> 113 us; at 512 its 43 and 147 stand against 48 and 164), from `tiles_gated_many_rows` on always (1,000 rows 88 -> 76,
+    # 323 -> 271), and beyond `tiles_gated_full_rows` up to `tiles_gated_most_rows` where the rounds of 256 x 256 tiles are full to
+    # `tiles_gated_full` (2,048 rows of the 7B shape, 0.925: 570 -> 490; of the 1.5B shape, 0.73: 136 and 138; at 4,096 rows the
+    # library is ahead again)
+    tiles_gated_min_out_features: int = 8192
+    tiles_gated_min_in_features: int = 1024
+    tiles_gated_few_rows: int = 128
+    tiles_gated_some_rows: int = 256
+    tiles_gated_odd_rows: int = 384
+    tiles_gated_many_rows: int = 961
+    tiles_gated_full_rows: int = 1024
+    tiles_gated_most_rows: int = 2304
+    tiles_gated_full: float = 0.9
+    # ... and the product whose parts of K the norm adds: K of at least `tiles_parts_min_in_features`, at most
+    # `library_split_max_out_features` columns, beyond `library_from_rows` rows up to so many, in as many parts as keep to
+    # `tiles_parts_workgroups` workgroups; with more than 64 rows not where K is so long beside that many columns that the tiles'
+    # rows of A are most of what is read (3,584 columns of 18,944 at 256 rows: the library's 59 us against 80)
+    tiles_parts_min_in_features: int = 3072
+    tiles_parts_most_rows: int = 256
+    tiles_parts_most_weights_many_rows: int = 32 << 20
+    tiles_parts_workgroups: int = 256
     # ---- the fused q|k|v projection + rotation + cache write (parts/attention.py): from more rows than this and a K
     # of at least that, the library's product followed by the rotation kernel is faster (the fused kernel cannot split K).
     fused_qkv_up_to_rows: int = 16

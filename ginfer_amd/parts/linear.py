@@ -1,7 +1,8 @@
 """y = x . W^T (+ b), W stored [out, in] as in the checkpoint (ginfer/core/layer/linear.cc:9-20).
 
 32-bit: the package's own FMA kernel (no matrix unit, no reduced-precision mode).  bfloat16: the
-package's matrix-core kernel for up to 64 rows (decode), the BLAS library for more rows (prefill), which
+package's matrix-core kernels for up to 64 rows (decode) and, where they are the fastest, over tiles through LDS for more, else
+the BLAS library for more rows (prefill), which
 is where the reference calls its library (ginfer/core/op/kernels/cuda/gemm_kernel/gemm_kernel.cu:42-164);
 both accumulate in 32-bit and add the bias before the one rounding.  From 17 rows on the library also takes
 the products with a wide output, where it was measured faster; replays of recorded steps that hold
@@ -21,6 +22,10 @@ def linear(x, weight, bias=None, out_dtype=None, parts_ok=False):
     if x.dtype == torch.float32:
         return ops.gemm_nt(x, weight, bias)
     float32_out = out_dtype == torch.float32
+    if parts_ok and bias is None and not float32_out:
+        parts = tiles_parts(x, weight)
+        if parts:
+            return ops.gemm_tiles_parts(x, weight, parts)
     skinny_ok = ops.gemm_skinny_supported(x, weight)
     plan = None
     if autotune.active():
@@ -30,6 +35,44 @@ def linear(x, weight, bias=None, out_dtype=None, parts_ok=False):
     if plan is None:
         plan = linear_plan(x.shape[0], weight.shape[0], x.shape[1], bias is not None, float32_out, parts_ok, skinny_ok)
     return run_linear_plan(plan, x, weight, bias, out_dtype)
+
+
+def tiles_parts(x, weight):
+    """Into how many parts of K the package's product over tiles is cut for a consumer that adds them, where it is the fastest
+    way (by sizes alone; the measurements stand in csrc/gemm_tiles.hip and beside the thresholds); 0: another way is."""
+    T, rows, (out_features, in_features) = TUNING, x.shape[0], weight.shape
+    if not T.library_from_rows < rows <= T.tiles_parts_most_rows or in_features < T.tiles_parts_min_in_features:
+        return 0
+    if out_features > T.library_split_max_out_features or not ops.gemm_tiles_supported(x, weight):
+        return 0
+    few = rows <= ops.SKINNY_MAX_ROWS
+    if not few and out_features * in_features > T.tiles_parts_most_weights_many_rows:
+        return 0
+    tiles = -(-out_features // (64 if few else 128)) * -(-rows // 64)
+    slabs = in_features // 64
+    return _parts_without_gaps(slabs, max(1, min(T.tiles_parts_workgroups // tiles, slabs // 8)))
+
+
+def _parts_without_gaps(slabs, parts):
+    """The largest number of parts up to `parts` that leaves none of them without a slab, every part but the last being
+    as long as the first."""
+    while (parts - 1) * -(-slabs // parts) >= slabs:
+        parts -= 1
+    return parts
+
+
+def tiles_gated(x, weight_gate_up):
+    """Whether the package's gated product over tiles is the fastest way, by sizes alone (measurements beside the thresholds)."""
+    T, rows, (out_features, in_features) = TUNING, x.shape[0], weight_gate_up.shape
+    if (rows <= T.library_from_rows or rows > T.tiles_gated_most_rows or out_features < T.tiles_gated_min_out_features
+            or in_features < T.tiles_gated_min_in_features or not ops.gemm_tiles_supported(x, weight_gate_up)):
+        return False
+    if rows <= T.tiles_gated_odd_rows:
+        return rows <= T.tiles_gated_few_rows or rows > T.tiles_gated_some_rows or -(-out_features // 128) <= 256
+    if rows <= T.tiles_gated_full_rows:
+        return rows >= T.tiles_gated_many_rows
+    tiles = -(-rows // 256) * -(-out_features // 256)
+    return tiles >= T.tiles_gated_full * 256 * -(-tiles // 256)
 
 
 def linear_plan(rows, out_features, in_features, has_bias, float32_out, parts_ok, skinny_ok):
@@ -247,6 +290,8 @@ def gated_linear(x, weight_gate_up):
     ops.ScaledRows."""
     if isinstance(x, ops.ScaledRows):
         return ops.gemm_skinny(x, weight_gate_up, gated=True)
+    if tiles_gated(x, weight_gate_up):
+        return ops.gemm_tiles_gated(x, weight_gate_up)
     skinny_ok = x.dtype == torch.bfloat16 and ops.gemm_skinny_supported(x, weight_gate_up)
     transposable = _transposable(x, weight_gate_up)
     plan = None

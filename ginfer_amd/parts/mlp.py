@@ -5,7 +5,7 @@ from ..kernels import ops
 from ..kernels.tuning import TUNING
 from ..weights.loader import WeightSpec
 from .base import Part
-from .linear import linear, gated_linear, gated_plan, linear_into_norm
+from .linear import linear, gated_linear, gated_plan, linear_into_norm, tiles_gated
 from .registry import register_feed_forward
 
 
@@ -33,7 +33,7 @@ class SwiGLU(Part):
         self.w_down = t["down_proj.weight"]
 
     def kernel_modules(self):
-        return ["activation", "gemm"] + (["gemm_skinny"] if self.dtype == torch.bfloat16 else [])
+        return ["activation", "gemm"] + (["gemm_skinny", "gemm_tiles"] if self.dtype == torch.bfloat16 else [])
 
     def forward(self, x, into_norm=None):
         """into_norm = (residual, norm): where the down projection's kernel can, the result is added to the
@@ -71,12 +71,14 @@ class ClampedGLU(Part):
         self.w_down = t["down"]
 
     def kernel_modules(self):
-        return ["activation", "gemm"] + (["gemm_skinny"] if self.dtype == torch.bfloat16 else [])
+        return ["activation", "gemm"] + (["gemm_skinny", "gemm_tiles"] if self.dtype == torch.bfloat16 else [])
 
     def forward(self, x, parts_ok=False):
         # few rows (decode): the weight-streaming product with the activation in its epilogue, where the rules would
         # take that kernel for the SiLU gate too; else the product and the activation's own pass
-        if (x.dtype == torch.bfloat16 and ops.gemm_skinny_supported(x, self.w_gate_up)
+        if tiles_gated(x, self.w_gate_up):
+            act = ops.gemm_tiles_gated(x, self.w_gate_up, bounds=(self.limit, self.alpha, self.shift))
+        elif (x.dtype == torch.bfloat16 and ops.gemm_skinny_supported(x, self.w_gate_up)
                 and gated_plan(x.shape[0], self.w_gate_up.shape[0], True, False) == ("skinny",)):
             act = ops.gemm_skinny(x, self.w_gate_up, gated=True, gate_bounds=(self.limit, self.alpha, self.shift))
         else:
@@ -103,7 +105,7 @@ class SquaredReLU(Part):
         self.w_up, self.w_down = t["up"], t["down"]
 
     def kernel_modules(self):
-        return ["activation", "gemm"] + (["gemm_skinny"] if self.dtype == torch.bfloat16 else [])
+        return ["activation", "gemm"] + (["gemm_skinny", "gemm_tiles"] if self.dtype == torch.bfloat16 else [])
 
     def forward(self, x):
         # the result may be partial sums of a K-split product: the norm that follows adds them up

@@ -1008,3 +1008,55 @@ def test_qkv_rope_skinny(M, pack, nh, nkv, hd, K, theta, ps):
     q2 = ops.qkv_rope_skinny(x, w, b, positions, cos.to(dev()), sin.to(dev()), slots.to(dev()), kp1, vp1, nh, nkv, hd,
                              write_kv=False, pack=pack)
     assert torch.equal(q2, q) and torch.equal(kp1.cpu(), kp0) and torch.equal(vp1.cpu(), vp0)
+
+
+@pytest.mark.parametrize("M", [1, 17, 63, 64, 65, 129, 255, 257, 1535, 1537])
+@pytest.mark.parametrize("cols,K", [(8, 64), (72, 128), (136, 192), (200, 256), (1000, 320)])
+def test_gated_product_over_tiles(M, cols, K):
+    """Rows, columns and K around the edges of every tile (64 to 256 rows, 32 to 128 columns) and of the buffers (two to four slabs
+    of 64), rows of a wider buffer, the three gates.  The sums are 32-bit sums of bfloat16 products and the result is rounded
+    once: an element is off by at most half a place of bfloat16 (2^-9 of itself) and by what the sums' rounding, some
+    sqrt(K) 2^-24 of |a||w| each, moves through the gate; 2^-8 of the value and 1e-3 of the results' size hold both."""
+    from ginfer_amd.kernels import ops
+    wide = rnd((M, K + 16), torch.bfloat16, 51)
+    a, w = wide[:, 8:8 + K], rnd((2 * cols, K), torch.bfloat16, 52)
+    g, u = (a.double() @ w.double().t()).split(cols, dim=1)
+    inf = float("inf")
+    for bounds in (None, (7.0, 1.702, 1.0), (inf, inf, 0.0)):
+        if bounds is None:
+            ref = g * torch.sigmoid(g) * u
+        else:
+            gc, uc = torch.clamp(g, max=bounds[0]), torch.clamp(u, -bounds[0], bounds[0])
+            ref = (torch.relu(gc) if bounds[1] == inf else gc * torch.sigmoid(bounds[1] * gc)) * (uc + bounds[2])
+        got = ops.gemm_tiles_gated(a, w, bounds=bounds).double()
+        assert got.shape == ref.shape
+        off = (got - ref).abs()
+        assert bool((off <= ref.abs() / 256 + 1e-3 * ref.pow(2).mean().sqrt()).all()), "%r: %g" % (bounds, float(off.max()))
+
+
+@pytest.mark.parametrize("M", [1, 63, 64, 65, 127, 256, 300])
+@pytest.mark.parametrize("N,K,parts", [(16, 64, 1), (80, 192, 3), (144, 320, 2), (1536, 640, 5), (64, 832, 13)])
+def test_product_over_tiles_in_parts(M, N, K, parts):
+    """Parts of one to five slabs, uneven ones too (five slabs in two parts): 32-bit sums of bfloat16 products, together the
+    whole product, each the product over its own piece of K."""
+    from ginfer_amd.kernels import ops
+    a, w = rnd((M, K), torch.bfloat16, 61), rnd((N, K), torch.bfloat16, 62)
+    got = ops.gemm_tiles_parts(a, w, parts).double()
+    per = -(-(K // 64) // parts) * 64
+    for p in range(parts):
+        ref = a[:, p * per:(p + 1) * per].double() @ w[:, p * per:(p + 1) * per].double().t()
+        close(got[p], ref, 2e-6)
+
+
+def test_products_over_tiles_refuse_what_they_do_not_take():
+    from ginfer_amd.kernels import ops
+    a, w = rnd((70, 128), torch.bfloat16, 1), rnd((32, 128), torch.bfloat16, 2)
+    assert ops.gemm_tiles_supported(a, w)
+    for x, y in ((a[:, :96], w[:, :96].contiguous()), (a.float(), w.float()), (a, w[:20].contiguous()), (a, w.t().contiguous().t()),
+                 (rnd((70, 129), torch.bfloat16, 3)[:, 1:], w)):
+        assert not ops.gemm_tiles_supported(x, y)
+        with pytest.raises(ops.KernelError):
+            ops.gemm_tiles_gated(x, y)
+    for parts in (0, 3):
+        with pytest.raises(ops.KernelError):
+            ops.gemm_tiles_parts(a, w, parts)
