@@ -22,28 +22,28 @@ def linear(x, weight, bias=None, out_dtype=None, parts_ok=False):
     if x.dtype == torch.float32:
         return ops.gemm_nt(x, weight, bias)
     float32_out = out_dtype == torch.float32
-    if parts_ok and bias is None and not float32_out:
-        parts = tiles_parts(x, weight)
-        if parts:
-            return ops.gemm_tiles_parts(x, weight, parts)
     skinny_ok = ops.gemm_skinny_supported(x, weight)
     plan = None
     if autotune.active():
         key = ("linear", autotune.rows_class(x.shape[0]), weight.shape[0], x.shape[1], bias is not None, float32_out,
                bool(parts_ok), skinny_ok)
         plan = autotune.choose(key, (weight, bias))
+    if plan is None and parts_ok and bias is None and not float32_out:
+        parts = tiles_parts(x.shape[0], weight.shape[0], x.shape[1])
+        if parts and ops.gemm_tiles_supported(x, weight):
+            plan = ("tiles", 1, parts)
     if plan is None:
         plan = linear_plan(x.shape[0], weight.shape[0], x.shape[1], bias is not None, float32_out, parts_ok, skinny_ok)
     return run_linear_plan(plan, x, weight, bias, out_dtype)
 
 
-def tiles_parts(x, weight):
+def tiles_parts(rows, out_features, in_features):
     """Into how many parts of K the package's product over tiles is cut for a consumer that adds them, where it is the fastest
     way (by sizes alone; the measurements stand in csrc/gemm_tiles.hip and beside the thresholds); 0: another way is."""
-    T, rows, (out_features, in_features) = TUNING, x.shape[0], weight.shape
+    T = TUNING
     if not T.library_from_rows < rows <= T.tiles_parts_most_rows or in_features < T.tiles_parts_min_in_features:
         return 0
-    if out_features > T.library_split_max_out_features or not ops.gemm_tiles_supported(x, weight):
+    if out_features > T.library_split_max_out_features or out_features % 16 or in_features % 64:
         return 0
     few = rows <= ops.SKINNY_MAX_ROWS
     if not few and out_features * in_features > T.tiles_parts_most_weights_many_rows:
@@ -77,7 +77,8 @@ def tiles_gated(x, weight_gate_up):
 
 def linear_plan(rows, out_features, in_features, has_bias, float32_out, parts_ok, skinny_ok):
     """The way a bfloat16 product is done, by the rules: ("skinny", tiles of W per wavefront, parts of K) for the
-    package's weight-streaming kernel, ("library", pieces of K) for the BLAS library.  More than one part or piece
+    package's weight-streaming kernel, ("library", pieces of K) for the BLAS library (the product over tiles, ("tiles", 1, parts
+    of K), stands before these rules: `tiles_parts`).  More than one part or piece
     means float32 partial sums [parts, M, N] for the consumer to add."""
     may_split = parts_ok and not float32_out
     if may_split and not has_bias:
@@ -109,6 +110,10 @@ def run_linear_plan(plan, x, weight, bias, out_dtype):
         if splits > 1:
             return ops.gemm_skinny(x, weight, bias, out_dtype=torch.float32, nt=nt, grid_splits=splits)
         return ops.gemm_skinny(x, weight, bias, out_dtype=out_dtype, nt=nt)
+    if plan[0] == "tiles":
+        if ops.gemm_tiles_supported(x, weight):
+            return ops.gemm_tiles_parts(x, weight, plan[2])
+        plan = ("library", 1)            # a plan kept for this class of sizes meets rows that the kernel does not take
     _, parts = plan
     if parts > 1:
         # the library, once, over `parts` pieces of K side by side (a batched product over views of x and
@@ -150,6 +155,9 @@ def linear_candidates(key):
                         add(("skinny", nt, parts))
     add(("library", 1))
     if may_split and not has_bias:
+        parts = tiles_parts(rows, out_features, in_features)
+        if parts and in_features % parts == 0:
+            add(("tiles", 1, parts))
         for parts in (2, 3, 4, 5, 7, 8, 10, 14, 16):
             if in_features % parts == 0 and (in_features // parts) % 8 == 0 and in_features // parts >= 512:
                 add(("library", parts))
