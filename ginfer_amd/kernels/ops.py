@@ -804,10 +804,21 @@ def paged_attention_mfma(q, k_pages, v_pages, block_table, step, num_heads, num_
         _check(lib.ga_attn_prefill(
             _ptr(out), _i64(out.stride(0)), _ptr(q), _i64(q.stride(0)), _ptr(k_pages), _ptr(v_pages), _ptr(block_table),
             _i(block_table.shape[1]), _ptr(plan["tiles"]), _i(plan["n_tiles"]), _i(tile_rows), _i(num_heads), _i(num_kv_heads),
-            _i(page_size), _i(w), _f(scale), _i(TUNING.prefill_fill_workgroups), _i(TUNING.prefill_prefer_workgroups),
+            _i(page_size), _i(w), _f(scale), _i(_prefill_fill(step, head_dim)), _i(TUNING.prefill_prefer_workgroups),
             _ptr(plan["parts"]), _ptr(plan["part_rows"]),
             _i(plan["n_part_rows"]), _i(plan["num_parts"]), _ptr(part_o), _ptr(part_ml), _ptr(sinks), *extras, _stream()), "attn_prefill")
     return out
+
+
+PREFILL_SHARED_DIMS = (64, 128, 256)     # head sizes with the prefill kernel that shares a kv head's operands through LDS
+
+
+def _prefill_fill(step, head_dim):
+    """How many workgroups a step's prompt rows have to make for heads to share them: fewer where that shares the operands
+    through LDS too and the tiles are all a prompt's (a recorded step's count holds padding)."""
+    if head_dim not in PREFILL_SHARED_DIMS or "static_plan" in (step.extra or {}):
+        return TUNING.prefill_fill_workgroups
+    return max(1, int(TUNING.prefill_fill_workgroups * TUNING.prefill_fill_real_tiles))
 
 
 def _prefill_workgroups(step, tile_rows, group, nkv, head_dim, window):
@@ -819,8 +830,8 @@ def _prefill_workgroups(step, tile_rows, group, nkv, head_dim, window):
     n_tiles = sum(-(-n // tile_rows) for n in step.host_q_len if n > 1)
     if n_tiles == 0:
         return None
-    fill, waves = TUNING.prefill_fill_workgroups, 8
-    if head_dim in (64, 128, 256):
+    fill, waves = _prefill_fill(step, head_dim), 8
+    if head_dim in PREFILL_SHARED_DIMS:
         heads = 1
         for d in range(waves - 1, 1, -1):
             if group % d == 0 and n_tiles * nkv * (group // d) >= fill:

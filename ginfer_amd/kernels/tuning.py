@@ -125,6 +125,12 @@ class Tuning:
     # workgroups; among the groupings that do, the one with the most heads that still makes `prefill_prefer_workgroups`
     # (one and a half rounds of the chip), else the one with the fewest heads
     prefill_fill_workgroups: int = 256
+    # ... and only so much of that where the sharing goes through LDS and the tiles are all a prompt's: one kv head's keys and
+    # values are then read once for all its heads.  Whole steps of the 7B shape (7 heads to a kv head: all or one), us, at 256 ->
+    # 128 workgroups: 2,000 tokens behind 2,048 beside 48 single ones (252 workgroups) 31,897 -> 28,487; 600 behind 3,000 (152)
+    # 15,465 -> 13,548; 1,000 alone (252) 16,105 -> 15,452.  Recorded steps count padding among their tiles and keep the full
+    # number: 256 rows behind 8,000 of the 1.5B shape, 96 workgroups with a row of their own, 5,250 -> 6,100.
+    prefill_fill_real_tiles: float = 0.5
     prefill_prefer_workgroups: int = 384
     # The keys of a step's heaviest prompt tiles can be dealt to several workgroups (merged by a second kernel): when the
     # step makes at most `prefill_split_max_workgroups` workgroups, the heaviest tile's walk is at least
