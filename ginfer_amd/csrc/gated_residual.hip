@@ -1,8 +1,11 @@
 // Sublayers that run side by side and enter the residual stream through gates of their own:
-//   residual[t] += sigmoid(z1[t]) * y1[t] (+ sigmoid(z2[t]) * y2[t])         z: 32-bit rows of gates * hidden numbers with a stride
+//   residual[t] += sigmoid(z1[t] + b1) * y1[t] (+ sigmoid(z2[t] + b2) * y2[t])    z: 32-bit rows of gates * hidden numbers with a
+//                                                                             stride; b: gates * hidden numbers (optional)
 //   next[t]      = g * residual[t] / sqrt(mean(residual[t]^2) + eps)         (optional: the norm that is read next)
 // The gated results are added to each other first and then to the stream.  All arithmetic in 32-bit; a row's sum of
 // squares is taken in an order that depends on its length alone.  A workgroup a token.
+// The bias is added here because the product that makes z is a library's for a prompt, which takes none with 32-bit results: a
+// pass of its own over the whole projection cost 22 us a layer at 2,048 tokens of some 5,000 columns.
 #include "common.h"
 #include "ginfer_amd.h"
 
@@ -12,6 +15,7 @@ __device__ __forceinline__ float grs_sigmoid(float z) { return 1.0f / (1.0f + ex
 
 template <typename Y, typename C>
 __global__ __launch_bounds__(GRS_THREADS) void gated_residual_add_kernel(float* __restrict__ residual, const float* __restrict__ z,
+                                                                          const float* __restrict__ z_bias,
                                                                           const Y* __restrict__ y1, const Y* __restrict__ y2,
                                                                           const float* __restrict__ next_gain, float next_eps,
                                                                           C* __restrict__ next, int hidden, int64_t z_stride) {
@@ -23,8 +27,8 @@ __global__ __launch_bounds__(GRS_THREADS) void gated_residual_add_kernel(float* 
   const Y* b = y2 ? y2 + t * hidden : nullptr;
   float ss = 0.f;
   for (int i = threadIdx.x; i < hidden; i += GRS_THREADS) {
-    float d = grs_sigmoid(zr[i]) * Num<Y>::ld(a + i);
-    if (b) d = fmaf(grs_sigmoid(zr[hidden + i]), Num<Y>::ld(b + i), d);
+    float d = grs_sigmoid(z_bias ? zr[i] + z_bias[i] : zr[i]) * Num<Y>::ld(a + i);
+    if (b) d = fmaf(grs_sigmoid(z_bias ? zr[hidden + i] + z_bias[hidden + i] : zr[hidden + i]), Num<Y>::ld(b + i), d);
     const float r = res[i] + d;
     res[i] = r;
     ss += r * r;
@@ -59,6 +63,7 @@ template <> struct Quad<bf16_t> {
 
 template <typename Y, typename C, int PER>
 __global__ __launch_bounds__(GRS_THREADS) void gated_residual_add_quad_kernel(float* __restrict__ residual, const float* __restrict__ z,
+                                                                               const float* __restrict__ z_bias,
                                                                                const Y* __restrict__ y1, const Y* __restrict__ y2,
                                                                                const float* __restrict__ next_gain, float next_eps,
                                                                                C* __restrict__ next, int hidden, int64_t z_stride) {
@@ -79,6 +84,14 @@ __global__ __launch_bounds__(GRS_THREADS) void gated_residual_add_quad_kernel(fl
       if (b) {
         zb[j] = Quad<float>::ld(zr + hidden + i);
         yb[j] = Quad<Y>::ld(b + i);
+      }
+      if (z_bias) {
+        const float4 ba = Quad<float>::ld(z_bias + i);
+        za[j] = make_float4(za[j].x + ba.x, za[j].y + ba.y, za[j].z + ba.z, za[j].w + ba.w);
+        if (b) {
+          const float4 bb = Quad<float>::ld(z_bias + hidden + i);
+          zb[j] = make_float4(zb[j].x + bb.x, zb[j].y + bb.y, zb[j].z + bb.z, zb[j].w + bb.w);
+        }
       }
     }
   }
@@ -113,15 +126,15 @@ __global__ __launch_bounds__(GRS_THREADS) void gated_residual_add_quad_kernel(fl
   }
 }
 
-extern "C" int ga_gated_residual_add(void* residual, const void* z, int64_t z_stride, const void* y1, const void* y2, int tokens, int hidden,
+extern "C" int ga_gated_residual_add(void* residual, const void* z, int64_t z_stride, const void* z_bias, const void* y1, const void* y2, int tokens, int hidden,
                                      int y_bf16, const void* next_gain, float next_eps, void* next, int next_bf16,
                                      hipStream_t stream) {
   if (tokens <= 0) return 0;
   if (hidden <= 0 || !z || !y1 || ((next != nullptr) != (next_gain != nullptr))) return -1;
   dim3 grid(tokens), block(GRS_THREADS);
-  if (hidden % 4 == 0 && hidden <= GRS_THREADS * 4 * 8 && z_stride % 4 == 0 && ((uintptr_t)z & 15) == 0) {
+  if (hidden % 4 == 0 && hidden <= GRS_THREADS * 4 * 8 && z_stride % 4 == 0 && (((uintptr_t)z | (uintptr_t)z_bias) & 15) == 0) {
 #define GQ(Y, C, PER) hipLaunchKernelGGL((gated_residual_add_quad_kernel<Y, C, PER>), grid, block, 0, stream, (float*)residual,   \
-                                         (const float*)z, (const Y*)y1, (const Y*)y2, (const float*)next_gain, next_eps, (C*)next, \
+                                         (const float*)z, (const float*)z_bias, (const Y*)y1, (const Y*)y2, (const float*)next_gain, next_eps, (C*)next, \
                                          hidden, z_stride)
 #define GP(Y, C) do { if (hidden <= GRS_THREADS * 4) GQ(Y, C, 1); else if (hidden <= GRS_THREADS * 8) GQ(Y, C, 2);              \
                       else if (hidden <= GRS_THREADS * 16) GQ(Y, C, 4); else GQ(Y, C, 8); } while (0)
@@ -132,7 +145,7 @@ extern "C" int ga_gated_residual_add(void* residual, const void* z, int64_t z_st
     return GA_CHECK_LAUNCH();
   }
 #define GO(Y, C) hipLaunchKernelGGL((gated_residual_add_kernel<Y, C>), grid, block, 0, stream, (float*)residual,          \
-                                    (const float*)z, (const Y*)y1, (const Y*)y2, (const float*)next_gain, next_eps, (C*)next, \
+                                    (const float*)z, (const float*)z_bias, (const Y*)y1, (const Y*)y2, (const float*)next_gain, next_eps, (C*)next, \
                                     hidden, z_stride)
   if (y_bf16) { if (next_bf16) GO(bf16_t, bf16_t); else GO(bf16_t, float); }
   else { if (next_bf16) GO(float, bf16_t); else GO(float, float); }

@@ -35,7 +35,7 @@ class _DecayedLinearAttention(Part):
         own = self.w_in.shape[0]
         self._extra = (own, own + weight.shape[0])
         self.w_in = torch.cat([self.w_in, weight], dim=0).contiguous()
-        self.b_in = torch.cat([torch.zeros((own,), dtype=bias.dtype, device=bias.device), bias]).contiguous()
+        self.b_in = None if bias is None else torch.cat([torch.zeros((own,), dtype=bias.dtype, device=bias.device), bias]).contiguous()
         return True
 
     def _project(self, x):

@@ -44,7 +44,7 @@ class SigmoidProjectionGate(Part):
         if not 1 <= len(self.names) <= 2:
             raise ValueError("a block gates one or two sublayers, got %r" % (names,))
         self.dtype, self.device = dtype, device
-        self.weight = self.bias = None
+        self.weight = self.bias = self.late_bias = None
 
     def weight_specs(self):
         H = self.hidden_size
@@ -68,12 +68,13 @@ class SigmoidProjectionGate(Part):
         return linear(x, self.weight, self.bias, out_dtype=torch.float32)
 
     def hand_over(self, taker):
-        """Gives the gates' matrix and bias to a part that reads the same rows and can stack them behind its own projection
-        (`append_columns(weight, bias)`; its forward then leaves the logits in `extra_columns`).  True if it took them: this
-        part then keeps no copy."""
+        """Gives the gates' matrix to a part that reads the same rows and can stack it behind its own projection
+        (`append_columns(weight, bias)`; its forward then leaves the columns in `extra_columns`).  The bias stays here and is
+        added by the launch that takes the sigmoids (bias None).  True if the matrix was taken: this part then keeps no copy."""
         take = getattr(taker, "append_columns", None)
-        if take is None or self.weight is None or not take(self.weight, self.bias):
+        if take is None or self.weight is None or not take(self.weight, None):
             return False
+        self.late_bias = self.bias.float().contiguous()
         self.weight = self.bias = None
         return True
 
@@ -84,6 +85,7 @@ class SigmoidProjectionGate(Part):
             raise ValueError("%d results for %d gates" % (len(results), len(self.names)))
         y2 = results[1] if len(results) > 1 else None
         if then is None:
-            return ops.gated_residual_add(residual, z, results[0], y2)
+            return ops.gated_residual_add(residual, z, results[0], y2, z_bias=self.late_bias)
         gain = then.weight if then.weight.dtype == torch.float32 else then.weight.float()
-        return ops.gated_residual_add(residual, z, results[0], y2, next_gain=gain, next_eps=then.eps, dtype=then.dtype)
+        return ops.gated_residual_add(residual, z, results[0], y2, next_gain=gain, next_eps=then.eps, dtype=then.dtype,
+                                      z_bias=self.late_bias)

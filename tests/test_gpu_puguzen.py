@@ -264,6 +264,23 @@ def test_recurrence_across_cuts_and_a_slot_that_was_used(heads, dim, vdim):
         assert torch.equal(state[3], final), kind
 
 
+@pytest.mark.parametrize("width", [7, 96, 1024, 1028, 4100])
+def test_gates_with_a_bias_are_the_gates_of_the_sum(width):
+    """A bias added to the gates' logits in the same launch gives the bits of logits that hold it, one gate or two, rows with a
+    stride, widths for either kernel."""
+    from ginfer_amd.kernels import ops
+    g = torch.Generator().manual_seed(width)
+    z = torch.randn((3, 2 * width + 4), generator=g).cuda()[:, 4:]
+    bias = torch.randn((2 * width,), generator=g).cuda()
+    y = [torch.randn((3, width), generator=g).cuda().to(torch.bfloat16) for _ in range(2)]
+    for gates in (1, 2):
+        a, b = torch.ones((3, width), device="cuda"), torch.ones((3, width), device="cuda")
+        zg, bg, y2 = z[:, :gates * width], bias[:gates * width].contiguous(), y[1] if gates == 2 else None
+        ops.gated_residual_add(a, zg, y[0], y2, z_bias=bg)
+        ops.gated_residual_add(b, zg + bg, y[0], y2)
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("dim", [16, 48, 64, 130, 250])
 @pytest.mark.parametrize("n", [1, 7, 8, 9, 16, 17, 40])
 def test_recurrences_of_many_entries_give_the_bits_of_one_alone(dim, n):
