@@ -237,7 +237,7 @@ static int gt_check(const void* C, const void* A, int64_t lda, const void* W, in
 // is nearly the same for 64 and for 128 rows then: the weights' way).  us, product and activation by the library's best way ->
 // here, as replays of a graph over several layers' weights: 17,920 rows of W, K 1,536: 17 rows 18.4 -> 16.1, 64 rows 21.0 -> 18.0,
 // 256 rows 33.9 -> 28.8, 384 rows 37.3 -> 32.1, 1,000 rows 88 -> 76; 37,888 rows, K 3,584: 384 rows 131 -> 118, 1,024 rows 309 -> 279,
-// 2,048 rows 570 -> 490.  What decides at many rows is how full the last round of tiles is (at 512 rows 43 here stand against
+// 2,048 rows 570 -> 490.  What decides at many rows is how full the last round of tiles is (at 512 rows the library's 43 stand against
 // 48 and 147 against 164): the caller's rule.
 extern "C" int ga_gemm_tiles_gated(void* C, int64_t ldc, const void* A, int64_t lda, const void* W, int M, int cols, int K, int kind,
                                    float limit, float alpha, float shift, hipStream_t stream) {
