@@ -20,6 +20,8 @@
 // q, k and v as the recurrence reads them: the projection's numbers or their silu, turned by position, scaled
 template <bool ROT>
 struct DecayRows {
+  struct Fixed {};
+  __device__ __forceinline__ Fixed fixed(int) const { return {}; }
   struct Plain { float q, k, a; };
   struct Turned { float q, k, a, q2, k2, c, s; };
   typedef typename std::conditional<ROT, Turned, Plain>::type Raw;
@@ -47,7 +49,7 @@ struct DecayRows {
     }
   }
   template <bool ACT>
-  __device__ __forceinline__ void finish(const Raw& x, int i, float& qv, float& kv, float& a) const {
+  __device__ __forceinline__ void finish(const Raw& x, const Fixed&, int i, float& qv, float& kv, float& a) const {
     qv = act<ACT>(x.q);
     kv = act<ACT>(x.k);
     if constexpr (ROT) {
@@ -68,10 +70,11 @@ struct DecayRows {
   __device__ __forceinline__ float finish_v(float x) const { return act<ACT>(x); }
 };
 
-// Measured on MI355X, 2,048 tokens of one request, 12 heads of 64 x 128, us, before (16 columns a workgroup whose every wavefront
-// brings, walks and adds up, operands in single reads, three barriers a tile) -> now: a decay per channel 412 -> 118, a
-// constant one with rotation 450 -> 143, with silu 463 -> 174; 28 heads 415 -> 167, 456 -> 286, 476 -> 236; five entries of 918
-// tokens 107 -> 52, 113 -> 73, 115 -> 68.  64 entries of one token: 18.7 -> 18.9 (reading and writing the state).
+// Measured on MI355X, the projection just written, us, before (16 columns a workgroup whose every wavefront brings, walks and adds
+// up, operands in single reads, three barriers a tile) -> now, a decay per channel and a constant one with rotation.  12 heads of
+// 64 x 128: 2,048 tokens of one request 421 -> 119, 459 -> 142; five entries of 918 207 -> 161, 217 -> 176; 495 tokens beside 16
+// single ones 110 -> 57, 120 -> 66; 64 entries of one token 20.7 -> 16.4, 21.3 -> 17.0 (reading and writing the state).  28 heads
+// of 128 x 128: 815 -> 459, 911 -> 500; 904 -> 486, 896 -> 511; 225 -> 162, 239 -> 171; 85 -> 70, 86 -> 70.
 template <int R, int COLS, int TILE, bool ROT>   // R rows of the state per thread: dim <= 16 * R
 __global__ __launch_bounds__(dw_threads(COLS)) void decay_scan_kernel(
     float* __restrict__ out, const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
@@ -306,11 +309,11 @@ __global__ __launch_bounds__(DS_THREADS) void wide_norm_gate_rows_kernel(T* __re
 
 extern "C" int ga_decay_scan(void* out, const void* q, const void* k, const void* v, int64_t stride, const void* decay,
                              const void* head_decay, const void* cos_t, const void* sin_t, int rot_dims, float q_scale,
-                             float k_scale, void* state, const void* slots, const void* cu, const void* q_start, int tokens, int entries,
+                             float k_scale, void* state, const void* slots, const void* cu, const void* q_start, int way, int entries,
                              int heads, int dim, int vdim, int silu_inputs, hipStream_t stream) {
   if (entries <= 0) return 0;
-  if (heads <= 0 || dim <= 0 || vdim <= 0 || dim > 16 * DW_SLICES) return -1;
-  if (heads > 65535 || (vdim + 15) / 16 > 65535 || stride >= (1ll << 27)) return -2;    // (a tile's offsets are 32-bit)
+  if (heads <= 0 || dim <= 0 || vdim <= 0 || dim > 16 * DW_SLICES || (way != 1 && way != 8 && way != 16)) return -1;
+  if (heads > 65535 || (vdim + (way == 8 ? 7 : 15)) / (way == 8 ? 8 : 16) > 65535 || stride >= (1ll << 27)) return -2;    // (a tile's offsets are 32-bit)
   if ((decay == nullptr) == (head_decay == nullptr)) return -3;
   if (rot_dims < 0 || rot_dims % 2 || rot_dims > dim || (rot_dims > 0 && (!cos_t || !sin_t))) return -4;
   const int rows = (dim + DW_SLICES - 1) / DW_SLICES;
@@ -320,11 +323,7 @@ extern "C" int ga_decay_scan(void* out, const void* q, const void* k, const void
                                  (float*)state, (const int64_t*)slots, (const int32_t*)cu, (const int32_t*)q_start, heads, dim, vdim,   \
                                  silu_inputs)
 #define GR(R, C, T) do { if (rot_dims > 0) GO(R, C, T, true); else GO(R, C, T, false); } while (0)
-  if (decay_walk_narrow(tokens, entries, heads, vdim)) {
-    DW_ROWS(rows, 8, GR);
-  } else {
-    DW_ROWS(rows, 16, GR);
-  }
+  DW_WAY(way, rows, GR);
 #undef GR
 #undef GO
   return GA_CHECK_LAUNCH();

@@ -10,7 +10,9 @@
 // What bounds it is the chain of tokens: with one wavefront a SIMD a token costs its 3 R + 4 vector instructions and the
 // LDS reads of its wavefronts.  Fewer columns a workgroup halve the reads a compute unit makes per token, which is what a
 // single prompt wants (its workgroups do not fill the chip anyway); many entries take 16 columns, which read a token's
-// operands half as often.  A result's bits depend on neither COLS nor TILE, nor on how tokens were cut into steps.
+// operands half as often.  Entries of one token (a decode step) are bound by the way of their state from memory and back: a
+// tile of one token leaves its LDS to as many workgroups as the registers allow.  The caller chooses (decay_walk_way in
+// kernels/ops.py, with both sides measured).  A result's bits depend on neither COLS nor TILE, nor on how tokens were cut into steps.
 #pragma once
 #include "common.h"
 #include <type_traits>
@@ -19,9 +21,9 @@
 
 __host__ __device__ constexpr int dw_threads(int cols) { return cols == 8 ? 384 : DW_SLICES * cols; }
 
-// Source: `Raw` (what a thread loads for one element of q, k and a), load(Raw&, start, token, channel), finish(Raw, channel, q, k,
-// a), load_v(start, token, column), finish_v(v); finish and finish_v are templates on whether `acts` is set.  `start` is the
-// same for all threads, tokens count from it.
+// Source: `Fixed` (what a channel has for all tokens), fixed(channel), `Raw` (what a thread loads for one element of q, k and a),
+// load(Raw&, start, token, channel), finish(Raw, Fixed, channel, q, k, a), load_v(start, token, column), finish_v(v); finish and
+// finish_v are templates on whether `acts` is set.  `start` is the same for all threads, tokens count from it.
 template <int R, int COLS, int TILE, class Source>
 __device__ __forceinline__ void decay_walk(float* __restrict__ out, const Source& source, float* __restrict__ state, bool fresh,
                                            int n, int heads, int dim, int vdim, int v0) {
@@ -42,7 +44,10 @@ __device__ __forceinline__ void decay_walk(float* __restrict__ out, const Source
     S[r] = (walks && !fresh && col_ok && i < dim) ? st[(int64_t)i * vdim] : 0.f;
   }
   typename Source::Raw raw[PER];
+  typename Source::Fixed fixed[PER];
   float raw_v = 0.f;
+#pragma unroll
+  for (int x = 0; x < PER; ++x) fixed[x] = source.fixed(min((tid + x * SERVERS) % DP, dim - 1));
   // Tiles are brought whole: the last one starts early enough to end with the last token, and is then walked from `t0 - start`
   // on.  So a thread's places in a tile never change, and an address is a uniform part and a constant one.  (An entry of
   // fewer tokens than a tile reads its last one again; channels and columns that do not exist read another and drop it.)
@@ -65,7 +70,7 @@ __device__ __forceinline__ void decay_walk(float* __restrict__ out, const Source
       const int idx = tid + x * SERVERS, tt = idx / DP, i = idx % DP;
       float q, k, a;
       if ((TILE * DP < SERVERS && tt >= TILE) || (decltype(few)::value && tt >= n)) break;
-      source.template finish<ACT>(raw[x], min(i, dim - 1), q, k, a);
+      source.template finish<ACT>(raw[x], fixed[x], min(i, dim - 1), q, k, a);
       ops[b][tt][0][i % DW_SLICES][i / DW_SLICES] = i < dim ? q : 0.f;
       ops[b][tt][1][i % DW_SLICES][i / DW_SLICES] = i < dim ? k : 0.f;
       ops[b][tt][2][i % DW_SLICES][i / DW_SLICES] = i < dim ? a : 0.f;
@@ -116,7 +121,7 @@ __device__ __forceinline__ void decay_walk(float* __restrict__ out, const Source
     }
   }
   int b = 0, t0 = 0;
-  for (; t0 + TILE <= n; t0 += TILE, b ^= 1) {               // (behind the last tile the last one is brought again)
+  for (; t0 + TILE <= n; t0 += TILE, b ^= 1) {               // (behind the last tile 8 columns bring the last one again)
     __syncthreads();                                         // this tile is staged; the partial sums of the one before are in
     if (walks && AHEAD == 0) {
 #pragma unroll 1
@@ -136,8 +141,10 @@ __device__ __forceinline__ void decay_walk(float* __restrict__ out, const Source
     }
     if (serves) {
       put(t0 - TILE, b ^ 1);
-      stage(b ^ 1, std::false_type());
-      fetch(t0 + 2 * TILE, std::false_type());
+      if (COLS == 8 || t0 + TILE < n) {                      // (a short entry's activations are a good part of its time)
+        stage(b ^ 1, std::false_type());
+        fetch(t0 + 2 * TILE, std::false_type());
+      }
     }
   }
   __syncthreads();
@@ -160,22 +167,24 @@ __device__ __forceinline__ void decay_walk(float* __restrict__ out, const Source
   }
 }
 
-// Whether a workgroup takes 8 columns, with wavefronts that only bring and put: where workgroups of 16 would not fill the
-// chip's 256 compute units, and where entries bring many tokens (the longest one's chain is then what a step waits for).
-static inline bool decay_walk_narrow(int tokens, int entries, int heads, int vdim) {
-  return ((int64_t)entries * heads * ((vdim + 15) / 16) < 256 || tokens >= 64 * (int64_t)entries) && (vdim + 7) / 8 <= 65535;
-}
-
 // GO(R, COLS, TILE) for a state of up to 16 * rows rows: as many tokens a tile as leave two workgroups of 16 columns (a
-// decode step's many) or one of 8 their LDS, and every thread a whole number of elements to bring
-#define DW_ROWS(rows, COLS, GO)                                            \
-  do {                                                                     \
-    if (rows <= 1) GO(1, COLS, 16);                                        \
-    else if (rows <= 2) GO(2, COLS, (COLS == 8 ? 16 : 8));                 \
-    else if (rows <= 3) GO(3, COLS, 16);                                   \
-    else if (rows <= 4) GO(4, COLS, (COLS == 8 ? 16 : 8));                 \
-    else if (rows <= 6) GO(6, COLS, 8);                                    \
-    else if (rows <= 8) GO(8, COLS, 8);                                    \
-    else if (rows <= 12) GO(12, COLS, 8);                                  \
-    else GO(16, COLS, 4);                                                  \
+// decode step's many) or one of 8 their LDS, and every thread a whole number of elements to bring; tokens: that many instead
+#define DW_TILE(TOKENS, OWN) (TOKENS > 0 ? TOKENS : OWN)
+#define DW_ROWS(rows, COLS, TOKENS, GO)                                                          \
+  do {                                                                                           \
+    if (rows <= 1) GO(1, COLS, DW_TILE(TOKENS, 16));                                       \
+    else if (rows <= 2) GO(2, COLS, DW_TILE(TOKENS, (COLS == 8 ? 16 : 8)));                \
+    else if (rows <= 3) GO(3, COLS, DW_TILE(TOKENS, 16));                                  \
+    else if (rows <= 4) GO(4, COLS, DW_TILE(TOKENS, (COLS == 8 ? 16 : 8)));                \
+    else if (rows <= 6) GO(6, COLS, DW_TILE(TOKENS, 8));                                   \
+    else if (rows <= 8) GO(8, COLS, DW_TILE(TOKENS, 8));                                   \
+    else if (rows <= 12) GO(12, COLS, DW_TILE(TOKENS, 8));                                 \
+    else GO(16, COLS, DW_TILE(TOKENS, 4));                                                 \
+  } while (0)
+// way: 1 tiles of one token in 16 columns, 8 and 16 that many columns
+#define DW_WAY(way, rows, GO)                       \
+  do {                                              \
+    if (way == 1) DW_ROWS(rows, 16, 1, GO);         \
+    else if (way == 8) DW_ROWS(rows, 8, 0, GO);     \
+    else DW_ROWS(rows, 16, 0, GO);                  \
   } while (0)

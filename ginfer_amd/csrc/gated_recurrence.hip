@@ -16,11 +16,13 @@ __device__ __forceinline__ float gr_sigmoid(float z) { return 1.0f / (1.0f + exp
 
 struct ForgetRows {
   struct Raw { float q, f; };
+  struct Fixed { float bias, lower; };
   const float *proj, *v;               // the entry's first token, the head's first channel or column
   const float *bias, *lower;           // the head's
   int64_t stride;
   int hd;
   static constexpr bool acts = false;
+  __device__ __forceinline__ Fixed fixed(int i) const { return {bias[i], lower[i]}; }
   __device__ __forceinline__ void load(Raw& x, int start, int t, int i) const {
     const float* p = proj + start * stride;
     const uint32_t at = (uint32_t)t * (uint32_t)stride + i;
@@ -28,10 +30,9 @@ struct ForgetRows {
     x.f = p[at + hd];
   }
   template <bool>
-  __device__ __forceinline__ void finish(const Raw& x, int i, float& q, float& k, float& f) const {
-    const float lo = lower[i];
+  __device__ __forceinline__ void finish(const Raw& x, const Fixed& c, int i, float& q, float& k, float& f) const {
     q = x.q * gr_sigmoid(x.q);
-    f = lo + (1.0f - lo) * gr_sigmoid(x.f + bias[i]);
+    f = c.lower + (1.0f - c.lower) * gr_sigmoid(x.f + c.bias);
     k = 1.0f - f;
   }
   __device__ __forceinline__ float load_v(int start, int t, int c) const {
@@ -41,8 +42,10 @@ struct ForgetRows {
   __device__ __forceinline__ float finish_v(float x) const { return x; }
 };
 
-// Measured on MI355X, us, before -> now: 2,048 tokens of one request, 12 heads of 64 x 128: 453 -> 165; 28 heads 459 -> 228; five
-// entries of 918 tokens 109 -> 65; 64 entries of one token 15.2 -> 16.0.
+// Measured on MI355X, the projection just written, us, before -> now.  12 heads of 64 x 128: 2,048 tokens of one request 454 -> 150;
+// five entries of 918 216 -> 168; 495 tokens beside 16 single ones 117 -> 64; 64 entries of one token 20.4 -> 17.0.  28 heads of 128 x
+// 128: 777 -> 498, 784 -> 544, 225 -> 172, 78 -> 69.  The one size seen that takes longer: 64 entries of 33 tokens, 16 heads of 32 x
+// 64, 27.9 -> 32.1.
 template <int R, int COLS, int TILE>          // R rows of the state per thread: dim <= 16 * R
 __global__ __launch_bounds__(dw_threads(COLS)) void hgrn2_scan_kernel(float* __restrict__ out, const float* __restrict__ proj,
                                                                        int64_t proj_stride, const float* __restrict__ f_bias,
@@ -80,20 +83,16 @@ __global__ __launch_bounds__(GR_THREADS) void headwise_rmsnorm_kernel(T* __restr
 }
 
 extern "C" int ga_hgrn2_scan(void* out, const void* proj, int64_t proj_stride, const void* f_bias, const void* lower,
-                             void* state, const void* slots, const void* cu, const void* q_start, int tokens, int entries, int heads,
-                             int dim, int vdim, hipStream_t stream) {
+                             void* state, const void* slots, const void* cu, const void* q_start, int way, int entries,
+                             int heads, int dim, int vdim, hipStream_t stream) {
   if (entries <= 0) return 0;
-  if (heads <= 0 || dim <= 0 || vdim <= 0 || dim > 16 * DW_SLICES) return -1;
-  if (heads > 65535 || (vdim + 15) / 16 > 65535 || proj_stride >= (1ll << 27)) return -2;    // (a tile's offsets are 32-bit)
+  if (heads <= 0 || dim <= 0 || vdim <= 0 || dim > 16 * DW_SLICES || (way != 1 && way != 8 && way != 16)) return -1;
+  if (heads > 65535 || (vdim + (way == 8 ? 7 : 15)) / (way == 8 ? 8 : 16) > 65535 || proj_stride >= (1ll << 27)) return -2;    // (a tile's offsets are 32-bit)
   const int rows = (dim + DW_SLICES - 1) / DW_SLICES;
 #define GO(R, C, T) hipLaunchKernelGGL((hgrn2_scan_kernel<R, C, T>), dim3(entries, heads, (vdim + C - 1) / C), dim3(dw_threads(C)), 0, stream, \
                                        (float*)out, (const float*)proj, proj_stride, (const float*)f_bias, (const float*)lower,            \
                                        (float*)state, (const int64_t*)slots, (const int32_t*)cu, (const int32_t*)q_start, heads, dim, vdim)
-  if (decay_walk_narrow(tokens, entries, heads, vdim)) {
-    DW_ROWS(rows, 8, GO);
-  } else {
-    DW_ROWS(rows, 16, GO);
-  }
+  DW_WAY(way, rows, GO);
 #undef GO
   return GA_CHECK_LAUNCH();
 }

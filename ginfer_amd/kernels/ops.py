@@ -1003,6 +1003,36 @@ def short_conv(x, weight, state, slots, step, dtype, add_input=True, update=True
 HGRN2_MAX_DIM = 256
 
 
+def decay_walk_way(tokens, entries, longest, heads, dim, vdim, turned=False):
+    """How the recurrences with a decay walk a step (csrc/decay_walk.h): 1 tiles of one token, else the value columns of a
+    workgroup, 8 or 16.  longest: tokens of the longest entry, 0 if not known (a recorded step: the mean stands for it); turned:
+    q and k are rotated.  Results do not depend on it.
+
+    One token an entry: the first (64 such entries, us, 16 columns -> tiles of one: 12 heads of 64 x 128 20.8 -> 16.8, 28 of
+    128 x 128 88 -> 68, 8 of 256 x 256 84 -> 72).  8 columns while the entries that are as long as the longest make no more
+    workgroups than the registers let a compute unit hold (three to a compute unit, two with a rotation and more than 32 rows
+    of state, one beyond 64 rows); then the chip is full, and reading a token's operands twice as often costs (12 entries of
+    300 tokens, 28 heads of 128 x 128: 376 us in 16 columns, 997 in 8; four, 12 heads of 64 x 128: 57 and 46, rotated 62 and
+    68).  And only while the longest entry's chain gains more than the smaller pieces cost the states of the entries beside it
+    (500 tokens beside 32 single ones, 12 heads of 64 x 128, 104 -> 81, but 8 of 256 x 256 320 -> 367, and 2,000 beside 32
+    1,045 -> 1,156; 157 and 101 beside 32, 12 heads, 42 -> 52)."""
+    T = TUNING
+    if tokens == entries and longest <= 1:
+        return 1
+    longest = longest if longest > 0 else -(-tokens // entries)
+    as_long = max(1, -(-(tokens - entries) // longest))
+    room = T.decay_narrow_workgroups // (1 if dim <= 32 or (dim <= 64 and not turned) else 1.5 if dim <= 64 else 3)
+    if -(-vdim // 8) > 65535 or as_long * heads * -(-vdim // 8) > room:
+        return 16
+    return 8 if longest * T.decay_narrow_state_a_token > (entries - as_long) * heads * dim * vdim else 16
+
+
+def _walk_of(step, tokens, entries, heads, dim, vdim, turned=False):
+    lens = getattr(step, "host_q_len", None)
+    known = lens is not None and "static_plan" not in (getattr(step, "extra", None) or {})
+    return decay_walk_way(tokens, entries, max(lens, default=0) if known else 0, heads, dim, vdim, turned)
+
+
 def hgrn2_scan(proj, f_bias, lower, state, slots, step, heads, dim, vdim, update=True):
     """proj float32 [T, 2 heads dim + heads vdim]: (q before its SiLU | forget-gate logits | v); f_bias, lower float32
     [heads dim]; state float32 [slots, heads, dim, vdim], advanced in place.  Returns float32 [T, heads, vdim]."""
@@ -1021,8 +1051,8 @@ def hgrn2_scan(proj, f_bias, lower, state, slots, step, heads, dim, vdim, update
     out = torch.empty((T, heads, vdim), dtype=torch.float32, device=proj.device)
     lib = build.load("gated_recurrence")
     _check(lib.ga_hgrn2_scan(_ptr(out), _ptr(proj), _i64(proj.stride(0)), _ptr(f_bias), _ptr(lower), _ptr(state), _ptr(slots),
-                             _ptr(step.cu_tokens), _ptr(step.q_start), _i(T), _i(E), _i(heads), _i(dim), _i(vdim), _stream()),
-           "hgrn2_scan")
+                             _ptr(step.cu_tokens), _ptr(step.q_start), _i(_walk_of(step, T, E, heads, dim, vdim)), _i(E), _i(heads),
+                             _i(dim), _i(vdim), _stream()), "hgrn2_scan")
     return out
 
 
@@ -1698,8 +1728,8 @@ def decay_scan(proj, q_start, k_start, v_start, state, slots, step, heads, dim, 
     lib = build.load("decay_scan")
     _check(lib.ga_decay_scan(_ptr(out), _ptr(q), _ptr(k), _ptr(v), _i64(proj.stride(0)), _ptr(decay), _ptr(head_decay),
                              _ptr(cos), _ptr(sin), _i(rot), _f(q_scale), _f(k_scale), _ptr(state), _ptr(slots),
-                             _ptr(step.cu_tokens), _ptr(step.q_start), _i(T), _i(E), _i(heads), _i(dim), _i(vdim),
-                             _i(1 if silu_inputs else 0), _stream()), "decay_scan")
+                             _ptr(step.cu_tokens), _ptr(step.q_start), _i(_walk_of(step, T, E, heads, dim, vdim, rot > 0)), _i(E), _i(heads),
+                             _i(dim), _i(vdim), _i(1 if silu_inputs else 0), _stream()), "decay_scan")
     return out
 
 

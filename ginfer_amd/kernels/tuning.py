@@ -156,6 +156,11 @@ class Tuning:
     # `pooled_decode_workgroups`, each with at least `pooled_decode_tiles_per_split` tiles (the partial sums just add)
     pooled_decode_workgroups: int = 2048
     pooled_decode_tiles_per_split: int = 4
+    # ---- the recurrences with a decay (decay_walk_way in kernels/ops.py, with the measurements): the workgroups of 8 columns that
+    # the longest entries may make (fewer with more registers), and the numbers of state beside them that a token of the longest
+    # one pays for
+    decay_narrow_workgroups: int = 768
+    decay_narrow_state_a_token: int = 6500
     # ---- routed feed-forwards (parts/mlp.py).  Steps of fewer rows than this run every expert over every row in one
     # product (rows that an expert does not own enter with zeros): no step that is recorded is longer, and up to some
     # hundred rows the experts' weights, which all come from memory either way, are what the step waits for.  Longer steps

@@ -862,3 +862,33 @@ def test_command_line_generates(folders):
     for _ in range(6):
         ids.append(int(torch.argmax(pp.logits(ids, w, cfg)[-1])))
     assert json.loads(out.stdout.strip().splitlines()[0])["token_ids"] == ids[5:]
+
+
+@pytest.mark.parametrize("dim", [5, 32, 48, 64, 90, 128, 192, 256])
+@pytest.mark.parametrize("lens", [[1], [1, 1, 1], [2], [1, 5, 16], [17, 1], [33]])
+def test_every_way_of_walking_gives_the_same_bits(dim, lens, monkeypatch):
+    """Tiles of one token, 8 columns and 16 columns (kernels/ops.py chooses by sizes): a token's arithmetic is the same, so
+    are the outputs and the states, for entries below, at and above what either walks at a time."""
+    from ginfer_amd.kernels import ops
+    E, T, heads, vdim = len(lens), sum(lens), 3, 21
+    g = torch.Generator().manual_seed(dim)
+    proj = torch.randn((T, 2 * heads * dim + heads * vdim), generator=g).cuda()
+    decay = (torch.rand((T, heads * dim), generator=g) * 0.9 + 0.1).cuda()
+    bias, lower = torch.randn((heads * dim,), generator=g).cuda(), torch.rand((heads * dim,), generator=g).cuda()
+    state = torch.randn((E, heads, dim, vdim), generator=g).cuda()
+    ang = torch.outer(torch.arange(64.0), torch.linspace(1.0, 0.01, 2)).cuda()
+    tables = dict(cos=torch.cos(ang).contiguous(), sin=torch.sin(ang).contiguous())
+    slots, step = torch.arange(E, device="cuda"), _Step(lens, [3 * (i % 2) for i in range(E)])
+    runs = {
+        "channel": lambda st: ops.decay_scan(proj, 0, heads * dim, 2 * heads * dim, st, slots, step, heads, dim, vdim, decay=decay),
+        "head": lambda st: ops.decay_scan(proj, 0, heads * dim, 2 * heads * dim, st, slots, step, heads, dim, vdim,
+                                          head_decay=lower[:heads].contiguous(), silu_inputs=True, **tables),
+        "hgrn2": lambda st: ops.hgrn2_scan(proj, bias, lower, st, slots, step, heads, dim, vdim)}
+    for kind, run in runs.items():
+        got = []
+        for way in (16, 8, 1):
+            monkeypatch.setattr(ops, "decay_walk_way", lambda *sizes: way)
+            st = state.clone()
+            got.append((run(st), st))
+        for out, st in got[1:]:
+            assert torch.equal(out, got[0][0]) and torch.equal(st, got[0][1]), kind
