@@ -1027,6 +1027,16 @@ def decay_walk_way(tokens, entries, longest, heads, dim, vdim, turned=False):
     return 8 if longest * T.decay_narrow_state_a_token > (entries - as_long) * heads * dim * vdim else 16
 
 
+DECAY_WALK_MAX_STRIDE = 1 << 27      # elements from token to token: the kernels count a tile's offsets in 32 bits
+
+
+def _near_rows(proj):
+    """`proj` [T, width] with rows that the recurrences' kernels can step over: a copy where they lie further apart."""
+    if proj.shape[0] == 1:
+        return proj.as_strided(proj.shape, (proj.shape[1], 1))       # one row has no next one, whatever its stride says
+    return proj if proj.stride(0) < DECAY_WALK_MAX_STRIDE else proj.contiguous()
+
+
 def _walk_of(step, tokens, entries, heads, dim, vdim, turned=False):
     lens = getattr(step, "host_q_len", None)
     known = lens is not None and "static_plan" not in (getattr(step, "extra", None) or {})
@@ -1048,6 +1058,7 @@ def hgrn2_scan(proj, f_bias, lower, state, slots, step, heads, dim, vdim, update
     E = step.cu_tokens.shape[0] - 1
     _need(slots.dtype == torch.int64 and slots.shape == (E,) and slots.is_contiguous(), "slots must be contiguous int64 [%d]", E)
     _need(update, "the recurrence always advances its state")
+    proj = _near_rows(proj)
     out = torch.empty((T, heads, vdim), dtype=torch.float32, device=proj.device)
     lib = build.load("gated_recurrence")
     _check(lib.ga_hgrn2_scan(_ptr(out), _ptr(proj), _i64(proj.stride(0)), _ptr(f_bias), _ptr(lower), _ptr(state), _ptr(slots),
@@ -1705,6 +1716,8 @@ def decay_scan(proj, q_start, k_start, v_start, state, slots, step, heads, dim, 
     entry's q_start is 0).  silu_inputs: the recurrence reads silu(q), silu(k) and silu(v).  Returns float32 [T, heads, vdim]."""
     _dev(proj, state, slots, decay, head_decay, cos, sin)
     T = proj.shape[0]
+    if proj.dim() == 2 and proj.stride(1) == 1:
+        proj = _near_rows(proj)
     q = _rows_of(proj, q_start, heads * dim, "q")
     k = _rows_of(proj, k_start, heads * dim, "k")
     v = _rows_of(proj, v_start, heads * vdim, "v")

@@ -892,3 +892,24 @@ def test_every_way_of_walking_gives_the_same_bits(dim, lens, monkeypatch):
             got.append((run(st), st))
         for out, st in got[1:]:
             assert torch.equal(out, got[0][0]) and torch.equal(st, got[0][1]), kind
+
+
+def test_recurrences_over_rows_far_apart():
+    """Rows of the projection 2^27 numbers apart (512 MB), and a single row with any stride: taken as rows side by side are."""
+    from ginfer_amd.kernels import ops
+    heads, dim, vdim, far = 2, 16, 8, 1 << 27
+    width = 2 * heads * dim + heads * vdim
+    g = torch.Generator().manual_seed(3)
+    near = torch.randn((2, width), generator=g).cuda()
+    apart = torch.empty((far + width,), device="cuda").as_strided((2, width), (far, 1))
+    apart.copy_(near)
+    bias, lower = torch.randn((heads * dim,), generator=g).cuda(), torch.rand((heads * dim,), generator=g).cuda()
+    slots = torch.arange(1, device="cuda")
+    runs = {"hgrn2": lambda p, st: ops.hgrn2_scan(p, bias, lower, st, slots, _Step([len(p)], [0]), heads, dim, vdim),
+            "decay": lambda p, st: ops.decay_scan(p, 0, heads * dim, 2 * heads * dim, st, slots, _Step([len(p)], [0]), heads, dim,
+                                                  vdim, head_decay=lower[:heads].contiguous())}
+    one = near[1:].as_strided((1, width), (far * 16, 1))
+    for kind, run in runs.items():
+        for a, b in ((near, apart), (near[1:], one)):
+            states = [torch.zeros((1, heads, dim, vdim), device="cuda") for _ in range(2)]
+            assert torch.equal(run(a, states[0]), run(b, states[1])) and torch.equal(*states), kind
