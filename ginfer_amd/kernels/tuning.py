@@ -21,8 +21,8 @@ from dataclasses import dataclass, field, fields
 
 @dataclass
 class Tuning:
-    # ---- bfloat16 products (parts/linear.py).  Up to 64 rows the package's weight-streaming kernel can take a product,
-    # beyond that only the BLAS library.
+    # ---- bfloat16 products (parts/linear.py).  Up to 64 rows the package's weight-streaming kernel can take a product;
+    # beyond that the BLAS library does, and from 17 rows on the package's products over tiles where they are faster (below).
     # From more rows than this, products with at least `library_min_out_features` output columns (gate-up, the head) go
     # to the library: the streaming kernel re-reads the rows once per 64 columns.
     library_from_rows: int = 16
@@ -65,12 +65,12 @@ class Tuning:
     library_square_min_features: int = 4096
     library_square_max_out_features: int = 8192
     library_square_many_rows: int = 128
-    # Sizes at which the library's own choice of kernel makes an exception of one plan: "class of the row count,output
-    # columns,elements of K" of a product whose consumer adds partial sums -> the plan measured fastest there, which
-    # stands before the rules (found with --autotune at the 7B shape: decode at batch 64 7.57 -> 7.20 ms a step).
-    measured_plans: dict = field(default_factory=lambda: {
-        "64,3584,18944": ("library", 2), "64,3584,3584": ("library", 2), "128,3584,3584": ("library", 2)})
-    # The same for the rows of prompt portions up to this many, in four pieces (the float32 parts cost the norm that
+    # Plans by size, before all rules: "class of the row count,output columns,elements of K" of a product whose consumer adds
+    # partial sums -> the plan.  None is needed at the sizes measured (the three that stood here, the library in halves for 64 and
+    # 128 rows of the 7B shape, take the product over tiles now, with the norm behind it: 64 rows, 3,584 columns of 18,944 49.6 ->
+    # 44.5 us, of 3,584 21.1 -> 18.6, 128 rows 24.7 -> 21.5).
+    measured_plans: dict = field(default_factory=dict)
+    # The library's product of a long K and few columns for the rows of prompt portions up to this many, in four pieces (the float32 parts cost the norm that
     # adds them more to read, so the gain is smaller and ends at 4,096 rows).
     library_split_portion_max_rows: int = 2048
     # with more output columns than `library_split_max_out_features`, a long K (as above) goes in halves up to this many rows

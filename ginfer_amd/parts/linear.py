@@ -23,17 +23,15 @@ def linear(x, weight, bias=None, out_dtype=None, parts_ok=False):
         return ops.gemm_nt(x, weight, bias)
     float32_out = out_dtype == torch.float32
     skinny_ok = ops.gemm_skinny_supported(x, weight)
+    tiles_ok = (parts_ok and bias is None and not float32_out and TUNING.library_from_rows < x.shape[0] <= TUNING.tiles_parts_most_rows
+                and ops.gemm_tiles_supported(x, weight))
     plan = None
     if autotune.active():
         key = ("linear", autotune.rows_class(x.shape[0]), weight.shape[0], x.shape[1], bias is not None, float32_out,
-               bool(parts_ok), skinny_ok)
+               bool(parts_ok), skinny_ok, tiles_ok)
         plan = autotune.choose(key, (weight, bias))
-    if plan is None and parts_ok and bias is None and not float32_out:
-        parts = tiles_parts(x.shape[0], weight.shape[0], x.shape[1])
-        if parts and ops.gemm_tiles_supported(x, weight):
-            plan = ("tiles", 1, parts)
     if plan is None:
-        plan = linear_plan(x.shape[0], weight.shape[0], x.shape[1], bias is not None, float32_out, parts_ok, skinny_ok)
+        plan = linear_plan(x.shape[0], weight.shape[0], x.shape[1], bias is not None, float32_out, parts_ok, skinny_ok, tiles_ok)
     return run_linear_plan(plan, x, weight, bias, out_dtype)
 
 
@@ -75,16 +73,19 @@ def tiles_gated(x, weight_gate_up):
     return tiles >= T.tiles_gated_full * 256 * -(-tiles // 256)
 
 
-def linear_plan(rows, out_features, in_features, has_bias, float32_out, parts_ok, skinny_ok):
+def linear_plan(rows, out_features, in_features, has_bias, float32_out, parts_ok, skinny_ok, tiles_ok=False):
     """The way a bfloat16 product is done, by the rules: ("skinny", tiles of W per wavefront, parts of K) for the
-    package's weight-streaming kernel, ("library", pieces of K) for the BLAS library (the product over tiles, ("tiles", 1, parts
-    of K), stands before these rules: `tiles_parts`).  More than one part or piece
-    means float32 partial sums [parts, M, N] for the consumer to add."""
+    package's weight-streaming kernel, ("tiles", 1, parts of K) for its product over tiles, ("library", pieces of K) for the BLAS
+    library; skinny_ok, tiles_ok: whether those kernels take the operands.  Tiles, and more than one part or piece, mean
+    float32 partial sums [parts, M, N] for the consumer to add."""
     may_split = parts_ok and not float32_out
     if may_split and not has_bias:
         measured = TUNING.measured_plans.get("%d,%d,%d" % (autotune.rows_class(rows), out_features, in_features))
-        if measured is not None and (skinny_ok or measured[0] != "skinny"):
+        if measured is not None and {"skinny": skinny_ok, "tiles": tiles_ok}.get(measured[0], True):
             return tuple(measured)
+        parts = tiles_parts(rows, out_features, in_features) if tiles_ok else 0
+        if parts:
+            return ("tiles", 1, parts)
         pieces = _library_long_k_pieces(rows, out_features, in_features)
         if pieces > 1:
             return ("library", pieces)
@@ -111,9 +112,7 @@ def run_linear_plan(plan, x, weight, bias, out_dtype):
             return ops.gemm_skinny(x, weight, bias, out_dtype=torch.float32, nt=nt, grid_splits=splits)
         return ops.gemm_skinny(x, weight, bias, out_dtype=out_dtype, nt=nt)
     if plan[0] == "tiles":
-        if ops.gemm_tiles_supported(x, weight):
-            return ops.gemm_tiles_parts(x, weight, plan[2])
-        plan = ("library", 1)            # a plan kept for this class of sizes meets rows that the kernel does not take
+        return ops.gemm_tiles_parts(x, weight, plan[2])
     _, parts = plan
     if parts > 1:
         # the library, once, over `parts` pieces of K side by side (a batched product over views of x and
@@ -135,8 +134,8 @@ def run_linear_plan(plan, x, weight, bias, out_dtype):
 
 def linear_candidates(key):
     """Every plan that does the product of an autotune key; the plan by the rules first."""
-    _, rows, out_features, in_features, has_bias, float32_out, parts_ok, skinny_ok = key
-    plans = [linear_plan(rows, out_features, in_features, has_bias, float32_out, parts_ok, skinny_ok)]
+    _, rows, out_features, in_features, has_bias, float32_out, parts_ok, skinny_ok, tiles_ok = key if len(key) > 8 else key + (False,)
+    plans = [linear_plan(rows, out_features, in_features, has_bias, float32_out, parts_ok, skinny_ok, tiles_ok)]
 
     def add(plan):
         if plan not in plans:
@@ -155,8 +154,8 @@ def linear_candidates(key):
                         add(("skinny", nt, parts))
     add(("library", 1))
     if may_split and not has_bias:
-        parts = tiles_parts(rows, out_features, in_features)
-        if parts and in_features % parts == 0:
+        parts = tiles_parts(rows, out_features, in_features) if tiles_ok else 0
+        if parts:
             add(("tiles", 1, parts))
         for parts in (2, 3, 4, 5, 7, 8, 10, 14, 16):
             if in_features % parts == 0 and (in_features // parts) % 8 == 0 and in_features // parts >= 512:
@@ -167,7 +166,7 @@ def linear_candidates(key):
 def _linear_timing(key, operands, device):
     """For the tuner: the product on random rows, followed, where it may come in parts, by the norm that adds them
     (more parts cost that norm more to read)."""
-    _, rows, out_features, in_features, _, float32_out, parts_ok, _ = key
+    _, rows, out_features, in_features, _, float32_out, parts_ok = key[:7]
     x = (torch.randn((rows, in_features), device=device) * 0.5).to(torch.bfloat16)
     residual = torch.zeros((rows, out_features), dtype=torch.float32, device=device) if parts_ok else None
     gain = torch.ones((out_features,), dtype=torch.bfloat16, device=device) if parts_ok else None

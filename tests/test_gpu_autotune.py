@@ -31,18 +31,19 @@ def test_every_candidate_plan_gives_the_product(rows, n, k):
                 x, w, b, xd, wd, bd = _operands(rows, n, k, rows + n + k, bias)
                 ref = xd @ wd.T + (bd if bias else 0.0)
                 skinny_ok = ops.gemm_skinny_supported(x, w)
-                key = ("linear", rows, n, k, bias, f32, parts_ok, skinny_ok)
+                tiles_ok = ops.gemm_tiles_supported(x, w)
+                key = ("linear", rows, n, k, bias, f32, parts_ok, skinny_ok, tiles_ok)
                 for plan in L.linear_candidates(key):
                     y = L.run_linear_plan(plan, x, w, b, torch.float32 if f32 else None)
                     parts = plan[-1] if (plan[0] == "library" or plan[2] > 1) and plan[-1] > 1 else 1
-                    if parts > 1:
+                    if parts > 1 or plan[0] == "tiles":
                         assert y.shape == (parts, rows, n) and y.dtype == torch.float32, (plan, y.shape)
                         y = y.double().sum(0)
                     else:
                         assert y.shape == (rows, n) and y.dtype == (torch.float32 if f32 else torch.bfloat16), (plan, y.dtype)
                     err = float((y.double().cpu() - ref).abs().max() / ref.abs().max())
                     # bfloat16 results carry one rounding (2^-9 of the value); 32-bit ones only the order of the sums
-                    tol = 1e-5 if (f32 or parts > 1) else 4e-3
+                    tol = 1e-5 if (f32 or parts > 1 or plan[0] == "tiles") else 4e-3
                     assert err <= tol, "plan %s of %s: %.3g" % (plan, key, err)
                     tried.add(plan)
     assert ("library", 1) in tried and len(tried) >= 3, tried
@@ -91,7 +92,7 @@ def test_a_runner_that_times_its_plans(tmp_path):
     assert runner.counts["autotuned_keys"] >= 3 and runner.counts["replayed_decode"] >= 3, runner.counts
     assert isinstance(runner.plans, autotune.Table)
     keys = [key for key, _, _ in runner.plans.report]
-    assert ("linear", 48, 3584, 18944, False, False, True, True) in keys, keys
+    assert ("linear", 48, 3584, 18944, False, False, True, True, True) in keys, keys
     for key, plan, times in runner.plans.report:
         print("%s -> %s (%d plans, %.1f to %.1f us)" % (key, plan, len(times), min(times.values()), max(times.values())))
         assert runner.plans[key] == plan and plan in times

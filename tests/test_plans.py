@@ -44,9 +44,7 @@ def test_a_long_k_of_few_rows_goes_to_the_library_in_pieces():
     assert plan(64, 5120, 5120) == ("library", 8) and plan(256, 5120, 5120) == ("library", 8)
     assert plan(64, 8192, 8192) == ("library", 1) and plan(128, 8192, 8192) == ("library", 4)
     assert plan(32, 5120, 5120) == ("library", 1)
-    # measured exceptions (the library's own choice of kernel at these very sizes)
-    assert plan(64, 3584, 18944) == ("library", 2) and plan(64, 3584, 3584) == ("library", 2)
-    assert plan(50, 3584, 18944) == ("library", 2)                  # rows share a plan in classes of 16
+    assert plan(64, 3584, 18944) == ("library", 8) and plan(64, 3584, 3584) == ("skinny", 4, 4)
     assert L.linear_plan(64, 3584, 18944, False, False, False, True)[0] == "skinny"     # nobody to add parts: no pieces
     assert L.linear_plan(64, 3584, 18944, True, False, True, True)[0] == "skinny"       # a bias: one product
     # the 0.5B and 1.5B shapes: as measured there
@@ -62,6 +60,52 @@ def test_a_long_k_of_few_rows_goes_to_the_library_in_pieces():
     for rows, n, k in ((64, 2048, 11008), (64, 8192, 29568), (32, 5120, 27648), (128, 8192, 8192), (64, 3584, 18944)):
         key = ("linear", rows, n, k, False, False, True, rows <= 64)
         assert L.linear_candidates(key)[0] == plan(rows, n, k)
+
+
+def test_products_over_tiles_in_parts_of_k():
+    """The rule for a consumer that adds parts, as linear() asks for it (operands that the kernel over tiles takes)."""
+    plan = lambda rows, n, k, has_bias=False, f32=False, parts_ok=True: L.linear_plan(rows, n, k, has_bias, f32, parts_ok, rows <= 64, True)
+    # as many parts as keep to one round of the chip, every one with a slab, none longer than the first
+    assert plan(64, 1536, 8960) == ("tiles", 1, 10) and plan(256, 1536, 8960) == ("tiles", 1, 5)
+    assert plan(64, 3584, 18944) == ("tiles", 1, 4) and plan(64, 3584, 3584) == ("tiles", 1, 4)
+    assert plan(128, 3584, 3584) == ("tiles", 1, 4) and plan(64, 2048, 11008) == ("tiles", 1, 8)
+    for rows in (17, 48, 64, 65, 100, 128, 192, 256):
+        for n, k in ((1024, 3072), (1536, 3072), (1536, 8960), (2048, 11008), (2560, 4096), (3584, 3584), (4096, 4096)):
+            way, _, parts = plan(rows, n, k)
+            slabs = k // 64
+            assert way == "tiles" and (parts - 1) * -(-slabs // parts) < slabs
+            tiles = -(-n // (64 if rows <= 64 else 128)) * -(-rows // 64)
+            assert parts == 1 or (parts * tiles <= 256 and parts * 8 <= slabs)
+    # outside its range, and for consumers that add no parts, the rules before it
+    assert plan(16, 1536, 8960)[0] == "skinny" and plan(257, 1536, 8960) == ("library", 4)
+    assert plan(64, 1536, 1536) == ("skinny", 1, 2) and plan(64, 4112, 8960)[0] == "library"
+    assert plan(64, 1528, 8960) == ("skinny", 4, 10)                # 1,528 columns are no multiple of 16
+    assert plan(65, 3584, 18944) == ("library", 8)                  # the rows of A are most of what is read
+    assert plan(64, 3584, 18944, parts_ok=False)[0] == "skinny" and plan(64, 3584, 18944, has_bias=True)[0] == "skinny"
+    assert plan(64, 3584, 18944, f32=True)[0] == "skinny"
+    assert L._parts_without_gaps(140, 10) == 10 and L._parts_without_gaps(9, 4) == 3 and L._parts_without_gaps(12, 5) == 4
+    assert L._parts_without_gaps(1, 1) == 1
+
+
+def test_measured_plans_stand_before_all_rules(monkeypatch):
+    monkeypatch.setattr(L.TUNING, "measured_plans", {"64,3584,18944": ("library", 2), "64,1536,8960": ("tiles", 1, 7)})
+    plan = lambda rows, n, k, tiles_ok=True: L.linear_plan(rows, n, k, False, False, True, rows <= 64, tiles_ok)
+    assert plan(64, 3584, 18944) == ("library", 2) and plan(50, 3584, 18944) == ("library", 2)      # classes of 16 rows
+    assert plan(64, 1536, 8960) == ("tiles", 1, 7)
+    assert plan(64, 1536, 8960, False) == ("skinny", 4, 10)         # operands that its kernel does not take
+    assert L.linear_plan(64, 3584, 18944, True, False, True, True, True)[0] == "skinny"             # a bias: no parts
+
+
+def test_the_tuner_starts_from_the_plan_that_runs():
+    for rows in (16, 17, 64, 128, 256):
+        for n, k in ((1536, 8960), (3584, 3584), (3072, 8192), (896, 4864), (3584, 18944)):
+            for tiles_ok in (False, True):
+                plans = L.linear_candidates(("linear", rows, n, k, False, False, True, rows <= 64, tiles_ok))
+                assert plans[0] == L.linear_plan(rows, n, k, False, False, True, rows <= 64, tiles_ok)
+                assert tiles_ok or not any(p[0] == "tiles" for p in plans)
+                assert len(set(plans)) == len(plans) and ("library", 1) in plans
+    # parts that do not divide K are candidates like any other
+    assert L.linear_candidates(("linear", 64, 3072, 8192, False, False, True, True, True))[0] == ("tiles", 1, 5)
 
 
 def test_measured_plans_can_be_set_from_json():
