@@ -173,7 +173,8 @@ struct KRange {
 // columns: the activation of the feed-forward without a pass over memory of its own.
 // The gate of a gated product: out = g * sigmoid(alpha g) * (u + shift) with g = min(gate, limit) and u = clamp(up, -limit,
 // limit).  limit = infinity, alpha = 1, shift = 0 is SiLU(gate) * up, bit for bit what stood here before the bounds; alpha =
-// infinity stands for the sigmoid's limit, a step at zero: relu(g) * (u + shift).
+// infinity stands for the sigmoid's limit, a step at zero: relu(g) * (u + shift).  (From 17 rows on the product over tiles may
+// stand here, whose sigmoid is the hardware's exp2 and reciprocal: csrc/gemm_tiles.hip has the two's errors.)
 struct GateAct {
   float limit, alpha, shift;
 };

@@ -34,7 +34,11 @@ template <int N>
 __device__ __forceinline__ void gt_wait_and_meet() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory"); }
 
 // act.kind 0: SiLU(v) * u; 1: g * sigmoid(alpha g) * (u + shift), g = min(v, limit), u = clamp(u, -limit, limit); 2: the same
-// with the sigmoid's limit, a step.  exp2 and the reciprocal are the hardware's (1 unit of the 32-bit result's last place).
+// with the sigmoid's limit, a step.  exp2 and the reciprocal are the hardware's: against 64 bits SiLU is off by at most 3 units of
+// the 32-bit result's last place for v > -0.5, 6 down to -4, 18 down to -20 and 65 (4e-6 of it) down to -87, below which it is 0;
+// with expf and a division, as the kernel for up to 16 rows has it, by at most 3.4 everywhere.  The one rounding that follows is
+// 2^-9 of the result.  expf and the division cost 1 us of 27 at 64 rows and 41 of 464 at 2,048 (one tile's 128 results a thread
+// are straight code that no one else has fetched yet), a correction of exp2's argument and one step on the reciprocal 21.
 struct GateAct {
   int kind;
   float limit, alpha, shift;
@@ -232,25 +236,27 @@ static int gt_check(const void* C, const void* A, int64_t lda, const void* W, in
   return 0;
 }
 
-// Tiles (rows of W x rows of A): up to 64 rows 128 x 64, up to 256 128 x 256, up to 1,535 256 x 128, beyond 256 x 256; and 256 x
-// 128 for few rows too where tiles of 128 rows of W would make more than a round of the chip's 256 compute units (a tile's time
-// is nearly the same for 64 and for 128 rows then: the weights' way).  us, product and activation by the library's best way ->
-// here, as replays of a graph over several layers' weights: 17,920 rows of W, K 1,536: 17 rows 18.4 -> 16.1, 64 rows 21.0 -> 18.0,
-// 256 rows 33.9 -> 28.8, 384 rows 37.3 -> 32.1, 1,000 rows 88 -> 76; 37,888 rows, K 3,584: 384 rows 131 -> 118, 1,024 rows 309 -> 279,
-// 2,048 rows 570 -> 490.  What decides at many rows is how full the last round of tiles is (at 512 rows the library's 43 stand against
-// 48 and 147 against 164): the caller's rule.
+// tiling: which tiles, rows of W x rows of A; the caller chooses by sizes and by how full they leave the chip's rounds
+// (gated_tiling in kernels/ops.py, tiles_gated in parts/linear.py, the fastest and the library beside each other).  us, product and
+// activation by the library's best way -> here, as replays of a graph over several layers' weights: 17,920 rows of W, K 1,536: 64 rows
+// 30.6 -> 26.9, 128 rows 35.1 -> 30.2 (tiles of 128 x 256, half of them rows that do not exist, 33.5), 256 rows 43.6 -> 37.2, 384
+// rows 45.9 -> 39.9; 37,888 rows, K 3,584: 128 rows 84.0 -> 79.3, 384 rows 133.9 -> 121.4, 1,000 rows 324 -> 272, 1,280 rows 386 ->
+// 291, 2,048 rows 552 -> 464; 19,456 rows, K 2,560: 128 rows 46.0 -> 44.0 (128 x 256 tiles 49.1), 384 rows 64.0 -> 57.8.
 extern "C" int ga_gemm_tiles_gated(void* C, int64_t ldc, const void* A, int64_t lda, const void* W, int M, int cols, int K, int kind,
-                                   float limit, float alpha, float shift, hipStream_t stream) {
+                                   float limit, float alpha, float shift, int tiling, hipStream_t stream) {
   if (M <= 0) return 0;
   const int rc = gt_check(C, A, lda, W, 2 * (int64_t)cols, M, cols, K);
   if (rc) return rc;
   if (kind < 0 || kind > 2 || ldc < cols || ldc % 8) return -1;
   const GateAct act = {kind, limit, alpha, shift};
-  const bool one_round = (cols + 63) / 64 <= 256;
-  if (M <= 64 && one_round) return gt_launch<2, 1, 2, 2, 3, true>(C, ldc, A, lda, W, M, cols, K, 1, act, stream);
-  if (M <= 256 && (one_round || M > 128)) return gt_launch<4, 2, 1, 4, 3, true>(C, ldc, A, lda, W, M, cols, K, 1, act, stream);
-  if (M < 1536) return gt_launch<4, 2, 2, 2, 3, true>(C, ldc, A, lda, W, M, cols, K, 1, act, stream);
-  return gt_launch<4, 4, 2, 2, 2, true>(C, ldc, A, lda, W, M, cols, K, 1, act, stream);
+  switch (tiling) {
+    case 0: return gt_launch<2, 1, 2, 2, 3, true>(C, ldc, A, lda, W, M, cols, K, 1, act, stream);     // 128 x 64
+    case 1: return gt_launch<4, 2, 1, 4, 3, true>(C, ldc, A, lda, W, M, cols, K, 1, act, stream);     // 128 x 256
+    case 2: return gt_launch<4, 2, 2, 2, 3, true>(C, ldc, A, lda, W, M, cols, K, 1, act, stream);     // 256 x 128
+    case 3: return gt_launch<4, 4, 2, 2, 2, true>(C, ldc, A, lda, W, M, cols, K, 1, act, stream);     // 256 x 256
+    case 4: return gt_launch<2, 2, 2, 2, 3, true>(C, ldc, A, lda, W, M, cols, K, 1, act, stream);     // 128 x 128
+  }
+  return -6;
 }
 
 // Up to 64 rows tiles of 64 x 64, beyond 128 x 64.  us with the norm that adds the parts, the best other way -> here, with as many

@@ -96,9 +96,9 @@ int ga_add_scalar_rmsnorm(void* residual, const void* y, const void* gain, void*
 
 // ---- gemm_tiles.hip: bfloat16 products over tiles through LDS; A [M, K] (row stride lda), W [rows, K] contiguous, 16-byte
 // addresses, K a multiple of 64, cols of 8.  gated: W is [2 cols, K], C [M, cols] bfloat16 = activation(A.gate^T) * (A.up^T), kind 0
-// SiLU, 1 bounded sigmoid, 2 bounded step; parts: C float [parts, M, cols], partial sums over K
+// SiLU, 1 bounded sigmoid, 2 bounded step; tiling 0 .. 4 (see there); parts: C float [parts, M, cols], partial sums over K
 int ga_gemm_tiles_gated(void* C, int64_t ldc, const void* A, int64_t lda, const void* W, int M, int cols, int K, int kind,
-                        float limit, float alpha, float shift, hipStream_t stream);
+                        float limit, float alpha, float shift, int tiling, hipStream_t stream);
 int ga_gemm_tiles_parts(void* C, const void* A, int64_t lda, const void* W, int M, int cols, int K, int parts, hipStream_t stream);
 
 // ---- embedding_sinusoid.hip: out float [tokens, hidden] = table_scale * table[ids] + (sin | cos)(position * freq[i / 2]), then the norm

@@ -6,6 +6,7 @@ fit; a kernel never sees a shape it was not written for.  Tensors are torch tens
 kernels run on torch's current stream.
 """
 import ctypes
+import math
 
 import torch
 
@@ -436,10 +437,28 @@ def gemm_tiles_supported(a, w):
             and w.numel() < 1 << 31 and a.shape[0] * a.stride(0) < 1 << 31)
 
 
-def gemm_tiles_gated(a, w, bounds=None):
+GATED_TILINGS = ((128, 64), (128, 256), (256, 128), (256, 256), (128, 128))      # rows of W, rows of A of a workgroup
+
+
+def gated_tiling(rows, out_features):
+    """The tiles of the gated product of `rows` rows by `out_features` rows of W: its number in GATED_TILINGS.  Few rows: the
+    smallest that hold them and keep to one round of the chip's 256 compute units; more: the fastest of what was measured."""
+    columns = -(-out_features // 128)
+    if rows <= 64 and columns <= 256:
+        return 0
+    if rows <= 128:
+        return 4 if columns <= 256 else 2
+    if rows <= 256:
+        return 4 if 2 * columns <= 256 else 1
+    if rows <= 384 and 3 * columns <= 256:
+        return 4
+    return 2 if rows <= 1024 else 3
+
+
+def gemm_tiles_gated(a, w, bounds=None, tiling=None):
     """a [M, K], w [2N, K] (gate over up) -> bfloat16 [M, N] = silu(a.gate^T) * (a.up^T), both sums in 32-bit and one
     rounding; with bounds = (limit, alpha, shift) g * sigmoid(alpha g) * (u + shift), g = min(gate, limit), u = clamp(up,
-    -limit, limit) (alpha = infinity: the sigmoid's limit, relu(g))."""
+    -limit, limit) (alpha = infinity: the sigmoid's limit, relu(g)).  tiling: its number in GATED_TILINGS (None: by sizes)."""
     _dev(a, w)
     _need(gemm_tiles_supported(a, w) and a.shape[1] == w.shape[1], "the kernel over tiles does not take %s %s x %s %s", a.dtype,
           tuple(a.shape), w.dtype, tuple(w.shape))
@@ -447,11 +466,13 @@ def gemm_tiles_gated(a, w, bounds=None):
     kind, (limit, alpha, shift) = 0, bounds or (0.0, 1.0, 0.0)
     if bounds is not None:
         _need(limit > 0, "the gate's bound must be positive, got %r", limit)
-        kind = 2 if alpha == float("inf") else 1
+        kind = 2 if math.isinf(alpha) else 1
+    if tiling is None:
+        tiling = gated_tiling(M, w.shape[0])
     out = torch.empty((M, N), dtype=a.dtype, device=a.device)
     lib = build.load("gemm_tiles")
     _check(lib.ga_gemm_tiles_gated(_ptr(out), _i64(N), _ptr(a), _i64(a.stride(0)), _ptr(w), _i(M), _i(N), _i(a.shape[1]), _i(kind),
-                                   _f(limit), _f(alpha), _f(shift), _stream()), "gemm_tiles_gated")
+                                   _f(limit), _f(alpha), _f(shift), _i(tiling), _stream()), "gemm_tiles_gated")
     return out
 
 

@@ -78,23 +78,30 @@ class Tuning:
     # The gate-up product lies transposed (weights as the library's first operand) for row counts from this on that
     # are a multiple of it: the library's tiles then fit the rows.
     transposed_gate_up_row_multiple: int = 256
-    # ---- the package's products over tiles through LDS (csrc/gemm_tiles.hip, with its measurements).  The gated product of at
-    # least so many rows of weights and elements of K: beyond `library_from_rows` rows up to `tiles_gated_few_rows` always,
-    # up to `tiles_gated_some_rows` while tiles of 128 rows of W make one round of the chip (7B shape, 256 rows: the library's 87 us
-    # against 115), up to `tiles_gated_odd_rows` again always (row counts the library's tiles do not fit: 300 rows 35 -> 30 and
-    # 125 -> 113 us; at 512 its 43 and 147 stand against 48 and 164), from `tiles_gated_many_rows` on always (1,000 rows 88 -> 76,
-    # 323 -> 271), and beyond `tiles_gated_full_rows` up to `tiles_gated_most_rows` where the rounds of 256 x 256 tiles are full to
-    # `tiles_gated_full` (2,048 rows of the 7B shape, 0.925: 570 -> 490; of the 1.5B shape, 0.73: 136 and 138; at 4,096 rows the
-    # library is ahead again)
+    # ---- the package's products over tiles through LDS (csrc/gemm_tiles.hip).  The gated product of at least so many rows of
+    # weights and elements of K, beyond `library_from_rows` rows; measured at twelve sizes of W from 8,192 x 1,024 to 59,136 x
+    # 8,192, in the tiles of ops.gated_tiling, the library's best way with the activation against it:
+    # - up to 256 rows, in one round of the chip's 256 compute units: a workgroup streams its K at a speed of its own, 12.5 ns an
+    #   element, however few others there are, the library at some 3.4 TB/s.  The two are level at `tiles_gated_level` tiles
+    #   (`tiles_gated_level_tall` where a tile has 256 rows of A); with fewer the kernel's shorter way to the activation pays for a
+    #   K times missing tiles of so much (64 rows: 96 tiles of K 3,072 34.4 -> 40.5 us, refused; 64 of 1,024 19.4 -> 15.1).  In two
+    #   rounds the library is ahead (37,888 rows of W at 256 rows 90 against 123);
+    # - up to 384 rows: one or two rounds, full to `tiles_gated_full_few_rounds` (17,920 x 1,536 0.82 45.9 -> 39.9, 37,888 x 3,584 0.87
+    #   133.9 -> 121.4; but 22,016 x 2,048 0.50 57.9 -> 68.4, 27,648 x 5,120 0.63 117 -> 161);
+    # - up to 1,024 rows: one round as full as that, or four and more full to `tiles_gated_full` (37,888 x 3,584 at 1,000 rows 324 -> 272;
+    #   the library is ahead by up to 20 % at 22,016 x 2,048, 28,672 x 4,096 and five others there; 17,920 x 1,536, three rounds 0.73 full,
+    #   would win 8 % of its 91 us);
+    # - up to `tiles_gated_most_rows`: rounds full to `tiles_gated_full` (37,888 x 3,584 at 1,280 rows 386 -> 291, at 2,048 552 -> 464;
+    #   17,920 x 1,536 at 1,700 rows 104 -> 99; at 2,304 rows and 4,096 the library is ahead again: 28,672 x 4,096 402 -> 431).
+    # Where the rule takes the kernel, the worst seen is 3 % more than the library.
     tiles_gated_min_out_features: int = 8192
     tiles_gated_min_in_features: int = 1024
-    tiles_gated_few_rows: int = 128
-    tiles_gated_some_rows: int = 256
-    tiles_gated_odd_rows: int = 384
-    tiles_gated_many_rows: int = 961
-    tiles_gated_full_rows: int = 1024
-    tiles_gated_most_rows: int = 2304
-    tiles_gated_full: float = 0.9
+    tiles_gated_level: int = 164
+    tiles_gated_level_tall: int = 209
+    tiles_gated_k_times_missing: int = 147000
+    tiles_gated_full_few_rounds: float = 0.8
+    tiles_gated_full: float = 0.92
+    tiles_gated_most_rows: int = 2048
     # ... and the product whose parts of K the norm adds: K of at least `tiles_parts_min_in_features`, at most
     # `library_split_max_out_features` columns, beyond `library_from_rows` rows up to so many, in as many parts as keep to
     # `tiles_parts_workgroups` workgroups; with more than 64 rows not where K is so long beside that many columns that the tiles'

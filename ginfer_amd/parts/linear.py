@@ -59,18 +59,27 @@ def _parts_without_gaps(slabs, parts):
     return parts
 
 
-def tiles_gated(x, weight_gate_up):
+def tiles_gated(rows, out_features, in_features):
     """Whether the package's gated product over tiles is the fastest way, by sizes alone (measurements beside the thresholds)."""
-    T, rows, (out_features, in_features) = TUNING, x.shape[0], weight_gate_up.shape
-    if (rows <= T.library_from_rows or rows > T.tiles_gated_most_rows or out_features < T.tiles_gated_min_out_features
-            or in_features < T.tiles_gated_min_in_features or not ops.gemm_tiles_supported(x, weight_gate_up)):
+    T = TUNING
+    if (not T.library_from_rows < rows <= T.tiles_gated_most_rows or out_features < T.tiles_gated_min_out_features
+            or in_features < T.tiles_gated_min_in_features):
         return False
-    if rows <= T.tiles_gated_odd_rows:
-        return rows <= T.tiles_gated_few_rows or rows > T.tiles_gated_some_rows or -(-out_features // 128) <= 256
-    if rows <= T.tiles_gated_full_rows:
-        return rows >= T.tiles_gated_many_rows
-    tiles = -(-rows // 256) * -(-out_features // 256)
-    return tiles >= T.tiles_gated_full * 256 * -(-tiles // 256)
+    tiling = ops.gated_tiling(rows, out_features)
+    of_w, of_a = ops.GATED_TILINGS[tiling]
+    tiles = -(-out_features // of_w) * -(-rows // of_a)
+    rounds = -(-tiles // 256)
+    full = tiles / (256.0 * rounds)
+    if rounds == 1 and (rows <= 256 or of_w == of_a == 128):
+        level = T.tiles_gated_level_tall if of_a == 256 else T.tiles_gated_level
+        return in_features * (level - tiles) <= T.tiles_gated_k_times_missing
+    if rows <= 256:
+        return False
+    if rows <= 384:
+        return rounds <= 2 and full >= T.tiles_gated_full_few_rounds
+    if rows <= 1024:
+        return full >= T.tiles_gated_full_few_rounds if rounds == 1 else (rounds >= 4 and full >= T.tiles_gated_full)
+    return full >= T.tiles_gated_full
 
 
 def linear_plan(rows, out_features, in_features, has_bias, float32_out, parts_ok, skinny_ok, tiles_ok=False):
@@ -292,28 +301,31 @@ def linear_into_norm(x, weight, bias, residual, norm):
     return ops.gemm_skinny(x, weight, bias, into_norm=(residual, norm.weight, norm.eps))
 
 
-def gated_linear(x, weight_gate_up):
-    """silu(x . Wg^T) * (x . Wu^T) with Wg over Wu stacked in one matrix [2I, K] -> [M, I].  x may be
-    ops.ScaledRows."""
+def gated_linear(x, weight_gate_up, bounds=None):
+    """silu(x . Wg^T) * (x . Wu^T) with Wg over Wu stacked in one matrix [2I, K] -> [M, I]; with bounds = (limit, alpha, shift)
+    the bounded gate of ops.clamped_glu.  x may be ops.ScaledRows (without bounds)."""
     if isinstance(x, ops.ScaledRows):
         return ops.gemm_skinny(x, weight_gate_up, gated=True)
-    if tiles_gated(x, weight_gate_up):
-        return ops.gemm_tiles_gated(x, weight_gate_up)
     skinny_ok = x.dtype == torch.bfloat16 and ops.gemm_skinny_supported(x, weight_gate_up)
-    transposable = _transposable(x, weight_gate_up)
+    transposable = bounds is None and _transposable(x, weight_gate_up)
+    rows, (out_features, in_features) = x.shape[0], weight_gate_up.shape
+    tiles_ok = (x.dtype == torch.bfloat16 and TUNING.library_from_rows < rows <= TUNING.tiles_gated_most_rows
+                and (bounds is None or bounds[0] > 0) and ops.gemm_tiles_supported(x, weight_gate_up))
     plan = None
     if autotune.active() and x.dtype == torch.bfloat16:
-        key = ("gated", autotune.rows_class(x.shape[0]), weight_gate_up.shape[0], x.shape[1], skinny_ok, transposable)
+        key = ("gated", autotune.rows_class(rows), out_features, in_features, skinny_ok, transposable, tiles_ok, bounds)
         plan = autotune.choose(key, (weight_gate_up,))
     if plan is None:
-        plan = gated_plan(x.shape[0], weight_gate_up.shape[0], skinny_ok, transposable)
-    return run_gated_plan(plan, x, weight_gate_up)
+        plan = gated_plan(rows, out_features, skinny_ok, transposable, in_features, tiles_ok)
+    return run_gated_plan(plan, x, weight_gate_up, bounds)
 
 
-def gated_plan(rows, out_features, skinny_ok, transposable):
-    """By the rules: ("skinny",) the weight-streaming kernel with the activation in its epilogue; ("transposed",) the
-    library with the weights as its first operand, which leaves the product transposed, [2I, M], and the activation on
-    that; ("library",) the usual product and the activation."""
+def gated_plan(rows, out_features, skinny_ok, transposable, in_features=0, tiles_ok=False):
+    """By the rules: ("skinny",) the weight-streaming kernel with the activation in its epilogue; ("tiles",) the product over
+    tiles with the same; ("transposed",) the library with the weights as its first operand, which leaves the product transposed,
+    [2I, M], and the activation on that; ("library",) the usual product and the activation."""
+    if tiles_ok and tiles_gated(rows, out_features, in_features):
+        return ("tiles",)
     if skinny_ok and not _library_is_faster(rows, out_features):
         return ("skinny",)
     if transposable and _transposed_product_is_faster(rows):
@@ -321,27 +333,35 @@ def gated_plan(rows, out_features, skinny_ok, transposable):
     return ("library",)
 
 
-def run_gated_plan(plan, x, weight_gate_up):
+def run_gated_plan(plan, x, weight_gate_up, bounds=None):
+    if plan[0] == "tiles":
+        return ops.gemm_tiles_gated(x, weight_gate_up, bounds=bounds)
     if plan[0] == "skinny":
-        return ops.gemm_skinny(x, weight_gate_up, gated=True)
+        return ops.gemm_skinny(x, weight_gate_up, gated=True, gate_bounds=bounds)
     if plan[0] == "transposed":
         return ops.silu_mul_transposed(torch.mm(weight_gate_up, x.t()))
-    return ops.silu_mul(linear(x, weight_gate_up))
+    gate_up = linear(x, weight_gate_up)
+    return ops.silu_mul(gate_up) if bounds is None else ops.clamped_glu(gate_up, *bounds)
+
+
+def _gated_key(key):
+    """(rows, out_features, in_features, skinny_ok, transposable, tiles_ok, bounds) of a key; the last two may be left out."""
+    return (key[1:] + (False, None))[:7] if len(key) < 8 else key[1:]
 
 
 def gated_candidates(key):
-    _, rows, out_features, _, skinny_ok, transposable = key
-    plans = [gated_plan(rows, out_features, skinny_ok, transposable)]
-    for plan, ok in ((("skinny",), skinny_ok), (("library",), True), (("transposed",), transposable)):
+    rows, out_features, in_features, skinny_ok, transposable, tiles_ok, _ = _gated_key(key)
+    plans = [gated_plan(rows, out_features, skinny_ok, transposable, in_features, tiles_ok)]
+    for plan, ok in ((("skinny",), skinny_ok), (("library",), True), (("transposed",), transposable), (("tiles",), tiles_ok)):
         if ok and plan not in plans:
             plans.append(plan)
     return plans
 
 
 def _gated_timing(key, operands, device):
-    _, rows, _, in_features, _, _ = key
+    rows, _, in_features, _, _, _, bounds = _gated_key(key)
     x = (torch.randn((rows, in_features), device=device) * 0.5).to(torch.bfloat16)
-    return lambda plan, i: run_gated_plan(plan, x, operands[i][0])
+    return lambda plan, i: run_gated_plan(plan, x, operands[i][0], bounds)
 
 
 autotune.register_kind("gated", gated_candidates, _gated_timing)

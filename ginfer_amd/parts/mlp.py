@@ -5,7 +5,7 @@ from ..kernels import ops
 from ..kernels.tuning import TUNING
 from ..weights.loader import WeightSpec
 from .base import Part
-from .linear import linear, gated_linear, gated_plan, linear_into_norm, tiles_gated
+from .linear import linear, gated_linear, linear_into_norm
 from .registry import register_feed_forward
 
 
@@ -74,15 +74,7 @@ class ClampedGLU(Part):
         return ["activation", "gemm"] + (["gemm_skinny", "gemm_tiles"] if self.dtype == torch.bfloat16 else [])
 
     def forward(self, x, parts_ok=False):
-        # few rows (decode): the weight-streaming product with the activation in its epilogue, where the rules would
-        # take that kernel for the SiLU gate too; else the product and the activation's own pass
-        if tiles_gated(x, self.w_gate_up):
-            act = ops.gemm_tiles_gated(x, self.w_gate_up, bounds=(self.limit, self.alpha, self.shift))
-        elif (x.dtype == torch.bfloat16 and ops.gemm_skinny_supported(x, self.w_gate_up)
-                and gated_plan(x.shape[0], self.w_gate_up.shape[0], True, False) == ("skinny",)):
-            act = ops.gemm_skinny(x, self.w_gate_up, gated=True, gate_bounds=(self.limit, self.alpha, self.shift))
-        else:
-            act = ops.clamped_glu(linear(x, self.w_gate_up), self.limit, self.alpha, self.shift)
+        act = gated_linear(x, self.w_gate_up, bounds=(self.limit, self.alpha, self.shift))
         return linear(act, self.w_down, parts_ok=parts_ok)
 
 

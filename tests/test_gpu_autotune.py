@@ -59,14 +59,19 @@ def test_every_candidate_plan_of_the_gated_product(rows, n, k):
     # the plain statement rounds the products to bfloat16 before the activation only where the kernels do; compare in
     # 64-bit with a tolerance of two roundings
     ref = gate * torch.sigmoid(gate) * up
-    key = ("gated", rows, 2 * n, k, ops.gemm_skinny_supported(x, w), L._transposable(x, w))
-    plans = L.gated_candidates(key)
-    assert len(plans) >= 2
-    for plan in plans:
-        y = L.run_gated_plan(plan, x, w)
-        assert y.shape == (rows, n) and y.dtype == torch.bfloat16
-        err = float((y.double().cpu() - ref).abs().max() / ref.abs().max())
-        assert err <= 1.2e-2, "plan %s: %.3g" % (plan, err)
+    bounds = (1.5, 1.702, 1.0)
+    bounded = torch.clamp(gate, max=bounds[0])
+    bounded = bounded * torch.sigmoid(bounds[1] * bounded) * (torch.clamp(up, -bounds[0], bounds[0]) + bounds[2])
+    for limits, want in ((None, ref), (bounds, bounded)):
+        key = ("gated", rows, 2 * n, k, ops.gemm_skinny_supported(x, w), limits is None and L._transposable(x, w),
+               ops.gemm_tiles_supported(x, w), limits)
+        plans = L.gated_candidates(key)
+        assert len(plans) >= 2 and (("tiles",) in plans) == (k % 64 == 0)
+        for plan in plans:
+            y = L.run_gated_plan(plan, x, w, limits)
+            assert y.shape == (rows, n) and y.dtype == torch.bfloat16
+            err = float((y.double().cpu() - want).abs().max() / want.abs().max())
+            assert err <= 1.2e-2, "plan %s: %.3g" % (plan, err)
 
 
 def test_a_runner_that_times_its_plans(tmp_path):

@@ -1034,6 +1034,21 @@ def test_gated_product_over_tiles(M, cols, K):
         assert bool((off <= ref.abs() / 256 + 1e-3 * ref.pow(2).mean().sqrt()).all()), "%r: %g" % (bounds, float(off.max()))
 
 
+@pytest.mark.parametrize("tiling", range(5))
+@pytest.mark.parametrize("M,cols,K", [(1, 8, 64), (63, 64, 128), (65, 72, 192), (127, 136, 256), (129, 128, 320), (257, 264, 640)])
+def test_gated_product_in_every_tiling(tiling, M, cols, K):
+    """One row or eight columns more or less than each tiling holds, K of one slab to ten (more than any has buffers): the same
+    sums as in the others, so the same bits; against 64 bits as above."""
+    from ginfer_amd.kernels import ops
+    a, w = rnd((M, K), torch.bfloat16, 53), rnd((2 * cols, K), torch.bfloat16, 54)
+    g, u = (a.double() @ w.double().t()).split(cols, dim=1)
+    ref = g * torch.sigmoid(g) * u
+    got = ops.gemm_tiles_gated(a, w, tiling=tiling)
+    assert torch.equal(got, ops.gemm_tiles_gated(a, w, tiling=0))
+    off = (got.double() - ref).abs()
+    assert bool((off <= ref.abs() / 256 + 1e-3 * ref.pow(2).mean().sqrt()).all()), float(off.max())
+
+
 @pytest.mark.parametrize("M", [1, 63, 64, 65, 127, 256, 300])
 @pytest.mark.parametrize("N,K,parts", [(16, 64, 1), (80, 192, 3), (144, 320, 2), (1536, 640, 5), (64, 832, 13)])
 def test_product_over_tiles_in_parts(M, N, K, parts):
@@ -1057,6 +1072,9 @@ def test_products_over_tiles_refuse_what_they_do_not_take():
         assert not ops.gemm_tiles_supported(x, y)
         with pytest.raises(ops.KernelError):
             ops.gemm_tiles_gated(x, y)
+    for tiling in (-1, 5):
+        with pytest.raises(ops.KernelError):
+            ops.gemm_tiles_gated(a, w, tiling=tiling)
     for parts in (0, 3):
         with pytest.raises(ops.KernelError):
             ops.gemm_tiles_parts(a, w, parts)

@@ -108,6 +108,53 @@ def test_the_tuner_starts_from_the_plan_that_runs():
     assert L.linear_candidates(("linear", 64, 3072, 8192, False, False, True, True, True))[0] == ("tiles", 1, 5)
 
 
+def test_tiles_of_the_gated_product():
+    """Which tiles a number of rows gets, and that the rule counts those: one place says it for both."""
+    from ginfer_amd.kernels import ops
+    tiles = lambda rows, n: ops.GATED_TILINGS[ops.gated_tiling(rows, n)]
+    assert tiles(17, 17920) == tiles(64, 17920) == (128, 64) and tiles(64, 37888) == (256, 128)
+    assert tiles(65, 17920) == tiles(128, 32768) == (128, 128) and tiles(128, 32770) == (256, 128)
+    assert tiles(129, 16384) == (128, 128) and tiles(129, 17920) == tiles(256, 37888) == (128, 256)
+    assert tiles(384, 8192) == (128, 128) and tiles(257, 17920) == tiles(1024, 17920) == (256, 128)
+    assert tiles(1025, 17920) == tiles(4096, 17920) == (256, 256)
+    for rows in range(1, 2100, 7):
+        for n in (16, 8192, 17920, 37888, 70000):
+            of_w, of_a = tiles(rows, n)
+            assert of_a >= min(rows, 64) and (rows > 384 or of_a < 2 * rows or of_a == 64 or of_w == of_a == 128 or of_w == 256)
+
+
+def test_gated_products_over_tiles_at_their_thresholds():
+    """The sizes the rule was measured at: taken where the kernel was the faster, refused where the library was."""
+    g = lambda rows, n, k: L.tiles_gated(rows, n, k)
+    assert not g(16, 17920, 1536) and g(17, 17920, 1536) and g(64, 8192, 1024)
+    assert not g(64, 8184, 1024) and not g(64, 8192, 1016) and not g(64, 12288, 3072) and not g(128, 10240, 1792)
+    assert all(g(rows, n, k) for rows in (65, 96, 128) for n, k in ((17920, 1536), (22016, 2048), (27648, 5120), (28672, 4096),
+                                                                     (19456, 2560), (16384, 1280), (37888, 3584), (59136, 8192)))
+    # two rounds of the chip beside few rows: the library
+    assert not g(129, 37888, 3584) and not g(256, 59136, 8192) and not g(128, 65792, 4096)
+    assert g(256, 17920, 1536) and g(256, 12288, 3072) and g(256, 27648, 5120)
+    # up to 384 rows full rounds, or a short K: the sizes where it had become up to 27 % slower than the library are refused
+    assert g(300, 17920, 1536) and g(384, 37888, 3584) and g(300, 10240, 1792) and g(384, 19456, 2560)
+    assert not any(g(rows, n, k) for rows in (257, 300, 384) for n, k in ((22016, 2048), (27648, 5120), (28672, 4096), (59136, 8192)))
+    # ... and around 1,000 rows up to 20 %
+    assert g(1000, 37888, 3584) and g(1024, 37888, 3584) and g(1000, 8192, 1024)
+    assert not any(g(1000, n, k) for n, k in ((22016, 2048), (27648, 5120), (28672, 4096), (59136, 8192), (16384, 1280), (10240, 1792)))
+    assert not any(g(rows, 17920, 1536) for rows in (385, 512, 700, 1000, 1025, 1500, 2048))
+    # by the tiles that run: 256 x 256 from 1,025 rows on
+    assert g(1025, 37888, 3584) and g(1280, 37888, 3584) and not g(1281, 37888, 3584) and not g(1536, 37888, 3584)
+    assert g(1700, 17920, 1536) and g(2048, 37888, 3584) and not g(2049, 37888, 3584)
+
+
+def test_the_gated_product_is_one_plan_of_several():
+    """The tuner starts from the plan that runs, can leave it, and tries tiles where the rule does not take them."""
+    key = lambda rows, n, k, tiles_ok=True, bounds=None: ("gated", rows, n, k, rows <= 64, bounds is None and rows % 8 == 0, tiles_ok, bounds)
+    assert L.gated_candidates(key(64, 17920, 1536)) == [("tiles",), ("skinny",), ("library",), ("transposed",)]
+    assert L.gated_candidates(key(512, 17920, 1536)) == [("transposed",), ("library",), ("tiles",)]
+    assert L.gated_candidates(key(300, 17920, 1536, False)) == [("library",)]
+    assert L.gated_candidates(key(100, 17920, 1536, True, (7.0, 1.702, 1.0))) == [("tiles",), ("library",)]
+    assert L.gated_plan(64, 17920, True, True, 1536, True) == ("tiles",) and L.gated_plan(64, 17920, True, True, 1536, False) == ("library",)
+
+
 def test_measured_plans_can_be_set_from_json():
     from ginfer_amd.kernels.tuning import Tuning
     t = Tuning()
