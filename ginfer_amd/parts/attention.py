@@ -86,7 +86,7 @@ class Attention(Part):
     def kernel_modules(self):
         mods = ["rope_kv", "attention_generic", "gemm"]
         if self.dtype == torch.bfloat16:
-            mods += ["gemm_skinny"]
+            mods += ["gemm_skinny", "gemm_tiles"]
             if self.hd in ops.MFMA_HEAD_DIMS:
                 mods += [("attention_mfma", {"HEAD_DIM": self.hd})]
         return mods

@@ -147,7 +147,7 @@ class ConvAttention(Part):
     def kernel_modules(self):
         mods = ["conv_rope_kv", "attention_generic", "gemm"]
         if self.dtype == torch.bfloat16:
-            mods += ["gemm_skinny"]
+            mods += ["gemm_skinny", "gemm_tiles"]
             if self.padded in ops.MFMA_HEAD_DIMS:
                 mods += [ops.attention_mfma_module(self.padded, self.soft_cap is not None)]
         return mods

@@ -36,7 +36,7 @@ class _DeltaMixer(Part):
         return [StateSpec(ops.delta_state_shape(self.nh, self.dk, self.dv), torch.float32), ring]
 
     def kernel_modules(self):
-        return ["delta_scan", "decay_scan", "gemm"] + (["delta_chunk", "gemm_skinny"] if self.dtype == torch.bfloat16 else [])
+        return ["delta_scan", "decay_scan", "gemm"] + (["delta_chunk", "gemm_skinny", "gemm_tiles"] if self.dtype == torch.bfloat16 else [])
 
     def _recurrence(self, proj, step, cache, **kw):
         state, ring = cache

@@ -49,7 +49,7 @@ class _DecayedLinearAttention(Part):
                 "o": WeightSpec((H, v))}
 
     def kernel_modules(self):
-        return ["decay_scan", "gemm"] + (["gemm_skinny"] if self.dtype == torch.bfloat16 else [])
+        return ["decay_scan", "gemm"] + (["gemm_skinny", "gemm_tiles"] if self.dtype == torch.bfloat16 else [])
 
     # column blocks of the stacked projection
     @property

@@ -186,7 +186,7 @@ class RoutedGLU(Part):
         self.w_down = torch.cat([t[n + ".down"] for n in names], dim=1).contiguous()
 
     def kernel_modules(self):
-        return ["routing", "activation", "gemm"] + (["gemm_skinny", "expert_gemm"] if self.dtype == torch.bfloat16 else [])
+        return ["routing", "activation", "gemm"] + (["gemm_skinny", "gemm_tiles", "expert_gemm"] if self.dtype == torch.bfloat16 else [])
 
     def route(self, x, own_out=None):
         """(ids int32 [T, top_k], weights float32 [T, top_k], the weights as rows over all experts that have tensors [T, E]);

@@ -66,7 +66,7 @@ class ParallelSum(Part):
         self.w_out = torch.cat(outs, dim=1).contiguous()
 
     def kernel_modules(self):
-        mods = ["activation", "gemm"] + (["gemm_skinny"] if self.dtype == torch.bfloat16 else [])
+        mods = ["activation", "gemm"] + (["gemm_skinny", "gemm_tiles"] if self.dtype == torch.bfloat16 else [])
         for b in self.branches:
             mods += [m for m in b.kernel_modules() if m not in mods]
         return mods

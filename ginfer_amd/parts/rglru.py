@@ -58,7 +58,7 @@ class RecurrentBlock(Part):
         self.w_o = t["o"]
 
     def kernel_modules(self):
-        return ["rglru", "short_conv", "gemm"] + (["gemm_skinny"] if self.dtype == torch.bfloat16 else [])
+        return ["rglru", "short_conv", "gemm"] + (["gemm_skinny", "gemm_tiles"] if self.dtype == torch.bfloat16 else [])
 
     def forward(self, x, step, cache):
         state, conv = cache
