@@ -105,10 +105,18 @@ class Tuning:
     # ... and the product whose parts of K the norm adds: K of at least `tiles_parts_min_in_features`, at most
     # `library_split_max_out_features` columns, beyond `library_from_rows` rows up to so many, in as many parts as keep to
     # `tiles_parts_workgroups` workgroups; with more than 64 rows not where K is so long beside that many columns that the tiles'
-    # rows of A are most of what is read (3,584 columns of 18,944 at 256 rows: the library's 59 us against 80)
+    # rows of A are most of what is read (3,584 columns of 18,944 at 256 rows: the library's 59 us against 80), with the most rows
+    # from fewer weights on (beyond `tiles_parts_many_rows`; 2,560 columns of 9,728 at 256 rows 37.7 against 41.6, at 192 47.4
+    # against 35.3); and with the fewest rows not a few columns, which the streaming kernel splits as well (896 of 4,864: 17 rows
+    # 11.5 against 13.0, 33 rows 13.5 and 13.3).  Twelve matrices at 17 to 256 rows, product and norm: at worst 4 % more than the
+    # best other way (2,048 columns of 8,192 at 224 rows), up to 54 % less (2,560 of 9,728 at 64).
     tiles_parts_min_in_features: int = 3072
     tiles_parts_most_rows: int = 256
+    tiles_parts_few_rows: int = 32
+    tiles_parts_few_rows_min_out_features: int = 1024
+    tiles_parts_many_rows: int = 224
     tiles_parts_most_weights_many_rows: int = 32 << 20
+    tiles_parts_most_weights_most_rows: int = 23 << 20
     tiles_parts_workgroups: int = 256
     # ---- the fused q|k|v projection + rotation + cache write (parts/attention.py): from more rows than this and a K
     # of at least that, the library's product followed by the rotation kernel is faster (the fused kernel cannot split K).

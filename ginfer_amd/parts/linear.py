@@ -44,7 +44,10 @@ def tiles_parts(rows, out_features, in_features):
     if out_features > T.library_split_max_out_features or out_features % 16 or in_features % 64:
         return 0
     few = rows <= ops.SKINNY_MAX_ROWS
-    if not few and out_features * in_features > T.tiles_parts_most_weights_many_rows:
+    if out_features < T.tiles_parts_few_rows_min_out_features and rows <= T.tiles_parts_few_rows:
+        return 0
+    most = T.tiles_parts_most_weights_many_rows if rows <= T.tiles_parts_many_rows else T.tiles_parts_most_weights_most_rows
+    if not few and out_features * in_features > most:
         return 0
     tiles = -(-out_features // (64 if few else 128)) * -(-rows // 64)
     slabs = in_features // 64

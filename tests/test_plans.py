@@ -81,6 +81,8 @@ def test_products_over_tiles_in_parts_of_k():
     assert plan(64, 1536, 1536) == ("skinny", 1, 2) and plan(64, 4112, 8960)[0] == "library"
     assert plan(64, 1528, 8960) == ("skinny", 4, 10)                # 1,528 columns are no multiple of 16
     assert plan(65, 3584, 18944) == ("library", 8)                  # the rows of A are most of what is read
+    assert plan(256, 2560, 9728) == ("library", 8) and plan(224, 2560, 9728)[0] == "tiles"
+    assert plan(32, 896, 4864) == ("skinny", 1, 4) and plan(33, 896, 4864) == ("tiles", 1, 9)       # few rows, few columns
     assert plan(64, 3584, 18944, parts_ok=False)[0] == "skinny" and plan(64, 3584, 18944, has_bias=True)[0] == "skinny"
     assert plan(64, 3584, 18944, f32=True)[0] == "skinny"
     assert L._parts_without_gaps(140, 10) == 10 and L._parts_without_gaps(9, 4) == 3 and L._parts_without_gaps(12, 5) == 4
