@@ -836,10 +836,11 @@ PREFILL_SHARED_DIMS = (64, 128, 256)     # head sizes with the prefill kernel th
 
 def _prefill_fill(step, head_dim):
     """How many workgroups a step's prompt rows have to make for heads to share them: fewer where that shares the operands
-    through LDS too and the tiles are all a prompt's (a recorded step's count holds padding)."""
-    if head_dim not in PREFILL_SHARED_DIMS or "static_plan" in (step.extra or {}):
+    through LDS too, which pays with wide heads, and the tiles are all a prompt's (a recorded step's count holds padding)."""
+    part = {128: TUNING.prefill_fill_real_tiles, 256: TUNING.prefill_fill_real_tiles_256}.get(head_dim)
+    if part is None or "static_plan" in (step.extra or {}):
         return TUNING.prefill_fill_workgroups
-    return max(1, int(TUNING.prefill_fill_workgroups * TUNING.prefill_fill_real_tiles))
+    return max(1, int(TUNING.prefill_fill_workgroups * part))
 
 
 def _prefill_workgroups(step, tile_rows, group, nkv, head_dim, window):

@@ -140,12 +140,17 @@ class Tuning:
     # workgroups; among the groupings that do, the one with the most heads that still makes `prefill_prefer_workgroups`
     # (one and a half rounds of the chip), else the one with the fewest heads
     prefill_fill_workgroups: int = 256
-    # ... and only so much of that where the sharing goes through LDS and the tiles are all a prompt's: one kv head's keys and
-    # values are then read once for all its heads.  Whole steps of the 7B shape (7 heads to a kv head: all or one), us, at 256 ->
-    # 128 workgroups: 2,000 tokens behind 2,048 beside 48 single ones (252 workgroups) 31,897 -> 28,487; 600 behind 3,000 (152)
-    # 15,465 -> 13,548; 1,000 alone (252) 16,105 -> 15,452.  Recorded steps count padding among their tiles and keep the full
-    # number: 256 rows behind 8,000 of the 1.5B shape, 96 workgroups with a row of their own, 5,250 -> 6,100.
-    prefill_fill_real_tiles: float = 0.5
+    # ... and, by head size, only so much of that where the sharing goes through LDS and the tiles are all a prompt's: one kv head's
+    # keys and values are then read once for all its heads.  Attention, us, at 256 -> so many workgroups, heads/kv heads: of 128,
+    # 28/4, 600 tokens alone 33.6 -> 24.9, behind 8,000 374 -> 213; 12/2, 520 alone 17.8 -> 16.4, 600 behind 8,000 156 -> 119; 16/2,
+    # 300 alone 14.5 -> 13.1; 64/8 and 32/8 at 300 to 1,500 tokens, and what makes 256 workgroups anyway, level.  Of 256 at half
+    # the number: 16/8, 300 alone 25.3 -> 21.3, but 8/2, 520 alone 25.0 -> 27.3; at three quarters the first is left and the second
+    # too, 800 alone 35.5 -> 35.0, 600 behind 8,000 (176 workgroups) is left at 302, 1,000 behind 8,000 316 -> 276.  Of 64 nothing is
+    # gained anywhere: 12/1, 520 alone 12.7 -> 13.4.  Whole steps of the 7B shape: 2,000 tokens behind 2,048 beside 48 single ones
+    # (252 workgroups) 31,897 -> 28,487.  Recorded steps count padding among their tiles and keep the full number: 256 rows
+    # behind 8,000 of the 1.5B shape, 96 workgroups with a row of their own, 5,250 -> 6,100.
+    prefill_fill_real_tiles: float = 0.5             # heads of 128
+    prefill_fill_real_tiles_256: float = 0.75        # heads of 256
     prefill_prefer_workgroups: int = 384
     # The keys of a step's heaviest prompt tiles can be dealt to several workgroups (merged by a second kernel): when the
     # step makes at most `prefill_split_max_workgroups` workgroups, the heaviest tile's walk is at least

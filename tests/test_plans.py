@@ -236,6 +236,19 @@ def test_kept_plans_answer_for_their_class_of_rows():
     assert not autotune.active()
 
 
+def test_how_many_workgroups_heads_share_a_prompts_tiles_from():
+    """Fewer than a round of the chip where the heads are wide and the tiles a prompt's own; small heads, other sizes and
+    recorded steps, whose tiles hold padding, wait for the full number."""
+    import types
+    from ginfer_amd.kernels import ops
+    own, none, recorded = (types.SimpleNamespace(extra=e) for e in ({}, None, {"static_plan": {}}))
+    full = ops.TUNING.prefill_fill_workgroups
+    assert ops._prefill_fill(own, 128) == ops._prefill_fill(none, 128) == full // 2
+    assert ops._prefill_fill(own, 256) == full * 3 // 4
+    assert ops._prefill_fill(own, 64) == ops._prefill_fill(own, 112) == full
+    assert all(ops._prefill_fill(recorded, d) == full for d in (64, 128, 256))
+
+
 def test_keys_of_a_short_prompt_are_dealt_out_and_those_of_other_steps_are_not(monkeypatch):
     """The rule that deals a tile's keys to several workgroups: one prompt of 2,048 tokens alone in a step (one round of
     workgroups, the last tile walking twice the mean) is split, every part within the mean share, the parts of a tile
