@@ -95,12 +95,14 @@ class Engine:
 
     def _warm_up(self):
         """Prompt portions of several lengths (the library picks other kernels for other numbers of rows, and loads each
-        at its first use), then decoded tokens, with sampling, through the model's own step; the request is given
-        back afterwards and leaves nothing behind (it is admitted without its tokens, so no page of it is remembered)."""
+        at its first use), then decoded tokens, with sampling, through the model's own step; short portions also beside a
+        request of a single token, as they arrive while others are answered: that is another recorded step.  The requests
+        are given back afterwards and leave nothing behind (they are admitted without their tokens, so no page of them is
+        remembered)."""
         runner, cfg = self.runner, self.config
         room = min(runner.max_model_len - 3, cfg.max_num_batched_tokens,
                    min(g.pool.num_free for g in runner.cache.groups) * runner.page_size - 3 if runner.cache.groups else 1 << 30)
-        rid = ("warm-up",)
+        rid, other = ("warm-up",), ("warm-up", "beside")
         greedy = [SamplingParams()]
         try:
             done = set()
@@ -120,9 +122,16 @@ class Engine:
                             logits = runner.step([StepEntry(rid, [0], [0])], borrow=True)
                             self.sampler.sample_on_device(logits, greedy, [0])
                     runner.release(rid)
+                beside = n > 1 and n + runner.page_size <= room and cfg.max_num_seqs > 1
+                for _ in range(runs if beside and n < TUNING.warmup_record_below else 0):
+                    logits = runner.step([StepEntry(rid, [0] * n, [n - 1]), StepEntry(other, [0], [0])], borrow=True)
+                    self.sampler.sample_on_device(logits, greedy * 2, [0, 0])
+                    runner.release(rid)
+                    runner.release(other)
             torch.cuda.synchronize()
         finally:
             runner.release(rid)
+            runner.release(other)
 
     def add_request(self, prompt_token_ids, params: Optional[SamplingParams] = None):
         params = params or SamplingParams()

@@ -145,7 +145,7 @@ class Tuning:
     # 28/4, 600 tokens alone 33.6 -> 24.9, behind 8,000 374 -> 213; 12/2, 520 alone 17.8 -> 16.4, 600 behind 8,000 156 -> 119; 16/2,
     # 300 alone 14.5 -> 13.1; 64/8 and 32/8 at 300 to 1,500 tokens, and what makes 256 workgroups anyway, level.  Of 256 at half
     # the number: 16/8, 300 alone 25.3 -> 21.3, but 8/2, 520 alone 25.0 -> 27.3; at three quarters the first is left and the second
-    # too, 800 alone 35.5 -> 35.0, 600 behind 8,000 (176 workgroups) is left at 302, 1,000 behind 8,000 316 -> 276.  Of 64 nothing is
+    # too, 800 alone 35.5 -> 35.0, 600 behind 8,000 (152 workgroups) is left at 302, 1,000 behind 8,000 316 -> 276.  Of 64 nothing is
     # gained anywhere: 12/1, 520 alone 12.7 -> 13.4.  Whole steps of the 7B shape: 2,000 tokens behind 2,048 beside 48 single ones
     # (252 workgroups) 31,897 -> 28,487.  Recorded steps count padding among their tiles and keep the full number: 256 rows
     # behind 8,000 of the 1.5B shape, 96 workgroups with a row of their own, 5,250 -> 6,100.
@@ -210,8 +210,8 @@ class Tuning:
     graph_keep: int = 128
     # ---- the engine's warm-up (engine/engine.py): prompt portions of these lengths run once before the first request
     # (the BLAS library picks other kernels for other numbers of rows and loads each at its first use); the ones under
-    # `warmup_record_below` run three times, so that the padded step a lone prompt of about that length is laid into is
-    # recorded and replayed before a request pays for it
+    # `warmup_record_below` run three times, and three times beside a single token, so that the padded steps that a prompt of
+    # about that length is laid into, alone and beside requests that decode, are recorded and replayed before a request pays for it
     warmup_portion_lengths: tuple = (2048, 1024, 512, 400, 256, 160, 96, 48, 8)
     warmup_record_below: int = 512
 

@@ -1005,3 +1005,25 @@ def test_the_pool_is_planned_from_free_memory_after_the_largest_step(folders, mo
     _greedy_as_plain(folders["C"], prompts, outs, "float32")
     eng.runner.cache.check()
     assert all(g.pool.num_free == g.pool.num_pages for g in eng.runner.cache.groups)
+
+
+def test_the_warm_up_records_portions_alone_and_beside_single_tokens(folders):
+    """The first short portion that a request brings finds its padded step recorded, alone in a step and beside requests
+    that decode (two recorded steps); nothing of the warm-up's requests is left."""
+    from ginfer_amd import Engine, EngineConfig, StepEntry
+    eng = Engine(EngineConfig(model_path=folders["A"], dtype="bfloat16", max_num_batched_tokens=128, max_num_seqs=4,
+                              max_seq_len=256, kvcache_block_size=16, num_kvcache_blocks=64))
+    runner = eng.runner
+    assert not runner.cache.has(("warm-up",)) and not runner.cache.has(("warm-up", "beside"))
+    before = dict(runner.counts)
+    runner.step([StepEntry("a", [5] * 20, [19])])
+    assert runner.counts["replayed_padded"] == before["replayed_padded"] + 1 and runner.counts["recorded"] == before["recorded"]
+    runner.step([StepEntry("a", [7], [0]), StepEntry("b", [9] * 30, [29])])
+    assert runner.counts["replayed_padded"] == before["replayed_padded"] + 2 and runner.counts["recorded"] == before["recorded"]
+    runner.release("a")
+    runner.release("b")
+    runner.cache.check()
+    # a server of one request at a time, and a pool with no page to spare, warm up as before
+    for kw in (dict(max_num_seqs=1, num_kvcache_blocks=64), dict(max_num_seqs=4, num_kvcache_blocks=2)):
+        Engine(EngineConfig(model_path=folders["A"], dtype="bfloat16", max_num_batched_tokens=128, max_seq_len=32,
+                            kvcache_block_size=16, **kw)).runner.cache.check()
