@@ -408,9 +408,7 @@ class ModelRunner:
         if R > e_pad:
             return None
         bucket = _context_bucket(host["max_kv"])
-        # a step of prompt portions alone gets no records of single tokens, so that nothing is launched for them (two kernels
-        # a layer over padding: 10.6 us of 115 in a step of 161 tokens at the 1.5B shape)
-        n_single = e_pad if len(host["decode_info"]) else 0
+        n_single = single_records(T, t_pad, e_pad, len(host["decode_info"]))
         key = ("padded", t_pad, e_pad, bucket, n_single)
         g = self._graphs.pop(key, None)
         if g is not None:
@@ -548,6 +546,14 @@ def reserve_for_step(cache, entries, max_model_len, reserved):
         elif cache.pending(e.request_id) != len(e.tokens):
             raise ValueError("request %r has %d tokens reserved but brings %d"
                              % (e.request_id, cache.pending(e.request_id), len(e.tokens)))
+
+
+def single_records(T, t_pad, e_pad, n_decode):
+    """Records of single tokens in a padded step of T tokens, `n_decode` of them single ones.  A step of prompt portions alone gets
+    none, so that nothing is launched for them (two kernels a layer over padding: 10.6 us of 115 in a step of 161 tokens at the
+    1.5B shape); unless its padding is one row: that entry's one token is a single token too, and a kernel for portions that
+    leaves those out would leave the row as it was allocated."""
+    return e_pad if n_decode or t_pad == T + 1 else 0
 
 
 def pad_step(host, t_pad, e_pad, width, pad_slot, n_single=None):

@@ -2,7 +2,7 @@
 import numpy as np
 import pytest
 
-from ginfer_amd.engine.runner import ModelRunner, pad_step
+from ginfer_amd.engine.runner import ModelRunner, pad_step, single_records
 from ginfer_amd.kernels import ops
 
 
@@ -87,3 +87,14 @@ def test_a_step_of_portions_alone_gets_no_records_of_single_tokens():
     assert p["decode_info"].shape == (0, 4)
     full = pad_step(host, 64, 8, 16, pad_slot=99)
     assert all(np.array_equal(p[k], full[k]) for k in ("ids", "pos", "ent", "cu", "q_len", "rows", "tiles", "state_slots"))
+
+
+def test_padding_of_one_row_has_a_record_of_its_own():
+    """An entry of one token is left out by kernels for portions: the row behind 63 tokens of portions is covered by the
+    records of single tokens, longer paddings by the portions' own way."""
+    assert single_records(62, 64, 8, 0) == 0 and single_records(100, 128, 16, 0) == 0
+    assert single_records(63, 64, 8, 0) == 8 and single_records(127, 128, 16, 0) == 16
+    assert single_records(40, 64, 8, 1) == 8 and single_records(63, 64, 8, 3) == 8
+    host = host_arrays([40, 23], [0, 16])
+    p = pad_step(host, 64, 8, 16, pad_slot=99, n_single=single_records(63, 64, 8, 0))
+    assert p["decode_info"].shape == (8, 4) and (p["decode_info"][:, 0] == 63).all() and p["q_len"][8] == 1
