@@ -19,7 +19,7 @@
 //   many rows  a workgroup takes 256 rows of the weight matrix by 64, 128 or 256 of the tile's rows, both brought into LDS in
 //              slabs of K, a slab ahead
 // A row's result does not depend on the rows beside it, and every sum has an order that depends on K alone.
-#include "common.h"
+#include "lds_load.h"
 #include "ginfer_amd.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
@@ -245,17 +245,6 @@ __global__ __launch_bounds__(KW * WAVE) void expert_few_kernel(void* __restrict_
 // memory into LDS, the next one on its way while one is multiplied.  A slab's rows are 128 bytes, eight 16-byte pieces; piece q
 // of row r lies at place q ^ (r & 7), so that the rows an operand reads lie in different banks.  K a multiple of 32 (the last slab may
 // be half a slab).
-typedef __attribute__((address_space(3))) unsigned char lds_byte_t;
-
-// 1 KB from memory into LDS, 16 bytes a lane from the lane's own address; the place is the same for all lanes.  Written out
-// because the compiler makes every LDS read wait for loads of this kind that are under way, also where they fill another
-// buffer; the loop below waits for them itself.  (s_nop: the place register must rest a cycle before it is read.)
-__device__ __forceinline__ void et_bring(uint32_t place, const bf16_t* src) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(place), "v"(src) : "memory");
-}
-// the wavefront's own loads are in, its LDS reads are through; then all meet
-__device__ __forceinline__ void et_wait_and_meet() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 #define ET_SLAB 64
 template <int MATS, int WN>
 __global__ __launch_bounds__(128 * WN, (WN == 1 ? 1 : 2)) void expert_many_kernel(
@@ -310,11 +299,11 @@ __global__ __launch_bounds__(128 * WN, (WN == 1 ? 1 : 2)) void expert_many_kerne
     // in a last slab of 32 the pieces behind K stand in for nothing: the ones before are brought twice
     const int back = (half && s == slabs - 1 && piece >= 4) ? 32 : 0;
 #pragma unroll
-    for (int j = 0; j < LOADS; ++j) et_bring(place + j * 1024, src[j] + (int64_t)s * ET_SLAB - back);
+    for (int j = 0; j < LOADS; ++j) lds_bring(place + j * 1024, src[j] + (int64_t)s * ET_SLAB - back);
   };
   bring(0);
   for (int s = 0; s < slabs; ++s) {
-    et_wait_and_meet();                   // slab s is in, and nobody reads the other buffer any more
+    lds_wait_and_meet();                   // slab s is in, and nobody reads the other buffer any more
     if (s + 1 < slabs) bring(s + 1);
     const unsigned char* cur = lds + (s & 1) * SLAB_BYTES;
     // a wavefront whose rows lie behind the tile's last has nothing to multiply: a group's last tile is often a short one

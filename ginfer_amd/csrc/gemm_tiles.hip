@@ -15,23 +15,13 @@
 //
 // What bounds it: many rows, the chip's power (products of random numbers run at 1,700 to 1,800 TFLOP/s, 2,400 of zeros) and the
 // way of a slab from memory; few rows, the weights' way from memory.
-#include "common.h"
+#include "lds_load.h"
 #include <type_traits>
 #include "ginfer_amd.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
-typedef __attribute__((address_space(3))) unsigned char lds_byte_t;
-
-// 1 KB from memory into LDS, 16 bytes a lane from `base` plus the lane's own offset; the place is the same for all lanes.
-// Written out because the compiler makes every LDS read wait for loads of this kind that are under way, also where they fill
-// another buffer; gt_wait_and_meet waits for all but the N youngest of them.  (s_nop: the place register must rest a cycle.)
-__device__ __forceinline__ void gt_bring(uint32_t place, uint32_t at, const void* base) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(place), "v"(at), "s"(base) : "memory");
-}
-template <int N>
-__device__ __forceinline__ void gt_wait_and_meet() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory"); }
 
 // act.kind 0: SiLU(v) * u; 1: g * sigmoid(alpha g) * (u + shift), g = min(v, limit), u = clamp(u, -limit, limit); 2: the same
 // with the sigmoid's limit, a step.  exp2 and the reciprocal are the hardware's: against 64 bits SiLU is off by at most 3 units of
@@ -99,8 +89,8 @@ __global__ __launch_bounds__(64 * WN * WM, 1) void gemm_tiles_kernel(
   const char* ap = reinterpret_cast<const char*>(A) + (int64_t)slab0 * ROW;
   uint32_t fill = base;                           // the buffer that the next slab goes to
   auto bring_one = [&](int j) {
-    if (j < LW) gt_bring(fill + (wave * LW + j) * 1024, src_w[j], wp);
-    else gt_bring(fill + TN * ROW + (wave * LA + j - LW) * 1024, src_a[j - LW], ap);
+    if (j < LW) lds_bring_from(fill + (wave * LW + j) * 1024, src_w[j], wp);
+    else lds_bring_from(fill + TN * ROW + (wave * LA + j - LW) * 1024, src_a[j - LW], ap);
   };
   auto brought = [&]() {
     wp += ROW;
@@ -153,21 +143,21 @@ __global__ __launch_bounds__(64 * WN * WM, 1) void gemm_tiles_kernel(
       for (int j = 0; j < LOADS; ++j) bring_one(j);
       brought();
     }
-  if (slabs >= NBUF) gt_wait_and_meet<(NBUF - 1) * LOADS>();
-  else gt_wait_and_meet<0>();
+  if (slabs >= NBUF) lds_wait_and_meet<(NBUF - 1) * LOADS>();
+  else lds_wait_and_meet<0>();
 #pragma unroll
   for (int y = 0; y < READS; ++y) read_one(0, y);
   int s = 0;
   for (; s + NBUF < slabs; ++s) {
     half_slab(0, std::false_type());
-    gt_wait_and_meet<(NBUF - 2) * LOADS>();
+    lds_wait_and_meet<(NBUF - 2) * LOADS>();
     cur = cur == lds + (NBUF - 1) * SLAB ? lds : cur + SLAB;
     half_slab(1, std::true_type());
     brought();
   }
   for (; s < slabs; ++s) {
     half_slab(0, std::false_type());
-    gt_wait_and_meet<0>();
+    lds_wait_and_meet<0>();
     cur = cur == lds + (NBUF - 1) * SLAB ? lds : cur + SLAB;
     half_slab(1, std::false_type());
   }

@@ -14,7 +14,7 @@
 // gate logits, and the write of c into its page.
 // latent_turned_prepare: the same for rows with a turned key part: RMS norm of the latent, the rotation of the key part and
 // of every head's query part, and the write of the row into its page.
-#include "common.h"
+#include "lds_load.h"
 #include "ginfer_amd.h"
 
 #define LA_MAX_HEADS_PER_WG 8
@@ -313,7 +313,6 @@ extern "C" int ga_latent_attention(void* out, int64_t out_t, int64_t out_h, cons
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(4))) short s16x4;
-typedef __attribute__((address_space(3))) unsigned char lds_byte_t;
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4_t;
 
 #define LT_LOG2E 1.4426950408889634f
@@ -331,15 +330,6 @@ __device__ __forceinline__ bf16x8 lt_pack8(const float* v) {
   return __builtin_bit_cast(bf16x8, make_uint4(w[0], w[1], w[2], w[3]));
 }
 __device__ __forceinline__ int lt_swizzle(int key) { return ((key & 3) << 1) | ((key >> 3) & 1); }
-
-// 1 KB from memory into LDS, 16 bytes a lane from the lane's own address; the place is the same for all lanes.  Written out
-// because the compiler makes every LDS read wait for loads of this kind that are under way, also where they fill another
-// buffer; the walk below waits for them itself.  (s_nop: the place register must rest a cycle before it is read.)
-__device__ __forceinline__ void lt_bring(uint32_t place, const bf16_t* src) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(place), "v"(src) : "memory");
-}
-// the wavefront's own loads are in, its LDS reads are through; then all wavefronts meet
-__device__ __forceinline__ void lt_wait_and_meet() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // A tile is brought 8 keys at a time, KP / 64 kilobytes each, which lie in one page.  Where a lane's 16 bytes of such a group come
 // from is the same for every tile: the table behind the tile buffers holds it, in elements from the group's first row, for
@@ -380,7 +370,7 @@ __device__ __forceinline__ void lt_bring_tile(const unsigned char* lds, uint32_t
     const bf16_t* rows = c_pages + (((int64_t)page << ps_shift) + in_page) * row;
     const uint16_t* table = reinterpret_cast<const uint16_t*>(lds + TileLayout<KP>::TABLE) + (group & 1) * TileLayout<KP>::PIECES + lane;
 #pragma unroll
-    for (int j = 0; j < KP / 64; ++j) lt_bring(place + group * (8 * KP * 2) + j * 1024, rows + table[64 * j]);
+    for (int j = 0; j < KP / 64; ++j) lds_bring(place + group * (8 * KP * 2) + j * 1024, rows + table[64 * j]);
   }
 }
 
@@ -405,12 +395,12 @@ __device__ __forceinline__ void lt_walk(f32x4 (&acc)[NS][RP / 16], float (&m_run
   if (tile_lo > tile_hi) return;                                            // the same for all wavefronts
   const int lane = 16 * g + c;
   int pages = lt_find_pages(bt, tile_lo, ps_shift, lo_min, hi_max, lane);
-  lt_wait_and_meet();                                                       // nobody reads the buffers of a walk before any more
+  lds_wait_and_meet();                                                       // nobody reads the buffers of a walk before any more
   lt_bring_tile<KP, WAVES>(lds, base, pages, c_pages, tile_lo, row, ps_shift, wave, lane);
   if (tile_lo + 32 <= tile_hi) pages = lt_find_pages(bt, tile_lo + 32, ps_shift, lo_min, hi_max, lane);
   int buf = 0;
   for (int k0 = tile_lo; k0 <= tile_hi; k0 += 32, buf ^= 1) {
-    lt_wait_and_meet();                   // this tile is in, and nobody reads the other buffer any more
+    lds_wait_and_meet();                   // this tile is in, and nobody reads the other buffer any more
     if (k0 + 32 <= tile_hi) {
       lt_bring_tile<KP, WAVES>(lds, base + (buf ^ 1) * TILE, pages, c_pages, k0 + 32, row, ps_shift, wave, lane);
       if (k0 + 64 <= tile_hi) pages = lt_find_pages(bt, k0 + 64, ps_shift, lo_min, hi_max, lane);

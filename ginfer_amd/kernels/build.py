@@ -31,7 +31,8 @@ MODULES = ("embedding", "norm", "rope_kv", "attention_generic", "attention_mfma"
 MODULE_FLAGS = {"random_fill": ["-ffp-contract=off"], "attention_generic": ["-ffp-contract=off"]}
 # headers beside common.h that a module includes (they enter its digest)
 MODULE_HEADERS = {"random_fill": ["random_normal.h"], "delta_scan": ["delta_common.h"], "delta_chunk": ["delta_common.h"],
-                  "decay_scan": ["decay_walk.h"], "gated_recurrence": ["decay_walk.h"]}
+                  "decay_scan": ["decay_walk.h"], "gated_recurrence": ["decay_walk.h"],
+                  "gemm_tiles": ["lds_load.h"], "expert_gemm": ["lds_load.h"], "latent_attention": ["lds_load.h"]}
 # plain C++ libraries for the host (no GPU runtime), built with the host compiler from csrc/host/
 HOST_MODULES = ("random_fill_host",)
 HOST_FLAGS = ["-O2", "-std=c++17", "-shared", "-fPIC", "-pthread", "-ffp-contract=off"]
