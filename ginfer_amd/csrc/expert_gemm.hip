@@ -374,8 +374,8 @@ static int eg_launch(void* out, const void* in, const void* w, int64_t w_expert,
   do {                                                                                                                        \
     const int64_t n = (int64_t)((cols + 256 / MATS - 1) / (256 / MATS)) * max_tiles;                                          \
     constexpr int bytes = (256 + 64 * WN) * 128 * 2;                                                                          \
-    static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void*>(expert_many_kernel<MATS, WN>),         \
-                                                         hipFuncAttributeMaxDynamicSharedMemorySize, bytes);                  \
+    const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void*>(expert_many_kernel<MATS, WN>),                \
+                                                  hipFuncAttributeMaxDynamicSharedMemorySize, bytes);                         \
     if (raised != hipSuccess) return (int)raised;                                                                             \
     if (K % 32 || n > 0x7ffffff0) return -2;                                                                                  \
     hipLaunchKernelGGL((expert_many_kernel<MATS, WN>), dim3((unsigned)((n + 7) / 8 * 8)), dim3(128 * WN), bytes, stream, OPERANDS, SIZES); \

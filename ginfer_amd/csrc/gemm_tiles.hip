@@ -207,8 +207,8 @@ static int gt_launch(void* C, int64_t ldc, const void* A, int64_t lda, const voi
   constexpr int TN = 32 * NI * WN, TM = 32 * MJ * WM, COLS = GATED ? TN / 2 : TN;
   constexpr int slabs_bytes = (TN + TM) * 128 * NBUF, out_bytes = GATED ? TM * (COLS + 8) * 2 : 0;
   constexpr int bytes = slabs_bytes > out_bytes ? slabs_bytes : out_bytes;
-  static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_tiles_kernel<NI, MJ, WN, WM, NBUF, GATED>),
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_tiles_kernel<NI, MJ, WN, WM, NBUF, GATED>),
+                                                hipFuncAttributeMaxDynamicSharedMemorySize, bytes);       // the current device's
   if (raised != hipSuccess) return (int)raised;
   const int64_t m_tiles = (M + TM - 1) / TM, n_tiles = (cols + COLS - 1) / COLS, groups = (m_tiles * n_tiles + 7) / 8 * 8;
   if (groups > 0x7fffffff / 256) return -2;

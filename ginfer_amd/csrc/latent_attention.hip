@@ -712,8 +712,8 @@ static bool lt_operands_ok(const void* out, int64_t out_t, int64_t out_h, const 
 #define LT_LAUNCH(KERNEL, KP, GRID, THREADS, ...)                                                                             \
   do {                                                                                                                        \
     constexpr int bytes = TileLayout<KP>::BYTES;                                                                                 \
-    static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void*>(&KERNEL),                              \
-                                                         hipFuncAttributeMaxDynamicSharedMemorySize, bytes);                  \
+    const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void*>(&KERNEL),                                     \
+                                                  hipFuncAttributeMaxDynamicSharedMemorySize, bytes);                         \
     if (raised != hipSuccess) return (int)raised;                                                                             \
     hipLaunchKernelGGL((KERNEL), GRID, dim3(THREADS), bytes, stream, __VA_ARGS__);                                            \
   } while (0)

@@ -16,3 +16,10 @@ def test_inline_assembly_names_the_place_register_that_it_writes():
                 found += 1
                 assert '"m0"' in statement.rsplit(":", 1)[1], "%s: %s" % (path, statement)
     assert found >= 2
+
+
+def test_no_launcher_keeps_what_one_device_allowed():
+    """How much LDS a kernel may ask for belongs to the device that is current: a static result would leave a second device
+    of the process at its default."""
+    for path in SOURCES:
+        assert not re.search(r"static[^;{}()]*=\s*hipFuncSetAttribute", open(path).read()), path
