@@ -942,6 +942,11 @@ def scalar_rmsnorm_rows(x, gain, eps, dtype, rows=None):
 ADD_SCALAR_NORM_PARTS_MAX = 4096     # columns up to which the kernel adds partial sums up itself
 
 
+def add_scalar_rmsnorm_adds_parts(width):
+    """Whether the kernel adds partial sums of rows this wide itself."""
+    return width % 4 == 0 and width <= ADD_SCALAR_NORM_PARTS_MAX
+
+
 def add_scalar_rmsnorm(residual, y, gain, eps, copy=False, copy_dtype=None):
     """residual float32 [T, H] += g * y / sqrt(mean(y^2) + eps), in place; y [T, H] float32 or bfloat16, or float32 partial
     sums [parts, T, H], added up in order.  With copy the new residual also comes back in y's dtype or `copy_dtype` (what the
@@ -953,10 +958,13 @@ def add_scalar_rmsnorm(residual, y, gain, eps, copy=False, copy_dtype=None):
     parts = 1
     if y.dim() == 3:
         _need(y.dtype == torch.float32, "partial sums must be float32, got %s", y.dtype)
-        if H % 4 or H > ADD_SCALAR_NORM_PARTS_MAX:
-            y = y.sum(dim=0)
-        else:
+        if add_scalar_rmsnorm_adds_parts(H):
             parts = y.shape[0]
+        else:
+            whole = y[0]
+            for p in range(1, y.shape[0]):       # (one by one: a reduction of the library's may clear memory in a way that a
+                whole = whole + y[p]             # recorded step does not repeat)
+            y = whole
     _need(tuple(y.shape[-2:]) == (T, H) and y.is_contiguous(), "y must be contiguous %s, got %s", (T, H), tuple(y.shape))
     out, out_dtype = None, copy_dtype or y.dtype
     _need(y.dtype == torch.float32 or out_dtype == y.dtype, "the copy of a bfloat16 y is bfloat16")

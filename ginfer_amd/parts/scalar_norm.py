@@ -14,12 +14,13 @@ class ScalarRMSNorm(Part):
 
     capturable = True
     accepts_partial_sums = False
-    adds_partial_sums = True     # add_normed takes float32 [parts, T, H] and adds the parts up in order
     foldable = False         # the products around it cannot fold it: it does not sit before a product
 
     def __init__(self, size, eps, dtype, device):
         self.size, self.eps, self.dtype, self.device = int(size), float(eps), dtype, device
         self.weight = None
+        # add_normed's launch takes float32 [parts, T, H] and adds the parts up in order
+        self.adds_partial_sums = ops.add_scalar_rmsnorm_adds_parts(self.size)
 
     def weight_specs(self):
         return {"": WeightSpec((), init="one_plus_normal", keep_32bit=True)}

@@ -122,3 +122,11 @@ def test_cache_manager_gives_slots_and_windowed_pages_back():
     cm.release("c")
     cm.check()
     assert cm.groups[0].pool.num_free == 6
+
+
+def test_the_feed_forward_leaves_parts_only_to_a_norm_that_adds_them():
+    """Rows wider than the norm's kernel holds, or of a width that is no multiple of four, come whole."""
+    import torch
+    from ginfer_amd.parts.scalar_norm import ScalarRMSNorm
+    adds = [ScalarRMSNorm(size, 1e-5, torch.bfloat16, None).adds_partial_sums for size in (4, 1536, 4096, 1538, 4100, 5120)]
+    assert adds == [True, True, True, False, False, False]
