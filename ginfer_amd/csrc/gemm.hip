@@ -151,7 +151,9 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_kernel(TC* __restrict__ 
 // elements of K with the four of a lane side by side (k = g, 4 + g, 8 + g, 12 + g): the operands of four instructions
 // come in one 16-byte read and need no exchange between lanes (with the row swaps of gfx950 after the read the chain of
 // a K of 8,960 took 91 us instead of 62), and with rows padded by four words neither side has bank conflicts.
-// Workgroups that share rows of W are neighbours on one XCD, whose L2 then reads W once.
+// Workgroups that share rows of W are neighbours on one XCD, whose L2 then reads W once: columns of tiles go to the XCDs in
+// turn, so that few columns leave some without work (2,048 rows by 32, a K of 1,536, 21.5 us on one XCD, 70.8 in the tiles before
+// these; the left-over columns dealt to all eight alike 14.5, but then 2,048 by 2,048 takes 140 where it takes 122).
 // Measured on MI355X, us, before (32 x 32 x 2 blocks in tiles of 64 x 64 to 128 x 128, two barriers a step) -> now, for
 // [rows] x 1,536 of a K of 8,960, x 2,048 of 1,536, and x 17,920 of 1,536: 65 rows 335 -> 62, 55 -> 13.6, 157 -> 62;
 // 256 rows 232 -> 99, 45 -> 21.6, 224 -> 124; 512 rows 232 -> 141, 47.5 -> 39, 327 -> 231; 2,048 rows 634 -> 433,
@@ -456,7 +458,7 @@ extern "C" int ga_gemm_nt(void* C, int64_t ldc, const void* A, int64_t lda, cons
   // many rows: the matrix cores, in tiles of 32 x 32, 64 x 64 or 64 x 96, whichever takes the least time by this sum.  A
   // chip of 256 compute units works off `rounds` tiles each; the first costs a tile's whole chain, further ones overlap
   // with it.  Measured in us at a K of 1,536 (alone / each further round): 13.2 / 8.5, 35.5 / 25.5, 47.5 / 39; the sums
-  // come within 6 % of what all the sizes above take in each tiling.
+  // come within 10 % of what the sizes above take (512 rows by 2,048: 35.5 against 39; 2,048 by 2,048: 112 against 122).
   const bool matrix = M > GEMM_MATRIX_FROM_ROWS;
   const int tile_m[3] = {32, 64, 64}, tile_n[3] = {32, 64, 96};
   const float alone[3] = {13.2f, 35.5f, 47.5f}, further[3] = {8.5f, 25.5f, 39.f};

@@ -215,13 +215,26 @@ def test_gemm_nt_on_the_matrix_cores_gives_the_bits_of_the_fma_kernel(dtype, M, 
     assert torch.equal(ops.gemm_nt(a[M - 1:].contiguous(), w, b, out_dtype=torch.float32)[0], full[M - 1])
 
 
-@pytest.mark.parametrize("M,N,K", [(65, 31, 64), (97, 33, 63), (96, 64, 65), (129, 100, 128), (70, 40, 193),       # 32 x 32
-                                   (2047, 1537, 31), (2049, 1500, 96), (2048, 1536, 100),                        # 64 x 64
-                                   (255, 4700, 32), (257, 4607, 95), (300, 4609, 224)])                          # 64 x 96
-def test_gemm_nt_tiles_at_their_edges(M, N, K):
+def _gemm_nt_tile(M, N):
+    """The tile that the launcher takes for more than 64 rows: the least of its three sums (csrc/gemm.hip)."""
+    sums = []
+    for tm, tn, alone, further in ((32, 32, 13.2, 8.5), (64, 64, 35.5, 25.5), (64, 96, 47.5, 39.0)):
+        tiles = -(-M // tm) * -(-N // tn)
+        sums.append((alone + further * (-(-tiles // 256) - 1), (tm, tn)))
+    return min(sums, key=lambda s: s[0])[1]
+
+
+@pytest.mark.parametrize("tile,M,N,K", [
+    ((32, 32), 65, 31, 64), ((32, 32), 97, 33, 63), ((32, 32), 96, 64, 65), ((32, 32), 129, 100, 128), ((32, 32), 70, 40, 193),
+    ((32, 32), 2049, 1500, 96), ((32, 32), 255, 4700, 32), ((32, 32), 1000, 20, 64), ((32, 32), 200, 300, 48),
+    ((64, 64), 2047, 1537, 31), ((64, 64), 2048, 1536, 100), ((64, 64), 2047, 1535, 64), ((64, 64), 2049, 1537, 33),
+    ((64, 96), 257, 4607, 95), ((64, 96), 300, 4609, 224), ((64, 96), 319, 4799, 32), ((64, 96), 320, 4801, 64), ((64, 96), 257, 4703, 96)])
+def test_gemm_nt_tiles_at_their_edges(tile, M, N, K):
     """One row, column or element of K more or less than the three tilings of the kernel for many rows hold, and K of one
-    step, an odd and an even number of steps: the bits of 16 rows at a time, which another kernel multiplies."""
+    step, an odd and an even number of steps, fewer and a few more columns of tiles than the chip has XCDs: the bits of 16
+    rows at a time, which another kernel multiplies."""
     from ginfer_amd.kernels import ops
+    assert _gemm_nt_tile(M, N) == tile, _gemm_nt_tile(M, N)
     a, w, b = rnd((M, K), torch.float32, 21), rnd((N, K), torch.float32, 22), rnd((N,), torch.float32, 23)
     full = ops.gemm_nt(a, w, b)
     for r in sorted({0, M // 2, M - 16}):
@@ -1050,10 +1063,11 @@ def test_gated_product_in_every_tiling(tiling, M, cols, K):
 
 
 @pytest.mark.parametrize("M", [1, 63, 64, 65, 127, 256, 300])
-@pytest.mark.parametrize("N,K,parts", [(16, 64, 1), (80, 192, 3), (144, 320, 2), (1536, 640, 5), (64, 832, 13)])
+@pytest.mark.parametrize("N,K,parts", [(16, 64, 1), (80, 192, 3), (144, 320, 2), (1536, 640, 5), (64, 832, 13), (80, 256, 1),
+                                       (144, 320, 1), (96, 576, 1), (64, 1088, 2), (208, 2112, 3)])
 def test_product_over_tiles_in_parts(M, N, K, parts):
-    """Parts of one to five slabs, uneven ones too (five slabs in two parts): 32-bit sums of bfloat16 products, together the
-    whole product, each the product over its own piece of K."""
+    """Parts of one to eleven slabs (the kernels have three and four buffers), uneven ones too (17 slabs in two parts): 32-bit
+    sums of bfloat16 products, together the whole product, each the product over its own piece of K."""
     from ginfer_amd.kernels import ops
     a, w = rnd((M, K), torch.bfloat16, 61), rnd((N, K), torch.bfloat16, 62)
     got = ops.gemm_tiles_parts(a, w, parts).double()
