@@ -152,8 +152,9 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_kernel(TC* __restrict__ 
 // come in one 16-byte read and need no exchange between lanes (with the row swaps of gfx950 after the read the chain of
 // a K of 8,960 took 91 us instead of 62), and with rows padded by four words neither side has bank conflicts.
 // Workgroups that share rows of W are neighbours on one XCD, whose L2 then reads W once: columns of tiles go to the XCDs in
-// turn, so that few columns leave some without work (2,048 rows by 32, a K of 1,536, 21.5 us on one XCD, 70.8 in the tiles before
-// these; the left-over columns dealt to all eight alike 14.5, but then 2,048 by 2,048 takes 140 where it takes 122).
+// turn, and the tiles of the columns that are left over to all eight alike (as whole columns they made a second round on the
+// XCDs that got one more: 300 rows by 4,864, 51 columns of tiles, K 1,536, 84 us, now 54.5; 1,536 by 640 60 and 39.7; 2,048 by
+// 32, one column, 21.5 and 14.5).
 // Measured on MI355X, us, before (32 x 32 x 2 blocks in tiles of 64 x 64 to 128 x 128, two barriers a step) -> now, for
 // [rows] x 1,536 of a K of 8,960, x 2,048 of 1,536, and x 17,920 of 1,536: 65 rows 335 -> 62, 55 -> 13.6, 157 -> 62;
 // 256 rows 232 -> 99, 45 -> 21.6, 224 -> 124; 512 rows 232 -> 141, 47.5 -> 39, 327 -> 231; 2,048 rows 634 -> 433,
@@ -172,9 +173,14 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_matrix_kernel(TC* __rest
   __shared__ float a_s[2][TM][PAD];
   __shared__ float w_s[2][TN][PAD];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, i16 = lane & 15, kq = lane >> 4;
-  const int at = blockIdx.x >> 3;
-  const int mt = at % m_tiles, nt = (at / m_tiles) * 8 + (blockIdx.x & 7);
-  if (nt >= n_tiles) return;
+  const int at = blockIdx.x >> 3, xcd = blockIdx.x & 7, whole = n_tiles / 8 * m_tiles;
+  int mt = at % m_tiles, nt = at / m_tiles * 8 + xcd;
+  if (at >= whole) {
+    const int rest = n_tiles % 8 * m_tiles, run = (rest + 7) / 8, id = xcd * run + at - whole;
+    if (at - whole >= run || id >= rest) return;
+    mt = id % m_tiles;
+    nt = n_tiles / 8 * 8 + id / m_tiles;
+  }
   const int m0 = mt * TM, n0 = nt * TN;
   const int wm = (wave >> 1) * (TM / 2), wn = (wave & 1) * (TN / 2);
   f32x4 acc[BM][BN];
@@ -478,7 +484,7 @@ extern "C" int ga_gemm_nt(void* C, int64_t ldc, const void* A, int64_t lda, cons
   dim3 grid((N + tn - 1) / tn, (M + tm - 1) / tm), block(GEMM_THREADS);
   if (matrix) {
     if ((M + 127) / 128 > 65535) return -2;
-    const int64_t groups = (int64_t)m_tiles * ((n_tiles + 7) / 8) * 8;     // one dimension: see the kernel's mapping
+    const int64_t groups = ((int64_t)m_tiles * (n_tiles / 8) + ((int64_t)m_tiles * (n_tiles % 8) + 7) / 8) * 8;    // see the kernel's mapping
     if (groups > 0x7fffffff / GEMM_THREADS) return -2;
     grid = dim3((unsigned)groups);
   }
