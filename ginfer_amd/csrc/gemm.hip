@@ -14,8 +14,8 @@
 // They are templated on storage, so that they also serve bfloat16 operands (the kernel tests' oracle and the
 // fallback for shapes the bfloat16 kernels refuse).
 //
-// A step of K is asked for (in 16-byte loads where rows allow it, consecutive lanes on consecutive elements)
-// while the step before is being multiplied.
+// A step of K is asked for (in 16-byte loads, in the first and the third kernel where rows allow it, consecutive lanes on
+// consecutive elements) while the step before is being multiplied.
 #include "common.h"
 #include "ginfer_amd.h"   // the entry points below are checked against their declarations
 
@@ -47,6 +47,20 @@ __device__ __forceinline__ void load4<bf16_t>(float (&v)[4], const bf16_t* p, in
 #pragma unroll
     for (int i = 0; i < 4; ++i) v[i] = i < valid ? bf16_to_f32(p[i]) : 0.f;
   }
+}
+
+// four consecutive elements at any address that an element may have, in one load all the same: the device takes vector loads
+// at such addresses, and a type that promises no more says so
+typedef float any_float4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint16_t any_half4 __attribute__((ext_vector_type(4), aligned(2)));
+__device__ __forceinline__ void load4_anywhere(float (&v)[4], const float* p) {
+  const any_float4 x = *reinterpret_cast<const any_float4*>(p);
+  v[0] = x[0]; v[1] = x[1]; v[2] = x[2]; v[3] = x[3];
+}
+__device__ __forceinline__ void load4_anywhere(float (&v)[4], const bf16_t* p) {
+  const any_half4 x = *reinterpret_cast<const any_half4*>(p);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = bf16_to_f32(x[i]);
 }
 
 // TM x TN: the workgroup's tile of C; TK: elements of K per step; a thread owns RM x RN elements, the threads
@@ -154,7 +168,8 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_kernel(TC* __restrict__ 
 // Workgroups that share rows of W are neighbours on one XCD, whose L2 then reads W once: columns of tiles go to the XCDs in
 // turn, and the tiles of the columns that are left over to all eight alike (as whole columns they made a second round on the
 // XCDs that got one more: 300 rows by 4,864, 51 columns of tiles, K 1,536, 84 us, now 54.5; 1,536 by 640 60 and 39.7; 2,048 by
-// 32, one column, 21.5 and 14.5).
+// 32, one column, 21.5 and 14.5).  Rows that are not aligned take the same loads (4,096 rows by 5,000 of a K of 521, us: 264 in the
+// tiles before, 330 element by element here, now 206; 256 by 1,536 of 1,537: 90, 49, 24).
 // Measured on MI355X, us, before (32 x 32 x 2 blocks in tiles of 64 x 64 to 128 x 128, two barriers a step) -> now, for
 // [rows] x 1,536 of a K of 8,960, x 2,048 of 1,536, and x 17,920 of 1,536: 65 rows 335 -> 62, 55 -> 13.6, 157 -> 62;
 // 256 rows 232 -> 99, 45 -> 21.6, 224 -> 124; 512 rows 232 -> 141, 47.5 -> 39, 327 -> 231; 2,048 rows 634 -> 433,
@@ -166,7 +181,7 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_matrix_kernel(TC* __rest
                                                                      const TA* __restrict__ A, int64_t lda,
                                                                      const TW* __restrict__ W,
                                                                      const TW* __restrict__ bias, int M, int N, int K,
-                                                                     int wide_a, int wide_w, int m_tiles, int n_tiles) {
+                                                                     int m_tiles, int n_tiles) {
   constexpr int TM = 32 * BM, TN = 32 * BN, PAD = TK + 4;
   constexpr int GA = TM * TK / 4 / GEMM_THREADS, GW = TN * TK / 4 / GEMM_THREADS;
   static_assert(GA >= 1 && GW >= 1 && TK % 16 == 0 && DEPTH % 2 == 0, "tile sizes");
@@ -204,9 +219,9 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_matrix_kernel(TC* __rest
   }
   auto fetch = [&](float (&xa)[GA][4], float (&xw)[GW][4], int k0) {
 #pragma unroll
-    for (int i = 0; i < GA; ++i) load4<TA>(xa[i], pa[i] + k0, 4, true);
+    for (int i = 0; i < GA; ++i) load4_anywhere(xa[i], pa[i] + k0);
 #pragma unroll
-    for (int i = 0; i < GW; ++i) load4<TW>(xw[i], pw[i] + k0, 4, true);
+    for (int i = 0; i < GW; ++i) load4_anywhere(xw[i], pw[i] + k0);
   };
   auto fetch_carefully = [&](float (&xa)[GA][4], float (&xw)[GW][4], int k0) {
     const int k = k0 + (tid % (TK / 4)) * 4, valid = k < K ? (K - k < 4 ? K - k : 4) : 0;
@@ -260,7 +275,7 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_matrix_kernel(TC* __rest
             acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[c][i][st], y[c][j][st], acc[i][j], 0, 0, 0);
     }
   };
-  const int steps = (wide_a && wide_w) ? K / TK : 0, last = (steps - 1) * TK;
+  const int steps = K / TK, last = (steps - 1) * TK;
   if (steps > 0) {
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d) fetch(ra[d], rw[d], d * TK < last ? d * TK : last);
@@ -509,16 +524,16 @@ extern "C" int ga_gemm_nt(void* C, int64_t ldc, const void* A, int64_t lda, cons
                          (const TA*)A, lda, (const TW*)W, (const TW*)bias, M, N, K, wide_a, wide_w);         \
     else if (matrix && tiling == 0)                                                                          \
       hipLaunchKernelGGL((gemm_nt_matrix_kernel<TA, TW, TC, 1, 1, 64, 2>), grid, block, 0, stream,           \
-                         (TC*)C, ldc, (const TA*)A, lda, (const TW*)W, (const TW*)bias, M, N, K, wide_a,     \
-                         wide_w, m_tiles, n_tiles);                                                          \
+                         (TC*)C, ldc, (const TA*)A, lda, (const TW*)W, (const TW*)bias, M, N, K, m_tiles,    \
+                         n_tiles);                                                                           \
     else if (matrix && tiling == 1)                                                                          \
       hipLaunchKernelGGL((gemm_nt_matrix_kernel<TA, TW, TC, 2, 2, 32, 2>), grid, block, 0, stream,           \
-                         (TC*)C, ldc, (const TA*)A, lda, (const TW*)W, (const TW*)bias, M, N, K, wide_a,     \
-                         wide_w, m_tiles, n_tiles);                                                          \
+                         (TC*)C, ldc, (const TA*)A, lda, (const TW*)W, (const TW*)bias, M, N, K, m_tiles,    \
+                         n_tiles);                                                                           \
     else if (matrix)                                                                                         \
       hipLaunchKernelGGL((gemm_nt_matrix_kernel<TA, TW, TC, 2, 3, 32, 2>), grid, block, 0, stream,           \
-                         (TC*)C, ldc, (const TA*)A, lda, (const TW*)W, (const TW*)bias, M, N, K, wide_a,     \
-                         wide_w, m_tiles, n_tiles);                                                          \
+                         (TC*)C, ldc, (const TA*)A, lda, (const TW*)W, (const TW*)bias, M, N, K, m_tiles,    \
+                         n_tiles);                                                                           \
     else                                                                                                     \
       hipLaunchKernelGGL((gemm_nt_kernel<TA, TW, TC, 64, 64, 32>), grid, block, 0, stream, (TC*)C, ldc,      \
                          (const TA*)A, lda, (const TW*)W, (const TW*)bias, M, N, K, wide_a, wide_w);         \

@@ -241,6 +241,20 @@ def test_gemm_nt_tiles_at_their_edges(tile, M, N, K):
         assert torch.equal(ops.gemm_nt(a[r:r + 16].contiguous(), w, b), full[r:r + 16]), "rows from %d" % r
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K", [(65, 40, 64), (130, 100, 77), (300, 4609, 97), (2049, 1537, 130)])
+def test_gemm_nt_takes_rows_at_any_address(dtype, M, N, K):
+    """Rows that start at every multiple of an element, A's with an odd stride and W's with an odd K: the bits of rows that are
+    aligned (K filled up with zeros, which add nothing)."""
+    from ginfer_amd.kernels import ops
+    wide, w = rnd((M, K + 6), dtype, 24), rnd((N, K), dtype, 25)
+    for at in (0, 1, 2, 3):
+        a = wide[:, at:at + K]
+        fill = torch.zeros((M, -K % 64), dtype=dtype, device=dev()), torch.zeros((N, -K % 64), dtype=dtype, device=dev())
+        want = ops.gemm_nt(torch.cat([a, fill[0]], dim=1), torch.cat([w, fill[1]], dim=1).contiguous(), out_dtype=torch.float32)
+        assert torch.equal(ops.gemm_nt(a, w, out_dtype=torch.float32), want), at
+
+
 @pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-4), (torch.bfloat16, 1e-2)])
 @pytest.mark.parametrize("T,nh,nkv,hd,rd,theta", [(128, 32, 8, 128, 128, 1e4), (64, 12, 12, 64, 64, 1e4),
                                                   (9, 6, 3, 48, 48, 5e5), (5, 4, 2, 32, 16, 1e6), (7, 3, 1, 24, 20, 1e4),
