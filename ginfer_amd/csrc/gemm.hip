@@ -483,14 +483,18 @@ extern "C" int ga_gemm_nt(void* C, int64_t ldc, const void* A, int64_t lda, cons
   const bool matrix = M > GEMM_MATRIX_FROM_ROWS;
   const int tile_m[3] = {32, 64, 64}, tile_n[3] = {32, 64, 96};
   const float alone[3] = {13.2f, 35.5f, 47.5f}, further[3] = {8.5f, 25.5f, 39.f};
-  int tiling = 0, m_tiles = 0, n_tiles = 0;
+  int tiling = -1, m_tiles = 0, n_tiles = 0;
+  int64_t groups = 0;
   float least = 0.f;
   for (int t = 0; matrix && t < 3; ++t) {
-    const int64_t mt = (M + tile_m[t] - 1) / tile_m[t], nt = (N + tile_n[t] - 1) / tile_n[t];
+    const int64_t mt = (M + (int64_t)tile_m[t] - 1) / tile_m[t], nt = (N + (int64_t)tile_n[t] - 1) / tile_n[t];
+    const int64_t blocks = (mt * (nt / 8) + (mt * (nt % 8) + 7) / 8) * 8;     // one dimension: see the kernel's mapping
+    if (blocks > 0xffffffffll / GEMM_THREADS) continue;                       // more threads than a launch may have
     const float us = alone[t] + further[t] * (float)((mt * nt + 255) / 256 - 1);
-    if (t == 0 || us < least) {
+    if (tiling < 0 || us < least) {
       least = us;
       tiling = t;
+      groups = blocks;
       m_tiles = (int)mt;
       n_tiles = (int)nt;
     }
@@ -498,9 +502,7 @@ extern "C" int ga_gemm_nt(void* C, int64_t ldc, const void* A, int64_t lda, cons
   const int tm = 64, tn = few ? 16 : 64;
   dim3 grid((N + tn - 1) / tn, (M + tm - 1) / tm), block(GEMM_THREADS);
   if (matrix) {
-    if ((M + 127) / 128 > 65535) return -2;
-    const int64_t groups = ((int64_t)m_tiles * (n_tiles / 8) + ((int64_t)m_tiles * (n_tiles % 8) + 7) / 8) * 8;    // see the kernel's mapping
-    if (groups > 0x7fffffff / GEMM_THREADS) return -2;
+    if ((M + 127) / 128 > 65535 || tiling < 0) return -2;
     grid = dim3((unsigned)groups);
   }
   if (grid.y > 65535) return -2;

@@ -255,6 +255,18 @@ def test_gemm_nt_takes_rows_at_any_address(dtype, M, N, K):
         assert torch.equal(ops.gemm_nt(a, w, out_dtype=torch.float32), want), at
 
 
+def test_gemm_nt_takes_more_columns_than_a_launch_has_small_tiles():
+    """65 rows by so many columns that tiles of 32 x 32 would be more threads than a launch may have: larger tiles take it.
+    A K of one: every result is one product, rounded once."""
+    from ginfer_amd.kernels import ops
+    N = 179_000_001
+    a, w = rnd((65, 1), torch.bfloat16, 26), rnd((1 << 20, 1), torch.bfloat16, 27)
+    w = w.repeat(-(-N // w.shape[0]), 1)[:N]
+    out = ops.gemm_nt(a, w)
+    for r in (0, 31, 32, 63, 64):
+        assert torch.equal(out[r], (a[r].float() * w[:, 0].float()).to(torch.bfloat16)), r
+
+
 @pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-4), (torch.bfloat16, 1e-2)])
 @pytest.mark.parametrize("T,nh,nkv,hd,rd,theta", [(128, 32, 8, 128, 128, 1e4), (64, 12, 12, 64, 64, 1e4),
                                                   (9, 6, 3, 48, 48, 5e5), (5, 4, 2, 32, 16, 1e6), (7, 3, 1, 24, 20, 1e4),
