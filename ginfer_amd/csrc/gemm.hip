@@ -171,9 +171,9 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_kernel(TC* __restrict__ 
 // 32, one column, 21.5 and 14.5).  Rows that are not aligned take the same loads (4,096 rows by 5,000 of a K of 521, us: 264 in the
 // tiles before, 330 element by element here, now 206; 256 by 1,536 of 1,537: 90, 49, 24).
 // Measured on MI355X, us, before (32 x 32 x 2 blocks in tiles of 64 x 64 to 128 x 128, two barriers a step) -> now, for
-// [rows] x 1,536 of a K of 8,960, x 2,048 of 1,536, and x 17,920 of 1,536: 65 rows 335 -> 62, 55 -> 13.6, 157 -> 62;
-// 256 rows 232 -> 99, 45 -> 21.6, 224 -> 124; 512 rows 232 -> 141, 47.5 -> 39, 327 -> 231; 2,048 rows 634 -> 433,
-// 136 -> 122, 905 -> 886 (127 of the 154 TFLOP/s that a large product reaches on this card).
+// [rows] x 1,536 of a K of 8,960, x 2,048 of 1,536, and x 17,920 of 1,536: 65 rows 335 -> 59, 55 -> 12.4, 157 -> 56;
+// 256 rows 232 -> 93, 45 -> 19.6, 224 -> 116; 512 rows 232 -> 136, 47.5 -> 36, 327 -> 229; 2,048 rows 634 -> 433,
+// 136 -> 105, 905 -> 868 (130 of the 154 TFLOP/s that a large product reaches on this card).
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 template <typename TA, typename TW, typename TC, int BM, int BN, int TK, int DEPTH>
@@ -479,7 +479,7 @@ extern "C" int ga_gemm_nt(void* C, int64_t ldc, const void* A, int64_t lda, cons
   // many rows: the matrix cores, in tiles of 32 x 32, 64 x 64 or 64 x 96, whichever takes the least time by this sum.  A
   // chip of 256 compute units works off `rounds` tiles each; the first costs a tile's whole chain, further ones overlap
   // with it.  Measured in us at a K of 1,536 (alone / each further round): 13.2 / 8.5, 35.5 / 25.5, 47.5 / 39; the sums
-  // come within 10 % of what the sizes above take (512 rows by 2,048: 35.5 against 39; 2,048 by 2,048: 112 against 122).
+  // are what the sizes above take at that K or up to 15 % more (512 rows by 2,048: 35.5 against 36; 65 by 17,920: 64 against 56).
   const bool matrix = M > GEMM_MATRIX_FROM_ROWS;
   const int tile_m[3] = {32, 64, 64}, tile_n[3] = {32, 64, 96};
   const float alone[3] = {13.2f, 35.5f, 47.5f}, further[3] = {8.5f, 25.5f, 39.f};
