@@ -20,6 +20,7 @@
 // q, k and v as the recurrence reads them: the projection's numbers or their silu, turned by position, scaled
 template <bool ROT>
 struct DecayRows {
+  static constexpr bool K_OF_A = false;
   struct Fixed {};
   __device__ __forceinline__ Fixed fixed(int) const { return {}; }
   struct Plain { float q, k, a; };
@@ -75,6 +76,10 @@ struct DecayRows {
 // 64 x 128: 2,048 tokens of one request 421 -> 119, 459 -> 142; five entries of 918 207 -> 161, 217 -> 176; 495 tokens beside 16
 // single ones 110 -> 57, 120 -> 66; 64 entries of one token 20.7 -> 16.4, 21.3 -> 17.0 (reading and writing the state).  28 heads
 // of 128 x 128: 815 -> 459, 911 -> 500; 904 -> 486, 896 -> 511; 225 -> 162, 239 -> 171; 85 -> 70, 86 -> 70.
+// Many short entries, the caches emptied before, a decay per channel, before -> with last tiles brought whole and 16 tokens a tile
+// for up to 16 and 33 to 48 rows of state -> now: 64 of 33 tokens, 16 heads of 16 x 32 18.5 -> 20.5 -> 18.8, of 32 x 64 38.6 -> 37.0 ->
+// 37.6, of 48 x 64 54.7 -> 58 -> 47.6, 12 of 64 x 128 80 -> 68 -> 66, 28 of 128 x 128 384 -> 279 -> 267; 300 of 5, 8 of 256 x 256 537 ->
+// 592 -> 475, 16 of 48 x 64 75 -> 89 -> 64.  Longer than before: 64 of 9 of 32 x 64 18.5 -> 20.3, 200 of 33 of 16 x 32 41 -> 43.
 template <int R, int COLS, int TILE, bool ROT>   // R rows of the state per thread: dim <= 16 * R
 __global__ __launch_bounds__(dw_threads(COLS)) void decay_scan_kernel(
     float* __restrict__ out, const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
@@ -323,7 +328,7 @@ extern "C" int ga_decay_scan(void* out, const void* q, const void* k, const void
                                  (float*)state, (const int64_t*)slots, (const int32_t*)cu, (const int32_t*)q_start, heads, dim, vdim,   \
                                  silu_inputs)
 #define GR(R, C, T) do { if (rot_dims > 0) GO(R, C, T, true); else GO(R, C, T, false); } while (0)
-  DW_WAY(way, rows, GR);
+  DW_WAY(way, rows, dw_many(entries, heads, vdim), GR);
 #undef GR
 #undef GO
   return GA_CHECK_LAUNCH();

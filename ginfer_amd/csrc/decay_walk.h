@@ -23,14 +23,16 @@ __host__ __device__ constexpr int dw_threads(int cols) { return cols == 8 ? 384 
 
 // Source: `Fixed` (what a channel has for all tokens), fixed(channel), `Raw` (what a thread loads for one element of q, k and a),
 // load(Raw&, start, token, channel), finish(Raw, Fixed, channel, q, k, a), load_v(start, token, column), finish_v(v); finish and
-// finish_v are templates on whether `acts` is set.  `start` is the same for all threads, tokens count from it.
+// finish_v are templates on whether `acts` is set.  `start` is the same for all threads, tokens count from it.  K_OF_A: k is 1 - a;
+// finish leaves it out and LDS, whose reads are what many entries wait for, does not hold it.
 template <int R, int COLS, int TILE, class Source>
 __device__ __forceinline__ void decay_walk(float* __restrict__ out, const Source& source, float* __restrict__ state, bool fresh,
                                            int n, int heads, int dim, int vdim, int v0) {
   constexpr int WALKERS = DW_SLICES * COLS, THREADS = dw_threads(COLS), SERVERS = THREADS > WALKERS ? THREADS - WALKERS : WALKERS;
   constexpr int DP = DW_SLICES * R, PER = (TILE * DP + SERVERS - 1) / SERVERS;
-  static_assert((TILE * DP % SERVERS == 0 || PER == 1) && TILE <= DW_SLICES, "tile sizes");
-  __shared__ __attribute__((aligned(16))) float ops[2][TILE][3][DW_SLICES][R];
+  constexpr int OPS = Source::K_OF_A ? 2 : 3;                // q, k, unless it is 1 - a, and a
+  static_assert(TILE <= DW_SLICES, "tile sizes");
+  __shared__ __attribute__((aligned(16))) float ops[2][TILE][OPS][DW_SLICES][R];
   __shared__ float vs[2][TILE][COLS], partial[2][TILE][DW_SLICES][COLS];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const bool walks = THREADS == WALKERS || wave < WALKERS / WAVE, serves = THREADS == WALKERS || !walks;
@@ -48,38 +50,42 @@ __device__ __forceinline__ void decay_walk(float* __restrict__ out, const Source
   float raw_v = 0.f;
 #pragma unroll
   for (int x = 0; x < PER; ++x) fixed[x] = source.fixed(min((tid + x * SERVERS) % DP, dim - 1));
-  // Tiles are brought whole: the last one starts early enough to end with the last token, and is then walked from `t0 - start`
-  // on.  So a thread's places in a tile never change, and an address is a uniform part and a constant one.  (An entry of
-  // fewer tokens than a tile reads its last one again; channels and columns that do not exist read another and drop it.)
-  auto start_of = [&](int t0) { return max(min(t0, n - TILE), 0); };
-  // FEW: of an entry with fewer tokens than a tile (a decode step's one), what lies behind them is left out.
-  auto fetch = [&](int t0, auto few) {
-    const int start = start_of(t0);
+  // WHOLE, with 8 columns: the last tile starts early enough to end with the last token, and is then walked from `t0 - start`
+  // on.  So a thread's places in a tile never change, and an address is a uniform part and a constant one.  With 16, where
+  // entries are short and their activations a good part of the time, a tile starts where it stands, its last token is brought
+  // again for those behind it, and only what is `left` is worked out (64 entries of 9 tokens, 8 heads of 256 x 256, us: 156 ->
+  // 123); but not where a thread has so many addresses to find anew that long entries lose more (a prompt of 2,048, 28 heads of
+  // 128 x 128: 492 -> 530).  No load is conditional either way: what is loaded
+  // must not be merged with what was there, which would wait for it.  (Channels and columns that do not exist read another and
+  // drop it.)
+  constexpr bool WHOLE = COLS == 8 || (R >= 6 && R <= 12 && !Source::K_OF_A);
+  auto start_of = [&](int t0) { return WHOLE ? max(min(t0, n - TILE), 0) : t0; };
+  auto fetch = [&](int t0) {
+    const int start = WHOLE ? start_of(t0) : min(t0, n - 1), last = min(TILE, WHOLE ? n : n - start) - 1;    // (WHOLE: of all tiles)
 #pragma unroll
     for (int x = 0; x < PER; ++x) {
       const int idx = tid + x * SERVERS;
-      if (decltype(few)::value && idx / DP >= n) break;
-      source.load(raw[x], start, min(min(idx / DP, TILE - 1), n - 1), min(idx % DP, dim - 1));
+      source.load(raw[x], start, min(idx / DP, last), min(idx % DP, dim - 1));
     }
-    raw_v = source.load_v(start, min(min(s, TILE - 1), n - 1), min(v0 + j, vdim - 1));      // thread (s, j): token s, column j
+    raw_v = source.load_v(start, min(s, last), min(v0 + j, vdim - 1));      // thread (s, j): token s, column j
   };
-  auto stage_with = [&](int b, auto act, auto few) {
+  auto stage_with = [&](int b, int left, auto act, auto few) {
     constexpr bool ACT = decltype(act)::value;
 #pragma unroll
     for (int x = 0; x < PER; ++x) {
       const int idx = tid + x * SERVERS, tt = idx / DP, i = idx % DP;
       float q, k, a;
-      if ((TILE * DP < SERVERS && tt >= TILE) || (decltype(few)::value && tt >= n)) break;
+      if ((TILE * DP % SERVERS != 0 && tt >= TILE) || (decltype(few)::value && tt >= left)) break;
       source.template finish<ACT>(raw[x], fixed[x], min(i, dim - 1), q, k, a);
       ops[b][tt][0][i % DW_SLICES][i / DW_SLICES] = i < dim ? q : 0.f;
-      ops[b][tt][1][i % DW_SLICES][i / DW_SLICES] = i < dim ? k : 0.f;
-      ops[b][tt][2][i % DW_SLICES][i / DW_SLICES] = i < dim ? a : 0.f;
+      if constexpr (!Source::K_OF_A) ops[b][tt][1][i % DW_SLICES][i / DW_SLICES] = i < dim ? k : 0.f;
+      ops[b][tt][OPS - 1][i % DW_SLICES][i / DW_SLICES] = i < dim ? a : 0.f;
     }
     if (s < TILE) vs[b][s][j] = source.template finish_v<ACT>(raw_v);
   };
-  auto stage = [&](int b, auto few) {
-    if (source.acts) stage_with(b, std::true_type(), few);
-    else stage_with(b, std::false_type(), few);
+  auto stage = [&](int b, int left, auto few) {                // FEW: `left` may be less than a tile
+    if (source.acts) stage_with(b, left, std::true_type(), few);
+    else stage_with(b, left, std::false_type(), few);
   };
   // the operands of AHEAD tokens are asked for from LDS before a token is worked off (none with 16 columns: a step of many
   // entries lives from many workgroups on a compute unit, and registers cost those)
@@ -88,9 +94,9 @@ __device__ __forceinline__ void decay_walk(float* __restrict__ out, const Source
   auto read = [&](int b, int tt, int at) {
     vx[at] = vs[b][tt][j];
 #pragma unroll
-    for (int r = 0; r < R; ++r) kx[at][r] = ops[b][tt][1][s][r];
+    for (int r = 0; r < R; ++r) kx[at][r] = Source::K_OF_A ? 0.f : ops[b][tt][1][s][r];
 #pragma unroll
-    for (int r = 0; r < R; ++r) ax[at][r] = ops[b][tt][2][s][r];
+    for (int r = 0; r < R; ++r) ax[at][r] = ops[b][tt][OPS - 1][s][r];
 #pragma unroll
     for (int r = 0; r < R; ++r) qx[at][r] = ops[b][tt][0][s][r];
   };
@@ -98,7 +104,7 @@ __device__ __forceinline__ void decay_walk(float* __restrict__ out, const Source
     float acc = 0.f;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      S[r] = fmaf(ax[at][r], S[r], kx[at][r] * vx[at]);
+      S[r] = fmaf(ax[at][r], S[r], (Source::K_OF_A ? 1.0f - ax[at][r] : kx[at][r]) * vx[at]);
       acc = fmaf(S[r], qx[at][r], acc);
     }
     partial[b][tt][s][j] = acc;
@@ -111,13 +117,12 @@ __device__ __forceinline__ void decay_walk(float* __restrict__ out, const Source
     out[(int64_t)(t0 + s) * heads * vdim + v0 + j] = o;
   };
   if (serves) {
+    fetch(0);
     if (n < TILE) {
-      fetch(0, std::true_type());
-      stage(0, std::true_type());
+      stage(0, n, std::true_type());
     } else {
-      fetch(0, std::false_type());
-      stage(0, std::false_type());
-      fetch(TILE, std::false_type());
+      stage(0, n, std::false_type());
+      fetch(TILE);
     }
   }
   int b = 0, t0 = 0;
@@ -141,10 +146,11 @@ __device__ __forceinline__ void decay_walk(float* __restrict__ out, const Source
     }
     if (serves) {
       put(t0 - TILE, b ^ 1);
-      if (COLS == 8 || t0 + TILE < n) {                      // (a short entry's activations are a good part of its time)
-        stage(b ^ 1, std::false_type());
-        fetch(t0 + 2 * TILE, std::false_type());
+      if (COLS == 8 || t0 + TILE < n) {
+        if (WHOLE) stage(b ^ 1, TILE, std::false_type());
+        else stage(b ^ 1, n - t0 - TILE, std::true_type());
       }
+      if (COLS == 8 || !WHOLE || t0 + TILE < n) fetch(t0 + 2 * TILE);
     }
   }
   __syncthreads();
@@ -167,24 +173,28 @@ __device__ __forceinline__ void decay_walk(float* __restrict__ out, const Source
   }
 }
 
-// GO(R, COLS, TILE) for a state of up to 16 * rows rows: as many tokens a tile as leave two workgroups of 16 columns (a
-// decode step's many) or one of 8 their LDS, and every thread a whole number of elements to bring; tokens: that many instead
+// GO(R, COLS, TILE) for a state of up to 16 * rows rows: as many tokens a tile as leave the workgroups of 16 columns (a step's
+// many) or one of 8 their LDS; tokens: that many instead.  With up to 16 rows of state 16 tokens leave four workgroups of 16 columns
+// a compute unit, 8 leave eight: `many` says that there are more than four (16 heads of 16 x 32, us, 16 -> 8 tokens: 64 entries of
+// 64 29 -> 26, 200 of 33 50 -> 43, but 16 entries of 129 22 -> 27).
 #define DW_TILE(TOKENS, OWN) (TOKENS > 0 ? TOKENS : OWN)
-#define DW_ROWS(rows, COLS, TOKENS, GO)                                                          \
+#define DW_ROWS(rows, COLS, TOKENS, many, GO)                                                    \
   do {                                                                                           \
-    if (rows <= 1) GO(1, COLS, DW_TILE(TOKENS, 16));                                       \
-    else if (rows <= 2) GO(2, COLS, DW_TILE(TOKENS, (COLS == 8 ? 16 : 8)));                \
-    else if (rows <= 3) GO(3, COLS, DW_TILE(TOKENS, 16));                                  \
-    else if (rows <= 4) GO(4, COLS, DW_TILE(TOKENS, (COLS == 8 ? 16 : 8)));                \
-    else if (rows <= 6) GO(6, COLS, DW_TILE(TOKENS, 8));                                   \
-    else if (rows <= 8) GO(8, COLS, DW_TILE(TOKENS, 8));                                   \
-    else if (rows <= 12) GO(12, COLS, DW_TILE(TOKENS, 8));                                 \
-    else GO(16, COLS, DW_TILE(TOKENS, 4));                                                 \
+    if (rows <= 1 && COLS == 16 && many) GO(1, COLS, DW_TILE(TOKENS, 8));                        \
+    else if (rows <= 1) GO(1, COLS, DW_TILE(TOKENS, 16));                                        \
+    else if (rows <= 2) GO(2, COLS, DW_TILE(TOKENS, (COLS == 8 ? 16 : 8)));                      \
+    else if (rows <= 3) GO(3, COLS, DW_TILE(TOKENS, (COLS == 8 ? 16 : 8)));                      \
+    else if (rows <= 4) GO(4, COLS, DW_TILE(TOKENS, (COLS == 8 ? 16 : 8)));                      \
+    else if (rows <= 6) GO(6, COLS, DW_TILE(TOKENS, 8));                                         \
+    else if (rows <= 8) GO(8, COLS, DW_TILE(TOKENS, 8));                                         \
+    else if (rows <= 12) GO(12, COLS, DW_TILE(TOKENS, 8));                                       \
+    else GO(16, COLS, DW_TILE(TOKENS, 4));                                                       \
   } while (0)
 // way: 1 tiles of one token in 16 columns, 8 and 16 that many columns
-#define DW_WAY(way, rows, GO)                       \
-  do {                                              \
-    if (way == 1) DW_ROWS(rows, 16, 1, GO);         \
-    else if (way == 8) DW_ROWS(rows, 8, 0, GO);     \
-    else DW_ROWS(rows, 16, 0, GO);                  \
+#define DW_WAY(way, rows, many, GO)                       \
+  do {                                                    \
+    if (way == 1) DW_ROWS(rows, 16, 1, false, GO);        \
+    else if (way == 8) DW_ROWS(rows, 8, 0, false, GO);    \
+    else DW_ROWS(rows, 16, 0, many, GO);                  \
   } while (0)
+static inline bool dw_many(int entries, int heads, int vdim) { return (int64_t)entries * heads * ((vdim + 15) / 16) > 4 * 256; }

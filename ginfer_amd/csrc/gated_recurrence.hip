@@ -21,7 +21,7 @@ struct ForgetRows {
   const float *bias, *lower;           // the head's
   int64_t stride;
   int hd;
-  static constexpr bool acts = false;
+  static constexpr bool acts = false, K_OF_A = true;
   __device__ __forceinline__ Fixed fixed(int i) const { return {bias[i], lower[i]}; }
   __device__ __forceinline__ void load(Raw& x, int start, int t, int i) const {
     const float* p = proj + start * stride;
@@ -30,10 +30,9 @@ struct ForgetRows {
     x.f = p[at + hd];
   }
   template <bool>
-  __device__ __forceinline__ void finish(const Raw& x, const Fixed& c, int i, float& q, float& k, float& f) const {
+  __device__ __forceinline__ void finish(const Raw& x, const Fixed& c, int i, float& q, float&, float& f) const {
     q = x.q * gr_sigmoid(x.q);
     f = c.lower + (1.0f - c.lower) * gr_sigmoid(x.f + c.bias);
-    k = 1.0f - f;
   }
   __device__ __forceinline__ float load_v(int start, int t, int c) const {
     return (v + start * stride)[(uint32_t)t * (uint32_t)stride + c];
@@ -42,10 +41,13 @@ struct ForgetRows {
   __device__ __forceinline__ float finish_v(float x) const { return x; }
 };
 
-// Measured on MI355X, the projection just written, us, before -> now.  12 heads of 64 x 128: 2,048 tokens of one request 454 -> 150;
-// five entries of 918 216 -> 168; 495 tokens beside 16 single ones 117 -> 64; 64 entries of one token 20.4 -> 17.0.  28 heads of 128 x
-// 128: 777 -> 498, 784 -> 544, 225 -> 172, 78 -> 69.  The one size seen that takes longer: 64 entries of 33 tokens, 16 heads of 32 x
-// 64, 27.9 -> 32.1.
+// Measured on MI355X, the caches emptied before, us, before the walk of decay_walk.h -> now.  12 heads of 64 x 128: 2,048 tokens of
+// one request 534 -> 177; five entries of 918 262 -> 181; 495 tokens beside 16 single ones 136 -> 64; 64 entries of 33 79 -> 65,
+// of 9 34.1 -> 33.3, of one 24.5 -> 20.2.  28 heads of 128 x 128: 934 -> 514, 880 -> 563, 252 -> 191, 310 -> 244, 129 -> 121, 80 ->
+// 70.  With k kept beside f in LDS, as the general walk has it, the reads of LDS made many entries slower than before (64 of 33
+// tokens, 16 heads of 32 x 64, 35.2 -> 37.9, now 35.4; of 48 x 64 47 -> 61, now 46; 300 of 5, 16 x 32, 20.7 -> 28.6, now 19.8).
+// What takes longer than before: 64 entries of 9 tokens of 32 x 64 and 48 x 64 (9 %), and 16 rows of state at 9 to 33 tokens of 64
+// to 200 entries (17.8 against 16.7, 41 against 37).
 template <int R, int COLS, int TILE>          // R rows of the state per thread: dim <= 16 * R
 __global__ __launch_bounds__(dw_threads(COLS)) void hgrn2_scan_kernel(float* __restrict__ out, const float* __restrict__ proj,
                                                                        int64_t proj_stride, const float* __restrict__ f_bias,
@@ -92,7 +94,7 @@ extern "C" int ga_hgrn2_scan(void* out, const void* proj, int64_t proj_stride, c
 #define GO(R, C, T) hipLaunchKernelGGL((hgrn2_scan_kernel<R, C, T>), dim3(entries, heads, (vdim + C - 1) / C), dim3(dw_threads(C)), 0, stream, \
                                        (float*)out, (const float*)proj, proj_stride, (const float*)f_bias, (const float*)lower,            \
                                        (float*)state, (const int64_t*)slots, (const int32_t*)cu, (const int32_t*)q_start, heads, dim, vdim)
-  DW_WAY(way, rows, GO);
+  DW_WAY(way, rows, dw_many(entries, heads, vdim), GO);
 #undef GO
   return GA_CHECK_LAUNCH();
 }

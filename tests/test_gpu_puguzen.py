@@ -310,6 +310,30 @@ def test_recurrences_of_many_entries_give_the_bits_of_one_alone(dim, n):
             assert torch.equal(one[e], many[e]), kind
 
 
+@pytest.mark.parametrize("n", [1, 2, 7, 8, 9, 16, 17, 25])
+@pytest.mark.parametrize("dim", [5, 16])
+def test_recurrences_of_so_many_entries_that_tiles_are_halved(dim, n):
+    """Up to 16 rows of state and more than 1,024 workgroups of 16 columns: 8 tokens at a time in place of 16, the same bits."""
+    from ginfer_amd.kernels import ops
+    E, heads, vdim = 65, 8, 17
+    assert E * heads * -(-vdim // 16) > 1024 and (n == 1 or ops.decay_walk_way(E * n, E, n, heads, dim, vdim) == 16)
+    g = torch.Generator().manual_seed(n)
+    proj = torch.randn((E * n, 2 * heads * dim + heads * vdim), generator=g).cuda()
+    decay = (torch.rand((E * n, heads * dim), generator=g) * 0.9 + 0.1).cuda()
+    bias, lower = torch.randn((heads * dim,), generator=g).cuda(), torch.rand((heads * dim,), generator=g).cuda()
+    state = torch.randn((E, heads, dim, vdim), generator=g).cuda()
+    runs = {
+        "channel": lambda p, d, st, sl, step: ops.decay_scan(p, 0, heads * dim, 2 * heads * dim, st, sl, step, heads, dim, vdim, decay=d),
+        "hgrn2": lambda p, d, st, sl, step: ops.hgrn2_scan(p, bias, lower, st, sl, step, heads, dim, vdim)}
+    for kind, run in runs.items():
+        many, one = state.clone(), state.clone()
+        got = run(proj, decay, many, torch.arange(E, device="cuda"), _Step([n] * E, [3] * E))
+        for e in (0, 31, E - 1):
+            rows = slice(e * n, (e + 1) * n)
+            alone = run(proj[rows], decay[rows].contiguous(), one, torch.tensor([e], device="cuda"), _Step([n], [3]))
+            assert torch.equal(alone, got[rows]) and torch.equal(one[e], many[e]), kind
+
+
 def test_heads_normed_and_gated():
     from ginfer_amd.kernels import ops
     g = torch.Generator().manual_seed(3)
