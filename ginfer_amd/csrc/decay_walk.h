@@ -23,14 +23,16 @@ __host__ __device__ constexpr int dw_threads(int cols) { return cols == 8 ? 384 
 
 // Source: `Fixed` (what a channel has for all tokens), fixed(channel), `Raw` (what a thread loads for one element of q, k and a),
 // load(Raw&, start, token, channel), finish(Raw, Fixed, channel, q, k, a), load_v(start, token, column), finish_v(v); finish and
-// finish_v are templates on whether `acts` is set.  `start` is the same for all threads, tokens count from it.  K_OF_A: k is 1 - a;
-// finish leaves it out and LDS, whose reads are what many entries wait for, does not hold it.
+// finish_v are templates on whether `acts` is set.  `start` is the same for all threads, tokens count from it.  K_OF_A: k is 1 - a,
+// and with 16 columns LDS, whose reads are what many entries wait for, does not hold it.  (With 8 columns it does: a chain waits for
+// its arithmetic, 2,048 tokens, 8 heads of 192 x 192, 443 us and 499 without.)
 template <int R, int COLS, int TILE, class Source>
 __device__ __forceinline__ void decay_walk(float* __restrict__ out, const Source& source, float* __restrict__ state, bool fresh,
                                            int n, int heads, int dim, int vdim, int v0) {
   constexpr int WALKERS = DW_SLICES * COLS, THREADS = dw_threads(COLS), SERVERS = THREADS > WALKERS ? THREADS - WALKERS : WALKERS;
   constexpr int DP = DW_SLICES * R, PER = (TILE * DP + SERVERS - 1) / SERVERS;
-  constexpr int OPS = Source::K_OF_A ? 2 : 3;                // q, k, unless it is 1 - a, and a
+  constexpr bool K_OF_A = Source::K_OF_A && COLS > 8;
+  constexpr int OPS = K_OF_A ? 2 : 3;                        // q, k, unless it is 1 - a, and a
   static_assert(TILE <= DW_SLICES, "tile sizes");
   __shared__ __attribute__((aligned(16))) float ops[2][TILE][OPS][DW_SLICES][R];
   __shared__ float vs[2][TILE][COLS], partial[2][TILE][DW_SLICES][COLS];
@@ -58,7 +60,7 @@ __device__ __forceinline__ void decay_walk(float* __restrict__ out, const Source
   // 128 x 128: 492 -> 530).  No load is conditional either way: what is loaded
   // must not be merged with what was there, which would wait for it.  (Channels and columns that do not exist read another and
   // drop it.)
-  constexpr bool WHOLE = COLS == 8 || (R >= 6 && R <= 12 && !Source::K_OF_A);
+  constexpr bool WHOLE = COLS == 8 || (R >= 6 && R <= 12 && !K_OF_A);
   auto start_of = [&](int t0) { return WHOLE ? max(min(t0, n - TILE), 0) : t0; };
   auto fetch = [&](int t0) {
     const int start = WHOLE ? start_of(t0) : min(t0, n - 1), last = min(TILE, WHOLE ? n : n - start) - 1;    // (WHOLE: of all tiles)
@@ -78,7 +80,7 @@ __device__ __forceinline__ void decay_walk(float* __restrict__ out, const Source
       if ((TILE * DP % SERVERS != 0 && tt >= TILE) || (decltype(few)::value && tt >= left)) break;
       source.template finish<ACT>(raw[x], fixed[x], min(i, dim - 1), q, k, a);
       ops[b][tt][0][i % DW_SLICES][i / DW_SLICES] = i < dim ? q : 0.f;
-      if constexpr (!Source::K_OF_A) ops[b][tt][1][i % DW_SLICES][i / DW_SLICES] = i < dim ? k : 0.f;
+      if constexpr (!K_OF_A) ops[b][tt][1][i % DW_SLICES][i / DW_SLICES] = i < dim ? k : 0.f;
       ops[b][tt][OPS - 1][i % DW_SLICES][i / DW_SLICES] = i < dim ? a : 0.f;
     }
     if (s < TILE) vs[b][s][j] = source.template finish_v<ACT>(raw_v);
@@ -94,7 +96,7 @@ __device__ __forceinline__ void decay_walk(float* __restrict__ out, const Source
   auto read = [&](int b, int tt, int at) {
     vx[at] = vs[b][tt][j];
 #pragma unroll
-    for (int r = 0; r < R; ++r) kx[at][r] = Source::K_OF_A ? 0.f : ops[b][tt][1][s][r];
+    for (int r = 0; r < R; ++r) kx[at][r] = K_OF_A ? 0.f : ops[b][tt][1][s][r];
 #pragma unroll
     for (int r = 0; r < R; ++r) ax[at][r] = ops[b][tt][OPS - 1][s][r];
 #pragma unroll
@@ -104,7 +106,7 @@ __device__ __forceinline__ void decay_walk(float* __restrict__ out, const Source
     float acc = 0.f;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      S[r] = fmaf(ax[at][r], S[r], (Source::K_OF_A ? 1.0f - ax[at][r] : kx[at][r]) * vx[at]);
+      S[r] = fmaf(ax[at][r], S[r], (K_OF_A ? 1.0f - ax[at][r] : kx[at][r]) * vx[at]);
       acc = fmaf(S[r], qx[at][r], acc);
     }
     partial[b][tt][s][j] = acc;
@@ -146,11 +148,15 @@ __device__ __forceinline__ void decay_walk(float* __restrict__ out, const Source
     }
     if (serves) {
       put(t0 - TILE, b ^ 1);
-      if (COLS == 8 || t0 + TILE < n) {
-        if (WHOLE) stage(b ^ 1, TILE, std::false_type());
-        else stage(b ^ 1, n - t0 - TILE, std::true_type());
+      if constexpr (WHOLE) {
+        if (COLS == 8 || t0 + TILE < n) {
+          stage(b ^ 1, TILE, std::false_type());
+          fetch(t0 + 2 * TILE);
+        }
+      } else {
+        if (t0 + TILE < n) stage(b ^ 1, n - t0 - TILE, std::true_type());
+        fetch(t0 + 2 * TILE);
       }
-      if (COLS == 8 || !WHOLE || t0 + TILE < n) fetch(t0 + 2 * TILE);
     }
   }
   __syncthreads();

@@ -30,9 +30,10 @@ struct ForgetRows {
     x.f = p[at + hd];
   }
   template <bool>
-  __device__ __forceinline__ void finish(const Raw& x, const Fixed& c, int i, float& q, float&, float& f) const {
+  __device__ __forceinline__ void finish(const Raw& x, const Fixed& c, int i, float& q, float& k, float& f) const {
     q = x.q * gr_sigmoid(x.q);
     f = c.lower + (1.0f - c.lower) * gr_sigmoid(x.f + c.bias);
+    k = 1.0f - f;
   }
   __device__ __forceinline__ float load_v(int start, int t, int c) const {
     return (v + start * stride)[(uint32_t)t * (uint32_t)stride + c];
@@ -42,8 +43,8 @@ struct ForgetRows {
 };
 
 // Measured on MI355X, the caches emptied before, us, before the walk of decay_walk.h -> now.  12 heads of 64 x 128: 2,048 tokens of
-// one request 534 -> 177; five entries of 918 262 -> 181; 495 tokens beside 16 single ones 136 -> 64; 64 entries of 33 79 -> 65,
-// of 9 34.1 -> 33.3, of one 24.5 -> 20.2.  28 heads of 128 x 128: 934 -> 514, 880 -> 563, 252 -> 191, 310 -> 244, 129 -> 121, 80 ->
+// one request 534 -> 181; five entries of 918 262 -> 183; 495 tokens beside 16 single ones 136 -> 64; 64 entries of 33 79 -> 65,
+// of 9 34.1 -> 33.3, of one 24.5 -> 20.2.  28 heads of 128 x 128: 934 -> 511, 880 -> 564, 252 -> 191, 310 -> 244, 129 -> 121, 80 ->
 // 70.  With k kept beside f in LDS, as the general walk has it, the reads of LDS made many entries slower than before (64 of 33
 // tokens, 16 heads of 32 x 64, 35.2 -> 37.9, now 35.4; of 48 x 64 47 -> 61, now 46; 300 of 5, 16 x 32, 20.7 -> 28.6, now 19.8).
 // What takes longer than before: 64 entries of 9 tokens of 32 x 64 and 48 x 64 (9 %), and 16 rows of state at 9 to 33 tokens of 64
