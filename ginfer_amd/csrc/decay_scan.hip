@@ -110,9 +110,12 @@ __global__ __launch_bounds__(dw_threads(COLS)) void decay_scan_kernel(
 }
 
 // decay[t, c] = exp(-softplus(-z) / tau), z = sum_r a2t[r, c] * low[t, r] + bias[c], the sum in ascending r.  a2t is the
-// widening matrix TRANSPOSED, [rank][channels]: neighbouring threads read neighbouring channels.  A workgroup takes GD_TOKENS
-// tokens and 256 channels; the tokens' narrow rows go through LDS and every element of a2t is read once for all of them.
+// widening matrix TRANSPOSED, [rank][channels]: neighbouring threads read neighbouring channels.  A workgroup takes 16 tokens and
+// 64 channels, a wavefront 4 of those tokens: what bounds it is the way of a2t's elements and the chain of the two exponentials and
+// the logarithm of a result, some hundred cycles each, so many short wavefronts go side by side; the four share a2t's rows in the
+// L1.  With 16 tokens to a thread and 256 channels to a workgroup 1 token took 13.9 us and 2,048 (768 channels, rank 64) 26.7, now 8.9 and 19.3.
 #define GD_TOKENS 16
+#define GD_EACH 4
 #define GD_BATCH 32
 __global__ __launch_bounds__(256) void gla_decay_kernel(float* __restrict__ decay, const float* __restrict__ low,
                                                         int64_t low_stride, const float* __restrict__ a2t,
@@ -120,37 +123,39 @@ __global__ __launch_bounds__(256) void gla_decay_kernel(float* __restrict__ deca
                                                         float inv_tau) {
   extern __shared__ float lows[];                      // [rank][GD_TOKENS]
   const int t0 = blockIdx.x * GD_TOKENS, nt = min(GD_TOKENS, tokens - t0);
-  for (int idx = threadIdx.x; idx < GD_TOKENS * rank; idx += 256) {
-    const int tt = idx / rank, r = idx % rank;
+  const int c = blockIdx.y * 64 + (threadIdx.x & 63), cc = min(c, channels - 1), first = (threadIdx.x >> 6) * GD_EACH;
+  float w[GD_BATCH];                                   // GD_BATCH elements of a2t are asked for at a time, the first of them
+  auto ask = [&](int r0) {                             // before the rows are laid out
+#pragma unroll
+    for (int j = 0; j < GD_BATCH; ++j) w[j] = a2t[(int64_t)min(r0 + j, rank - 1) * channels + cc];
+  };
+  if (first < nt) ask(0);
+  for (int tt = threadIdx.x % GD_TOKENS, r = threadIdx.x / GD_TOKENS; r < rank; r += 256 / GD_TOKENS)
     lows[r * GD_TOKENS + tt] = tt < nt ? low[(int64_t)(t0 + tt) * low_stride + r] : 0.f;
-  }
   __syncthreads();
-  const int c = blockIdx.y * 256 + threadIdx.x;
-  if (c >= channels) return;
-  float z[GD_TOKENS];
+  if (first >= nt || c >= channels) return;
+  float z[GD_EACH];
 #pragma unroll
-  for (int tt = 0; tt < GD_TOKENS; ++tt) z[tt] = 0.f;
-  for (int r0 = 0; r0 < rank; r0 += GD_BATCH) {        // GD_BATCH elements of a2t are asked for at a time: in a decode step
-    float w[GD_BATCH];                                 // every one comes from memory, a microsecond away
-#pragma unroll
-    for (int j = 0; j < GD_BATCH; ++j) w[j] = r0 + j < rank ? a2t[(int64_t)(r0 + j) * channels + c] : 0.f;
+  for (int tt = 0; tt < GD_EACH; ++tt) z[tt] = 0.f;
+  for (int r0 = 0; r0 < rank; r0 += GD_BATCH) {
+    if (r0) ask(r0);
 #pragma unroll
     for (int j = 0; j < GD_BATCH; ++j) {
       if (r0 + j < rank) {
-        const float* lo = lows + (r0 + j) * GD_TOKENS;
+        const float* lo = lows + (r0 + j) * GD_TOKENS + first;
 #pragma unroll
-        for (int tt = 0; tt < GD_TOKENS; ++tt) z[tt] = fmaf(w[j], lo[tt], z[tt]);
+        for (int tt = 0; tt < GD_EACH; ++tt) z[tt] = fmaf(w[j], lo[tt], z[tt]);
       }
     }
   }
   const float b = bias[c];
 #pragma unroll
-  for (int tt = 0; tt < GD_TOKENS; ++tt) {
-    if (tt < nt) {
+  for (int tt = 0; tt < GD_EACH; ++tt) {
+    if (first + tt < nt) {
       const float v = z[tt] + b;
       // log(sigmoid(v)) = -softplus(-v); far out the softplus is its argument
       const float sp = -v > 30.f ? -v : log1pf(expf(-v));
-      decay[(int64_t)(t0 + tt) * channels + c] = expf(-sp * inv_tau);
+      decay[(int64_t)(t0 + first + tt) * channels + c] = expf(-sp * inv_tau);
     }
   }
 }
@@ -339,7 +344,7 @@ extern "C" int ga_gla_decay(void* decay, const void* low, int64_t low_stride, co
   if (tokens <= 0) return 0;
   if (channels <= 0 || rank <= 0 || !(tau > 0.f)) return -1;
   if ((size_t)GD_TOKENS * rank * sizeof(float) > 48 * 1024) return -2;
-  dim3 grid((tokens + GD_TOKENS - 1) / GD_TOKENS, (channels + 255) / 256);
+  dim3 grid((tokens + GD_TOKENS - 1) / GD_TOKENS, (channels + 63) / 64);
   hipLaunchKernelGGL(gla_decay_kernel, grid, dim3(256), GD_TOKENS * rank * sizeof(float), stream, (float*)decay,
                      (const float*)low, low_stride, (const float*)a2t, (const float*)bias, tokens, channels, rank, 1.0f / tau);
   return GA_CHECK_LAUNCH();

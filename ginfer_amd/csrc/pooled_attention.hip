@@ -108,60 +108,86 @@ __device__ __forceinline__ int64_t pa_row(const int32_t* __restrict__ table, int
   return page < 0 ? -1 : (int64_t)page * page_size + (p - b * page_size);
 }
 
-// The mean over the block that ends at `pos` of one channel: eight rows are asked for at a time, without a branch in
-// between (a row that is not there is read at row 0 and left out), and added in the order of the positions.
-template <bool KEYS, typename TC>
+// The mean over the block that ends at `pos` of one channel, added in the order of the positions.  What bounds it is the way to
+// memory, which is gone twice for 64 rows: a lane looks up the page of one row, then all rows are asked for (16 at a time without a
+// branch in between; a row that has no page is read at row 0 and left out), of values, which lie position by position, 8 in one
+// load where blocks and pages are multiples of 8 (WIDE).  2,048 tokens of 2 heads of 128 in blocks of 64: 60 us with the pages
+// looked up for 8 rows at a time and a division for every one of them, now 11 with the workgroups below.
+template <bool KEYS, bool WIDE, typename TC>
 __device__ __forceinline__ float pa_block_mean(const TC* __restrict__ rows, const int32_t* __restrict__ bt, int width, int pos,
                                                int pool, int page_size, int nkv, int g, int w, int c) {
+  constexpr int BATCH = 64, GROUP = 16, STEP = WIDE ? 8 : 1;
+  const int lane = threadIdx.x & 63;
   float sum = 0.f;
-  for (int p0 = pos + 1 - pool; p0 <= pos; p0 += 8) {
-    int page[8], at[8];
+  for (int done = 0; done < pool; done += BATCH) {
+    const int p = pos + 1 - pool + done + lane, b = p / page_size, at_row = p - b * page_size;
+    const int page_row = done + lane < pool && b < width ? bt[b] : -1;
+    const uint64_t there = __ballot(page_row >= 0);
+    float x[BATCH];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int p = p0 + j <= pos ? p0 + j : pos;
-      const int b = p / page_size;
-      at[j] = p - b * page_size;
-      page[j] = bt[b < width ? b : width - 1];
-      if (b >= width || p0 + j > pos) page[j] = -1;
+    for (int j0 = 0; j0 < BATCH; j0 += GROUP) {
+      if (done + j0 >= pool) break;
+#pragma unroll
+      for (int j = j0; j < j0 + GROUP; j += STEP) {
+        const int page = __builtin_amdgcn_readlane(page_row, j), at = __builtin_amdgcn_readlane(at_row, j);
+        const int64_t pg = page < 0 ? 0 : page;
+        if constexpr (KEYS) {
+          x[j] = Num<TC>::ld(rows + ((pg * page_size + at) * nkv + g) * (int64_t)w + c);
+        } else {
+          const TC* src = rows + ((pg * nkv + g) * (int64_t)w + c) * page_size + at;
+          if constexpr (WIDE) {
+            struct alignas(16) Eight { TC v[8]; };
+            const Eight e = *reinterpret_cast<const Eight*>(src);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) x[j + i] = Num<TC>::ld(e.v + i);
+          } else {
+            x[j] = Num<TC>::ld(src);
+          }
+        }
+      }
     }
-    float x[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int64_t pg = page[j] < 0 ? 0 : page[j];
-      x[j] = KEYS ? Num<TC>::ld(rows + ((pg * page_size + at[j]) * nkv + g) * (int64_t)w + c)
-                  : Num<TC>::ld(rows + ((pg * nkv + g) * (int64_t)w + c) * page_size + at[j]);
-    }
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-      if (page[j] >= 0) sum += x[j];
+    for (int j = 0; j < BATCH; ++j)
+      if (there >> j & 1) sum += x[j];
   }
   return sum / (float)pool;
 }
 
-// grid (tokens, 2 nkv): the keys' and the values' heads of the block that a token ends
-template <typename TC>
+// grid (tokens / each, 2 nkv): the keys' and the values' heads of the blocks that `each` tokens end, one after the other.  A
+// workgroup whose token ends no block still has to be started: one a token cost 13 of 20 us at 2,048 tokens.
+template <bool WIDE, typename TC>
 __global__ __launch_bounds__(256) void pwa_pool_kernel(float* __restrict__ pk_rows, float* __restrict__ pv_rows,
                                                        const TC* __restrict__ k_rows, const TC* __restrict__ v_rows,
                                                        const int32_t* __restrict__ positions,
                                                        const int32_t* __restrict__ token_entry,
                                                        const int32_t* __restrict__ table, int width,
-                                                       const int64_t* __restrict__ pool_slots, int nkv, int dim, int vdim,
-                                                       int pool, int page_size) {
-  const int64_t t = blockIdx.x;
-  const int pos = positions[t];
-  if ((pos + 1) % pool) return;
-  const int64_t dst_row = pool_slots[t];
-  if (dst_row < 0) return;
-  const int32_t* bt = table + (int64_t)token_entry[t] * width;
-  if (blockIdx.y < (unsigned)nkv) {
-    const int g = blockIdx.y;
-    for (int c = threadIdx.x; c < dim; c += blockDim.x)
-      pk_rows[(dst_row * nkv + g) * (int64_t)dim + c] = pa_block_mean<true, TC>(k_rows, bt, width, pos, pool, page_size, nkv, g, dim, c);
-  } else {
-    const int g = blockIdx.y - nkv;
-    for (int c = threadIdx.x; c < vdim; c += blockDim.x)
-      pv_rows[pa_value_at(dst_row, g, c, nkv, vdim, page_size)] =
-          pa_block_mean<false, TC>(v_rows, bt, width, pos, pool, page_size, nkv, g, vdim, c);
+                                                       const int64_t* __restrict__ pool_slots, int tokens, int each, int nkv,
+                                                       int dim, int vdim, int pool, int page_size) {
+  const int64_t t0 = (int64_t)blockIdx.x * each;
+  const int lane = threadIdx.x & 63;
+  const bool ends = lane < each && t0 + lane < tokens && (positions[t0 + lane] + 1) % pool == 0;
+  for (uint64_t left = __ballot(ends); left; left &= left - 1) {
+    const int64_t t = t0 + __builtin_ctzll(left);
+    const int64_t dst_row = pool_slots[t];
+    if (dst_row < 0) continue;
+    const int pos = positions[t];
+    const int32_t* bt = table + (int64_t)token_entry[t] * width;
+    // all lanes look up pages, also those beyond the width
+    if (blockIdx.y < (unsigned)nkv) {
+      const int g = blockIdx.y;
+      for (int c0 = 0; c0 < dim; c0 += blockDim.x) {
+        const int c = c0 + threadIdx.x;
+        const float mean = pa_block_mean<true, false, TC>(k_rows, bt, width, pos, pool, page_size, nkv, g, dim, min(c, dim - 1));
+        if (c < dim) pk_rows[(dst_row * nkv + g) * (int64_t)dim + c] = mean;
+      }
+    } else {
+      const int g = blockIdx.y - nkv;
+      for (int c0 = 0; c0 < vdim; c0 += blockDim.x) {
+        const int c = c0 + threadIdx.x;
+        const float mean = pa_block_mean<false, WIDE, TC>(v_rows, bt, width, pos, pool, page_size, nkv, g, vdim, min(c, vdim - 1));
+        if (c < vdim) pv_rows[pa_value_at(dst_row, g, c, nkv, vdim, page_size)] = mean;
+      }
+    }
   }
 }
 
@@ -266,10 +292,15 @@ extern "C" int ga_pwa_pool(void* pk_rows, void* pv_rows, const void* k_rows, con
   if (tokens <= 0) return 0;
   if (nkv <= 0 || 2 * nkv > 65535 || dim <= 0 || vdim <= 0 || pool <= 0 || page_size <= 0 || width <= 0) return -1;
   const int widest = dim > vdim ? dim : vdim;          // a thread a channel: the chains of a block's sum run side by side
-  dim3 grid(tokens, 2 * nkv), block(widest <= 64 ? 64 : widest <= 128 ? 128 : 256);
-#define GO(T) hipLaunchKernelGGL(pwa_pool_kernel<T>, grid, block, 0, stream, (float*)pk_rows, (float*)pv_rows,            \
+  // few tokens, mostly single ones whose blocks end as it happens: a workgroup each, so that no two wait for one another; many are
+  // mostly neighbours, of which one in `pool` ends a block
+  const int each = tokens < 512 ? 1 : 8;
+  dim3 grid((tokens + each - 1) / each, 2 * nkv), block(widest <= 64 ? 64 : widest <= 128 ? 128 : 256);
+  const bool wide = pool % 8 == 0 && page_size % 8 == 0 && (uintptr_t)v_rows % 16 == 0;
+#define GO(T) hipLaunchKernelGGL((wide ? pwa_pool_kernel<true, T> : pwa_pool_kernel<false, T>), grid, block, 0, stream,   \
+                                 (float*)pk_rows, (float*)pv_rows,                                                        \
                                  (const T*)k_rows, (const T*)v_rows, (const int32_t*)positions, (const int32_t*)token_entry, \
-                                 (const int32_t*)table, width, (const int64_t*)pool_slots, nkv, dim, vdim, pool, page_size)
+                                 (const int32_t*)table, width, (const int64_t*)pool_slots, tokens, each, nkv, dim, vdim, pool, page_size)
   if (cache_bf16) GO(bf16_t); else GO(float);
 #undef GO
   return GA_CHECK_LAUNCH();

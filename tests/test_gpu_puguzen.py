@@ -390,6 +390,62 @@ class _AttentionCase:
         return torch.cat(out)
 
 
+@pytest.mark.parametrize("tokens", [5, 511, 513, 1030])          # a workgroup a token, and one for eight of them
+@pytest.mark.parametrize("pool, page", [(1, 8), (7, 16), (8, 8), (12, 4), (24, 16), (64, 16), (72, 8), (130, 16)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_block_means_are_the_sums_in_order(tokens, pool, page, dtype):
+    """Bit for bit the mean of the block's rows, added in the order of their positions; rows without a page are left out."""
+    from types import SimpleNamespace
+    from ginfer_amd.kernels import ops
+    g = torch.Generator().manual_seed(tokens + pool)
+    nkv, dim, vdim = 2, 66, 130
+    lengths = [tokens - 2 * (tokens // 3), tokens // 3, tokens // 3]
+    starts = [pool + 3, 0, 2 * pool - 1]
+    width = -(-max(s + n for s, n in zip(starts, lengths)) // page)
+    pages = 3 * width
+    table = torch.randperm(pages, generator=g).to(torch.int32).view(3, width)
+    table[0, 0] = -1                                              # a page that was given back
+    k = torch.randn((pages, page, nkv, dim), generator=g).to(dtype)
+    v = torch.randn((pages, nkv, vdim, page), generator=g).to(dtype)
+    pos = torch.cat([torch.arange(s, s + n) for s, n in zip(starts, lengths)]).to(torch.int32)
+    ent = torch.repeat_interleave(torch.arange(3), torch.tensor(lengths)).to(torch.int32)
+    ends = [t for t in range(tokens) if (int(pos[t]) + 1) % pool == 0]
+    slots = torch.full((tokens,), -1, dtype=torch.int64)
+    for i, t in enumerate(ends[:-1] if len(ends) > 2 else ends):  # one that ends a block keeps no mean
+        slots[t] = i
+    out_pages = max(1, -(-len(ends) // page))
+    pk, pv = torch.zeros((out_pages * page, nkv, dim)).cuda(), torch.zeros((out_pages, nkv, vdim, page)).cuda()
+    step = SimpleNamespace(positions=pos.cuda(), token_entry=ent.cuda(), cu_tokens=torch.zeros(4, dtype=torch.int32).cuda())
+    ops.pooled_attention_pool(pk, pv, k.view(-1, nkv, dim).cuda(), v.cuda(), step, table.cuda(), slots.cuda(), nkv, dim, vdim, pool, page)
+    pk, pv = pk.cpu(), pv.cpu()
+    for t in ends[:20] + ends[-20:]:
+        i = int(slots[t])
+        if i < 0:
+            continue
+        sk, sv = torch.zeros((nkv, dim)), torch.zeros((nkv, vdim))
+        for p in range(int(pos[t]) + 1 - pool, int(pos[t]) + 1):
+            pg = int(table[int(ent[t]), p // page])
+            if pg >= 0:
+                sk, sv = sk + k[pg, p % page].float(), sv + v[pg, :, :, p % page].float()
+        assert torch.equal(pk[i], sk / pool) and torch.equal(pv[i // page, :, :, i % page], sv / pool), (t, i)
+    used = int((slots >= 0).sum())
+    assert not pk[used:].any()
+
+
+@pytest.mark.parametrize("tokens", [1, 4, 5, 15, 16, 17, 33])     # a wavefront's four, a workgroup's sixteen
+@pytest.mark.parametrize("channels, rank", [(63, 31), (64, 32), (65, 33), (200, 70)])
+def test_decay_at_the_edges_of_its_workgroups(tokens, channels, rank):
+    from ginfer_amd.kernels import ops
+    g = torch.Generator().manual_seed(tokens)
+    proj = torch.randn((tokens, 3 + rank), generator=g)
+    a2, b = torch.randn((channels, rank), generator=g), torch.randn((channels,), generator=g)
+    got = ops.gla_decay(proj.cuda(), 3, a2.t().contiguous().cuda(), b.cuda(), 16.0).cpu()
+    want = torch.sigmoid(proj[:, 3:].double() @ a2.double().T + b.double()) ** (1 / 16.0)
+    # a result below 1: half a place of it is 3e-8; the sum of up to 70 products, some 50 at most, is off by 70 * 50 * 6e-8 at worst
+    # and enters by 1/16
+    assert got.shape == want.shape and float((got.double() - want).abs().max()) < 70 * 50 * 6e-8 / 16
+
+
 def _split(proj, nh, nkv, dim, vdim, dtype):
     """q, k, v of a projection as the kernels hold them: q in 32-bit, k and v rounded as the cache rounds them."""
     T = proj.shape[0]
