@@ -7,27 +7,18 @@
 // A workgroup of 8 wavefronts owns NT*16 rows of W (output columns) and all M rows of A; the wavefronts
 // split K and add their parts up through LDS in a fixed order.  v_mfma_f32_16x16x32_bf16 with W as the
 // first operand: lane l supplies W[n0 + l%16][k-slots] and A[l%16][k-slots] and receives
-// D[n = (l/16)*4+i][m = l%16].  Both operands come straight from global memory in 16-byte loads, no LDS
-// staging: the k-slots of a lane are 8 consecutive elements, and since a sum over k may take its terms
-// in any order as long as both operands agree, lane group g = l/16 takes the 16 elements
-// [k + 16g, k + 16g + 16) of every 64-element step as two products, so that the four lanes of a row read
-// 128 consecutive bytes.
+// D[n = (l/16)*4+i][m = l%16].  Both operands come from global memory in 16-byte loads, 8 lanes to a row, and turn into
+// that layout in the wavefront's own piece of LDS (SkinnyTrip).
 #include "common.h"
 #include "ginfer_amd.h"   // the entry points below are checked against their declarations
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
+typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 
 #define SK_WAVES 8
 #define SK_THREADS (SK_WAVES * 64)
 
-__device__ __forceinline__ bf16x8 zero8() {
-  uint4 z = {0u, 0u, 0u, 0u};
-  return __builtin_bit_cast(bf16x8, z);
-}
-__device__ __forceinline__ bf16x8 load8(const bf16_t* p) {
-  return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(p));
-}
 
 // A root-mean-square norm folded into the two products around it (ginfer/core/op/kernels/cuda/rmsnorm_kernel.cu:27-66
 // is the norm itself: y = x * g / sqrtf(sum(x^2) / width + eps)).  The product BEFORE the norm adds its result
@@ -82,49 +73,92 @@ struct NormInLoads {
 };
 
 // The wavefront's share of the sum over k: UNROLL steps of 64 elements per trip, all loads of a trip issued
-// before its products.  The trips run over [kb, kend), the same for every lane; a lane's own pointers may be
+// before its products.  The trips run over [0, kend), the same for every lane; a lane's own pointers may be
 // shifted (a packed tile, below) and its own range ends at ke: the guard on every 8-element piece makes the
 // tail safe (a piece past the end is zeros and touches no memory).  The terms are added in ascending k.
+//
+// A load brings 8 rows of an operand's tile of 16, 128 bytes of each: lane l brings piece l % 8 of row l / 8.  The matrix cores
+// want row l % 16 in lane l, but neighbouring lanes in different rows cost the address unit a cycle a lane, 16 bytes a cycle and
+// compute unit, measured from L2 and L1 alike, where 8 lanes to 128 bytes get 56: that rate, of weights and rows of A together, was
+// what these products waited for wherever A is not small beside the weights.  So every tile goes through LDS, a wavefront's own
+// 2 KB, two of them in turn: written and read by one wavefront, in order, without a barrier; the sums are the same, in the
+// same order.  us as replays of a graph over many layers' weights, before -> after, at 1, 8 and 16 rows: 1,536 columns of a K of 8,960
+// with the folded norm 9.1 -> 9.2, 12.4 -> 9.9, 16.7 -> 13.5; 3,584 of 18,944 28.5 -> 27.4, 35.5 -> 27.1, 43.5 -> 30.8; q|k|v of 28
+// heads and K 3,584 13.1 -> 10.0, 15.2 -> 10.8, 16.1 -> 11.1; at 64 rows 28.1 -> 18.3.
+// UNROLL is 1 wherever several workgroups share a compute unit: their wavefronts cover each other's trips, and longer trips were up
+// to three times slower, spread over fewer of them.  A workgroup alone on its unit with a long K takes 3 (K 8,960: 11.6 us with 1,
+// 10.1 with 2, 9.2 with 3, 10.1 with 4); two trips under way at once were slower than one everywhere.
+template <int NT, int MB>
+struct SkinnySource {
+  const bf16_t* wp[NT][2];                 // the lane's rows of each tile: l / 8 and 8 more
+  const bf16_t* ap[MB][2];
+  bool wok[NT][2], aok[MB][2];
+  int ke[2], kend;
+};
+// 16 rows of 8 pieces of 16 bytes; piece p of row r lies at p ^ (r / 2): 16 lanes that read one piece of 16 rows meet all banks once
+#define SK_TILE_PIECES 128
 template <int NT, int MB, int UNROLL>
 struct SkinnyTrip {
-  bf16x8 a[UNROLL][2][NT], b[UNROLL][2][MB];
-  __device__ __forceinline__ void load(const bf16_t* const (&wp)[NT], const bool (&wok)[NT],
-                                       const bf16_t* const (&ap)[MB], const bool (&aok)[MB], int k, int ke, int g) {
+  u32x4 a[UNROLL][NT][2], b[UNROLL][MB][2];
+  __device__ __forceinline__ void load(const SkinnySource<NT, MB>& src, int k, int lane) {
+    const u32x4 zero = {0u, 0u, 0u, 0u};
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u)
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        const int kk = k + u * 64 + j * 32 + g * 8;
-        const bool ok = kk < ke;
+        const int kk = k + u * 64 + (lane & 7) * 8;
+        const bool ok = kk < src.ke[j];
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) a[u][j][nt] = (ok && wok[nt]) ? load8(wp[nt] + kk) : zero8();
+        for (int nt = 0; nt < NT; ++nt) a[u][nt][j] = (ok && src.wok[nt][j]) ? *reinterpret_cast<const u32x4*>(src.wp[nt][j] + kk) : zero;
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) b[u][j][mb] = (ok && aok[mb]) ? load8(ap[mb] + kk) : zero8();
+        for (int mb = 0; mb < MB; ++mb) b[u][mb][j] = (ok && src.aok[mb][j]) ? *reinterpret_cast<const u32x4*>(src.ap[mb][j] + kk) : zero;
       }
   }
-  __device__ __forceinline__ void multiply(f32x4 (&acc)[NT][MB]) const {
+  __device__ __forceinline__ void multiply(f32x4 (&acc)[NT][MB], u32x4* area, int lane) const {
+    const int row = lane >> 3, piece = lane & 7, m = lane & 15, g = lane >> 4;
+    u32x4* const put[2] = {area + row * 8 + (piece ^ (row >> 1)), area + (row + 8) * 8 + (piece ^ ((row + 8) >> 1))};
+    const u32x4* const get[2] = {area + m * 8 + (g ^ (m >> 1)), area + m * 8 + ((4 + g) ^ (m >> 1))};
+    auto through = [&](const u32x4 (&v)[2], bf16x8 (&out)[2], int slot) {
 #pragma unroll
-    for (int u = 0; u < UNROLL; ++u)
+      for (int j = 0; j < 2; ++j) put[j][slot * SK_TILE_PIECES] = v[j];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int h = 0; h < 2; ++h) out[h] = __builtin_bit_cast(bf16x8, get[h][slot * SK_TILE_PIECES]);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    };
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
+    for (int u = 0; u < UNROLL; ++u) {
+      bf16x8 y[MB][2];
 #pragma unroll
-          for (int mb = 0; mb < MB; ++mb)
-            acc[nt][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][j][nt], b[u][j][mb], acc[nt][mb], 0, 0, 0);
+      for (int mb = 0; mb < MB; ++mb) through(b[u][mb], y[mb], (u * (NT + MB) + mb) & 1);
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) {
+        bf16x8 x[2];
+        through(a[u][nt], x, (u * (NT + MB) + MB + nt) & 1);
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int mb = 0; mb < MB; ++mb) acc[nt][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[h], y[mb][h], acc[nt][mb], 0, 0, 0);
+      }
+    }
   }
 };
 
-template <int NT, int MB, int UNROLL = ((NT * MB <= 4) ? 4 : 2)>
-__device__ __forceinline__ void skinny_accumulate(f32x4 (&acc)[NT][MB], const bf16_t* const (&wp)[NT],
-                                                  const bool (&wok)[NT], const bf16_t* const (&ap)[MB],
-                                                  const bool (&aok)[MB], int kb, int kend, int ke, int g) {
-  for (int k = kb; k < kend; k += 64 * UNROLL) {
+template <int NT, int MB, int UNROLL>
+__device__ __forceinline__ void skinny_accumulate(f32x4 (&acc)[NT][MB], const SkinnySource<NT, MB>& src, u32x4* area, int lane) {
+  for (int k = 0; k < src.kend; k += 64 * UNROLL) {
     SkinnyTrip<NT, MB, UNROLL> trip;
-    trip.load(wp, wok, ap, aok, k, ke, g);
-    trip.multiply(acc);
+    trip.load(src, k, lane);
+    __builtin_amdgcn_sched_barrier(0);         // no load moves behind a product
+    trip.multiply(acc, area, lane);
   }
 }
+// a wavefront's LDS: two tiles under way, and in their place, at the end, its sums: [NT * 16][MB * 16 + 1]
+template <int NT, int MB>
+struct SkinnyArea {
+  static constexpr int SUMS = NT * 16 * (MB * 16 + 1) * 4, TILES = 2 * SK_TILE_PIECES * 16;
+  static constexpr int BYTES = ((SUMS > TILES ? SUMS : TILES) + 15) / 16 * 16;
+};
 
 // A PACKED tile (PACK == 2, at most 8 rows of A): with so few rows half of the matrix core's 16 x 16 tile
 // would hold nothing, so the tile takes 8 rows of W twice, for the two halves of the wavefront's K range:
@@ -135,9 +169,8 @@ __device__ __forceinline__ void skinny_accumulate(f32x4 (&acc)[NT][MB], const bf
 template <int PACK>
 struct Packed {
   static constexpr int CP = 16 / PACK;     // columns of W in a tile = most rows of A
-  // lane row r of a tile: its column of W (and row of A), and its half of K
+  // row r of a tile: its column of W (and row of A); its half of K is r / CP
   static __device__ __forceinline__ int col(int r) { return r % CP; }
-  static __device__ __forceinline__ int seg(int r) { return r / CP; }
 };
 
 // How K is dealt out: in steps of 64 elements, as evenly as whole steps allow, to `units` consumers (the
@@ -147,17 +180,16 @@ struct Packed {
 // trips (the longer of its halves).
 template <int PACK>
 struct KRange {
-  int shift, ke, kend;
-  __device__ __forceinline__ KRange(int first_unit, int seg, int steps, int units, int K) {
+  int shift[2], ke[2], kend;               // of tile rows 0 to 7 and 8 to 15
+  __device__ __forceinline__ KRange(int first_unit, int steps, int units, int K) {
     int longest = 0;
 #pragma unroll
-    for (int q = 0; q < PACK; ++q) {
+    for (int j = 0; j < 2; ++j) {
+      const int q = PACK == 2 ? j : 0;
       const int b = (int)(((int64_t)(first_unit + q) * steps) / units), e = (int)(((int64_t)(first_unit + q + 1) * steps) / units);
       longest = e - b > longest ? e - b : longest;
-      if (q == seg) {
-        shift = b * 64;
-        ke = (e * 64 < K ? e * 64 : K) - b * 64;
-      }
+      shift[j] = b * 64;
+      ke[j] = (e * 64 < K ? e * 64 : K) - b * 64;
     }
     kend = longest * 64;
   }
@@ -185,7 +217,7 @@ __device__ __forceinline__ float gate_act(float v, float u, const GateAct act) {
   return (v * (1.0f / (1.0f + expf(-(act.alpha * v))))) * (u + act.shift);
 }
 
-template <int NT, int MB, int KS, typename TC, bool GATED, int PACK>
+template <int NT, int MB, int KS, typename TC, bool GATED, int PACK, int UNROLL = 1>
 __global__ __launch_bounds__(SK_THREADS) void gemm_skinny_kernel(TC* __restrict__ C, int64_t ldc,
                                                                  const bf16_t* __restrict__ A, int64_t lda,
                                                                  const bf16_t* __restrict__ W,
@@ -193,12 +225,14 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_skinny_kernel(TC* __restrict_
                                                                  int K, int ksteps, NormIn norm_in,
                                                                  NormOut norm_out, int fold_cols, GateAct act) {
   static_assert(PACK == 1 || MB == 1, "a packed tile holds at most 8 rows of A");
-  __shared__ float red[SK_WAVES][NT * 16][MB * 16 + 1];
+  using Area = SkinnyArea<NT, MB>;
+  __shared__ __attribute__((aligned(16))) unsigned char area[SK_WAVES][Area::BYTES];
   __shared__ float rstd[16];
   using P = Packed<PACK>;
   constexpr int CP = P::CP;
   constexpr int GROUPS = SK_WAVES / KS;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+  auto red = [&](int w, int n, int m) -> float& { return reinterpret_cast<float*>(area[w])[n * (MB * 16 + 1) + m]; };
   const int grp = wave / KS, ks = wave % KS;
   constexpr int NCOL = GATED ? CP : NT * CP;       // output columns of a group
   // A product that folds the norm after it owns `fold_cols` (<= CP) columns per workgroup: as many as spread the
@@ -207,24 +241,25 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_skinny_kernel(TC* __restrict_
   const bool fuse_out = !GATED && NT == 1 && KS == SK_WAVES && MB == 1 && norm_out.residual != nullptr;
   const int my_cols = fuse_out ? fold_cols : NCOL;
   const int n0 = fuse_out ? blockIdx.x * fold_cols : (blockIdx.x * GROUPS + grp) * NCOL;
-  const KRange<PACK> kr((blockIdx.y * KS + ks) * PACK, P::seg(r), ksteps, gridDim.y * KS * PACK, K);
-  const int shift = kr.shift;
-
-  const bf16_t* wp[NT];
-  bool wok[NT];
+  const KRange<PACK> kr((blockIdx.y * KS + ks) * PACK, ksteps, gridDim.y * KS * PACK, K);
+  SkinnySource<NT, MB> src;
+  src.kend = kr.kend;
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    const int n = GATED ? n0 + P::col(r) : n0 + nt * CP + P::col(r);
-    wok[nt] = n < N && (!fuse_out || P::col(r) < my_cols);
-    wp[nt] = W + ((int64_t)(wok[nt] ? n : 0) + (GATED ? (int64_t)nt * N : 0)) * K + shift;
-  }
-  const bf16_t* ap[MB];
-  bool aok[MB];
+  for (int j = 0; j < 2; ++j) {
+    const int tr = (lane >> 3) + 8 * j;            // the row of a tile that the lane brings a piece of
+    src.ke[j] = kr.ke[j];
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb) {
-    const int m = mb * 16 + P::col(r);
-    aok[mb] = m < M;
-    ap[mb] = A + (int64_t)(aok[mb] ? m : 0) * lda + shift;
+    for (int nt = 0; nt < NT; ++nt) {
+      const int n = GATED ? n0 + P::col(tr) : n0 + nt * CP + P::col(tr);
+      src.wok[nt][j] = n < N && (!fuse_out || P::col(tr) < my_cols);
+      src.wp[nt][j] = W + ((int64_t)(src.wok[nt][j] ? n : 0) + (GATED ? (int64_t)nt * N : 0)) * K + kr.shift[j];
+    }
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+      const int m = mb * 16 + P::col(tr);
+      src.aok[mb][j] = m < M;
+      src.ap[mb][j] = A + (int64_t)(src.aok[mb][j] ? m : 0) * lda + kr.shift[j];
+    }
   }
   f32x4 acc[NT][MB];
 #pragma unroll
@@ -244,7 +279,7 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_skinny_kernel(TC* __restrict_
     }
   }
 
-  skinny_accumulate<NT, MB>(acc, wp, wok, ap, aok, 0, kr.kend, kr.ke, g);
+  skinny_accumulate<NT, MB, UNROLL>(acc, src, reinterpret_cast<u32x4*>(area[wave]), lane);
   if (MB == 1) in_loads.finish(norm_in, rstd, M, wave, lane);
   // the KS parts of a group meet in LDS and are added in wavefront order, the halves of a packed tile in theirs
 #pragma unroll
@@ -252,7 +287,7 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_skinny_kernel(TC* __restrict_
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) red[wave][nt * 16 + g * 4 + i][mb * 16 + r] = acc[nt][mb][i];
+      for (int i = 0; i < 4; ++i) red(wave, nt * 16 + g * 4 + i, mb * 16 + r) = acc[nt][mb][i];
   __syncthreads();
   const bool scale_rows = MB == 1 && norm_in.sumsq != nullptr;
   // element (column nl of tile t, row m) of group gi, summed over its wavefronts and halves
@@ -261,7 +296,7 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_skinny_kernel(TC* __restrict_
 #pragma unroll
     for (int w = 0; w < KS; ++w)
 #pragma unroll
-      for (int q = 0; q < PACK; ++q) v += red[gi * KS + w][t * 16 + q * CP + nl][(m / CP) * 16 + q * CP + m % CP];
+      for (int q = 0; q < PACK; ++q) v += red(gi * KS + w, t * 16 + q * CP + nl, (m / CP) * 16 + q * CP + m % CP);
     return v;
   };
   if (fuse_out) {
@@ -323,48 +358,52 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_even_kernel(TC* __restrict__ 
                                                                int ksteps, NormIn norm_in, GateAct act) {
   static_assert(!GATED || TILES % 2 == 0, "as many tiles of the gate as of the up matrix");
   constexpr int PER = GATED ? TILES / 2 : TILES;             // tiles of one matrix
-  __shared__ float red[SK_WAVES][TILES * 16][16 + 1];
+  using Area = SkinnyArea<TILES, 1>;
+  __shared__ __attribute__((aligned(16))) unsigned char area[SK_WAVES][Area::BYTES];
   __shared__ float rstd[16];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+  auto red = [&](int w, int n, int m) -> float& { return reinterpret_cast<float*>(area[w])[n * 17 + m]; };
   const int c0 = (int)(((int64_t)blockIdx.x * N) / gridDim.x), c1 = (int)(((int64_t)(blockIdx.x + 1) * N) / gridDim.x);
   const int cols = c1 - c0;                                  // <= PER * 16 by the launcher's choice of the grid
-  const KRange<1> kr(wave, 0, ksteps, SK_WAVES, K);
-  const bf16_t* wp[TILES];
-  bool wok[TILES];
+  const KRange<1> kr(wave, ksteps, SK_WAVES, K);
+  SkinnySource<TILES, 1> src;
+  src.kend = kr.kend;
 #pragma unroll
-  for (int t = 0; t < TILES; ++t) {
-    const int cl = (t % PER) * 16 + r;                       // the lane's column within the workgroup's range
-    wok[t] = cl < cols;
-    wp[t] = W + ((int64_t)(wok[t] ? c0 + cl : 0) + (GATED && t >= PER ? (int64_t)N : 0)) * K + kr.shift;
+  for (int j = 0; j < 2; ++j) {
+    const int tr = (lane >> 3) + 8 * j;                      // the row of a tile that the lane brings a piece of
+    src.ke[j] = kr.ke[j];
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) {
+      const int cl = (t % PER) * 16 + tr;                    // its column within the workgroup's range
+      src.wok[t][j] = cl < cols;
+      src.wp[t][j] = W + ((int64_t)(src.wok[t][j] ? c0 + cl : 0) + (GATED && t >= PER ? (int64_t)N : 0)) * K + kr.shift[j];
+    }
+    src.aok[0][j] = tr < M;
+    src.ap[0][j] = A + (int64_t)(src.aok[0][j] ? tr : 0) * lda + kr.shift[j];
   }
-  const bf16_t* ap[1];
-  bool aok[1];
-  aok[0] = r < M;
-  ap[0] = A + (int64_t)(aok[0] ? r : 0) * lda + kr.shift;
   f32x4 acc[TILES][1];
 #pragma unroll
   for (int t = 0; t < TILES; ++t) acc[t][0] = f32x4{0.f, 0.f, 0.f, 0.f};
   NormInLoads in_loads;
   in_loads.load(norm_in, M, wave, lane);
-  // steps of K asked for at once: fewer with more tiles, whose loads fill the registers
-  skinny_accumulate<TILES, 1, (TILES <= 2 ? 4 : TILES <= 4 ? 2 : 1)>(acc, wp, wok, ap, aok, 0, kr.kend, kr.ke, g);
+  skinny_accumulate<TILES, 1, 1>(acc, src, reinterpret_cast<u32x4*>(area[wave]), lane);
   in_loads.finish(norm_in, rstd, M, wave, lane);
 #pragma unroll
   for (int t = 0; t < TILES; ++t)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) red[wave][t * 16 + g * 4 + i][r] = acc[t][0][i];
+    for (int i = 0; i < 4; ++i) red(wave, t * 16 + g * 4 + i, r) = acc[t][0][i];
   __syncthreads();
   const bool scale_rows = norm_in.sumsq != nullptr;
   for (int idx = threadIdx.x; idx < cols * M; idx += SK_THREADS) {
     const int cl = idx % cols, m = idx / cols;
     float v = 0.f;
 #pragma unroll
-    for (int w = 0; w < SK_WAVES; ++w) v += red[w][cl][m];            // in wavefront order, as in the kernel above
+    for (int w = 0; w < SK_WAVES; ++w) v += red(w, cl, m);            // in wavefront order, as in the kernel above
     if (scale_rows) v *= rstd[m];
     if (GATED) {
       float u = 0.f;
 #pragma unroll
-      for (int w = 0; w < SK_WAVES; ++w) u += red[w][PER * 16 + cl][m];
+      for (int w = 0; w < SK_WAVES; ++w) u += red(w, PER * 16 + cl, m);
       if (scale_rows) u *= rstd[m];
       v = gate_act(v, u, act);
     } else if (bias) {
@@ -393,32 +432,21 @@ static int auto_pack(int M, int workgroups_of_full_tiles) {
 // The gated product of up to 16 rows goes to the kernel that deals its columns evenly from this many (activation)
 // columns on: a workgroup then has at least 8 of them.
 #define GA_GATED_EVEN_MIN_COLUMNS 2048
-// Its workgroups: the multiple of GA_FOLD_TARGET that comes nearest to 12 columns a workgroup with up to 4 rows (and up
-// to 8 rows of a K of up to 2,048), 28 with up to 8 rows, 32 beyond, and never more than 48 (three tiles).  Measured on
-// MI355X as replays of a graph that walks 28 layers' weights, in us, before -> after (columns a workgroup), at 1, 8 and
-// 16 rows: 8,960 x 1,536: 16.7 -> 13.2 (12), 18.2 -> 15.7 (12), 20.5 -> 17.1 (35); 4,864 x 896: 8.5 -> 6.5 (10),
-// 9.2 -> 7.2 (10), 10.0 -> 8.0 (19); 11,008 x 2,048: 22.7 -> 18.9 (11), 24.8 -> 23.3 (11), 27.2 -> 26.7 (43);
-// 18,944 x 3,584: 57.4 -> 51.0 (13), 63.1 -> 60.3 (25), 71.7 -> 63.5 (37); 13,824 x 5,120: 63.9 -> 54.8 (11),
-// 71.6 -> 63.6 (27), 82.3 -> 68.7 (27); 29,568 x 8,192: 183 -> 169 (12), 200 -> 191 (29), 234 -> 206 (29).
+// Its workgroups: the multiple of GA_FOLD_TARGET that comes nearest to 14 columns a workgroup, and never more than 48 (three
+// tiles).  Measured on MI355X as replays of a graph that walks many layers' weights, in us, at 1, 8 and 16 rows: 8,960 x 1,536:
+// 13.1, 13.3, 13.8 with 35 columns, 13.4, 13.5, 13.8 with 18, 13.0, 12.9, 13.4 with 12, 12.6, 12.9, 14.5 with 9; 11,008 x 2,048:
+// 21.4, 21.1, 21.9 with 43, 20.6, 20.1, 20.8 with 22, 18.5, 18.9, 19.8 with 14; 18,944 x 3,584: 48 to 50 from 12 columns to 37, at 16
+// rows 52 with 12.  (With operands that came straight from memory in the matrix cores' layout: 13.1, 15.9, 17.0; 18.9, 23.3, 26.7;
+// 53.1, 59.9, 63.7.)
 // The plain product of up to 16 rows and at least this many columns (the head) is dealt the same way, to workgroups of
-// up to 6 tiles; 0: the kernel above keeps it.  Its thousands of small workgroups are even enough by their number, so
-// less is gained: measured on MI355X at 151,936 x 1,536 with 32-bit sums out, in us, before -> after (columns a
-// workgroup) at 1, 8 and 16 rows: 92.5 -> 86.0 (25), 109.9 -> 106.9 (75), 129.4 -> 113.5 (75); 152,064 x 3,584:
-// 186 -> 183 (16), 237 -> 227 (85), 298 -> 240 (85); 152,064 x 8,192: 410 and 410 (16), 486 -> 481 (60), 625 -> 515 (85).
+// up to 6 tiles, of about 64 columns: 151,936 x 1,536 with 32-bit sums out, in us at 1, 8 and 16 rows: 85.3, 88.3, 94.2 with 85
+// columns, 81.7, 88.1, 93.9 with 66, 83.2, 91.8, 100.7 with 33 (before: 88.8, 108.6, 115.6); 152,064 x 3,584: 188, 191, 196 with 66,
+// 188, 197, 220 with 25 (before: 187, 235, 248).
 #define GA_PLAIN_EVEN_MIN_COLUMNS 16384
-static int plain_even_workgroups(int M, int N, int K) {
-  if (M <= 4 && K > 2048) return 0;
-  const int target = M <= 4 ? 24 : 80;
+static int even_workgroups(int N, int target, int most) {
   int rounds = (N + GA_FOLD_TARGET * target / 2) / (GA_FOLD_TARGET * target);
   if (rounds < 1) rounds = 1;
-  while ((N + GA_FOLD_TARGET * rounds - 1) / (GA_FOLD_TARGET * rounds) > 96) ++rounds;
-  return GA_FOLD_TARGET * rounds;
-}
-static int gated_even_workgroups(int M, int N, int K) {
-  const int target = M <= 4 ? 12 : M <= 8 ? (K <= 2048 ? 12 : 28) : 32;
-  int rounds = (N + GA_FOLD_TARGET * target / 2) / (GA_FOLD_TARGET * target);
-  if (rounds < 1) rounds = 1;
-  while ((N + GA_FOLD_TARGET * rounds - 1) / (GA_FOLD_TARGET * rounds) > 48) ++rounds;
+  while ((N + GA_FOLD_TARGET * rounds - 1) / (GA_FOLD_TARGET * rounds) > most) ++rounds;
   return GA_FOLD_TARGET * rounds;
 }
 static int fold_cols(int M, int N) {
@@ -470,10 +498,9 @@ static int gemm_skinny_launch(void* C, int64_t ldc, const void* A, int64_t lda, 
   const int groups = SK_WAVES / ks;
   if (pack == 0) pack = (grid_splits == 1 && !gated) ? auto_pack(M, (N + groups * nt * 16 - 1) / (groups * nt * 16)) : 1;
   if (pack != 1 && (pack != 2 || M > 8)) return -2;
-  const bool plain_even = !gated && grid_splits == 1 && !norm_out.residual && ks == SK_WAVES &&
-                          N >= GA_PLAIN_EVEN_MIN_COLUMNS && plain_even_workgroups(M, N, K) > 0;
+  const bool plain_even = !gated && grid_splits == 1 && !norm_out.residual && ks == SK_WAVES && N >= GA_PLAIN_EVEN_MIN_COLUMNS;
   if (mb == 1 && pack == 1 && ((gated && N >= GA_GATED_EVEN_MIN_COLUMNS) || plain_even)) {
-    const int workgroups = gated ? gated_even_workgroups(M, N, K) : plain_even_workgroups(M, N, K);
+    const int workgroups = gated ? even_workgroups(N, 14, 48) : even_workgroups(N, 64, 96);
     const int most = (N + workgroups - 1) / workgroups, per = (most + 15) / 16;      // tiles of one matrix
     const int ksteps = (K + 63) / 64;
     dim3 grid(workgroups), block(SK_THREADS);
@@ -499,6 +526,17 @@ static int gemm_skinny_launch(void* C, int64_t ldc, const void* A, int64_t lda, 
   if (norm_out.residual) {
     fcols = fold_cols(M, N);
     grid.x = (N + fcols - 1) / fcols;
+  }
+  // workgroups that are alone on their compute units, with a long K: longer trips
+  if (mb == 1 && nt == 1 && ks == SK_WAVES && !gated && (int64_t)grid.x * grid.y <= GA_FOLD_TARGET &&
+      ksteps >= 8 * SK_WAVES * pack * grid_splits) {
+#define LAUNCH_LONG(TC, PK)                                                                                        \
+  hipLaunchKernelGGL((gemm_skinny_kernel<1, 1, SK_WAVES, TC, false, PK, 3>), grid, block, 0, stream, (TC*)C, ldc, \
+                     (const bf16_t*)A, lda, (const bf16_t*)W, (const bf16_t*)bias, M, N, K, ksteps, norm_in, norm_out, fcols, act)
+    if (out_f32) { if (pack == 2) LAUNCH_LONG(float, 2); else LAUNCH_LONG(float, 1); }
+    else { if (pack == 2) LAUNCH_LONG(bf16_t, 2); else LAUNCH_LONG(bf16_t, 1); }
+#undef LAUNCH_LONG
+    return GA_CHECK_LAUNCH();
   }
 #define LAUNCH(NT, MB, KS, TC, G, PK)                                                                     \
   hipLaunchKernelGGL((gemm_skinny_kernel<NT, MB, KS, TC, G, PK>), grid, block, 0, stream, (TC*)C, ldc,   \
@@ -575,8 +613,10 @@ __global__ __launch_bounds__(SK_THREADS) void qkv_rope_skinny_kernel(
     int ksteps, NormIn norm_in, int ucols) {
   static_assert(PACK == 1 || MB == 1, "a packed tile holds at most 8 rows of A");
   static_assert(PACK == 1 || !HALF, "a tile is packed or half empty, not both");
-  __shared__ float red[SK_WAVES][32][MB * 16 + 1];
+  using Area = SkinnyArea<2, MB>;
+  __shared__ __attribute__((aligned(16))) unsigned char area[SK_WAVES][Area::BYTES];
   __shared__ float rstd[16];
+  auto red = [&](int w, int n, int m) -> float& { return reinterpret_cast<float*>(area[w])[n * (MB * 16 + 1) + m]; };
   using P = Packed<PACK>;
   constexpr int CP = HALF ? 8 : P::CP;
   constexpr int GROUPS = SK_WAVES / KS;
@@ -601,19 +641,23 @@ __global__ __launch_bounds__(SK_THREADS) void qkv_rope_skinny_kernel(
       row1 = row0 + ucols;
     }
   }
-  const KRange<PACK> kr(ks * PACK, P::seg(r), ksteps, KS * PACK, K);
-  const int shift = kr.shift;
-  const int wrow = HALF ? (r & 7) : P::col(r);
-  const bool lane_ok = unit_ok && (!HALF || r < 8) && wrow < ucols;
-  const bf16_t* wp[2] = {W + (int64_t)(row0 + wrow) * K + shift, W + (int64_t)(row1 + wrow) * K + shift};
-  const bool wok[2] = {lane_ok, lane_ok};
-  const bf16_t* ap[MB];
-  bool aok[MB];
+  const KRange<PACK> kr(ks * PACK, ksteps, KS * PACK, K);
+  SkinnySource<2, MB> src;
+  src.kend = kr.kend;
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb) {
-    const int m = mb * 16 + P::col(r);
-    aok[mb] = m < M;
-    ap[mb] = A + (int64_t)(aok[mb] ? m : 0) * lda + shift;
+  for (int j = 0; j < 2; ++j) {
+    const int tr = (lane >> 3) + 8 * j;            // the row of a tile that the lane brings a piece of
+    src.ke[j] = kr.ke[j];
+    const int wrow = HALF ? (tr & 7) : P::col(tr);
+    src.wok[0][j] = src.wok[1][j] = unit_ok && (!HALF || tr < 8) && wrow < ucols;
+    src.wp[0][j] = W + (int64_t)(row0 + wrow) * K + kr.shift[j];
+    src.wp[1][j] = W + (int64_t)(row1 + wrow) * K + kr.shift[j];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+      const int m = mb * 16 + P::col(tr);
+      src.aok[mb][j] = m < M;
+      src.ap[mb][j] = A + (int64_t)(src.aok[mb][j] ? m : 0) * lda + kr.shift[j];
+    }
   }
   // What the epilogue needs from memory (position, slot, cosine and sine, bias) is asked for now, so that
   // it arrives while the weights stream: an epilogue item is (unit of the workgroup, column, row of A).
@@ -656,7 +700,7 @@ __global__ __launch_bounds__(SK_THREADS) void qkv_rope_skinny_kernel(
     for (int mb = 0; mb < MB; ++mb) acc[nt][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
   NormInLoads in_loads;
   if (MB == 1) in_loads.load(norm_in, M, wave, lane);
-  skinny_accumulate<2, MB>(acc, wp, wok, ap, aok, 0, kr.kend, kr.ke, g);
+  skinny_accumulate<2, MB, 1>(acc, src, reinterpret_cast<u32x4*>(area[wave]), lane);
   if (MB == 1) in_loads.finish(norm_in, rstd, M, wave, lane);
   const bool scale_rows = MB == 1 && norm_in.sumsq != nullptr;
 #pragma unroll
@@ -664,7 +708,7 @@ __global__ __launch_bounds__(SK_THREADS) void qkv_rope_skinny_kernel(
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) red[wave][nt * 16 + g * 4 + i][mb * 16 + r] = acc[nt][mb][i];
+      for (int i = 0; i < 4; ++i) red(wave, nt * 16 + g * 4 + i, mb * 16 + r) = acc[nt][mb][i];
   __syncthreads();
 #pragma unroll
   for (int it = 0; it < ITEMS; ++it) {
@@ -679,8 +723,8 @@ __global__ __launch_bounds__(SK_THREADS) void qkv_rope_skinny_kernel(
 #pragma unroll
       for (int q = 0; q < PACK; ++q) {
         const int col = PACK == 1 ? m : q * CP + m;
-        lo += red[gi * KS + w][q * CP + nl][col];
-        hi += red[gi * KS + w][16 + q * CP + nl][col];
+        lo += red(gi * KS + w, q * CP + nl, col);
+        hi += red(gi * KS + w, 16 + q * CP + nl, col);
       }
     if (scale_rows) {
       lo *= rstd[m];

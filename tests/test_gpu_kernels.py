@@ -890,6 +890,33 @@ def test_gemm_skinny_gated(M, I, K):
         close(ops.gemm_skinny(a, w, gated=True, pack=pack), ref, 1e-2)
 
 
+@pytest.mark.parametrize("M", [1, 7, 8, 9, 15, 16, 17, 31, 33, 64])
+@pytest.mark.parametrize("K", [8, 56, 64, 72, 1032, 4096, 8960])     # pieces, steps and trips that end in the middle; the long K of few workgroups
+def test_products_of_few_rows_bring_every_element_to_its_place(M, K):
+    """Small whole numbers, whose sums 32-bit holds exactly in any order (each below 9 * K < 2^24): bit for bit the product."""
+    from ginfer_amd.kernels import ops
+    g = torch.Generator().manual_seed(M * K)
+    whole = lambda *size: torch.randint(-3, 4, size, generator=g).to(torch.bfloat16).to(dev())
+    a, w = whole(M, K), whole(2310, K)
+    want = lambda n: (a.double() @ w[:n].double().t()).float()
+    for n in (1, 15, 40, 1000, 2310):
+        for pack in (0, 1) if M <= 8 else (0,):
+            assert torch.equal(ops.gemm_skinny(a, w[:n], out_dtype=torch.float32, pack=pack), want(n)), (n, pack)
+    for nt in (1, 2, 4):
+        if K >= 1032:
+            parts = ops.gemm_skinny(a, w, out_dtype=torch.float32, nt=nt, grid_splits=2)
+            assert torch.equal(parts.sum(dim=0), want(2310)), nt
+    if M <= 16:
+        residual, gain = torch.zeros((M, 1000), device=dev()), torch.ones((1000,), dtype=torch.bfloat16, device=dev())
+        ops.gemm_skinny(a, w[:1000], into_norm=(residual, gain, 1e-6))
+        assert torch.equal(residual, want(1000))
+        wide = whole(16390, K)
+        assert torch.equal(ops.gemm_skinny(a, wide, out_dtype=torch.float32), (a.double() @ wide.double().t()).float())
+        gated = ops.gemm_skinny(a, w[:2 * 1100], gated=True, gate_bounds=(float("inf"), float("inf"), 0.0), out_dtype=torch.float32)
+        sums = want(2 * 1100)
+        assert torch.equal(gated, sums[:, :1100].clamp(min=0) * sums[:, 1100:])
+
+
 @pytest.mark.parametrize("M", [1, 3, 8, 16])
 @pytest.mark.parametrize("N,K,bias,gain_dtype", [(1536, 1536, False, torch.bfloat16), (1536, 8960, False, torch.float32),
                                                  (88, 136, True, torch.bfloat16), (200, 64, True, torch.float32),
