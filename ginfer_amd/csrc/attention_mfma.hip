@@ -414,13 +414,25 @@ __device__ __forceinline__ void load_q(bf16x8 (&q)[KB], const bf16_t* row /* nul
 // part_o: [n_tokens][nh][splits][HD] float; part_ml: [n_tokens][nh][splits][2] float (max, sum).
 // With one split the normalised result goes straight to `out`.
 #define DEC_WAVES 4
+// Keys of a token's split: its own keys dealt evenly to the launch's splits, in whole tiles and no fewer than `least`.  The number of
+// splits fits the longest context that the step is recorded for (a power of two), the length the token itself: with lengths
+// made for the longest, 4 requests at 13,001 to 16,384 in a launch for 32,768 left half of the workgroups without a key, and a request of
+// 2,049 keys in one for 4,096 had 2,048 of them in one split and one in the other.
+struct Splits {
+  int count, least;
+  uint32_t inverse;                  // 2^32 / count, rounded up: x * inverse >> 32 is x / count for x * count < 2^32
+};
+__device__ __forceinline__ int split_length(int span, const Splits& sp) {
+  const int even = sp.count == 1 ? span : (int)__umulhi((uint32_t)(span + sp.count - 1), sp.inverse);
+  return (max(even, sp.least) + 31) & ~31;
+}
 
 __global__ __launch_bounds__(64 * DEC_WAVES) void attn_decode_split_kernel(
     bf16_t* __restrict__ out, int64_t out_stride, float* __restrict__ part_o, float* __restrict__ part_ml,
     const bf16_t* __restrict__ q, int64_t q_stride, const bf16_t* __restrict__ k_pages,
     const bf16_t* __restrict__ v_pages, const int32_t* __restrict__ block_table, int table_width,
     const int4* __restrict__ decode_info, int nh, int nkv, int head_blocks, int ps_shift, int window,
-    float scale, int split_keys, int num_splits, const HeadExtras ex) {
+    float scale, const Splits splits, const HeadExtras ex) {
   __shared__ float o_s[DEC_WAVES][HD][17];
   __shared__ float m_s[DEC_WAVES][16], l_s[DEC_WAVES][16], mx_s[16], lsum_s[16];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;
@@ -428,7 +440,7 @@ __global__ __launch_bounds__(64 * DEC_WAVES) void attn_decode_split_kernel(
   const int kvh = blockIdx.y / head_blocks, hb = blockIdx.y % head_blocks;
   const int group = nh / nkv;
   const int4 info = decode_info[ti];       // (row of the step, position, entry of the block table, -): one load
-  const int t = info.x, pos = info.y;
+  const int t = info.x, pos = __builtin_amdgcn_readfirstlane(info.y), num_splits = splits.count;
   const int lo = first_visible_key(pos, window);
   const bool col_ok = hb * 16 + c < group;
   const int head = kvh * group + hb * 16 + c;
@@ -436,9 +448,10 @@ __global__ __launch_bounds__(64 * DEC_WAVES) void attn_decode_split_kernel(
   f32x4 o[1][DB];
   float m[1], l[1];
   init_state<1>(o, m, l);
-  const int begin = (lo / 32) * 32 + split * split_keys;
+  const int first = (lo / 32) * 32, length = split_length(pos + 1 - first, splits);
+  const int begin = first + split * length;
   if (begin <= pos) {
-    int end = begin + split_keys;
+    int end = begin + length;
     if (end > pos + 1) end = ((pos + 32) / 32) * 32;
     bf16x8 qr[1][KB];
     load_q(qr[0], col_ok ? q + (int64_t)t * q_stride + (int64_t)head * HD : nullptr, g);
@@ -501,61 +514,74 @@ __global__ __launch_bounds__(64 * DEC_WAVES) void attn_decode_split_kernel(
   }
 }
 
-// grid (decode tokens, nh), 64 threads: merges the splits of one (token, head) in ascending order.
-// EARLY > 0 (at most that many splits, the usual case): every partial output this lane will need is asked for at
-// once, before the weights are worked out: one trip to memory instead of one after the other.  The sums are the same,
-// in the same order.
+// grid (decode tokens, nh), WAVES wavefronts: merges the splits of one (token, head).  Wavefront w adds the splits [w EARLY, (w + 1) EARLY) in
+// ascending order, and the wavefronts' sums are added in theirs.  What bounds it is the way to memory: every partial output that a
+// lane will need is asked for at once, before the weights are worked out.  (More than 32 splits went through one wavefront, 8 at a
+// time; a decode step of one token at 16,000 with 128 of them 1,467 us, now 1,440.  Which splits have no keys is not asked either:
+// waiting for the token's position before the loads cost 0.7 us of a launch, and reading what nobody wrote 1.1.)
 #define MAX_SPLITS 256
-template <int EARLY>
-__global__ __launch_bounds__(64) void attn_decode_combine_kernel(
+template <int EARLY, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void attn_decode_combine_kernel(
     bf16_t* __restrict__ out, int64_t out_stride, const float* __restrict__ part_o,
     const float* __restrict__ part_ml, const int4* __restrict__ decode_info, int nh, int num_splits,
     const HeadExtras ex) {
-  __shared__ float w_s[MAX_SPLITS];
-  const int ti = blockIdx.x, head = blockIdx.y, lane = threadIdx.x;
+  static_assert(WAVES == 1 || EARLY == 32, "a wavefront's splits");
+  constexpr int DPL = (HD + 63) / 64, SLOTS = WAVES * EARLY;
+  __shared__ float w_s[SLOTS];
+  __shared__ float sums_s[WAVES > 1 ? WAVES : 1][WAVES > 1 ? DPL * 64 : 1];
+  const int ti = blockIdx.x, head = blockIdx.y, lane = threadIdx.x & 63;
+  const int s0 = WAVES == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * EARLY;      // a scalar: 64 addresses hang on it
   const int64_t base = ((int64_t)ti * nh + head) * num_splits;
-  constexpr int DPL = (HD + 63) / 64;
-  float o[DPL][EARLY > 0 ? EARLY : 1];
+  float o[DPL][EARLY];
   const int row = decode_info[ti].x;
-  if (EARLY > 0) {
 #pragma unroll
-    for (int i = 0; i < DPL; ++i) {
-      const int d = lane + 64 * i < HD ? lane + 64 * i : 0;
+  for (int i = 0; i < DPL; ++i) {
+    const int d = lane + 64 * i < HD ? lane + 64 * i : 0;
 #pragma unroll
-      for (int s = 0; s < EARLY; ++s) o[i][s] = part_o[(base + (s < num_splits ? s : 0)) * HD + d];
-    }
+    for (int s = 0; s < EARLY; ++s) o[i][s] = part_o[(base + (s0 + s < num_splits ? s0 + s : 0)) * HD + d];
+  }
+  constexpr int MINE = (SLOTS + 63) / 64;
+  float ms[MINE], ls[MINE];
+#pragma unroll
+  for (int j = 0; j < MINE; ++j) {
+    const int s = lane + 64 * j < num_splits ? lane + 64 * j : 0;
+    ms[j] = part_ml[(base + s) * 2];
+    ls[j] = part_ml[(base + s) * 2 + 1];
   }
   float mx = -INFINITY;
-  for (int s = lane; s < num_splits; s += 64) mx = fmaxf(mx, part_ml[(base + s) * 2]);
+#pragma unroll
+  for (int j = 0; j < MINE; ++j) mx = lane + 64 * j < num_splits ? fmaxf(mx, ms[j]) : mx;
   mx = wave_max(mx);
   float total = 0.f;
-  for (int s = lane; s < num_splits; s += 64) {
-    const float ms = part_ml[(base + s) * 2];
-    const float w = ms == -INFINITY ? 0.f : fast_exp2(ms - mx);
-    w_s[s] = w;
-    total += w * part_ml[(base + s) * 2 + 1];
-  }
+#pragma unroll
+  for (int j = 0; j < MINE; ++j)
+    if (lane + 64 * j < num_splits) {                     // every wavefront works out all of them, and the same
+      const float w = ms[j] == -INFINITY ? 0.f : fast_exp2(ms[j] - mx);
+      w_s[lane + 64 * j] = w;
+      total += w * ls[j];
+    }
   total = wave_sum(total);
   __syncthreads();
   const float inv = 1.f / sink_sum(total, mx, ex.sinks, head) * head_gate(ex, row, head);
   bf16_t* op = out + (int64_t)row * out_stride + (int64_t)head * HD;
-  if (EARLY > 0) {
 #pragma unroll
-    for (int i = 0; i < DPL; ++i) {
-      const int d = lane + 64 * i;
+  for (int i = 0; i < DPL; ++i) {
+    const int d = lane + 64 * i;
+    float acc = 0.f;
+#pragma unroll
+    for (int s = 0; s < EARLY; ++s)
+      if (s0 + s < num_splits) acc += o[i][s] * w_s[s0 + s];
+    if constexpr (WAVES > 1) sums_s[threadIdx.x >> 6][d] = acc;
+    else if (d < HD) op[d] = f32_to_bf16(acc * inv);
+  }
+  if constexpr (WAVES > 1) {
+    __syncthreads();
+    for (int d = threadIdx.x; d < HD; d += 64 * WAVES) {
       float acc = 0.f;
 #pragma unroll
-      for (int s = 0; s < EARLY; ++s)
-        if (s < num_splits) acc += o[i][s] * w_s[s];
-      if (d < HD) op[d] = f32_to_bf16(acc * inv);
+      for (int w = 0; w < WAVES; ++w) acc += sums_s[w][d];
+      op[d] = f32_to_bf16(acc * inv);
     }
-    return;
-  }
-  for (int d = lane; d < HD; d += 64) {
-    float acc = 0.f;
-#pragma unroll 8
-    for (int s = 0; s < num_splits; ++s) acc += part_o[(base + s) * HD + d] * w_s[s];
-    op[d] = f32_to_bf16(acc * inv);
   }
 }
 
@@ -992,22 +1018,26 @@ extern "C" int ga_attn_decode(void* out, int64_t out_stride, const void* q, int6
   if (num_splits > MAX_SPLITS) return -5;
   HeadExtras ex = {(const float*)sinks, cap, (const float*)gate, gate_stride, gate_scale};
   if (!bound_scores(scale, ex)) return -20;
+  // no split shorter than a tile for each wavefront, unless the caller's own are
+  const Splits splits = {num_splits, split_keys < 32 * DEC_WAVES ? split_keys : 32 * DEC_WAVES,
+                         num_splits > 1 ? 0xffffffffu / (uint32_t)num_splits + 1u : 0u};
   dim3 grid(n_tokens, nkv * head_blocks, num_splits);
   hipLaunchKernelGGL(attn_decode_split_kernel, grid, dim3(64 * DEC_WAVES), 0, stream, (bf16_t*)out, out_stride,
                      (float*)workspace_o, (float*)workspace_ml, (const bf16_t*)q, q_stride,
                      (const bf16_t*)k_pages, (const bf16_t*)v_pages, (const int32_t*)block_table, table_width,
-                     (const int4*)decode_info, nh, nkv, head_blocks, ps_shift, window, scale * LOG2E, split_keys,
-                     num_splits, ex);
+                     (const int4*)decode_info, nh, nkv, head_blocks, ps_shift, window, scale * LOG2E, splits, ex);
   int rc = GA_CHECK_LAUNCH();
   if (rc || num_splits == 1) return rc;
-#define COMBINE(EARLY)                                                                                       \
-  hipLaunchKernelGGL(attn_decode_combine_kernel<EARLY>, dim3(n_tokens, nh), dim3(64), 0, stream, (bf16_t*)out, \
+#define COMBINE(EARLY, WAVES)                                                                                \
+  hipLaunchKernelGGL((attn_decode_combine_kernel<EARLY, WAVES>), dim3(n_tokens, nh), dim3(64 * WAVES), 0, stream, (bf16_t*)out, \
                      out_stride, (const float*)workspace_o, (const float*)workspace_ml,                        \
                      (const int4*)decode_info, nh, num_splits, ex)
-  if (num_splits <= 8) COMBINE(8);
-  else if (num_splits <= 16) COMBINE(16);
-  else if (num_splits <= 32) COMBINE(32);
-  else COMBINE(0);
+  if (num_splits <= 8) COMBINE(8, 1);
+  else if (num_splits <= 16) COMBINE(16, 1);
+  else if (num_splits <= 32) COMBINE(32, 1);
+  else if (num_splits <= 64) COMBINE(32, 2);
+  else if (num_splits <= 128) COMBINE(32, 4);
+  else COMBINE(32, 8);
 #undef COMBINE
   return GA_CHECK_LAUNCH();
 }
@@ -1039,9 +1069,8 @@ extern "C" int ga_attn_prefill(void* out, int64_t out_stride, const void* q, int
                               tile_rows, nh, nkv, page_size, window, scale, fill_workgroups, prefer_workgroups, parts, part_o,
                               part_ml, ex, stream);
   if (rc || n_part_rows == 0) return rc;
-  hipLaunchKernelGGL(attn_decode_combine_kernel<8>, dim3(n_part_rows, nh), dim3(64), 0, stream, (bf16_t*)out, out_stride,
-                     (const float*)part_o, (const float*)part_ml, (const int4*)part_rows, nh, num_parts,
-                     ex);
+  hipLaunchKernelGGL((attn_decode_combine_kernel<8, 1>), dim3(n_part_rows, nh), dim3(64), 0, stream, (bf16_t*)out, out_stride,
+                     (const float*)part_o, (const float*)part_ml, (const int4*)part_rows, nh, num_parts, ex);
   return GA_CHECK_LAUNCH();
 }
 

@@ -630,6 +630,24 @@ MFMA_SEQS = ATTN_SEQS + [[(1, 31), (1, 32), (1, 33), (1, 64), (1, 65)], [(31, 31
                          [(1, 5000)], [(300, 700)]]
 
 
+@pytest.mark.parametrize("span", [256, 4096, 32768])
+@pytest.mark.parametrize("most", [1, 8, 9, 32, 33, 64, 65, 128, 129, 256])    # the merge: one wavefront, two, four and eight
+@pytest.mark.parametrize("window", [None, 70])
+def test_keys_of_single_tokens_dealt_to_splits(span, most, window, monkeypatch):
+    """Contexts far below the longest that the number of splits is made for, and up to it: splits of a tile and of many, empty ones."""
+    from ginfer_amd.kernels import ops
+    monkeypatch.setattr(ops.TUNING, "decode_target_workgroups", 1 << 20)
+    monkeypatch.setattr(ops.TUNING, "decode_min_split_keys", 32)
+    monkeypatch.setattr(ops.TUNING, "decode_max_splits", most)
+    lengths = [n for n in (1, 31, 33, 128, 129, 255, 256, 1000, 4095, 4096) if n <= span]
+    seqs = [(1, n) for n in lengths]
+    a, ref, _ = _paged_case(seqs, 6, 2, 64, 16, torch.bfloat16, seed=most, window=window)
+    step = _Step(seqs, a)
+    step.extra = {"decode_span": span}
+    out = ops.paged_attention_mfma(a["q"], a["k_pages"], a["v_pages"], a["block_table"], step, 6, 2, 64, 1.0 / math.sqrt(64), window=window)
+    close(out, ref, 2e-2)
+
+
 @pytest.mark.parametrize("wide", [False, True])
 @pytest.mark.parametrize("nh,nkv,hd", ATTN_HEADS + [(40, 2, 64), (3, 1, 256), (18, 1, 16), (7, 1, 64), (8, 4, 256)])
 @pytest.mark.parametrize("seqs", MFMA_SEQS)
