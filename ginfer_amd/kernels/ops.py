@@ -455,10 +455,36 @@ def gated_tiling(rows, out_features):
     return 2 if rows <= 1024 else 3
 
 
+GATED_WIDE_TILINGS = {6: (192, 64), 7: (192, 128), 8: (192, 256)}
+
+
+def gated_wide_tiling(rows, out_features, in_features):
+    """The tiles of 192 rows of W that the gated product takes in place of gated_tiling's, or None: where they fill one round of the
+    chip's 256 compute units, or few, better.  us beside the tiles that they replace, or beside the library where those are not
+    taken, as replays of a graph over several layers' weights: 37,888 rows of W, K 3,584: 64 rows 62.2 -> 54.6 (198 workgroups for 148),
+    128 rows 67.8 -> 61.1; 28,672 rows, K 4,096 the other way, 53.0 -> 59.6 (150 for 224).  17,920 rows, K 1,536: 161 rows 27.4 -> 24.4
+    (188 workgroups for 140), 256 rows 29.1 -> 26.5; 22,016 rows, K 2,048: 256 rows 36.9 -> 35.6 (230 for 172).  A round of 192 x 256 takes
+    0.82 (K 3,584) to 0.89 (K 1,536) of one of 256 x 256: beyond 1,024 rows it stands where it makes that up in rounds, nearly full:
+    17,920 rows of W: 1,025 rows 79.8 -> 77.2, 1,280 86.9 -> 82.0, 2,048 129 -> 119 (752 tiles in 3 rounds; 560 of 256 x 256 in 3), but 4,096 rows
+    226 -> 238 (6 rounds for 5); 22,016: 512 rows 56.5 -> 52.0, 1,536 152 -> 144, but 2,048 175 -> 188 (4 for 3).  With a longer K the library
+    has most of that many rows: 28,672, K 4,096 1,025 rows 227 -> 251; 12,288, K 3,072 2,048 rows 138 -> 137."""
+    wide, rounds = -(-out_features // 192), lambda of_w, of_a: -(-(-(-out_features // of_w) * -(-rows // of_a)) // 256)
+    if rows <= 128:
+        return (6 if rows <= 64 else 7) if rounds(128, 128) > 1 and wide <= 256 else None
+    if rows <= 256:
+        return 7 if rounds(128, 128) > 1 and rounds(192, 128) == 1 else None
+    tiles = wide * -(-rows // 256)
+    if 384 < rows <= 512 and 0.85 * 256 <= tiles <= 256:
+        return 8
+    few = rounds(192, 256)
+    return 8 if rows > 1024 and in_features <= 3072 and tiles >= 0.89 * 256 * few and 0.9 * few < rounds(256, 256) else None
+
+
 def gemm_tiles_gated(a, w, bounds=None, tiling=None):
     """a [M, K], w [2N, K] (gate over up) -> bfloat16 [M, N] = silu(a.gate^T) * (a.up^T), both sums in 32-bit and one
     rounding; with bounds = (limit, alpha, shift) g * sigmoid(alpha g) * (u + shift), g = min(gate, limit), u = clamp(up,
-    -limit, limit) (alpha = infinity: the sigmoid's limit, relu(g)).  tiling: its number in GATED_TILINGS (None: by sizes)."""
+    -limit, limit) (alpha = infinity: the sigmoid's limit, relu(g)).  tiling: its number in GATED_TILINGS or GATED_WIDE_TILINGS (None: by
+    sizes)."""
     _dev(a, w)
     _need(gemm_tiles_supported(a, w) and a.shape[1] == w.shape[1], "the kernel over tiles does not take %s %s x %s %s", a.dtype,
           tuple(a.shape), w.dtype, tuple(w.shape))
@@ -468,7 +494,7 @@ def gemm_tiles_gated(a, w, bounds=None, tiling=None):
         _need(limit > 0, "the gate's bound must be positive, got %r", limit)
         kind = 2 if math.isinf(alpha) else 1
     if tiling is None:
-        tiling = gated_tiling(M, w.shape[0])
+        tiling = gated_wide_tiling(M, w.shape[0], w.shape[1]) or gated_tiling(M, w.shape[0])
     out = torch.empty((M, N), dtype=a.dtype, device=a.device)
     lib = build.load("gemm_tiles")
     _check(lib.ga_gemm_tiles_gated(_ptr(out), _i64(N), _ptr(a), _i64(a.stride(0)), _ptr(w), _i(M), _i(N), _i(a.shape[1]), _i(kind),

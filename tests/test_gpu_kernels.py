@@ -1118,6 +1118,16 @@ def test_gated_product_over_tiles(M, cols, K):
         assert bool((off <= ref.abs() / 256 + 1e-3 * ref.pow(2).mean().sqrt()).all()), "%r: %g" % (bounds, float(off.max()))
 
 
+@pytest.mark.parametrize("tiling", [6, 7, 8])
+@pytest.mark.parametrize("M,cols,K", [(1, 8, 64), (64, 88, 128), (65, 96, 192), (128, 104, 256), (129, 192, 320), (256, 200, 64), (257, 296, 640)])
+def test_gated_product_in_tiles_of_192_rows(tiling, M, cols, K):
+    """Around 64, 128 and 256 rows of A and 96 columns; the same sums as in the other tilings, so the same bits."""
+    from ginfer_amd.kernels import ops
+    a, w = rnd((M, K), torch.bfloat16, 61), rnd((2 * cols, K), torch.bfloat16, 62)
+    for bounds in (None, (7.0, 1.702, 1.0)):
+        assert torch.equal(ops.gemm_tiles_gated(a, w, bounds=bounds, tiling=tiling), ops.gemm_tiles_gated(a, w, bounds=bounds, tiling=0))
+
+
 @pytest.mark.parametrize("tiling", range(5))
 @pytest.mark.parametrize("M,cols,K", [(1, 8, 64), (63, 64, 128), (65, 72, 192), (127, 136, 256), (129, 128, 320), (257, 264, 640)])
 def test_gated_product_in_every_tiling(tiling, M, cols, K):

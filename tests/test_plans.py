@@ -147,6 +147,20 @@ def test_gated_products_over_tiles_at_their_thresholds():
     assert g(1700, 17920, 1536) and g(2048, 37888, 3584) and not g(2049, 37888, 3584)
 
 
+def test_gated_products_in_tiles_of_192_rows_at_their_thresholds():
+    """Taken where they fill the chip's rounds better than the other tiles, refused where those, or the library, were the faster."""
+    from ginfer_amd.kernels import ops
+    wide = lambda rows, n, k: ops.GATED_WIDE_TILINGS.get(ops.gated_wide_tiling(rows, n, k))
+    assert wide(64, 37888, 3584) == (192, 64) and wide(65, 37888, 3584) == wide(128, 37888, 3584) == (192, 128)
+    assert wide(64, 32768, 3584) is None and wide(64, 49152, 1024) == (192, 64) and wide(64, 49344, 1024) is None
+    assert wide(129, 17920, 1536) == wide(256, 22016, 2048) == (192, 128) and wide(256, 16384, 1280) is None and wide(256, 37888, 3584) is None
+    assert wide(400, 22016, 2048) == (192, 256) and wide(400, 17920, 1536) is None and wide(384, 22016, 2048) is None
+    assert all(wide(rows, 17920, 1536) == (192, 256) for rows in (1025, 1280, 1900, 2048))
+    assert not any(wide(rows, 17920, 1536) for rows in (513, 1024, 1300, 1536, 1792, 4096)) and wide(2048, 22016, 2048) is None
+    assert wide(1025, 28672, 4096) is None and wide(2048, 12288, 3072) == (192, 256)
+    assert L.gated_plan(2048, 17920, False, True, 1536, True) == ("tiles",) and L.gated_plan(512, 17920, False, True, 1536, True) == ("transposed",)
+
+
 def test_the_gated_product_is_one_plan_of_several():
     """The tuner starts from the plan that runs, can leave it, and tries tiles where the rule does not take them."""
     key = lambda rows, n, k, tiles_ok=True, bounds=None: ("gated", rows, n, k, rows <= 64, bounds is None and rows % 8 == 0, tiles_ok, bounds)
