@@ -118,15 +118,25 @@ class Tuning:
     tiles_parts_most_weights_many_rows: int = 32 << 20
     tiles_parts_most_weights_most_rows: int = 23 << 20
     tiles_parts_workgroups: int = 256
+    # ---- the gated product of few rows beyond `library_from_rows`: up to so many the weight-streaming kernel, while W is no larger
+    # than these (us of the tiles, or the library where they are not taken -> of it at 17 and at 32 rows: 17,920 x 1,536 16.8 -> 15.2,
+    # 17.5 -> 17.3; 22,016 x 2,048 26.1 -> 21.8, 25.6 -> 23.2; 16,384 x 1,280 15.6 -> 11.3, 16.2 -> 12.4; 10,240 x 1,792 16.7 -> 12.6, 17.1 ->
+    # 14.1; the other way 37,888 x 3,584 55.0 -> 56.7, 55.9 -> 62.3; 27,648 x 5,120 54.7 -> 61.3, 56.4 -> 70.1)
+    gated_skinny_up_to_rows: int = 32
+    gated_skinny_most_out_features: int = 22528
+    gated_skinny_most_in_features: int = 2560
     # ---- the fused q|k|v projection + rotation + cache write (parts/attention.py): from more rows than this and a K
-    # of at least that, the library's product followed by the rotation kernel is faster (the fused kernel cannot split K).
+    # of at least that, the library's product followed by the rotation kernel is faster (the fused kernel cannot split K): us of the
+    # two -> fused at 17, 32 and 64 rows: 4,608 columns, K 3,584 14.6 -> 10.7, 14.7 -> 11.5, 18.5 -> 15.5; 6,144, K 4,096 19.3 -> 15.1,
+    # 20.1 -> 16.5, 22.9 -> 22.3; 7,168, K 5,120 23.2 -> 20.3, 24.3 -> 21.4, but 27.9 -> 29.1; 15,360, K 5,120 39.6 -> 40.2 at 32, 43.2 -> 52.9
+    # at 64; 10,240, K 8,192 43.9 -> 44.0, 45.3 -> 49.4, 47.7 -> 65.8.
     fused_qkv_up_to_rows: int = 16
-    fused_qkv_unless_in_features: int = 3072
-    # With a shorter K than that, from this many rows on the product goes to the weight-streaming kernel with K split over
-    # workgroups, into K // `qkv_in_parts_min_k` parts (at most `qkv_in_parts_most`), which the rotation kernel adds up
-    # (2,048 columns of a K of 1,536 in a decode step of 64 rows: the fused kernel 13.6 us, product 6.7 + rotation over the
-    # parts 5.9; decode at batch 64 18,340 -> 18,450 tok/s, at batch 48 15,760 -> 15,900).
-    qkv_in_parts_from_rows: int = 48
+    fused_qkv_unless_in_features: int = 4608
+    # With a shorter K than that, from this many rows on the product can go to the weight-streaming kernel with K split over
+    # workgroups, into K // `qkv_in_parts_min_k` parts (at most `qkv_in_parts_most`), which the rotation kernel adds up.  More rows than
+    # that kernel takes (the default): never; since it reads 8 lanes to a row the fused kernel is ahead everywhere (2,048 columns, K
+    # 1,536: 64 rows 8.1 us, product in 4 parts and rotation 10.4; 48 rows 7.0 and 9.7).
+    qkv_in_parts_from_rows: int = 65
     qkv_in_parts_min_k: int = 384
     qkv_in_parts_most: int = 4
     # ---- attention on the matrix cores (kernels/ops.py)

@@ -12,19 +12,16 @@ from .registry import register_mixer
 
 
 def _library_then_rotation_is_faster(rows, in_features):
-    """The fused projection kernel cannot split K over workgroups (its epilogue needs whole sums).  Measured on
-    MI355X at a 7B model's sizes (K 3584, 4608 outputs): from 17 rows on the BLAS library's product followed by
-    the rotation kernel is faster (32 rows: 17.6 us against 20.6; 64 rows: 23.4 against 28.1); at a 1.5B model's
-    (K 1536) the fused kernel stays ahead or level up to 64 rows."""
+    """The fused projection kernel cannot split K over workgroups (its epilogue needs whole sums): from 17 rows and some K on the
+    BLAS library's product followed by the rotation kernel is faster (the figures stand beside the thresholds)."""
     return rows > TUNING.fused_qkv_up_to_rows and in_features >= TUNING.fused_qkv_unless_in_features
 
 
 def _projection_in_parts(x, w_qkv, head_dim, rotary_dim):
     """Into how many parts of K the q|k|v product of these rows is split, its parts to be added by the rotation kernel;
     0: not this way.  The fused kernel cannot split K, and each of its workgroups reads all rows of x, which from some
-    48 rows on is most of what it reads.  Measured on MI355X in a decode step of 64 rows (2,048 columns of a K of 1,536):
-    the fused kernel 13.6 us, the product in four parts 6.7 + the rotation kernel over them 5.9; with fewer rows the fused
-    kernel's time falls faster than the pair's (32 rows: 9.2 us)."""
+    48 rows on is most of what it reads; it is ahead all the same (the figures stand beside the thresholds), so that the
+    defaults never take this way."""
     if isinstance(x, ops.ScaledRows) or x.dtype != torch.bfloat16:
         return 0
     rows, K = x.shape

@@ -327,6 +327,9 @@ def gated_plan(rows, out_features, skinny_ok, transposable, in_features=0, tiles
     """By the rules: ("skinny",) the weight-streaming kernel with the activation in its epilogue; ("tiles",) the product over
     tiles with the same; ("transposed",) the library with the weights as its first operand, which leaves the product transposed,
     [2I, M], and the activation on that; ("library",) the usual product and the activation."""
+    if (skinny_ok and tiles_ok and TUNING.library_from_rows < rows <= TUNING.gated_skinny_up_to_rows
+            and out_features <= TUNING.gated_skinny_most_out_features and in_features <= TUNING.gated_skinny_most_in_features):
+        return ("skinny",)
     if tiles_ok and (tiles_gated(rows, out_features, in_features) or ops.gated_wide_tiling(rows, out_features, in_features) == 8):
         return ("tiles",)
     if skinny_ok and not _library_is_faster(rows, out_features):

@@ -159,6 +159,9 @@ def test_gated_products_in_tiles_of_192_rows_at_their_thresholds():
     assert not any(wide(rows, 17920, 1536) for rows in (513, 1024, 1300, 1536, 1792, 4096)) and wide(2048, 22016, 2048) is None
     assert wide(1025, 28672, 4096) is None and wide(2048, 12288, 3072) == (192, 256)
     assert L.gated_plan(2048, 17920, False, True, 1536, True) == ("tiles",) and L.gated_plan(512, 17920, False, True, 1536, True) == ("transposed",)
+    # the weight-streaming kernel up to 32 rows, while W is small
+    assert L.gated_plan(17, 17920, True, False, 1536, True) == L.gated_plan(32, 22016, True, True, 2048, True) == ("skinny",)
+    assert L.gated_plan(33, 17920, True, False, 1536, True) == L.gated_plan(17, 37888, True, False, 3584, True) == ("tiles",)
 
 
 def test_the_gated_product_is_one_plan_of_several():
