@@ -114,6 +114,9 @@ int ga_embedding_sinusoid_norm(void* out, const void* table, const void* ids, co
 int ga_short_conv_apply(void* out, const void* x, const void* w, const void* state, const void* slots,
                         const void* token_entry, const void* cu, const void* q_start, int tokens, int width, int taps,
                         int add_input, int out_bf16, int64_t x_stride, const void* bias, hipStream_t stream);
+int ga_short_conv_step(void* out, const void* x, const void* w, void* state, const void* slots, const void* cu, const void* q_start,
+                       int entries, int width, int taps, int add_input, int out_bf16, int64_t x_stride, const void* bias,
+                       hipStream_t stream);
 int ga_short_conv_update(void* state, const void* x, const void* slots, const void* cu, const void* q_start, int entries,
                          int width, int taps, int64_t x_stride, hipStream_t stream);
 

@@ -1047,6 +1047,12 @@ def short_conv(x, weight, state, slots, step, dtype, add_input=True, update=True
         _need(slots.dtype == torch.int64 and slots.shape == (E,) and slots.is_contiguous(), "slots must be contiguous int64 [%d]", E)
     out = torch.empty((T, W), dtype=dtype, device=x.device)
     lib = build.load("short_conv")
+    lens = getattr(step, "host_q_len", None)
+    if update and taps > 1 and lens and max(lens) == 1:        # single tokens: one launch (right for any lengths, but token after token)
+        _check(lib.ga_short_conv_step(_ptr(out), _ptr(x), _ptr(weight), _ptr(state), _ptr(slots), _ptr(step.cu_tokens), _ptr(step.q_start),
+                                      _i(E), _i(W), _i(taps), _i(1 if add_input else 0), _i(_is_bf16(dtype)), _i64(x.stride(0)),
+                                      _ptr(bias), _stream()), "short_conv_step")
+        return out
     _check(lib.ga_short_conv_apply(_ptr(out), _ptr(x), _ptr(weight), _ptr(state), _ptr(slots), _ptr(step.token_entry),
                                    _ptr(step.cu_tokens), _ptr(step.q_start), _i(T), _i(W), _i(taps), _i(1 if add_input else 0),
                                    _i(_is_bf16(dtype)), _i64(x.stride(0)), _ptr(bias), _stream()), "short_conv_apply")

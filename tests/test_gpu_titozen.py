@@ -213,6 +213,32 @@ def test_short_convolution_across_cuts_and_slots(taps):
             at[k] += n
 
 
+@pytest.mark.parametrize("taps", [2, 3, 4, 5, 16])
+@pytest.mark.parametrize("lens", [[1] * 17, [1], [3, 0, 1, 20, 2]])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_short_convolution_in_one_launch(taps, lens, dtype):
+    """The launch for steps of single tokens, also as a recorded step replays it, where other lengths than the ones it was recorded
+    with may come: bit for bit what the two launches give, outputs and state."""
+    from types import SimpleNamespace
+    from ginfer_amd.kernels import ops
+    W, E = 300, len(lens)
+    g = torch.Generator().manual_seed(taps)
+    x, w = torch.randn((sum(lens), 2 * W), generator=g).cuda()[:, W:], torch.randn((W, taps), generator=g).cuda()
+    bias, state = torch.randn((W,), generator=g).cuda(), torch.randn((E + 3, taps - 1, W), generator=g).cuda()
+    slots = (torch.randperm(E + 3, generator=g)[:E]).cuda()
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32).cuda()
+    entry = torch.repeat_interleave(torch.arange(E), torch.tensor(lens)).to(torch.int32).cuda()
+    start = torch.tensor([0 if e % 3 == 0 else 5 for e in range(E)], dtype=torch.int32).cuda()
+    got = []
+    for host in ([1] * E, None):
+        step, st = SimpleNamespace(token_entry=entry, cu_tokens=cu, q_start=start, host_q_len=host), state.clone()
+        for add, b in ((True, None), (False, bias)):
+            got.append(ops.short_conv(x, w, st, slots, step, dtype, add_input=add, bias=b))
+        got.append(st)
+    for a, b in zip(got[:3], got[3:]):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("heads,dim,vdim", [(1, 5, 3), (3, 40, 72), (2, 130, 20), (2, 16, 100), (1, 256, 16)])
 def test_gated_recurrence_across_cuts(heads, dim, vdim):
     """The recurrence of one request in portions of 1 to 40 tokens beside another request, against the plain loop; the
