@@ -98,3 +98,8 @@ def test_padding_of_one_row_has_a_record_of_its_own():
     host = host_arrays([40, 23], [0, 16])
     p = pad_step(host, 64, 8, 16, pad_slot=99, n_single=single_records(63, 64, 8, 0))
     assert p["decode_info"].shape == (8, 4) and (p["decode_info"][:, 0] == 63).all() and p["q_len"][8] == 1
+
+
+def test_rows_of_recorded_steps():
+    from ginfer_amd.engine.runner import padded_rows
+    assert [padded_rows(n) for n in (1, 64, 65, 128, 129, 256, 257, 384, 385, 512, 513, 1025)] == [64, 64, 128, 128, 256, 256, 384, 384, 512, 512, 1024, 2048]
