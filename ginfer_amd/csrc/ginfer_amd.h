@@ -400,7 +400,7 @@ int ga_pwa_attend_mfma(void* out, void* partial, const void* q, const void* k_ro
 // ---- gated_residual.hip: residual float [tokens, hidden] += sigmoid(z[:, :hidden]) * y1 (+ sigmoid(z[:, hidden:]) * y2, y2
 // may be null; z: float rows with the stride z_stride; z_bias: float, one number per column of z, or null); with next: next = rmsnorm(residual) * next_gain (float [hidden])
 int ga_gated_residual_add(void* residual, const void* z, int64_t z_stride, const void* z_bias, const void* y1, const void* y2,
-                          int tokens, int hidden, int y_bf16,
+                          int parts1, int parts2, int tokens, int hidden, int y_bf16,
                           const void* next_gain, float next_eps, void* next, int next_bf16, hipStream_t stream);
 
 // ---- hyper_connection.hip: the residual stream as S streams side by side, X float [tokens, S, width].  open: every stream

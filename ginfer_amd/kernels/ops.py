@@ -2096,7 +2096,7 @@ def gated_residual_add(residual, z, y1, y2=None, next_gain=None, next_eps=0.0, d
     """residual float32 [T, H] += sigmoid(z[:, :H]) * y1 (+ sigmoid(z[:, H:]) * y2), the gated results added to each other
     first; z float32 [T, H] or [T, 2H] (rows may have a stride: columns of a wider projection), z_bias float32, one number
     per column, is added to it; y1, y2 [T, H] in float32 or
-    bfloat16.  With next_gain (float32 [H]) the rows of the norm
+    bfloat16, or float32 partial sums [parts, T, H] of a product cut along K, which are added up.  With next_gain (float32 [H]) the rows of the norm
     that is read next, rmsnorm(residual) * next_gain in `dtype`, come back; else None."""
     _dev(residual, z, y1, y2, next_gain, z_bias)
     _need(residual.dtype == torch.float32 and residual.dim() == 2 and residual.is_contiguous(), "residual must be contiguous float32 [T, H]")
@@ -2104,8 +2104,16 @@ def gated_residual_add(residual, z, y1, y2=None, next_gain=None, next_eps=0.0, d
     gates = 1 if y2 is None else 2
     _need(z.dtype == torch.float32 and tuple(z.shape) == (T, gates * H) and z.stride(1) == 1,
           "z must be float32 [%d, %d] with unit inner stride (it may be columns of a wider projection)", T, gates * H)
-    for name, y in (("y1", y1), ("y2", y2)):
-        _need(y is None or (y.shape == (T, H) and y.is_contiguous() and y.dtype == y1.dtype), "%s must be contiguous [%d, %d] in one dtype", name, T, H)
+    summed = [y for y in (y1, y2) if y is not None and y.dim() == 3]
+    if summed and not (H % 4 == 0 and H <= 8192 and z.stride(0) % 4 == 0
+                       and all(t.data_ptr() % 16 == 0 for t in (z, z_bias, *summed) if t is not None)):      # rows the launch that adds does not take
+        whole = [y.dtype for y in (y1, y2) if y is not None and y.dim() == 2]
+        y1, y2 = (y.sum(dim=0).to(whole[0] if whole else y.dtype) if y is not None and y.dim() == 3 else y for y in (y1, y2))
+    parts = [y.shape[0] if y is not None and y.dim() == 3 else 0 for y in (y1, y2)]
+    plain = [y for y, n in zip((y1, y2), parts) if y is not None and n == 0]
+    for name, y, n in (("y1", y1, parts[0]), ("y2", y2, parts[1])):
+        _need(y is None or (tuple(y.shape[-2:]) == (T, H) and y.is_contiguous() and y.dtype == (torch.float32 if n else plain[0].dtype)),
+              "%s must be contiguous [%d, %d] in one dtype, or float32 parts of that", name, T, H)
     if z_bias is not None:
         _f32(z_bias, (gates * H,), "z_bias")
     nxt = None
@@ -2113,8 +2121,8 @@ def gated_residual_add(residual, z, y1, y2=None, next_gain=None, next_eps=0.0, d
         _f32(next_gain, (H,), "next_gain")
         nxt = torch.empty((T, H), dtype=dtype, device=residual.device)
     lib = build.load("gated_residual")
-    _check(lib.ga_gated_residual_add(_ptr(residual), _ptr(z), _i64(z.stride(0)), _ptr(z_bias), _ptr(y1), _ptr(y2), _i(T), _i(H),
-                                     _i(_is_bf16(y1.dtype)),
+    _check(lib.ga_gated_residual_add(_ptr(residual), _ptr(z), _i64(z.stride(0)), _ptr(z_bias), _ptr(y1), _ptr(y2), _i(parts[0]), _i(parts[1]),
+                                     _i(T), _i(H), _i(_is_bf16(plain[0].dtype) if plain else 0),
                                      _ptr(next_gain), _f(next_eps), _ptr(nxt), _i(_is_bf16(dtype) if nxt is not None else 0),
                                      _stream()), "gated_residual_add")
     return nxt

@@ -245,9 +245,11 @@ class ParallelGatedBlock(Arrangement):
         else:
             z = self.gate.logits(n)
             results = [self.mixer.forward(n, step, cache)]
+        adds = getattr(self.gate, "adds_partial_sums", False)
         if self.feed_forward is not None:
-            results.append(self.feed_forward.forward(n))
-        rows = self.gate.add(residual, z, [whole(r).to(n.dtype) if r.dim() == 3 else r for r in results], then=into_norm)
+            parts = adds and getattr(self.feed_forward, "makes_partial_sums", False)
+            results.append(self.feed_forward.forward(n, parts_ok=True) if parts else self.feed_forward.forward(n))
+        rows = self.gate.add(residual, z, results if adds else [whole(r).to(n.dtype) if r.dim() == 3 else r for r in results], then=into_norm)
         return NormedRows(rows) if into_norm is not None else None
 
 

@@ -38,6 +38,7 @@ class SigmoidProjectionGate(Part):
     the norm that is read next."""
 
     capturable = True
+    adds_partial_sums = True         # results may be float32 [parts, T, H]
 
     def __init__(self, hidden_size, names, dtype, device):
         self.hidden_size, self.names = int(hidden_size), [str(n) for n in names]

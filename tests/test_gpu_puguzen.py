@@ -166,6 +166,27 @@ def test_gated_sum_into_the_stream_and_the_next_norm():
             assert H.rel_err(r1.cpu(), want1) < 2e-6
 
 
+@pytest.mark.parametrize("width", [7, 96, 1536, 4100])                # 7: rows of no multiple of 4, added up before the launch
+@pytest.mark.parametrize("p1, p2", [(0, 1), (0, 4), (5, 0), (2, 9), (3, None)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_gated_sum_of_results_in_parts(width, p1, p2, dtype):
+    """Whole results in `dtype` beside 32-bit partial sums, against 64 bits: up to 9 parts of size 1 round by at most 9 * 3 * 2^-24 of
+    the stream's size, 3; a result that is added up before the launch is rounded to the other's dtype."""
+    from ginfer_amd.kernels import ops
+    g = torch.Generator().manual_seed(width + p1)
+    T, sig = 6, torch.sigmoid
+    res, z = torch.randn((T, width), generator=g) * 3, torch.randn((T, 2 * width), generator=g)
+    make = lambda p: torch.randn((p, T, width), generator=g) if p else torch.randn((T, width), generator=g).to(dtype)
+    y1, y2 = make(p1), None if p2 is None else make(p2)
+    total = lambda y: y.double().sum(dim=0) if y.dim() == 3 else y.double()
+    want = res.double() + sig(z[:, :width].double()) * total(y1)
+    if y2 is not None:
+        want = want + sig(z[:, width:].double()) * total(y2)
+    got, gates = res.cuda(), z if y2 is not None else z[:, :width].contiguous()
+    ops.gated_residual_add(got, gates.cuda(), y1.cuda(), None if y2 is None else y2.cuda())
+    assert H.rel_err(got.cpu(), want) < (2e-6 if width % 4 == 0 or dtype == torch.float32 else 1e-2)
+
+
 def test_relu_as_the_limit_of_the_bounded_gate():
     """relu(gate) * up from the gated activation with no bound, a step in place of the sigmoid and no shift: its own
     pass over a product, and the epilogue of the weight-streaming product (few rows, bfloat16)."""
