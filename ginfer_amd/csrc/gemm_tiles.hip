@@ -20,7 +20,9 @@
 #include "ginfer_amd.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 
 // act.kind 0: SiLU(v) * u; 1: g * sigmoid(alpha g) * (u + shift), g = min(v, limit), u = clamp(u, -limit, limit); 2: the same
@@ -226,6 +228,205 @@ static int gt_check(const void* C, const void* A, int64_t lda, const void* W, in
   return 0;
 }
 
+// ---- up to 512 rows, dealt evenly to the chip
+// W's rows come in units of eight: four columns' gates and the same columns' ups.  Column group b of G owns the units [b U / G, (b + 1)
+// U / G), row tile t of T the rows [t R, (t + 1) R), and G T workgroups make whole rounds of the chip's compute units, so that each
+// takes in the same bytes, whatever the sizes; a tile has room for NB blocks of 16 rows of W and TM rows of A, and what of that
+// it does not own is not loaded.  Eight wavefronts, WN x WM of the tile's blocks of v_mfma_f32_16x16x32_bf16 and WK of a slab's K.
+//
+// What bounds it: loads return in order, so a compute unit's stream of lines, some from its L2 and some from memory, goes at the
+// pace of the latter: 45 to 50 GB/s a compute unit in every mixture, 110 from L2 alone.  So the bytes a compute unit takes in
+// are what counts: all 256 at work with a few rows fewer each, not the 188 of tiles of 192 x 128 (256 rows by 17,920 rows of W, K 1,536:
+// the loads alone 20.8 us there, 18.0 here, of 26.0 and 22.9 whole).  W is asked for as memory that is read once (nt), so that A
+// stays in the L2s: 18.1 -> 17.4 us with a line of W wanted twice, 11.5 -> 10.6 with it wanted once (64 rows).  Slabs of 128 elements
+// where the tile leaves room (WK 2): half the meetings, 5 % of the loads' time.
+template <int NI, int MJ, int WN, int WM, int WK, int NBUF>
+struct SpreadTile {
+  static constexpr int WAVES = WN * WM * WK, TM = 16 * MJ * WM, NB = NI * WN, TW = 16 * NB, BK = 64 * WK;
+  static constexpr int ROW = 2 * BK, RPL = 1024 / ROW, LPR = ROW / 16;           // bytes a row of a slab; rows a load brings, lanes a row
+  static constexpr int LW = (TW / RPL + WAVES - 1) / WAVES, LA = (TM / RPL + WAVES - 1) / WAVES, LOADS = LW + LA, SLAB = (TW + TM) * ROW;
+  static constexpr int SUMS = WK == 2 ? (NI * MJ + 1) / 2 * WAVES * 1024 : 0, PITCH = 8 * NB + 4, OUT = TM * PITCH * 2;
+  static constexpr int SLABS = SLAB * NBUF, LDS = SLABS > SUMS ? (SLABS > OUT ? SLABS : OUT) : (SUMS > OUT ? SUMS : OUT);
+  static_assert(TW % RPL == 0 && TM % RPL == 0 && LDS <= 160 * 1024 && LOADS <= 7 && LOADS * (NBUF - 1) < 64, "tile");
+};
+
+template <int NI, int MJ, int WN, int WM, int WK, int NBUF>
+__global__ __launch_bounds__(64 * WN * WM * WK, 1) void gemm_spread_gated_kernel(
+    bf16_t* __restrict__ C, int64_t ldc, const bf16_t* __restrict__ A, int64_t lda, const bf16_t* __restrict__ W, int M, int cols,
+    int K, int m_tiles, int tile_rows, int groups, GateAct act) {
+  using S = SpreadTile<NI, MJ, WN, WM, WK, NBUF>;
+  constexpr int WAVES = S::WAVES, ROW = S::ROW, RPL = S::RPL, LPR = S::LPR, LW = S::LW, LA = S::LA, LOADS = S::LOADS;
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  const int total = m_tiles * groups, run = (total + 7) / 8, at8 = blockIdx.x / 8, id = (blockIdx.x % 8) * run + at8;
+  if (at8 >= run || id >= total) return;
+  const int mt = id % m_tiles, b = id / m_tiles, m0 = mt * tile_rows, units = cols / 4;
+  const int u0 = __builtin_amdgcn_readfirstlane((int)((int64_t)b * units / groups));
+  const int own = __builtin_amdgcn_readfirstlane((int)((int64_t)(b + 1) * units / groups)) - u0, c0 = 4 * u0;      // units; at most 2 NB
+  const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave % WM, wn = wave / WM % WN, wk = wave / (WM * WN);
+  const uint32_t base = (uint32_t)(uintptr_t)(lds_byte_t*)lds + wave * 1024;
+  const int slabs = K / S::BK, live = min(tile_rows, M - m0);
+  // load l of W or of A is wavefront l % WAVES's; how many a slab takes of it
+  const int of_w = own * 8 / RPL, of_a = (live + RPL - 1) / RPL;
+  const int mine_w = of_w > wave ? (of_w - wave + WAVES - 1) / WAVES : 0, mine_a = of_a > wave ? (of_a - wave + WAVES - 1) / WAVES : 0;
+  const int mine = mine_w + mine_a;
+  uint32_t src_w[LW], src_a[LA];
+#pragma unroll
+  for (int j = 0; j < LW; ++j) {      // rows 0 to 3 of a unit are gates, 4 to 7 ups; piece p of row r lies at place p ^ (r % LPR)
+    const int r = min(wave + j * WAVES, of_w - 1) * RPL + lane / LPR, piece = (lane % LPR) ^ (r & (LPR - 1));
+    src_w[j] = ((uint32_t)(c0 + (r / 8) * 4 + (r & 3) + ((r & 4) ? cols : 0)) * (uint32_t)K + 8 * piece) * 2u;
+  }
+#pragma unroll
+  for (int j = 0; j < LA; ++j) {
+    const int r = (wave + j * WAVES) * RPL + lane / LPR, piece = (lane % LPR) ^ (r & (LPR - 1));
+    src_a[j] = ((uint32_t)min(m0 + r, M - 1) * (uint32_t)lda + 8 * piece) * 2u;
+  }
+  const char* wp = reinterpret_cast<const char*>(W);
+  const char* ap = reinterpret_cast<const char*>(A);
+  uint32_t fill = base;                           // the buffer that the next slab goes to
+  int fill_at = 0, read_at = 0;
+  auto bring_one = [&](int j) {
+    if (j < LW) {
+      if (j < mine_w) lds_bring_once_from(fill + j * WAVES * 1024, src_w[j], wp);
+    } else if (j - LW < mine_a) {
+      lds_bring_from(fill + S::TW * ROW + (j - LW) * WAVES * 1024, src_a[j - LW], ap);
+    }
+  };
+  auto brought = [&]() {
+    wp += ROW;
+    ap += ROW;
+    fill_at = fill_at == NBUF - 1 ? 0 : fill_at + 1;
+    fill = base + fill_at * S::SLAB;
+  };
+  // all but the youngest n slabs' loads are in, and all wavefronts meet
+  auto wait_for = [&](auto n) {
+    constexpr int N = decltype(n)::value;
+    switch (mine) {
+      case 1: lds_wait_and_meet<N>(); break;
+      case 2: lds_wait_and_meet<2 * N>(); break;
+      case 3: lds_wait_and_meet<3 * N>(); break;
+      case 4: lds_wait_and_meet<4 * N>(); break;
+      case 5: lds_wait_and_meet<5 * N>(); break;
+      case 6: lds_wait_and_meet<6 * N>(); break;
+      case 7: lds_wait_and_meet<7 * N>(); break;
+      default: lds_wait_and_meet<0>();
+    }
+  };
+  f32x4 acc[NI][MJ];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < MJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  int at[2];                                      // a wavefront has two steps of 32 of every slab
+#pragma unroll
+  for (int k = 0; k < 2; ++k) at[k] = (((wk * 2 + k) * 4 + g) ^ (c & (LPR - 1))) * 16 + c * ROW;
+  const unsigned char* cur = lds;
+  bf16x8 a[2][NI], bb[2][MJ];
+  constexpr int READS = MJ + NI;
+  auto read_one = [&](int k, int y) {
+    if (y < MJ) bb[k][y] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(cur + at[k] + (S::TW + (wm * MJ + y) * 16) * ROW));
+    else a[k][y - MJ] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(cur + at[k] + (wn * NI + y - MJ) * 16 * ROW));
+  };
+  // the products of one step, beside the reads of the next and the loads of a later slab
+  auto step = [&](int k, auto loads) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      if (decltype(loads)::value) {
+#pragma unroll
+        for (int j = 0; j < LOADS; ++j)
+          if (j * NI / LOADS == i) bring_one(j);
+      }
+#pragma unroll
+      for (int y = 0; y < READS; ++y)
+        if (y * (NI - 1) / READS == i) read_one(1 - k, y);
+#pragma unroll
+      for (int j = 0; j < MJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[k][i], bb[k][j], acc[i][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  auto turn = [&]() {
+    read_at = read_at == NBUF - 1 ? 0 : read_at + 1;
+    cur = lds + read_at * S::SLAB;
+  };
+#pragma unroll
+  for (int s = 0; s < NBUF; ++s)
+    if (s < slabs) {
+#pragma unroll
+      for (int j = 0; j < LOADS; ++j) bring_one(j);
+      brought();
+    }
+  if (slabs >= NBUF) wait_for(std::integral_constant<int, NBUF - 1>());
+  else lds_wait_and_meet<0>();
+#pragma unroll
+  for (int y = 0; y < READS; ++y) read_one(0, y);
+  int s = 0;
+  for (; s + NBUF < slabs; ++s) {                 // in mid-slab its operands are all in registers, and its buffer is free
+    step(0, std::false_type());
+    wait_for(std::integral_constant<int, NBUF - 2>());
+    turn();
+    step(1, std::true_type());
+    brought();
+  }
+  for (; s < slabs; ++s) {
+    step(0, std::false_type());
+    lds_wait_and_meet<0>();
+    turn();
+    step(1, std::false_type());
+  }
+  __syncthreads();
+  constexpr int T = NI * MJ;
+  if constexpr (WK == 2) {                        // the parts of K meet: block t's sums are the wavefront's with wk = t % 2
+    constexpr int PER = (T + 1) / 2;
+    f32x4* area = reinterpret_cast<f32x4*>(lds);
+    const int other = wave ^ (WM * WN);
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+      if (t % 2 != wk) area[(wave * PER + t / 2) * 64 + lane] = acc[t / MJ][t % MJ];
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+      if (t % 2 == wk) {
+        const f32x4 v = area[(other * PER + t / 2) * 64 + lane], h = acc[t / MJ][t % MJ];
+        acc[t / MJ][t % MJ] = wk ? v + h : h + v;
+      }
+    __syncthreads();
+  }
+  // Lanes with even g hold gates, the 16 behind them the same columns' ups: exchanged so that a lane has both of two columns.  Through
+  // LDS, so that a row's columns leave side by side.
+  bf16_t* tile = reinterpret_cast<bf16_t*>(lds);
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+    if (WK == 1 || t % 2 == wk) {
+      const int i = t / MJ, j = t % MJ;
+      const f32x4 v = acc[i][j];
+      const auto even = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[0]), __float_as_uint(v[2]), false, false);
+      const auto odd = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[1]), __float_as_uint(v[3]), false, false);
+      const bf16x2 y = {(__bf16)gt_act(__uint_as_float(even[0]), __uint_as_float(even[1]), act),
+                        (__bf16)gt_act(__uint_as_float(odd[0]), __uint_as_float(odd[1]), act)};
+      *reinterpret_cast<uint32_t*>(tile + ((wm * MJ + j) * 16 + c) * S::PITCH + (wn * NI + i) * 8 + 2 * g) = __builtin_bit_cast(uint32_t, y);
+    }
+  __syncthreads();
+  for (int idx = tid; idx < S::TM * 2 * S::NB; idx += 64 * WAVES) {
+    const int m = idx / (2 * S::NB), q = idx % (2 * S::NB);
+    if (m < live && q < own)
+      *reinterpret_cast<uint2*>(C + (int64_t)(m0 + m) * ldc + c0 + 4 * q) = *reinterpret_cast<const uint2*>(tile + m * S::PITCH + 4 * q);
+  }
+}
+
+template <int NI, int MJ, int WN, int WM, int WK, int NBUF>
+static int gt_spread(void* C, int64_t ldc, const void* A, int64_t lda, const void* W, int M, int cols, int K, int m_tiles, int groups,
+                     GateAct act, hipStream_t stream) {
+  using S = SpreadTile<NI, MJ, WN, WM, WK, NBUF>;
+  const int tile_rows = ((M + m_tiles - 1) / m_tiles + 15) / 16 * 16, units = cols / 4;
+  if (K % S::BK || tile_rows > S::TM || (int64_t)(m_tiles - 1) * tile_rows >= M || groups > units || (units + groups - 1) / groups > 2 * S::NB) return -7;
+  const auto kernel = gemm_spread_gated_kernel<NI, MJ, WN, WM, WK, NBUF>;
+  const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, S::LDS);
+  if (raised != hipSuccess) return (int)raised;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)((m_tiles * groups + 7) / 8 * 8)), dim3(64 * S::WAVES), S::LDS, stream, (bf16_t*)C, ldc,
+                     (const bf16_t*)A, lda, (const bf16_t*)W, M, cols, K, m_tiles, tile_rows, groups, act);
+  return GA_CHECK_LAUNCH();
+}
+
 // tiling: which tiles, rows of W x rows of A; the caller chooses by sizes and by how full they leave the chip's rounds
 // (gated_tiling in kernels/ops.py, tiles_gated in parts/linear.py, the fastest and the library beside each other).  us, product and
 // activation by the library's best way -> here, as replays of a graph over several layers' weights: 17,920 rows of W, K 1,536: 64 rows
@@ -252,6 +453,34 @@ extern "C" int ga_gemm_tiles_gated(void* C, int64_t ldc, const void* A, int64_t 
     case 6: return gt_launch<6, 1, 1, 2, 4, true>(C, ldc, A, lda, W, M, cols, K, 1, act, stream);     // 192 x 64
     case 7: return gt_launch<6, 1, 1, 4, 3, true>(C, ldc, A, lda, W, M, cols, K, 1, act, stream);     // 192 x 128
     case 8: return gt_launch<6, 2, 1, 4, 2, true>(C, ldc, A, lda, W, M, cols, K, 1, act, stream);     // 192 x 256
+  }
+  return -6;
+}
+
+// shape: the tile, the rows of A and of W that it has room for; m_tiles row tiles of equal numbers of rows times `groups` groups of columns
+// (spread_plan in kernels/ops.py chooses them, spread_is_faster in parts/linear.py where the product goes this way at all).  us of the other
+// ways -> here, as replays of a graph over weights beyond the 256 MB cache: 17,920 rows of W, K 1,536: 17 rows 15.3 -> 12.5, 64 18.9 -> 13.7, 128
+// 22.5 -> 16.7, 256 26.6 -> 23.7, 384 31.4 -> 28.7, 512 43.6 -> 35.2; 37,888, K 3,584: 64 rows 55.9 -> 45.3 (6.0 TB/s of weights), 128 61.3 ->
+// 52.3, 192 83.7 -> 61.5, 256 84.1 -> 73.1; 9,728, K 896: 64 11.6 -> 8.1, 256 18.4 -> 11.6.  480 products of 40 sizes of W: 1.22 times as fast
+// in the geometric mean.
+extern "C" int ga_gemm_spread_gated(void* C, int64_t ldc, const void* A, int64_t lda, const void* W, int M, int cols, int K, int kind,
+                                    float limit, float alpha, float shift, int shape, int m_tiles, int groups, hipStream_t stream) {
+  if (M <= 0) return 0;
+  const int rc = gt_check(C, A, lda, W, 2 * (int64_t)cols, M, cols, K);
+  if (rc) return rc;
+  if (kind < 0 || kind > 2 || ldc < cols || ldc % 4 || m_tiles < 1 || m_tiles > M || groups < 1 || (int64_t)m_tiles * groups > 1 << 20) return -1;
+  const GateAct act = {kind, limit, alpha, shift};
+  switch (shape) {
+    case 0: return gt_spread<5, 1, 1, 4, 2, 4>(C, ldc, A, lda, W, M, cols, K, m_tiles, groups, act, stream);     // 64 rows of A, 80 of W
+    case 1: return gt_spread<5, 2, 1, 4, 2, 3>(C, ldc, A, lda, W, M, cols, K, m_tiles, groups, act, stream);     // 128, 80
+    case 2: return gt_spread<5, 1, 2, 4, 1, 5>(C, ldc, A, lda, W, M, cols, K, m_tiles, groups, act, stream);     // 64, 160
+    case 3: return gt_spread<5, 2, 2, 4, 1, 4>(C, ldc, A, lda, W, M, cols, K, m_tiles, groups, act, stream);     // 128, 160
+    case 4: return gt_spread<5, 3, 2, 4, 1, 3>(C, ldc, A, lda, W, M, cols, K, m_tiles, groups, act, stream);     // 192, 160
+    case 5: return gt_spread<5, 4, 2, 4, 1, 3>(C, ldc, A, lda, W, M, cols, K, m_tiles, groups, act, stream);     // 256, 160
+    case 6: return gt_spread<4, 1, 2, 4, 1, 6>(C, ldc, A, lda, W, M, cols, K, m_tiles, groups, act, stream);     // 64, 128
+    case 7: return gt_spread<4, 2, 2, 4, 1, 5>(C, ldc, A, lda, W, M, cols, K, m_tiles, groups, act, stream);     // 128, 128
+    case 8: return gt_spread<4, 3, 2, 4, 1, 4>(C, ldc, A, lda, W, M, cols, K, m_tiles, groups, act, stream);     // 192, 128
+    case 9: return gt_spread<4, 4, 2, 4, 1, 3>(C, ldc, A, lda, W, M, cols, K, m_tiles, groups, act, stream);     // 256, 128
   }
   return -6;
 }

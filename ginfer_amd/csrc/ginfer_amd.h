@@ -102,6 +102,8 @@ int ga_add_scalar_rmsnorm(void* residual, const void* y, const void* gain, void*
 // SiLU, 1 bounded sigmoid, 2 bounded step; tiling 0 .. 4 (see there); parts: C float [parts, M, cols], partial sums over K
 int ga_gemm_tiles_gated(void* C, int64_t ldc, const void* A, int64_t lda, const void* W, int M, int cols, int K, int kind,
                         float limit, float alpha, float shift, int tiling, hipStream_t stream);
+int ga_gemm_spread_gated(void* C, int64_t ldc, const void* A, int64_t lda, const void* W, int M, int cols, int K, int kind,
+                         float limit, float alpha, float shift, int shape, int m_tiles, int groups, hipStream_t stream);
 int ga_gemm_tiles_parts(void* C, const void* A, int64_t lda, const void* W, int M, int cols, int K, int parts, hipStream_t stream);
 
 // ---- embedding_sinusoid.hip: out float [tokens, hidden] = table_scale * table[ids] + (sin | cos)(position * freq[i / 2]), then the norm

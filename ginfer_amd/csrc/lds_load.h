@@ -14,6 +14,10 @@ __device__ __forceinline__ void lds_bring(uint32_t place, const bf16_t* src) {
 __device__ __forceinline__ void lds_bring_from(uint32_t place, uint32_t at, const void* base) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(place), "v"(at), "s"(base) : "memory", "m0");
 }
+// the same for memory that this launch reads once or nearly so: it is the first to leave the caches
+__device__ __forceinline__ void lds_bring_once_from(uint32_t place, uint32_t at, const void* base) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(place), "v"(at), "s"(base) : "memory", "m0");
+}
 // all but the wavefront's N youngest loads are in, its LDS reads are through; then all wavefronts meet
 template <int N = 0>
 __device__ __forceinline__ void lds_wait_and_meet() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory"); }

@@ -486,8 +486,8 @@ def gated_wide_tiling(rows, out_features, in_features):
 def gemm_tiles_gated(a, w, bounds=None, tiling=None):
     """a [M, K], w [2N, K] (gate over up) -> bfloat16 [M, N] = silu(a.gate^T) * (a.up^T), both sums in 32-bit and one
     rounding; with bounds = (limit, alpha, shift) g * sigmoid(alpha g) * (u + shift), g = min(gate, limit), u = clamp(up,
-    -limit, limit) (alpha = infinity: the sigmoid's limit, relu(g)).  tiling: its number in GATED_TILINGS or GATED_WIDE_TILINGS (None: by
-    sizes)."""
+    -limit, limit) (alpha = infinity: the sigmoid's limit, relu(g)).  tiling: its number in GATED_TILINGS or GATED_WIDE_TILINGS, or a
+    plan as spread_plan makes them (None: by sizes)."""
     _dev(a, w)
     _need(gemm_tiles_supported(a, w) and a.shape[1] == w.shape[1], "the kernel over tiles does not take %s %s x %s %s", a.dtype,
           tuple(a.shape), w.dtype, tuple(w.shape))
@@ -497,12 +497,53 @@ def gemm_tiles_gated(a, w, bounds=None, tiling=None):
         _need(limit > 0, "the gate's bound must be positive, got %r", limit)
         kind = 2 if math.isinf(alpha) else 1
     if tiling is None:
-        tiling = gated_wide_tiling(M, w.shape[0], w.shape[1]) or gated_tiling(M, w.shape[0])
+        tiling = (spread_plan(M, w.shape[0], w.shape[1]) or gated_wide_tiling(M, w.shape[0], w.shape[1])
+                  or gated_tiling(M, w.shape[0]))
     out = torch.empty((M, N), dtype=a.dtype, device=a.device)
     lib = build.load("gemm_tiles")
+    if isinstance(tiling, tuple):
+        _check(lib.ga_gemm_spread_gated(_ptr(out), _i64(N), _ptr(a), _i64(a.stride(0)), _ptr(w), _i(M), _i(N), _i(a.shape[1]), _i(kind),
+                                        _f(limit), _f(alpha), _f(shift), *(_i(v) for v in tiling), _stream()), "gemm_spread_gated")
+        return out
     _check(lib.ga_gemm_tiles_gated(_ptr(out), _i64(N), _ptr(a), _i64(a.stride(0)), _ptr(w), _i(M), _i(N), _i(a.shape[1]), _i(kind),
                                    _f(limit), _f(alpha), _f(shift), _i(tiling), _stream()), "gemm_tiles_gated")
     return out
+
+
+SPREAD_SHAPES = ((64, 80, 128), (128, 80, 128), (64, 160, 64), (128, 160, 64), (192, 160, 64), (256, 160, 64),
+                 (64, 128, 64), (128, 128, 64), (192, 128, 64), (256, 128, 64))     # room for rows of A and of W, elements of a slab
+
+
+def spread_plan(rows, out_features, in_features):
+    """(number in SPREAD_SHAPES, row tiles, groups of columns) of the gated product of 17 to 512 rows by `out_features` rows of W
+    dealt evenly to the chip (csrc/gemm_tiles.hip), or None where the tiles of gated_tiling and gated_wide_tiling are the faster or
+    no shape holds it.  One workgroup to each of the 256 compute units, in the split that has them read the fewest rows, and up to
+    64 rows two, one after the other, where one cannot hold its share of W.  Beyond 128 rows the other tiles are better where they
+    fit one round about as well: a compute unit's rows there, the mean of its rows of A, against here; us, rows of the
+    two: 17,920 x 1,536 at 256 rows 320 and 272, 26.6 -> 23.7; 9,088 x 2,880 at 256 256 and 200, 32.0 -> 27.1; the other way 21,120 x
+    1,792 at 253 318 and 344, 30.9 -> 31.8; 10,496 x 3,584 at 264 216 and 224, 33.5 -> 36.3; 15,360 x 6,144 at 136 196 and 200, 58.4 -> 61.0."""
+    if not 17 <= rows <= 512:
+        return None
+    units, best = out_features // 8, None
+    for m_tiles in range(1, 5):
+        tile_rows = -(-(-(-rows // m_tiles)) // 16) * 16
+        if (m_tiles - 1) * tile_rows >= rows:
+            continue
+        groups = min(units, 256 // m_tiles)
+        if m_tiles == 1 and rows <= 64 and units > 20 * groups:
+            groups = min(units, 512)
+        of_w = -(-units // groups) * 8
+        fits = [(tm * tw, n) for n, (tm, tw, bk) in enumerate(SPREAD_SHAPES) if tm >= tile_rows and tw >= of_w and in_features % bk == 0]
+        if fits and (best is None or tile_rows + of_w <= best[0]):
+            best = (tile_rows + of_w, (min(fits)[1], m_tiles, groups))
+    if best is None or rows <= 128:
+        return best and best[1]
+    number = gated_wide_tiling(rows, out_features, in_features)
+    of_w, of_a = GATED_WIDE_TILINGS[number] if number else GATED_TILINGS[gated_tiling(rows, out_features)]
+    tiles = -(-rows // of_a)
+    if -(-out_features // of_w) * tiles <= 256 and best[0] > 0.92 * (of_w + rows / tiles):
+        return None
+    return best[1]
 
 
 def gemm_tiles_parts(a, w, parts):

@@ -10,6 +10,7 @@ these calls are checked bit for bit against eager steps in the tests."""
 import torch
 
 from ..kernels import autotune, ops
+from ..kernels.ops import SKINNY_MAX_ROWS
 from ..kernels.tuning import TUNING      # every threshold below is a field of this table, with what it was measured on
 
 
@@ -320,7 +321,23 @@ def gated_linear(x, weight_gate_up, bounds=None):
         plan = autotune.choose(key, (weight_gate_up,))
     if plan is None:
         plan = gated_plan(rows, out_features, skinny_ok, transposable, in_features, tiles_ok)
+        if tiles_ok and spread_is_faster(plan, rows, out_features, in_features):
+            plan = ("tiles",)
     return run_gated_plan(plan, x, weight_gate_up, bounds)
+
+
+def spread_is_faster(plan, rows, out_features, in_features):
+    """Whether the product over tiles that are dealt evenly to the chip stands in for `plan`, the other rules' (by sizes alone; the
+    measurements stand beside the thresholds and ops.spread_plan)."""
+    T = TUNING
+    if plan == ("tiles",) or ops.spread_plan(rows, out_features, in_features) is None:
+        return False
+    if plan == ("skinny",):
+        return (out_features >= T.spread_few_rows_min_out_features
+                or rows > T.spread_beyond_rows and out_features * in_features >= T.spread_min_weights)
+    if rows > SKINNY_MAX_ROWS and in_features > T.spread_most_k_of_columns * out_features:
+        return False
+    return rows <= T.spread_long_k_up_to_rows or in_features <= T.spread_most_in_features
 
 
 def gated_plan(rows, out_features, skinny_ok, transposable, in_features=0, tiles_ok=False):

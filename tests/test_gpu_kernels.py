@@ -1205,6 +1205,35 @@ def test_gated_product_in_every_tiling(tiling, M, cols, K):
     assert bool((off <= ref.abs() / 256 + 1e-3 * ref.pow(2).mean().sqrt()).all()), float(off.max())
 
 
+@pytest.mark.parametrize("shape", range(10))
+@pytest.mark.parametrize("fill,m_tiles,K", [(0.3, 1, 128), (0.99, 1, 384), (1.0, 1, 1152), (1.0, 2, 256), (0.6, 3, 512)])
+def test_gated_product_dealt_evenly(shape, fill, m_tiles, K):
+    """Every shape with a share of its rows of A and its columns full, one to three row tiles, groups that own one unit of four columns more
+    than others, K of one slab to more than there are buffers; bounds as for the other tiles."""
+    from ginfer_amd.kernels import ops
+    tm, tw, _ = ops.SPREAD_SHAPES[shape]
+    M = max(1, int(fill * tm)) * m_tiles - (m_tiles - 1)
+    most = max(2, int(fill * tw) // 8)                 # units of the largest group
+    groups = 5
+    cols = 4 * (most * groups - 3) // 8 * 8
+    wide = rnd((M, K + 16), torch.bfloat16, 71)
+    a, w = wide[:, 8:8 + K], rnd((2 * cols, K), torch.bfloat16, 72)
+    g, u = (a.double() @ w.double().t()).split(cols, dim=1)
+    for bounds in (None, (7.0, 1.702, 1.0), (float("inf"), float("inf"), 0.0)):
+        if bounds is None:
+            ref = g * torch.sigmoid(g) * u
+        else:
+            gc, uc = torch.clamp(g, max=bounds[0]), torch.clamp(u, -bounds[0], bounds[0])
+            ref = (torch.relu(gc) if bounds[1] == float("inf") else gc * torch.sigmoid(bounds[1] * gc)) * (uc + bounds[2])
+        got = ops.gemm_tiles_gated(a, w, bounds=bounds, tiling=(shape, m_tiles, groups)).double()
+        off = (got - ref).abs()
+        assert bool((off <= ref.abs() / 256 + 1e-3 * ref.pow(2).mean().sqrt()).all()), "%r: %g" % (bounds, float(off.max()))
+    # no such shape, more row tiles than rows, more groups than units, a group with more columns than the tile has room for
+    for plan in ((10, m_tiles, groups), (shape, M + 1, groups), (shape, m_tiles, cols // 4 + 1)) + (((shape, m_tiles, 1),) if cols > tw // 2 else ()):
+        with pytest.raises(ops.KernelError):
+            ops.gemm_tiles_gated(a, w, tiling=plan)
+
+
 @pytest.mark.parametrize("M", [1, 63, 64, 65, 127, 256, 300])
 @pytest.mark.parametrize("N,K,parts", [(16, 64, 1), (80, 192, 3), (144, 320, 2), (1536, 640, 5), (64, 832, 13), (80, 256, 1),
                                        (144, 320, 1), (96, 576, 1), (64, 1088, 2), (208, 2112, 3)])

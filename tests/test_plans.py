@@ -169,6 +169,30 @@ def test_gated_products_in_tiles_of_192_rows_at_their_thresholds():
     assert L.gated_plan(33, 17920, True, False, 1536, True) == L.gated_plan(17, 37888, True, False, 3584, True) == ("tiles",)
 
 
+def test_gated_products_dealt_evenly():
+    """A plan's tiles hold what it deals out, in one round of the chip (two for the fewest rows of the widest), and stand where they were
+    measured the faster."""
+    from ginfer_amd.kernels import ops
+    for rows in list(range(17, 513, 9)) + [64, 65, 128, 129, 192, 193, 256, 257, 384, 512]:
+        for n, k in ((16, 64), (1024, 320), (8192, 1024), (9728, 896), (17920, 1536), (22016, 2048), (37888, 3584), (59136, 8192), (131072, 128)):
+            plan = ops.spread_plan(rows, n, k)
+            if plan is None:
+                continue
+            (tm, tw, bk), m_tiles, groups = ops.SPREAD_SHAPES[plan[0]], plan[1], plan[2]
+            tile_rows = -(-(-(-rows // m_tiles)) // 16) * 16
+            assert tile_rows <= tm and (m_tiles - 1) * tile_rows < rows and k % bk == 0 and 1 <= groups <= n // 8
+            assert -(-(n // 8) // groups) * 8 <= tw and m_tiles * groups <= (512 if rows <= 64 else 256)
+    plan = ops.spread_plan
+    assert plan(64, 17920, 1536) == (0, 1, 256) and plan(128, 17920, 1536) == (1, 1, 256) and plan(161, 17920, 1536) == plan(256, 17920, 1536) == (3, 2, 128)
+    assert plan(384, 17920, 1536) == (4, 2, 128) and plan(64, 37888, 3584) == (2, 1, 256) and plan(64, 59136, 8192) == (6, 1, 512)
+    assert plan(16, 17920, 1536) is None and plan(513, 17920, 1536) is None and plan(65, 59136, 8192) is None
+    assert plan(253, 21120, 1792) is None and plan(264, 10496, 3584) is None and plan(256, 9088, 2880) == (7, 2, 128)
+    faster = lambda plan, rows, n, k: L.spread_is_faster((plan,), rows, n, k)
+    assert faster("skinny", 17, 17920, 1536) and not faster("skinny", 17, 9728, 896) and faster("skinny", 33, 3072, 2048) and not faster("skinny", 34, 2688, 512)
+    assert faster("library", 400, 17920, 1536) and faster("transposed", 512, 17920, 1536) and not faster("library", 92, 2048, 6144)
+    assert faster("library", 384, 11136, 8192) and not faster("library", 508, 11136, 8192) and not faster("tiles", 64, 17920, 1536)
+
+
 def test_steps_of_a_trip():
     """Products of few rows: a short K in one way to memory, then two, then three steps at a time."""
     from ginfer_amd.kernels import build
