@@ -250,39 +250,35 @@ struct SpreadTile {
   static_assert(TW % RPL == 0 && TM % RPL == 0 && LDS <= 160 * 1024 && LOADS <= 7 && LOADS * (NBUF - 1) < 64, "tile");
 };
 
-template <int NI, int MJ, int WN, int WM, int WK, int NBUF>
-__global__ __launch_bounds__(64 * WN * WM * WK, 1) void gemm_spread_gated_kernel(
-    bf16_t* __restrict__ C, int64_t ldc, const bf16_t* __restrict__ A, int64_t lda, const bf16_t* __restrict__ W, int M, int cols,
-    int K, int m_tiles, int tile_rows, int groups, GateAct act) {
+// A tile's sums over the slabs [slab0, slab0 + slabs) of K: acc of wavefront (wn, wm, wk), block (i, j) the rows 16 (wn NI + i) of the tile of
+// W by the rows 16 (wm MJ + j) of A; with WK 2 block t = i MJ + j is whole in the wavefront with wk = t % 2.  row_of_w(r): which row of W
+// is row r of the tile, for r below 8 `own`.  Afterwards the LDS is free.
+template <int NI, int MJ, int WN, int WM, int WK, int NBUF, typename RowOfW>
+__device__ __forceinline__ void spread_sums(f32x4 (&acc)[NI][MJ], unsigned char* lds, const bf16_t* __restrict__ A, int64_t lda,
+                                            const bf16_t* __restrict__ W, int K, int slab0, int slabs, int m0, int live, int own,
+                                            RowOfW row_of_w) {
   using S = SpreadTile<NI, MJ, WN, WM, WK, NBUF>;
   constexpr int WAVES = S::WAVES, ROW = S::ROW, RPL = S::RPL, LPR = S::LPR, LW = S::LW, LA = S::LA, LOADS = S::LOADS;
-  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  const int total = m_tiles * groups, run = (total + 7) / 8, at8 = blockIdx.x / 8, id = (blockIdx.x % 8) * run + at8;
-  if (at8 >= run || id >= total) return;
-  const int mt = id % m_tiles, b = id / m_tiles, m0 = mt * tile_rows, units = cols / 4;
-  const int u0 = __builtin_amdgcn_readfirstlane((int)((int64_t)b * units / groups));
-  const int own = __builtin_amdgcn_readfirstlane((int)((int64_t)(b + 1) * units / groups)) - u0, c0 = 4 * u0;      // units; at most 2 NB
-  const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave % WM, wn = wave / WM % WN, wk = wave / (WM * WN);
+  const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave % WM, wn = wave / WM % WN, wk = wave / (WM * WN);
   const uint32_t base = (uint32_t)(uintptr_t)(lds_byte_t*)lds + wave * 1024;
-  const int slabs = K / S::BK, live = min(tile_rows, M - m0);
   // load l of W or of A is wavefront l % WAVES's; how many a slab takes of it
   const int of_w = own * 8 / RPL, of_a = (live + RPL - 1) / RPL;
   const int mine_w = of_w > wave ? (of_w - wave + WAVES - 1) / WAVES : 0, mine_a = of_a > wave ? (of_a - wave + WAVES - 1) / WAVES : 0;
   const int mine = mine_w + mine_a;
   uint32_t src_w[LW], src_a[LA];
 #pragma unroll
-  for (int j = 0; j < LW; ++j) {      // rows 0 to 3 of a unit are gates, 4 to 7 ups; piece p of row r lies at place p ^ (r % LPR)
+  for (int j = 0; j < LW; ++j) {      // piece p of row r of a tile lies at place p ^ (r % LPR)
     const int r = min(wave + j * WAVES, of_w - 1) * RPL + lane / LPR, piece = (lane % LPR) ^ (r & (LPR - 1));
-    src_w[j] = ((uint32_t)(c0 + (r / 8) * 4 + (r & 3) + ((r & 4) ? cols : 0)) * (uint32_t)K + 8 * piece) * 2u;
+    src_w[j] = ((uint32_t)row_of_w(r) * (uint32_t)K + 8 * piece) * 2u;
   }
 #pragma unroll
   for (int j = 0; j < LA; ++j) {
     const int r = (wave + j * WAVES) * RPL + lane / LPR, piece = (lane % LPR) ^ (r & (LPR - 1));
-    src_a[j] = ((uint32_t)min(m0 + r, M - 1) * (uint32_t)lda + 8 * piece) * 2u;
+    src_a[j] = ((uint32_t)(m0 + min(r, live - 1)) * (uint32_t)lda + 8 * piece) * 2u;
   }
-  const char* wp = reinterpret_cast<const char*>(W);
-  const char* ap = reinterpret_cast<const char*>(A);
+  const char* wp = reinterpret_cast<const char*>(W) + (int64_t)slab0 * ROW;
+  const char* ap = reinterpret_cast<const char*>(A) + (int64_t)slab0 * ROW;
   uint32_t fill = base;                           // the buffer that the next slab goes to
   int fill_at = 0, read_at = 0;
   auto bring_one = [&](int j) {
@@ -312,7 +308,6 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 1) void gemm_spread_gated_kernel
       default: lds_wait_and_meet<0>();
     }
   };
-  f32x4 acc[NI][MJ];
 #pragma unroll
   for (int i = 0; i < NI; ++i)
 #pragma unroll
@@ -391,41 +386,194 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 1) void gemm_spread_gated_kernel
       }
     __syncthreads();
   }
-  // Lanes with even g hold gates, the 16 behind them the same columns' ups: exchanged so that a lane has both of two columns.  Through
-  // LDS, so that a row's columns leave side by side.
-  bf16_t* tile = reinterpret_cast<bf16_t*>(lds);
-#pragma unroll
-  for (int t = 0; t < T; ++t)
-    if (WK == 1 || t % 2 == wk) {
-      const int i = t / MJ, j = t % MJ;
-      const f32x4 v = acc[i][j];
-      const auto even = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[0]), __float_as_uint(v[2]), false, false);
-      const auto odd = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[1]), __float_as_uint(v[3]), false, false);
-      const bf16x2 y = {(__bf16)gt_act(__uint_as_float(even[0]), __uint_as_float(even[1]), act),
-                        (__bf16)gt_act(__uint_as_float(odd[0]), __uint_as_float(odd[1]), act)};
-      *reinterpret_cast<uint32_t*>(tile + ((wm * MJ + j) * 16 + c) * S::PITCH + (wn * NI + i) * 8 + 2 * g) = __builtin_bit_cast(uint32_t, y);
-    }
-  __syncthreads();
-  for (int idx = tid; idx < S::TM * 2 * S::NB; idx += 64 * WAVES) {
-    const int m = idx / (2 * S::NB), q = idx % (2 * S::NB);
-    if (m < live && q < own)
-      *reinterpret_cast<uint2*>(C + (int64_t)(m0 + m) * ldc + c0 + 4 * q) = *reinterpret_cast<const uint2*>(tile + m * S::PITCH + 4 * q);
+}
+
+// What workgroup `id` of m_tiles x groups owns: rows of A from m0 on, `live` of them, and units of W from u0 on, `own` of them.  Workgroups
+// that share rows of W are neighbours on one XCD.
+struct SpreadShare {
+  int m0, live, u0, own;
+  __device__ __forceinline__ bool take(int M, int units, int m_tiles, int tile_rows, int groups) {
+    const int total = m_tiles * groups, run = (total + 7) / 8, at8 = blockIdx.x / 8, id = (blockIdx.x % 8) * run + at8;
+    if (at8 >= run || id >= total) return false;
+    const int b = id / m_tiles;
+    m0 = id % m_tiles * tile_rows;
+    live = min(tile_rows, M - m0);
+    u0 = __builtin_amdgcn_readfirstlane((int)((int64_t)b * units / groups));
+    own = __builtin_amdgcn_readfirstlane((int)((int64_t)(b + 1) * units / groups)) - u0;
+    return true;
   }
+};
+// Lanes of even g hold four columns' first rows of W (gates, a head's lower half), the 16 lanes behind them the second ones: exchanged
+// so that every lane has both of two columns, 2 g and 2 g + 1 of the block's eight.
+struct SpreadPairs {
+  float first[2], second[2];
+  __device__ __forceinline__ explicit SpreadPairs(const f32x4& v) {
+    const auto even = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[0]), __float_as_uint(v[2]), false, false);
+    const auto odd = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[1]), __float_as_uint(v[3]), false, false);
+    first[0] = __uint_as_float(even[0]);
+    second[0] = __uint_as_float(even[1]);
+    first[1] = __uint_as_float(odd[0]);
+    second[1] = __uint_as_float(odd[1]);
+  }
+};
+__device__ __forceinline__ uint32_t gt_round2(float a, float b) {
+  const bf16x2 r = {(__bf16)a, (__bf16)b};
+  return __builtin_bit_cast(uint32_t, r);
 }
 
 template <int NI, int MJ, int WN, int WM, int WK, int NBUF>
-static int gt_spread(void* C, int64_t ldc, const void* A, int64_t lda, const void* W, int M, int cols, int K, int m_tiles, int groups,
-                     GateAct act, hipStream_t stream) {
+__global__ __launch_bounds__(64 * WN * WM * WK, 1) void gemm_spread_gated_kernel(
+    bf16_t* __restrict__ C, int64_t ldc, const bf16_t* __restrict__ A, int64_t lda, const bf16_t* __restrict__ W, int M, int cols,
+    int K, int m_tiles, int tile_rows, int groups, GateAct act) {
   using S = SpreadTile<NI, MJ, WN, WM, WK, NBUF>;
-  const int tile_rows = ((M + m_tiles - 1) / m_tiles + 15) / 16 * 16, units = cols / 4;
-  if (K % S::BK || tile_rows > S::TM || (int64_t)(m_tiles - 1) * tile_rows >= M || groups > units || (units + groups - 1) / groups > 2 * S::NB) return -7;
-  const auto kernel = gemm_spread_gated_kernel<NI, MJ, WN, WM, WK, NBUF>;
-  const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, S::LDS);
-  if (raised != hipSuccess) return (int)raised;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)((m_tiles * groups + 7) / 8 * 8)), dim3(64 * S::WAVES), S::LDS, stream, (bf16_t*)C, ldc,
-                     (const bf16_t*)A, lda, (const bf16_t*)W, M, cols, K, m_tiles, tile_rows, groups, act);
-  return GA_CHECK_LAUNCH();
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  SpreadShare mine;
+  if (!mine.take(M, cols / 4, m_tiles, tile_rows, groups)) return;
+  const int c0 = 4 * mine.u0;
+  f32x4 acc[NI][MJ];
+  // rows 0 to 3 of a unit are gates, 4 to 7 the same columns' ups
+  spread_sums<NI, MJ, WN, WM, WK, NBUF>(acc, lds, A, lda, W, K, 0, K / S::BK, mine.m0, mine.live, mine.own,
+                                        [&](int r) { return c0 + (r / 8) * 4 + (r & 3) + ((r & 4) ? cols : 0); });
+  const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave % WM, wn = wave / WM % WN, wk = wave / (WM * WN);
+  bf16_t* tile = reinterpret_cast<bf16_t*>(lds);       // through LDS, so that a row's columns leave side by side
+#pragma unroll
+  for (int t = 0; t < NI * MJ; ++t)
+    if (WK == 1 || t % 2 == wk) {
+      const int i = t / MJ, j = t % MJ;
+      const SpreadPairs v(acc[i][j]);
+      *reinterpret_cast<uint32_t*>(tile + ((wm * MJ + j) * 16 + c) * S::PITCH + (wn * NI + i) * 8 + 2 * g) =
+          gt_round2(gt_act(v.first[0], v.second[0], act), gt_act(v.first[1], v.second[1], act));
+    }
+  __syncthreads();
+  for (int idx = threadIdx.x; idx < S::TM * 2 * S::NB; idx += 64 * S::WAVES) {
+    const int m = idx / (2 * S::NB), q = idx % (2 * S::NB);
+    if (m < mine.live && q < mine.own)
+      *reinterpret_cast<uint2*>(C + (int64_t)(mine.m0 + m) * ldc + c0 + 4 * q) = *reinterpret_cast<const uint2*>(tile + m * S::PITCH + 4 * q);
+  }
 }
+
+// The same for partial sums [parts][M][cols]: the grid's y is the part of K, a unit eight neighbouring columns.
+template <int NI, int MJ, int WN, int WM, int WK, int NBUF>
+__global__ __launch_bounds__(64 * WN * WM * WK, 1) void gemm_spread_parts_kernel(
+    float* __restrict__ C, const bf16_t* __restrict__ A, int64_t lda, const bf16_t* __restrict__ W, int M, int cols, int K, int m_tiles,
+    int tile_rows, int groups, int slabs_per_part) {
+  using S = SpreadTile<NI, MJ, WN, WM, WK, NBUF>;
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  SpreadShare mine;
+  if (!mine.take(M, cols / 8, m_tiles, tile_rows, groups)) return;
+  const int c0 = 8 * mine.u0, slab0 = blockIdx.y * slabs_per_part;
+  f32x4 acc[NI][MJ];
+  spread_sums<NI, MJ, WN, WM, WK, NBUF>(acc, lds, A, lda, W, K, slab0, min(slabs_per_part, K / S::BK - slab0), mine.m0, mine.live, mine.own,
+                                        [&](int r) { return c0 + r; });
+  const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave % WM, wn = wave / WM % WN, wk = wave / (WM * WN);
+  float* P = C + ((int64_t)blockIdx.y * M + mine.m0) * cols + c0;
+#pragma unroll
+  for (int t = 0; t < NI * MJ; ++t)
+    if (WK == 1 || t % 2 == wk) {
+      const int i = t / MJ, m = (wm * MJ + t % MJ) * 16 + c, n = (wn * NI + i) * 16 + 4 * g;
+      const f32x4 v = acc[i][t % MJ];
+      if (m < mine.live && n < 8 * mine.own) *reinterpret_cast<float4*>(P + (int64_t)m * cols + n) = make_float4(v[0], v[1], v[2], v[3]);
+    }
+}
+
+// The fused q|k|v projection of a step of 17 to 512 rows with its epilogue: bias, NeoX rotation of q and k on the 32-bit sums, q to its own
+// buffer, k and v into the paged cache (layouts and formula as in rope_kv.hip).  A unit is four columns of a head and their rotation
+// partners half a head on, or eight columns of a v head.
+struct SpreadQkv {
+  const bf16_t* bias;
+  const int32_t* positions;
+  const float *cos_t, *sin_t;
+  const int64_t* slots;
+  bf16_t *k_pages, *v_pages;
+  int nh, nkv, hd, page_size, write_kv;
+};
+template <int NI, int MJ, int WN, int WM, int WK, int NBUF>
+__global__ __launch_bounds__(64 * WN * WM * WK, 1) void gemm_spread_qkv_kernel(
+    bf16_t* __restrict__ q_out, const bf16_t* __restrict__ A, int64_t lda, const bf16_t* __restrict__ W, int M, int K, int m_tiles,
+    int tile_rows, int groups, const SpreadQkv x) {
+  using S = SpreadTile<NI, MJ, WN, WM, WK, NBUF>;
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  SpreadShare mine;
+  if (!mine.take(M, (x.nh + 2 * x.nkv) * x.hd / 8, m_tiles, tile_rows, groups)) return;
+  const int half = x.hd / 2, per_head = x.hd / 8, turned = (x.nh + x.nkv) * per_head;      // units of a head; of q and k
+  // the first row of W of a unit, and how far on its second four rows lie
+  auto unit_row = [&](int u) { return u < turned ? u / per_head * x.hd + u % per_head * 4 : u * 8; };
+  auto unit_step = [&](int u) { return u < turned ? half : 4; };
+  f32x4 acc[NI][MJ];
+  spread_sums<NI, MJ, WN, WM, WK, NBUF>(acc, lds, A, lda, W, K, 0, K / S::BK, mine.m0, mine.live, mine.own, [&](int r) {
+    const int u = mine.u0 + r / 8;
+    return unit_row(u) + (r & 3) + ((r & 4) ? unit_step(u) : 0);
+  });
+  const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave % WM, wn = wave / WM % WN, wk = wave / (WM * WN);
+#pragma unroll
+  for (int t = 0; t < NI * MJ; ++t)
+    if (WK == 1 || t % 2 == wk) {
+      const int i = t / MJ, row = (wm * MJ + t % MJ) * 16 + c, m = mine.m0 + row;
+      const int lu = (wn * NI + i) * 2 + (g >> 1), u = mine.u0 + lu;
+      const SpreadPairs v(acc[i][t % MJ]);
+      if (row >= mine.live || lu >= mine.own) continue;
+      const int n = unit_row(u) + 2 * (g & 1), step = unit_step(u);          // columns n, n + 1 and their partners
+      float lo[2] = {v.first[0], v.first[1]}, hi[2] = {v.second[0], v.second[1]};
+      if (x.bias) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          lo[e] += bf16_to_f32(x.bias[n + e]);
+          hi[e] += bf16_to_f32(x.bias[n + step + e]);
+        }
+      }
+      const int64_t slot = x.write_kv && u >= x.nh * per_head ? x.slots[m] : -1;
+      int64_t page = 0, off = 0;
+      if (slot >= 0) slot_page(slot, x.page_size, page, off);
+      if (u < turned) {
+        const int j = n % x.hd, head = n / x.hd;
+        const int64_t at = (int64_t)x.positions[m] * half + j;
+        const float c0 = x.cos_t[at], c1 = x.cos_t[at + 1], s0 = x.sin_t[at], s1 = x.sin_t[at + 1];
+        const uint32_t a = gt_round2(lo[0] * c0 - hi[0] * s0, lo[1] * c1 - hi[1] * s1), b = gt_round2(lo[0] * s0 + hi[0] * c0, lo[1] * s1 + hi[1] * c1);
+        bf16_t* o = nullptr;
+        if (head < x.nh) o = q_out + ((int64_t)m * x.nh + head) * x.hd + j;
+        else if (slot >= 0) o = x.k_pages + ((page * x.nkv + (head - x.nh)) * x.page_size + off) * x.hd + j;
+        if (o) {
+          *reinterpret_cast<uint32_t*>(o) = a;
+          *reinterpret_cast<uint32_t*>(o + half) = b;
+        }
+      } else if (slot >= 0) {
+        const int d = n - (x.nh + x.nkv) * x.hd;                     // column of the v heads
+        bf16_t* o = x.v_pages + (page * x.nkv * x.hd + d) * (int64_t)x.page_size + off;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          o[(int64_t)e * x.page_size] = f32_to_bf16(lo[e]);
+          o[(int64_t)(step + e) * x.page_size] = f32_to_bf16(hi[e]);
+        }
+      }
+    }
+}
+
+// The tiles: NI, MJ, WN, WM, WK, buffers; room for 16 MJ WM rows of A and 16 NI WN of W.  The first ten serve the gated product, all of
+// them the others, whose columns are few.
+#define GA_SPREAD_GATED(X)                                                                                             \
+  X(0, 5, 1, 1, 4, 2, 4) X(1, 5, 2, 1, 4, 2, 3) X(2, 5, 1, 2, 4, 1, 5) X(3, 5, 2, 2, 4, 1, 4) X(4, 5, 3, 2, 4, 1, 3) \
+  X(5, 5, 4, 2, 4, 1, 3) X(6, 4, 1, 2, 4, 1, 6) X(7, 4, 2, 2, 4, 1, 5) X(8, 4, 3, 2, 4, 1, 4) X(9, 4, 4, 2, 4, 1, 3)
+#define GA_SPREAD_NARROW(X) X(10, 1, 1, 1, 4, 2, 7) X(11, 2, 1, 1, 4, 2, 6) X(12, 2, 2, 1, 4, 2, 4) X(13, 3, 1, 1, 4, 2, 5) X(14, 3, 2, 1, 4, 2, 3)
+
+// Whether a tile holds what a launch deals out; the rows of A of a row tile
+template <int NI, int MJ, int WN, int WM, int WK, int NBUF>
+static bool spread_fits(int M, int units, int slabs_of_64, int m_tiles, int groups, int& tile_rows) {
+  using S = SpreadTile<NI, MJ, WN, WM, WK, NBUF>;
+  tile_rows = ((M + m_tiles - 1) / m_tiles + 15) / 16 * 16;
+  return slabs_of_64 % WK == 0 && tile_rows <= S::TM && (int64_t)(m_tiles - 1) * tile_rows < M && groups <= units &&
+         (units + groups - 1) / groups <= 2 * S::NB;
+}
+template <typename Kernel>
+static int spread_room(Kernel kernel, int bytes) {
+  return (int)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);      // the current device's
+}
+static int spread_check(int M, int m_tiles, int groups) {
+  return m_tiles < 1 || m_tiles > M || groups < 1 || (int64_t)m_tiles * groups > 1 << 20 ? -1 : 0;
+}
+#define GA_SPREAD_GRID(parts) dim3((unsigned)((m_tiles * groups + 7) / 8 * 8), parts)
 
 // tiling: which tiles, rows of W x rows of A; the caller chooses by sizes and by how full they leave the chip's rounds
 // (gated_tiling in kernels/ops.py, tiles_gated in parts/linear.py, the fastest and the library beside each other).  us, product and
@@ -468,19 +616,84 @@ extern "C" int ga_gemm_spread_gated(void* C, int64_t ldc, const void* A, int64_t
   if (M <= 0) return 0;
   const int rc = gt_check(C, A, lda, W, 2 * (int64_t)cols, M, cols, K);
   if (rc) return rc;
-  if (kind < 0 || kind > 2 || ldc < cols || ldc % 4 || m_tiles < 1 || m_tiles > M || groups < 1 || (int64_t)m_tiles * groups > 1 << 20) return -1;
+  if (kind < 0 || kind > 2 || ldc < cols || ldc % 4 || spread_check(M, m_tiles, groups)) return -1;
   const GateAct act = {kind, limit, alpha, shift};
+  int tile_rows;
   switch (shape) {
-    case 0: return gt_spread<5, 1, 1, 4, 2, 4>(C, ldc, A, lda, W, M, cols, K, m_tiles, groups, act, stream);     // 64 rows of A, 80 of W
-    case 1: return gt_spread<5, 2, 1, 4, 2, 3>(C, ldc, A, lda, W, M, cols, K, m_tiles, groups, act, stream);     // 128, 80
-    case 2: return gt_spread<5, 1, 2, 4, 1, 5>(C, ldc, A, lda, W, M, cols, K, m_tiles, groups, act, stream);     // 64, 160
-    case 3: return gt_spread<5, 2, 2, 4, 1, 4>(C, ldc, A, lda, W, M, cols, K, m_tiles, groups, act, stream);     // 128, 160
-    case 4: return gt_spread<5, 3, 2, 4, 1, 3>(C, ldc, A, lda, W, M, cols, K, m_tiles, groups, act, stream);     // 192, 160
-    case 5: return gt_spread<5, 4, 2, 4, 1, 3>(C, ldc, A, lda, W, M, cols, K, m_tiles, groups, act, stream);     // 256, 160
-    case 6: return gt_spread<4, 1, 2, 4, 1, 6>(C, ldc, A, lda, W, M, cols, K, m_tiles, groups, act, stream);     // 64, 128
-    case 7: return gt_spread<4, 2, 2, 4, 1, 5>(C, ldc, A, lda, W, M, cols, K, m_tiles, groups, act, stream);     // 128, 128
-    case 8: return gt_spread<4, 3, 2, 4, 1, 4>(C, ldc, A, lda, W, M, cols, K, m_tiles, groups, act, stream);     // 192, 128
-    case 9: return gt_spread<4, 4, 2, 4, 1, 3>(C, ldc, A, lda, W, M, cols, K, m_tiles, groups, act, stream);     // 256, 128
+#define CASE(n, ...)                                                                                                                     \
+  case n: {                                                                                                                              \
+    if (!spread_fits<__VA_ARGS__>(M, cols / 4, K / 64, m_tiles, groups, tile_rows)) return -7;                                           \
+    constexpr int bytes = SpreadTile<__VA_ARGS__>::LDS;                                                                                  \
+    if (const int raised = spread_room(gemm_spread_gated_kernel<__VA_ARGS__>, bytes)) return raised;                                     \
+    hipLaunchKernelGGL((gemm_spread_gated_kernel<__VA_ARGS__>), GA_SPREAD_GRID(1), dim3(64 * SpreadTile<__VA_ARGS__>::WAVES), bytes,     \
+                       stream, (bf16_t*)C, ldc, (const bf16_t*)A, lda, (const bf16_t*)W, M, cols, K, m_tiles, tile_rows, groups, act);   \
+    return GA_CHECK_LAUNCH();                                                                                                            \
+  }
+    GA_SPREAD_GATED(CASE)
+#undef CASE
+  }
+  return -6;
+}
+
+// Which shape, row tiles and groups: spread_few_columns in kernels/ops.py; how many parts, and where the other plans are the faster: spread_parts
+// in parts/linear.py, with the figures.  570 products of 70 sizes of W with the norm that adds their parts, 17 to 384 rows: 1.18 times as
+// fast in the geometric mean.
+extern "C" int ga_gemm_spread_parts(void* C, const void* A, int64_t lda, const void* W, int M, int cols, int K, int parts, int shape,
+                                    int m_tiles, int groups, hipStream_t stream) {
+  if (M <= 0) return 0;
+  const int rc = gt_check(C, A, lda, W, cols, M, cols, K);
+  if (rc) return rc;
+  if (spread_check(M, m_tiles, groups) || parts < 1 || parts > K / 64 || parts > 65535) return -1;
+  const int per_part = (K / 64 + parts - 1) / parts;                   // slabs of 64
+  if ((parts - 1) * per_part >= K / 64) return -4;       // a part without a slab
+  int tile_rows;
+  switch (shape) {
+#define CASE(n, ...)                                                                                                                     \
+  case n: {                                                                                                                              \
+    constexpr int slab = SpreadTile<__VA_ARGS__>::BK / 64, bytes = SpreadTile<__VA_ARGS__>::LDS;                                         \
+    if (!spread_fits<__VA_ARGS__>(M, cols / 8, K / 64, m_tiles, groups, tile_rows) || (parts > 1 && per_part % slab)) return -7;         \
+    if (const int raised = spread_room(gemm_spread_parts_kernel<__VA_ARGS__>, bytes)) return raised;                                     \
+    hipLaunchKernelGGL((gemm_spread_parts_kernel<__VA_ARGS__>), GA_SPREAD_GRID(parts), dim3(64 * SpreadTile<__VA_ARGS__>::WAVES), bytes, \
+                       stream, (float*)C, (const bf16_t*)A, lda, (const bf16_t*)W, M, cols, K, m_tiles, tile_rows, groups,               \
+                       per_part / slab);                                                                                                 \
+    return GA_CHECK_LAUNCH();                                                                                                            \
+  }
+    GA_SPREAD_GATED(CASE) GA_SPREAD_NARROW(CASE)
+#undef CASE
+  }
+  return -6;
+}
+
+// us of the fused kernel for few rows (up to 64 rows), or the library and the rotation -> here: 2,048 columns, K 1,536: 17 rows 6.2 -> 6.0, 64
+// 8.4 -> 6.8, 128 12.4 -> 7.7, 256 13.5 -> 9.3, 512 14.6 -> 12.9; 4,608, K 3,584: 64 rows 19.2 -> 14.3, 256 40.6 -> 23.4, 512 37.5 -> 32.0; 1,152, K
+// 896: 128 rows 10.5 -> 5.5; 10,240, K 8,192: 65 rows 81.9 -> 43.7; of 72 the slowest 2 % behind (6,144, K 4,096 at 512 rows 44.2 -> 45.0).
+// W [(nh + 2 nkv) hd, K], bias [the same] or null, hd a multiple of 8 that is rotated whole; the rest as ga_qkv_rope_skinny
+extern "C" int ga_qkv_spread(void* q_out, const void* A, int64_t lda, const void* W, const void* bias, const void* positions,
+                             const void* cos_t, const void* sin_t, const void* slot_mapping, void* k_pages, void* v_pages, int M, int K,
+                             int nh, int nkv, int hd, int page_size, int write_kv, int shape, int m_tiles, int groups,
+                             hipStream_t stream) {
+  if (M <= 0) return 0;
+  if (nh <= 0 || nkv <= 0 || hd <= 0 || hd % 8 || page_size <= 0 || (write_kv && (!slot_mapping || !k_pages || !v_pages))) return -1;
+  const int64_t cols = ((int64_t)nh + 2 * nkv) * hd;
+  if (cols > 1 << 24) return -1;
+  const int rc = gt_check(q_out, A, lda, W, cols, M, (int)cols, K);
+  if (rc) return rc;
+  if (spread_check(M, m_tiles, groups)) return -1;
+  const SpreadQkv x = {(const bf16_t*)bias, (const int32_t*)positions, (const float*)cos_t, (const float*)sin_t, (const int64_t*)slot_mapping,
+                       (bf16_t*)k_pages, (bf16_t*)v_pages, nh, nkv, hd, page_size, write_kv};
+  int tile_rows;
+  switch (shape) {
+#define CASE(n, ...)                                                                                                                     \
+  case n: {                                                                                                                              \
+    if (!spread_fits<__VA_ARGS__>(M, (int)(cols / 8), K / 64, m_tiles, groups, tile_rows)) return -7;                                    \
+    constexpr int bytes = SpreadTile<__VA_ARGS__>::LDS;                                                                                  \
+    if (const int raised = spread_room(gemm_spread_qkv_kernel<__VA_ARGS__>, bytes)) return raised;                                       \
+    hipLaunchKernelGGL((gemm_spread_qkv_kernel<__VA_ARGS__>), GA_SPREAD_GRID(1), dim3(64 * SpreadTile<__VA_ARGS__>::WAVES), bytes,       \
+                       stream, (bf16_t*)q_out, (const bf16_t*)A, lda, (const bf16_t*)W, M, K, m_tiles, tile_rows, groups, x);            \
+    return GA_CHECK_LAUNCH();                                                                                                            \
+  }
+    GA_SPREAD_GATED(CASE) GA_SPREAD_NARROW(CASE)
+#undef CASE
   }
   return -6;
 }

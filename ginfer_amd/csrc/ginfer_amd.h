@@ -104,6 +104,11 @@ int ga_gemm_tiles_gated(void* C, int64_t ldc, const void* A, int64_t lda, const 
                         float limit, float alpha, float shift, int tiling, hipStream_t stream);
 int ga_gemm_spread_gated(void* C, int64_t ldc, const void* A, int64_t lda, const void* W, int M, int cols, int K, int kind,
                          float limit, float alpha, float shift, int shape, int m_tiles, int groups, hipStream_t stream);
+int ga_gemm_spread_parts(void* C, const void* A, int64_t lda, const void* W, int M, int cols, int K, int parts, int shape, int m_tiles,
+                         int groups, hipStream_t stream);
+int ga_qkv_spread(void* q_out, const void* A, int64_t lda, const void* W, const void* bias, const void* positions, const void* cos_t,
+                  const void* sin_t, const void* slot_mapping, void* k_pages, void* v_pages, int M, int K, int nh, int nkv, int hd,
+                  int page_size, int write_kv, int shape, int m_tiles, int groups, hipStream_t stream);
 int ga_gemm_tiles_parts(void* C, const void* A, int64_t lda, const void* W, int M, int cols, int K, int parts, hipStream_t stream);
 
 // ---- embedding_sinusoid.hip: out float [tokens, hidden] = table_scale * table[ids] + (sin | cos)(position * freq[i / 2]), then the norm

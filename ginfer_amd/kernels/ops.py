@@ -6,6 +6,7 @@ fit; a kernel never sees a shape it was not written for.  Tensors are torch tens
 kernels run on torch's current stream.
 """
 import ctypes
+import functools
 import math
 
 import torch
@@ -514,6 +515,7 @@ SPREAD_SHAPES = ((64, 80, 128), (128, 80, 128), (64, 160, 64), (128, 160, 64), (
                  (64, 128, 64), (128, 128, 64), (192, 128, 64), (256, 128, 64))     # room for rows of A and of W, elements of a slab
 
 
+@functools.lru_cache(maxsize=4096)
 def spread_plan(rows, out_features, in_features):
     """(number in SPREAD_SHAPES, row tiles, groups of columns) of the gated product of 17 to 512 rows by `out_features` rows of W
     dealt evenly to the chip (csrc/gemm_tiles.hip), or None where the tiles of gated_tiling and gated_wide_tiling are the faster or
@@ -546,8 +548,40 @@ def spread_plan(rows, out_features, in_features):
     return best[1]
 
 
-def gemm_tiles_parts(a, w, parts):
-    """a [M, K] . w [N, K]^T as float32 partial sums [parts, M, N] over parts of K, for the consumer to add in order."""
+SPREAD_NARROW_SHAPES = ((64, 16, 128), (64, 32, 128), (128, 32, 128), (64, 48, 128), (128, 48, 128))     # beside the others, for few columns
+
+
+@functools.lru_cache(maxsize=4096)
+def spread_few_columns(rows, out_features, in_features, parts=1):
+    """(what a compute unit reads, in rows; (number in SPREAD_SHAPES + SPREAD_NARROW_SHAPES, row tiles, groups)) of a product of few columns
+    dealt evenly to the chip in `parts` parts of K, or None where no shape holds it.  A row of W that several row tiles read counts a
+    tenth more for each of them (7,168 x 5,120 at 65 rows in one row tile 25.4 us, in two, of fewer rows each, 28.8), and a row that the
+    tile has room for and does not own a quarter (its operands are read from LDS all the same: 1,536 x 8,960 at 25 rows in four parts of
+    24 rows of W in a tile of 128 17.2 us, in eight parts of 48 in one of 48 11.9)."""
+    slabs, units, best = in_features // 64, out_features // 8, None
+    of_part = -(-slabs // parts)
+    if (parts - 1) * of_part >= slabs:
+        return None
+    for m_tiles in range(1, 13):
+        tile_rows = -(-(-(-rows // m_tiles)) // 16) * 16
+        groups = min(units, 256 // (m_tiles * parts))
+        if (m_tiles - 1) * tile_rows >= rows or groups < 1:
+            continue
+        of_w = -(-units // groups) * 8
+        fits = [(tm * tw, n, tw) for n, (tm, tw, bk) in enumerate(SPREAD_SHAPES + SPREAD_NARROW_SHAPES)
+                if tm >= tile_rows and tw >= of_w and slabs % (bk // 64) == 0 and (parts == 1 or of_part % (bk // 64) == 0)]
+        if not fits:
+            continue
+        _, number, tw = min(fits)
+        cost = tile_rows + of_w * (1.0 + 0.1 * (m_tiles - 1)) + 0.25 * (tw - of_w)
+        if best is None or cost < best[0]:
+            best = (cost, (number, m_tiles, groups))
+    return best
+
+
+def gemm_tiles_parts(a, w, parts, plan=None):
+    """a [M, K] . w [N, K]^T as float32 partial sums [parts, M, N] over parts of K, for the consumer to add in order.  plan: None for tiles
+    of 64 or 128 columns, or (shape, row tiles, groups) of the kernel that deals them evenly (spread_few_columns)."""
     _dev(a, w)
     _need(gemm_tiles_supported(a, w) and a.shape[1] == w.shape[1], "the kernel over tiles does not take %s %s x %s %s", a.dtype,
           tuple(a.shape), w.dtype, tuple(w.shape))
@@ -556,6 +590,10 @@ def gemm_tiles_parts(a, w, parts):
     M, N = a.shape[0], w.shape[0]
     out = torch.empty((parts, M, N), dtype=torch.float32, device=a.device)
     lib = build.load("gemm_tiles")
+    if plan is not None:
+        _check(lib.ga_gemm_spread_parts(_ptr(out), _ptr(a), _i64(a.stride(0)), _ptr(w), _i(M), _i(N), _i(a.shape[1]), _i(parts), *(_i(v) for v in plan),
+                                        _stream()), "gemm_spread_parts")
+        return out
     _check(lib.ga_gemm_tiles_parts(_ptr(out), _ptr(a), _i64(a.stride(0)), _ptr(w), _i(M), _i(N), _i(a.shape[1]), _i(parts), _stream()),
            "gemm_tiles_parts")
     return out
@@ -685,6 +723,45 @@ def qkv_rope_skinny(x, w, bias, positions, cos, sin, slot_mapping, k_pages, v_pa
                                   _ptr(sin), _ptr(slot_mapping), _ptr(k_pages), _ptr(v_pages), _i(M), _i(K), _i(num_heads),
                                   _i(num_kv_heads), _i(head_dim), _i(page_size), _i(1 if write_kv else 0), _i(pack),
                                   ctypes.byref(norm) if norm is not None else _vp(0), _stream()), "qkv_rope_skinny")
+    return q
+
+
+def qkv_spread_plan(x, w, head_dim, rotary_dim):
+    """The plan by which the q|k|v projection of 17 to 512 rows with its rotation and cache write is one kernel (csrc/gemm_tiles.hip), or None
+    where its operands are not of the kind."""
+    if (isinstance(x, ScaledRows) or not gemm_tiles_supported(x, w) or not 17 <= x.shape[0] <= 512 or head_dim % 8 or rotary_dim != head_dim):
+        return None
+    best = spread_few_columns(x.shape[0], w.shape[0], w.shape[1])
+    return best and best[1]
+
+
+def qkv_spread(x, w, bias, positions, cos, sin, slot_mapping, k_pages, v_pages, num_heads, num_kv_heads, head_dim, write_kv=True,
+               plan=None):
+    """qkv_rope_skinny for more rows: x [M, K] . w^T + bias, NeoX rotation of whole heads on the 32-bit sums, q returned as [M, nh*hd], k and
+    v written into the paged cache at slot_mapping.  plan: as qkv_spread_plan makes them (None: that)."""
+    _dev(x, w, bias, positions, cos, sin, slot_mapping, k_pages, v_pages)
+    M, K = x.shape
+    width = (num_heads + 2 * num_kv_heads) * head_dim
+    _need(w.shape == (width, K), "qkv weight must be [%d, %d], got %s", width, K, tuple(w.shape))
+    _need(gemm_tiles_supported(x, w) and head_dim % 8 == 0, "the kernel over tiles does not take %s %s x %s %s in heads of %d", x.dtype,
+          tuple(x.shape), w.dtype, tuple(w.shape), head_dim)
+    if bias is not None:
+        _need(bias.dtype == torch.bfloat16 and bias.shape == (width,) and bias.is_contiguous(), "qkv bias must be bfloat16 [%d]", width)
+    _need(positions.dtype == torch.int32 and positions.shape == (M,) and positions.is_contiguous(), "positions must be int32 [M]")
+    _need(cos.dtype == torch.float32 and sin.dtype == torch.float32 and cos.shape == sin.shape and cos.is_contiguous()
+          and sin.is_contiguous() and 2 * cos.shape[1] == head_dim, "cos and sin must be contiguous float32 [P, head_dim/2]")
+    page_size = 1
+    if write_kv:
+        _need(slot_mapping is not None and slot_mapping.dtype == torch.int64 and slot_mapping.shape == (M,)
+              and slot_mapping.is_contiguous(), "slot_mapping must be contiguous int64 [M]")
+        page_size = _check_pages(k_pages, v_pages, torch.bfloat16, num_kv_heads, head_dim)
+    plan = plan or qkv_spread_plan(x, w, head_dim, head_dim)
+    _need(plan is not None, "no tiles hold q|k|v of %d rows, %d x %d", M, width, K)
+    q = torch.empty((M, num_heads * head_dim), dtype=torch.bfloat16, device=x.device)
+    lib = build.load("gemm_tiles")
+    _check(lib.ga_qkv_spread(_ptr(q), _ptr(x), _i64(x.stride(0)), _ptr(w), _ptr(bias), _ptr(positions), _ptr(cos), _ptr(sin), _ptr(slot_mapping),
+                             _ptr(k_pages), _ptr(v_pages), _i(M), _i(K), _i(num_heads), _i(num_kv_heads), _i(head_dim), _i(page_size),
+                             _i(1 if write_kv else 0), *(_i(v) for v in plan), _stream()), "qkv_spread")
     return q
 
 

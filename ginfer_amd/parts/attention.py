@@ -33,7 +33,7 @@ def _projection_in_parts(rows, in_features, out_features):
 
 
 def _projection_way(x, w_qkv, head_dim, rotary_dim):
-    """("fused",), ("parts", n) or ("library",): how rows x become q, k and v."""
+    """("fused",), ("parts", n) or ("library",): how rows x become q, k and v where their product is not dealt evenly to the chip."""
     rows, K = x.shape
     if ops.qkv_rope_skinny_supported(x, w_qkv, head_dim, rotary_dim):
         return ("library",) if _library_then_rotation_is_faster(rows, K, w_qkv.shape[0]) else ("fused",)
@@ -104,11 +104,16 @@ class Attention(Part):
         """into_norm = (residual, norm): where the output projection's kernel can, the result is added to the
         residual here and the rows of `norm` come back as ops.ScaledRows; else the result comes back as ever."""
         cos, sin = self.position.tables()
-        way = _projection_way(x, self.w_qkv, self.hd, self.position.rotary_dim)
+        spread = ops.qkv_spread_plan(x, self.w_qkv, self.hd, self.position.rotary_dim)
+        way = ("spread",) if spread else _projection_way(x, self.w_qkv, self.hd, self.position.rotary_dim)
         if way[0] == "fused":
             # few rows (decode): projection, rotation and cache write in one kernel
             qkv = ops.qkv_rope_skinny(x, self.w_qkv, self.b_qkv, step.positions, cos, sin, cache.slot_mapping,
                                       cache.k_pages, cache.v_pages, self.nh, self.nkv, self.hd, write_kv=cache.owner)
+        elif way[0] == "spread":
+            # more rows: the same, over tiles that are dealt evenly to the chip
+            qkv = ops.qkv_spread(x, self.w_qkv, self.b_qkv, step.positions, cos, sin, cache.slot_mapping, cache.k_pages, cache.v_pages,
+                                 self.nh, self.nkv, self.hd, write_kv=cache.owner, plan=spread)
         elif way[0] == "parts":
             # the product with K split over workgroups (every workgroup then reads a share of the rows only), its 32-bit
             # parts added up by the kernel that rotates and writes the cache

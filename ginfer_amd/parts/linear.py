@@ -7,6 +7,8 @@ is where the reference calls its library (ginfer/core/op/kernels/cuda/gemm_kerne
 both accumulate in 32-bit and add the bias before the one rounding.  From 17 rows on the library also takes
 the products with a wide output, where it was measured faster; replays of recorded steps that hold
 these calls are checked bit for bit against eager steps in the tests."""
+import math
+
 import torch
 
 from ..kernels import autotune, ops
@@ -26,6 +28,7 @@ def linear(x, weight, bias=None, out_dtype=None, parts_ok=False):
     skinny_ok = ops.gemm_skinny_supported(x, weight)
     tiles_ok = (parts_ok and bias is None and not float32_out and TUNING.library_from_rows < x.shape[0] <= TUNING.tiles_parts_most_rows
                 and ops.gemm_tiles_supported(x, weight))
+    spread_ok = parts_ok and bias is None and not float32_out and ops.gemm_tiles_supported(x, weight)
     plan = None
     if autotune.active():
         key = ("linear", autotune.rows_class(x.shape[0]), weight.shape[0], x.shape[1], bias is not None, float32_out,
@@ -33,7 +36,58 @@ def linear(x, weight, bias=None, out_dtype=None, parts_ok=False):
         plan = autotune.choose(key, (weight, bias))
     if plan is None:
         plan = linear_plan(x.shape[0], weight.shape[0], x.shape[1], bias is not None, float32_out, parts_ok, skinny_ok, tiles_ok)
+        if spread_ok:
+            plan = spread_parts(plan, x.shape[0], weight.shape[0], x.shape[1]) or plan
     return run_linear_plan(plan, x, weight, bias, out_dtype)
+
+
+def _dealing_number(shape, m_tiles, groups):
+    """The second number of a ("tiles", number, parts) plan whose tiles are dealt evenly to the chip; 1 stands for those of 64 and 128
+    columns."""
+    return (groups * 100 + m_tiles) * 100 + shape
+
+
+def _dealing(number):
+    return None if number == 1 else (number % 100, number // 100 % 100, number // 10000)
+
+
+def _parts_estimate(rows, out_features, in_features, read, parts):
+    """us that a product in parts of K and the norm that adds them are taken to differ by: a compute unit's rows of W and A at the 50 GB/s it
+    takes in and all of W at 5.2 TB/s, which hide each other in part, the parts' way to memory and back, and what the norm's loop over
+    a number of parts it was not compiled for costs."""
+    streams = math.hypot(read * 2 * in_features / parts / 50e3, out_features * in_features * 2 / 5.2e6)
+    return streams + parts * rows * out_features * 8 / 3e6 + (0 if parts in (1, 2, 4, 8) else 3)
+
+
+def spread_parts(plan, rows, out_features, in_features):
+    """The plan of a product whose parts of K the consumer adds, over tiles that are dealt evenly to the chip, where it is faster than `plan`,
+    the other rules' (by sizes alone; the measurements stand beside the thresholds); else None."""
+    T = TUNING
+    if (not T.library_from_rows < rows <= T.spread_parts_most_rows or out_features % 16 or in_features % 64
+            or in_features < T.spread_parts_min_in_features or T.measured_plans):
+        return None
+    if plan[0] == "skinny" and rows <= T.spread_parts_beyond_rows:
+        return None
+    if rows > 256 and in_features <= T.spread_parts_short_k:
+        return None
+    if (plan[0] == "library" and out_features * in_features > T.spread_parts_library_weights
+            and T.spread_parts_library_from_rows < rows <= 256):
+        return None
+    best = None
+    for parts in (1, 2, 4, 8):
+        found = ops.spread_few_columns(rows, out_features, in_features, parts) if in_features >= parts * T.spread_parts_min_k else None
+        if found:
+            cost = _parts_estimate(rows, out_features, in_features, found[0], parts)
+            if best is None or cost < best[0]:
+                best = (cost, ("tiles", _dealing_number(*found[1]), parts))
+    if best is None:
+        return None
+    if plan[0] == "tiles":
+        tile = 64 if rows <= SKINNY_MAX_ROWS else 128
+        other = _parts_estimate(rows, out_features, in_features, 64 + tile, plan[2])
+        if best[0] > T.spread_parts_share_of_tiles * other or (rows <= 128 and best[1][2] == plan[2]):
+            return None
+    return best[1]
 
 
 def tiles_parts(rows, out_features, in_features):
@@ -88,7 +142,8 @@ def tiles_gated(rows, out_features, in_features):
 
 def linear_plan(rows, out_features, in_features, has_bias, float32_out, parts_ok, skinny_ok, tiles_ok=False):
     """The way a bfloat16 product is done, by the rules: ("skinny", tiles of W per wavefront, parts of K) for the
-    package's weight-streaming kernel, ("tiles", 1, parts of K) for its product over tiles, ("library", pieces of K) for the BLAS
+    package's weight-streaming kernel, ("tiles", 1, parts of K) for its product over tiles (another number than 1: over tiles dealt evenly,
+    `_dealing`), ("library", pieces of K) for the BLAS
     library; skinny_ok, tiles_ok: whether those kernels take the operands.  Tiles, and more than one part or piece, mean
     float32 partial sums [parts, M, N] for the consumer to add."""
     may_split = parts_ok and not float32_out
@@ -125,7 +180,7 @@ def run_linear_plan(plan, x, weight, bias, out_dtype):
             return ops.gemm_skinny(x, weight, bias, out_dtype=torch.float32, nt=nt, grid_splits=splits)
         return ops.gemm_skinny(x, weight, bias, out_dtype=out_dtype, nt=nt)
     if plan[0] == "tiles":
-        return ops.gemm_tiles_parts(x, weight, plan[2])
+        return ops.gemm_tiles_parts(x, weight, plan[2], _dealing(plan[1]))
     _, parts = plan
     if parts > 1:
         # the library, once, over `parts` pieces of K side by side (a batched product over views of x and
@@ -170,6 +225,9 @@ def linear_candidates(key):
         parts = tiles_parts(rows, out_features, in_features) if tiles_ok else 0
         if parts:
             add(("tiles", 1, parts))
+        spread = spread_parts(plans[0], rows, out_features, in_features) if tiles_ok else None
+        if spread:
+            add(spread)
         for parts in (2, 3, 4, 5, 7, 8, 10, 14, 16):
             if in_features % parts == 0 and (in_features // parts) % 8 == 0 and in_features // parts >= 512:
                 add(("library", parts))

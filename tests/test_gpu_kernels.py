@@ -1234,6 +1234,71 @@ def test_gated_product_dealt_evenly(shape, fill, m_tiles, K):
             ops.gemm_tiles_gated(a, w, tiling=plan)
 
 
+@pytest.mark.parametrize("shape", range(15))
+@pytest.mark.parametrize("fill,m_tiles,K,parts", [(0.3, 1, 128, 1), (1.0, 1, 1280, 2), (0.99, 2, 2304, 6), (0.6, 3, 384, 3)])
+def test_product_of_few_columns_dealt_evenly(shape, fill, m_tiles, K, parts):
+    """As above, K whole and in parts (uneven ones too) of one slab to more than there are buffers, groups of uneven numbers of units."""
+    from ginfer_amd.kernels import ops
+    tm, tw, bk = (ops.SPREAD_SHAPES + ops.SPREAD_NARROW_SHAPES)[shape]
+    M = max(1, int(fill * tm)) * m_tiles - (m_tiles - 1)
+    most = max(1, int(fill * tw) // 8)
+    groups, N = 6, (8 * most * 6 - 16) // 16 * 16 or 16
+    groups = min(groups, N // 8)
+    wide = rnd((M, K + 16), torch.bfloat16, 73)
+    a, w = wide[:, 8:8 + K], rnd((N, K), torch.bfloat16, 74)
+    got = ops.gemm_tiles_parts(a, w, parts, (shape, m_tiles, groups)).double()
+    per = -(-(K // 64) // parts) * 64
+    for p in range(parts):
+        close(got[p], a[:, p * per:(p + 1) * per].double() @ w[:, p * per:(p + 1) * per].double().t(), 2e-6)
+    for plan in ((15, m_tiles, groups), (shape, M + 1, groups), (shape, m_tiles, N // 8 + 1)):
+        with pytest.raises(ops.KernelError):
+            ops.gemm_tiles_parts(a, w, parts, plan)
+    if bk == 128:                                      # a part that is no whole number of slabs
+        with pytest.raises(ops.KernelError):
+            ops.gemm_tiles_parts(rnd((M, 192), torch.bfloat16, 1), rnd((N, 192), torch.bfloat16, 2), 1, (shape, m_tiles, groups))
+
+
+@pytest.mark.parametrize("M,hd,nh,nkv,K", [(17, 64, 3, 1, 128), (40, 48, 4, 2, 320), (64, 128, 12, 2, 256), (100, 80, 2, 2, 192), (161, 128, 4, 1, 384),
+                                           (290, 8, 6, 3, 64), (512, 32, 8, 2, 128)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_projection_dealt_evenly(M, hd, nh, nkv, K, bias):
+    """q|k|v of 17 to 512 rows, heads of 8 to 128, against 64 bits: one rounding of 32-bit sums; tokens whose slots skip a page or are left
+    out, places nobody writes as they were, a run that reads another layer's cache writes nothing."""
+    from ginfer_amd.kernels import ops
+    ps, width = 16, (nh + 2 * nkv) * hd
+    x, w = rnd((M, K), torch.bfloat16, 75), rnd((width, K), torch.bfloat16, 76, 0.05)
+    b = rnd((width,), torch.bfloat16, 77) if bias else None
+    ang = torch.arange(600, dtype=torch.float32)[:, None] * (10000.0 ** (-2.0 * torch.arange(hd // 2) / hd))[None]
+    cos, sin = torch.cos(ang), torch.sin(ang)
+    positions = torch.randint(0, 600, (M,), generator=torch.Generator().manual_seed(3)).to(torch.int32)
+    slots = torch.randperm((M // ps + 2) * ps, generator=torch.Generator().manual_seed(4))[:M].to(torch.int64)
+    slots[::7] = -1
+    pages = M // ps + 2
+    kp0, vp0 = rnd((pages, nkv, ps, hd), torch.bfloat16, 78).cpu(), rnd((pages, nkv, hd, ps), torch.bfloat16, 79).cpu()
+    kp, vp = kp0.clone().to(dev()), vp0.clone().to(dev())
+    args = (positions.to(dev()), cos.to(dev()), sin.to(dev()), slots.to(dev()))
+    assert ops.qkv_spread_plan(x, w, hd, hd) is not None
+    q = ops.qkv_spread(x, w, b, *args, kp, vp, nh, nkv, hd)
+    full = (x.double() @ w.double().t() + (b.double() if bias else 0.0)).cpu().view(M, nh + 2 * nkv, hd)
+    c, s = cos[positions.long()].double()[:, None], sin[positions.long()].double()[:, None]
+    lo, hi = full[:, :nh + nkv, :hd // 2], full[:, :nh + nkv, hd // 2:]
+    turned = torch.cat([lo * c - hi * s, lo * s + hi * c], dim=-1)
+    close(q.view(M, nh, hd), turned[:, :nh], 1e-2)
+    kr, vr = kp0.double(), vp0.double()
+    for t in range(M):
+        if int(slots[t]) >= 0:
+            kr[int(slots[t]) // ps, :, int(slots[t]) % ps] = turned[t, nh:]
+            vr[int(slots[t]) // ps, :, :, int(slots[t]) % ps] = full[t, nh + nkv:]
+    close(kp, kr, 1e-2)
+    close(vp, vr, 1e-2)
+    unwritten = torch.ones(pages * ps, dtype=torch.bool)
+    unwritten[slots[slots >= 0]] = False
+    page, off = (torch.nonzero(unwritten)[:, 0] // ps), (torch.nonzero(unwritten)[:, 0] % ps)
+    assert torch.equal(kp.cpu()[page, :, off], kp0[page, :, off]) and torch.equal(vp.cpu()[page, :, :, off], vp0[page, :, :, off])
+    kp1, vp1 = kp0.clone().to(dev()), vp0.clone().to(dev())
+    assert torch.equal(ops.qkv_spread(x, w, b, *args, kp1, vp1, nh, nkv, hd, write_kv=False), q) and torch.equal(kp1.cpu(), kp0) and torch.equal(vp1.cpu(), vp0)
+
+
 @pytest.mark.parametrize("M", [1, 63, 64, 65, 127, 256, 300])
 @pytest.mark.parametrize("N,K,parts", [(16, 64, 1), (80, 192, 3), (144, 320, 2), (1536, 640, 5), (64, 832, 13), (80, 256, 1),
                                        (144, 320, 1), (96, 576, 1), (64, 1088, 2), (208, 2112, 3)])

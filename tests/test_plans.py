@@ -193,6 +193,33 @@ def test_gated_products_dealt_evenly():
     assert faster("library", 384, 11136, 8192) and not faster("library", 508, 11136, 8192) and not faster("tiles", 64, 17920, 1536)
 
 
+def test_few_columns_dealt_evenly():
+    """A plan's tiles hold what it deals out, its parts of K are whole slabs, and it stands where it was measured the faster."""
+    from ginfer_amd.kernels import ops
+    shapes = ops.SPREAD_SHAPES + ops.SPREAD_NARROW_SHAPES
+    for rows in list(range(17, 513, 11)) + [64, 65, 128, 192, 256, 384, 512]:
+        for n, k in ((16, 64), (896, 4864), (1536, 1536), (1536, 8960), (2048, 1536), (3584, 18944), (4608, 3584), (10240, 8192), (2048, 704)):
+            for parts in (1, 2, 4, 8):
+                found = ops.spread_few_columns(rows, n, k, parts)
+                if found is None:
+                    continue
+                number, m_tiles, groups = found[1]
+                (tm, tw, bk), tile_rows, of_part = shapes[number], -(-(-(-rows // m_tiles)) // 16) * 16, -(-(k // 64) // parts)
+                assert tile_rows <= tm and (m_tiles - 1) * tile_rows < rows and m_tiles * groups * parts <= 256 and 1 <= groups <= n // 8
+                assert -(-(n // 8) // groups) * 8 <= tw and k % bk == 0 and (parts == 1 or of_part * 64 % bk == 0) and (parts - 1) * of_part < k // 64
+    assert ops.spread_few_columns(64, 2048, 1536)[1] == (10, 2, 128) and ops.spread_few_columns(65, 7168, 5120)[1] == (12, 1, 256)
+    assert ops.spread_few_columns(64, 16, 64, 2) is None and ops.spread_few_columns(512, 131072, 64) is None
+    def parts(rows, n, k):
+        plan = L.linear_plan(rows, n, k, False, False, True, rows <= 64, True)
+        return L.spread_parts(plan, rows, n, k)
+    assert parts(64, 1536, 8960) == ("tiles", 320113, 8) and L._dealing(320113) == (13, 1, 32) and L._dealing(1) is None and parts(128, 3584, 18944)[2] == 8 and parts(64, 3584, 18944)[2] == 8
+    assert parts(96, 1536, 1536)[2] == 2 and parts(64, 2048, 2048) and parts(17, 5120, 13824)
+    assert not any(parts(rows, n, k) for rows, n, k in ((16, 1536, 8960), (48, 1536, 1536), (64, 2048, 11008), (91, 3584, 3584), (250, 4096, 14336),
+                                                         (300, 2304, 1536), (385, 1536, 8960), (128, 1536, 960), (64, 1528, 8960)))
+    key = ("linear", 128, 1536, 8960, False, False, True, False, True)
+    assert L.linear_candidates(key)[0] == L.linear_plan(*key[1:]) and ("tiles", L._dealing_number(14, 1, 32), 8) in L.linear_candidates(key)
+
+
 def test_steps_of_a_trip():
     """Products of few rows: a short K in one way to memory, then two, then three steps at a time."""
     from ginfer_amd.kernels import build
