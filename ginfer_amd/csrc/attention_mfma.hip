@@ -694,7 +694,11 @@ __global__ __launch_bounds__(64 * PREFILL_WAVES) void attn_prefill_kernel(
   f32x4 o[NB][DB];
   float m[NB], l[NB];
   init_state<NB>(o, m, l);
-  if (head_ok) {
+  // The wavefronts of a head that have a tile of keys; the others ask for no queries and bring nothing to the meeting, whose sums they
+  // would leave as they are.  A short tile is bound by that chain of queries, LDS and exponentials, not by its keys: 10 prompts of 13
+  // to 19 tokens, where one wavefront of eight has keys, 10.0 -> 8.8 us
+  const int meeting = min(splits, max(1, (kp.end - kp.begin + 31) >> 5));
+  if (head_ok && split < meeting) {
     bf16x8 qr[NB][KB];
     int cpos[NB], clo[NB];
 #pragma unroll
@@ -716,7 +720,7 @@ __global__ __launch_bounds__(64 * PREFILL_WAVES) void attn_prefill_kernel(
     finish_sums<NB>(l);
   }
   if (splits > 1) {
-    if (head_ok && split > 0) {
+    if (head_ok && split > 0 && split < meeting) {
       float* st = lds + (int64_t)((hl * (splits - 1) + split - 1) * NB) * STATE;
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) {
@@ -736,13 +740,13 @@ __global__ __launch_bounds__(64 * PREFILL_WAVES) void attn_prefill_kernel(
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
       float mx = m[nb];
-      for (int sp = 1; sp < splits; ++sp)
+      for (int sp = 1; sp < meeting; ++sp)
         mx = fmaxf(mx, lds[(int64_t)((hl * (splits - 1) + sp - 1) * NB + nb) * STATE + HD * 17 + c]);
       const float f0 = m[nb] == -INFINITY ? 0.f : fast_exp2(m[nb] - mx);
       l[nb] *= f0;
 #pragma unroll
       for (int db = 0; db < DB; ++db) o[nb][db] *= f0;
-      for (int sp = 1; sp < splits; ++sp) {      // in split order
+      for (int sp = 1; sp < meeting; ++sp) {     // in split order
         const float* sn = lds + (int64_t)((hl * (splits - 1) + sp - 1) * NB + nb) * STATE;
         const float ms = sn[HD * 17 + c];
         const float f = ms == -INFINITY ? 0.f : fast_exp2(ms - mx);
@@ -945,9 +949,9 @@ __global__ __launch_bounds__(64 * PREFILL_WAVES) void attn_prefill_shared_kernel
   }
   // the wavefronts of a head meet as in the kernel above; first everybody is through with the ring
   __syncthreads();
-  const int split = stream;
+  const int split = stream, meeting = min(splits, max(1, (tile_end - first + 31) >> 5));
   if (splits > 1) {
-    if (head_ok && split > 0) {
+    if (head_ok && split > 0 && split < meeting) {
       float* st = lds + (int64_t)((hl * (splits - 1) + split - 1) * NB) * STATE;
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) {
@@ -967,13 +971,13 @@ __global__ __launch_bounds__(64 * PREFILL_WAVES) void attn_prefill_shared_kernel
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
       float mx = m[nb];
-      for (int sp = 1; sp < splits; ++sp)
+      for (int sp = 1; sp < meeting; ++sp)
         mx = fmaxf(mx, lds[(int64_t)((hl * (splits - 1) + sp - 1) * NB + nb) * STATE + HD * 17 + c]);
       const float f0 = m[nb] == -INFINITY ? 0.f : fast_exp2(m[nb] - mx);
       l[nb] *= f0;
 #pragma unroll
       for (int db = 0; db < DB; ++db) o[nb][db] *= f0;
-      for (int sp = 1; sp < splits; ++sp) {      // in split order
+      for (int sp = 1; sp < meeting; ++sp) {     // in split order
         const float* sn = lds + (int64_t)((hl * (splits - 1) + sp - 1) * NB + nb) * STATE;
         const float ms = sn[HD * 17 + c];
         const float f = ms == -INFINITY ? 0.f : fast_exp2(ms - mx);

@@ -692,6 +692,21 @@ def test_paged_attention_mfma_heads_side_by_side(nh, nkv, hd, seqs, wide, monkey
         close(out, ref, 2e-2)
 
 
+@pytest.mark.parametrize("fill", [1, 1 << 30])                               # heads side by side, or one with its keys split eight ways
+@pytest.mark.parametrize("window", [None, 40])
+@pytest.mark.parametrize("keys", [2, 31, 32, 33, 64, 65, 96, 127, 129, 225, 256, 257])
+def test_paged_attention_mfma_where_wavefronts_have_no_keys(keys, window, fill, monkeypatch):
+    """One tile of 32 keys to more tiles than a workgroup has wavefronts: those without one leave what the others meet as it is."""
+    from ginfer_amd.kernels import ops
+    monkeypatch.setattr(ops.TUNING, "prefill_fill_workgroups", fill)
+    nh, nkv, hd = 6, 2, 64
+    seqs = [(min(keys, 19), keys), (2, keys), (min(keys, 33), keys)]
+    a, ref, _ = _paged_case(seqs, nh, nkv, hd, 16, torch.bfloat16, seed=keys, window=window)
+    out = ops.paged_attention_mfma(a["q"], a["k_pages"], a["v_pages"], a["block_table"], _Step(seqs, a), nh, nkv, hd,
+                                   1.0 / math.sqrt(hd), window=window)
+    close(out, ref, 2e-2)
+
+
 @pytest.mark.parametrize("wide", [False, True])
 @pytest.mark.parametrize("window", [1, 5, 16, 40, 64, 100])
 def test_paged_attention_mfma_heads_side_by_side_window(window, wide, monkeypatch):
