@@ -10,11 +10,16 @@
 // LDS; operands come out of LDS half a slab ahead of their products.  In the middle of a slab its second half's operands are in
 // registers: there all wait for the next slab and meet, once a slab, and from there on the slab's own buffer is filled with the
 // slab NBUF on.  Loads and LDS reads are dealt between the products, so that no wavefront waits to issue them.  In the gated
-// product a wavefront's first half of rows is the gate's and its second the up matrix's of the same columns, so that both
+// product the first half of a block's rows is the gate's and its second the up matrix's of the same columns, so that both
 // sums of a result lie in one lane.  Workgroups that share rows of W are neighbours on one XCD, whose L2 then reads W once.
 //
 // What bounds it: many rows, the chip's power (products of random numbers run at 1,700 to 1,800 TFLOP/s, 2,400 of zeros) and the
-// way of a slab from memory; few rows, the weights' way from memory.
+// way of a slab from memory; few rows, the weights' way from memory.  192 x 256 tiles of 2,048 rows, 17,920 rows of W, K 1,536, us: the products
+// alone 73, the loads alone 64 (whatever order the tiles come in), both 85, with the LDS reads 95, with the activation 120; the last is a
+// third of that where eight wavefronts share it rather than four: 105, though they read a quarter more from LDS.  Tiles beyond 128 x 128
+// have eight, us of four and eight: 256 x 256 (37,888 rows, K 3,584, 2,048 rows) 467 -> 455, 128 x 256 (17,920, K 1,536, 1,024 rows) 69.6 -> 65.6, 256 x
+// 128 68.9 -> 63.7, 192 x 128 59.1 -> 57.5; 128 x 128 has four, 65.9 against 68.1.  Loads dealt faster than evenly are slower (all at once
+// 105 -> 109), W or A read past the caches too (114, 126).
 #include "lds_load.h"
 #include <type_traits>
 #include "ginfer_amd.h"
@@ -73,13 +78,8 @@ __global__ __launch_bounds__(64 * WN * WM, 1) void gemm_tiles_kernel(
   for (int j = 0; j < LW; ++j) {
     const int r = (wave * LW + j) * RPL + lrow;
     int col;
-    if (GATED) {
-      constexpr int H = 16 * NI;                  // of a wavefront's 32 NI rows, half are gate's
-      const int w = r / (2 * H), q = r % (2 * H) / H;
-      col = min(c0 + w * H + r % H, cols - 1) + q * cols;
-    } else {
-      col = min(c0 + r, cols - 1);
-    }
+    if (GATED) col = min(c0 + r / 32 * 16 + r % 16, cols - 1) + r % 32 / 16 * cols;      // of a block's 32 rows, 16 are the gate's
+    else col = min(c0 + r, cols - 1);
     src_w[j] = ((uint32_t)col * (uint32_t)K + 8 * piece) * 2u;
   }
 #pragma unroll
@@ -179,19 +179,19 @@ __global__ __launch_bounds__(64 * WN * WM, 1) void gemm_tiles_kernel(
     }
   } else {
     // through LDS, so that rows leave in 16-byte pieces side by side
-    constexpr int PITCH = COLS + 8, OI = NI / 2;
+    constexpr int PITCH = COLS + 8;
     __syncthreads();
     bf16_t* tile = reinterpret_cast<bf16_t*>(lds);
 #pragma unroll
-    for (int i = 0; i < OI; ++i)
+    for (int i = 0; i < NI; ++i)
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
+      for (int q = 0; q < 2; ++q)
 #pragma unroll
         for (int j = 0; j < MJ; ++j) {
           float y[4];
 #pragma unroll
-          for (int x = 0; x < 4; ++x) y[x] = gt_act(acc[i][j][4 * q + x], acc[i + OI][j][4 * q + x], act);
-          *reinterpret_cast<uint2*>(tile + ((wm * MJ + j) * 32 + c) * PITCH + (wn * OI + i) * 32 + 8 * q + 4 * g) = gt_round4(y);
+          for (int x = 0; x < 4; ++x) y[x] = gt_act(acc[i][j][4 * q + x], acc[i][j][8 + 4 * q + x], act);
+          *reinterpret_cast<uint2*>(tile + ((wm * MJ + j) * 32 + c) * PITCH + (wn * NI + i) * 16 + 8 * q + 4 * g) = gt_round4(y);
         }
     __syncthreads();
     bf16_t* out = reinterpret_cast<bf16_t*>(C);
@@ -594,13 +594,13 @@ extern "C" int ga_gemm_tiles_gated(void* C, int64_t ldc, const void* A, int64_t 
   const GateAct act = {kind, limit, alpha, shift};
   switch (tiling) {
     case 0: return gt_launch<2, 1, 2, 2, 3, true>(C, ldc, A, lda, W, M, cols, K, 1, act, stream);     // 128 x 64
-    case 1: return gt_launch<4, 2, 1, 4, 3, true>(C, ldc, A, lda, W, M, cols, K, 1, act, stream);     // 128 x 256
-    case 2: return gt_launch<4, 2, 2, 2, 3, true>(C, ldc, A, lda, W, M, cols, K, 1, act, stream);     // 256 x 128
-    case 3: return gt_launch<4, 4, 2, 2, 2, true>(C, ldc, A, lda, W, M, cols, K, 1, act, stream);     // 256 x 256
+    case 1: return gt_launch<2, 2, 2, 4, 3, true>(C, ldc, A, lda, W, M, cols, K, 1, act, stream);     // 128 x 256
+    case 2: return gt_launch<2, 2, 4, 2, 3, true>(C, ldc, A, lda, W, M, cols, K, 1, act, stream);     // 256 x 128
+    case 3: return gt_launch<2, 4, 4, 2, 2, true>(C, ldc, A, lda, W, M, cols, K, 1, act, stream);     // 256 x 256
     case 4: return gt_launch<2, 2, 2, 2, 3, true>(C, ldc, A, lda, W, M, cols, K, 1, act, stream);     // 128 x 128
     case 6: return gt_launch<6, 1, 1, 2, 4, true>(C, ldc, A, lda, W, M, cols, K, 1, act, stream);     // 192 x 64
-    case 7: return gt_launch<6, 1, 1, 4, 3, true>(C, ldc, A, lda, W, M, cols, K, 1, act, stream);     // 192 x 128
-    case 8: return gt_launch<6, 2, 1, 4, 2, true>(C, ldc, A, lda, W, M, cols, K, 1, act, stream);     // 192 x 256
+    case 7: return gt_launch<3, 1, 2, 4, 3, true>(C, ldc, A, lda, W, M, cols, K, 1, act, stream);     // 192 x 128
+    case 8: return gt_launch<3, 2, 2, 4, 2, true>(C, ldc, A, lda, W, M, cols, K, 1, act, stream);     // 192 x 256
   }
   return -6;
 }
