@@ -579,6 +579,13 @@ def spread_few_columns(rows, out_features, in_features, parts=1):
     return best
 
 
+def spread_many_columns(rows, out_features):
+    """(number in SPREAD_SHAPES, row tiles, groups of columns) of a product of up to 64 rows by more columns than one round of the chip holds, dealt evenly to
+    as many rounds as tiles of 160 rows of W make (151,936 x 1,536 at 33 rows 92.8 us, over tiles of 128 rows 94.4, of 32 101)."""
+    units = out_features // 8
+    return (2, 1, min(units, -(-units // (256 * 20)) * 256))
+
+
 def gemm_tiles_parts(a, w, parts, plan=None):
     """a [M, K] . w [N, K]^T as float32 partial sums [parts, M, N] over parts of K, for the consumer to add in order.  plan: None for tiles
     of 64 or 128 columns, or (shape, row tiles, groups) of the kernel that deals them evenly (spread_few_columns)."""

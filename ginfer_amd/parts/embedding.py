@@ -128,7 +128,7 @@ class LMHead(Part):
         self.weight = embedding_weight
 
     def kernel_modules(self):
-        return (["gemm"] + (["gemm_skinny"] if self.dtype == torch.bfloat16 else [])
+        return (["gemm"] + (["gemm_skinny", "gemm_tiles"] if self.dtype == torch.bfloat16 else [])
                 + (["activation"] if self.soft_cap is not None else []))
 
     def forward(self, x):

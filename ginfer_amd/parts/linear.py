@@ -26,7 +26,8 @@ def linear(x, weight, bias=None, out_dtype=None, parts_ok=False):
         return ops.gemm_nt(x, weight, bias)
     float32_out = out_dtype == torch.float32
     skinny_ok = ops.gemm_skinny_supported(x, weight)
-    tiles_ok = (parts_ok and bias is None and not float32_out and TUNING.library_from_rows < x.shape[0] <= TUNING.tiles_parts_most_rows
+    wide = float32_out and bias is None and head_is_wide(x.shape[0], weight.shape[0], x.shape[1])
+    tiles_ok = ((wide or (parts_ok and bias is None and not float32_out and TUNING.library_from_rows < x.shape[0] <= TUNING.tiles_parts_most_rows))
                 and ops.gemm_tiles_supported(x, weight))
     spread_ok = parts_ok and bias is None and not float32_out and ops.gemm_tiles_supported(x, weight)
     plan = None
@@ -36,9 +37,12 @@ def linear(x, weight, bias=None, out_dtype=None, parts_ok=False):
         plan = autotune.choose(key, (weight, bias))
     if plan is None:
         plan = linear_plan(x.shape[0], weight.shape[0], x.shape[1], bias is not None, float32_out, parts_ok, skinny_ok, tiles_ok)
-        if spread_ok:
+        if wide and tiles_ok:
+            plan = wide_plan(x.shape[0], weight.shape[0])
+        elif spread_ok:
             plan = spread_parts(plan, x.shape[0], weight.shape[0], x.shape[1]) or plan
-    return run_linear_plan(plan, x, weight, bias, out_dtype)
+    y = run_linear_plan(plan, x, weight, bias, out_dtype)
+    return y[0] if float32_out and plan[0] == "tiles" else y
 
 
 def _dealing_number(shape, m_tiles, groups):
@@ -88,6 +92,19 @@ def spread_parts(plan, rows, out_features, in_features):
         if best[0] > T.spread_parts_share_of_tiles * other or (rows <= 128 and best[1][2] == plan[2]):
             return None
     return best[1]
+
+
+def head_is_wide(rows, out_features, in_features):
+    """Whether a 32-bit product of few rows by so many columns is faster over tiles dealt evenly to several rounds of the chip (by sizes alone;
+    the measurements stand beside the thresholds)."""
+    T = TUNING
+    if not T.library_from_rows < rows <= SKINNY_MAX_ROWS or out_features < T.spread_wide_min_out_features or out_features % 16 or in_features % 64:
+        return False
+    return rows <= T.spread_wide_few_rows or (in_features < T.spread_wide_long_k and out_features * in_features <= T.spread_wide_most_weights)
+
+
+def wide_plan(rows, out_features):
+    return ("tiles", _dealing_number(*ops.spread_many_columns(rows, out_features)), 1)
 
 
 def tiles_parts(rows, out_features, in_features):
@@ -210,6 +227,8 @@ def linear_candidates(key):
             plans.append(plan)
 
     may_split = parts_ok and not float32_out
+    if tiles_ok and float32_out and not has_bias and head_is_wide(rows, out_features, in_features):
+        add(wide_plan(rows, out_features))
     if skinny_ok:
         tiles = (1, 4) if rows > 16 else (1,)
         for nt in tiles:

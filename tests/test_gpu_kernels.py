@@ -1273,6 +1273,17 @@ def test_product_of_few_columns_dealt_evenly(shape, fill, m_tiles, K, parts):
             ops.gemm_tiles_parts(rnd((M, 192), torch.bfloat16, 1), rnd((N, 192), torch.bfloat16, 2), 1, (shape, m_tiles, groups))
 
 
+@pytest.mark.parametrize("M", [16, 17, 48, 49, 64, 65])
+@pytest.mark.parametrize("N,K", [(24576, 64), (41120, 128), (25008, 5120)])
+def test_head_of_many_columns(M, N, K):
+    """Logits in 32 bits on both sides of the rule's lines, a number of columns that leaves groups of two sizes."""
+    from ginfer_amd.parts.linear import linear
+    x, w = rnd((M, K), torch.bfloat16, 91), rnd((N, K), torch.bfloat16, 92, 0.05)
+    y = linear(x, w, None, out_dtype=torch.float32)
+    assert y.shape == (M, N) and y.dtype == torch.float32 and y.is_contiguous()
+    close(y, x.double() @ w.double().t(), 1e-5)
+
+
 @pytest.mark.parametrize("M,hd,nh,nkv,K", [(17, 64, 3, 1, 128), (40, 48, 4, 2, 320), (64, 128, 12, 2, 256), (100, 80, 2, 2, 192), (161, 128, 4, 1, 384),
                                            (290, 8, 6, 3, 64), (512, 32, 8, 2, 128)])
 @pytest.mark.parametrize("bias", [False, True])

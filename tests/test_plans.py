@@ -220,6 +220,19 @@ def test_few_columns_dealt_evenly():
     assert L.linear_candidates(key)[0] == L.linear_plan(*key[1:]) and ("tiles", L._dealing_number(14, 1, 32), 8) in L.linear_candidates(key)
 
 
+def test_heads_of_many_columns():
+    """Where the head of 17 to 64 rows leaves the library, and that the tiles hold what its plan deals out."""
+    from ginfer_amd.kernels import ops
+    assert all(L.head_is_wide(rows, 151936, k) for rows in (17, 33, 64) for k in (896, 1536, 3584)) and L.head_is_wide(48, 65024, 5120)
+    assert not any(L.head_is_wide(*x) for x in ((16, 151936, 1536), (65, 151936, 1536), (64, 65024, 5120), (64, 256000, 3584), (33, 24560, 1536),
+                                                (33, 151936, 1500), (33, 50257, 768)))
+    for n in (24576, 32768, 50304, 151936, 256000):
+        shape, m_tiles, groups = ops.spread_many_columns(64, n)
+        assert shape == 2 and m_tiles == 1 and groups % 256 == 0 and -(-(n // 8) // groups) * 8 <= ops.SPREAD_SHAPES[shape][1]
+    key = ("linear", 64, 151936, 1536, False, True, False, True, True)
+    assert L.linear_candidates(key)[:2] == [("library", 1), L.wide_plan(64, 151936)]
+
+
 def test_steps_of_a_trip():
     """Products of few rows: a short K in one way to memory, then two, then three steps at a time."""
     from ginfer_amd.kernels import build
