@@ -580,11 +580,10 @@ static int spread_check(int M, int m_tiles, int groups) {
 // activation by the library's best way -> here, as replays of a graph over several layers' weights: 17,920 rows of W, K 1,536: 64 rows
 // 30.6 -> 26.9, 128 rows 35.1 -> 30.2 (tiles of 128 x 256, half of them rows that do not exist, 33.5), 256 rows 43.6 -> 37.2, 384
 // rows 45.9 -> 39.9; 37,888 rows, K 3,584: 128 rows 84.0 -> 79.3, 384 rows 133.9 -> 121.4, 1,000 rows 324 -> 272, 1,280 rows 386 ->
-// 291, 2,048 rows 552 -> 464; 19,456 rows, K 2,560: 128 rows 46.0 -> 44.0 (128 x 256 tiles 49.1), 384 rows 64.0 -> 57.8.
+// 291, 2,048 rows 552 -> 464; 19,456 rows, K 2,560: 128 rows 46.0 -> 44.0 (128 x 256 tiles 49.1), 384 rows 64.0 -> 57.8 (all with four
+// wavefronts to a tile; what eight give stands above).
 // Tiles of 192 rows of W stand beside the others (6 to 8) where those leave the chip's rounds emptier (gated_wide_tiling in
-// kernels/ops.py has the rule and the figures): many rows run at 1.5 to 1.7 GHz, which is the power they may draw, with the
-// matrix cores busy 0.61 (192 x 256, K 1,536) to 0.68 of the time (256 x 256, K 3,584) and wavefronts waiting 0.21 and 0.14 of it, so
-// that only less padding, not a busier loop, gains much.
+// kernels/ops.py has the rule and the figures).
 extern "C" int ga_gemm_tiles_gated(void* C, int64_t ldc, const void* A, int64_t lda, const void* W, int M, int cols, int K, int kind,
                                    float limit, float alpha, float shift, int tiling, hipStream_t stream) {
   if (M <= 0) return 0;

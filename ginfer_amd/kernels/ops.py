@@ -521,9 +521,28 @@ def spread_plan(rows, out_features, in_features):
     dealt evenly to the chip (csrc/gemm_tiles.hip), or None where the tiles of gated_tiling and gated_wide_tiling are the faster or
     no shape holds it.  One workgroup to each of the 256 compute units, in the split that has them read the fewest rows, and up to
     64 rows two, one after the other, where one cannot hold its share of W.  Beyond 128 rows the other tiles are better where they
-    fit one round about as well: a compute unit's rows there, the mean of its rows of A, against here; us, rows of the
-    two: 17,920 x 1,536 at 256 rows 320 and 272, 26.6 -> 23.7; 9,088 x 2,880 at 256 256 and 200, 32.0 -> 27.1; the other way 21,120 x
-    1,792 at 253 318 and 344, 30.9 -> 31.8; 10,496 x 3,584 at 264 216 and 224, 33.5 -> 36.3; 15,360 x 6,144 at 136 196 and 200, 58.4 -> 61.0."""
+    fit one round and read fewer rows with their padding, or are of 128 x 128 and fill most of it, against three row tiles here, or
+    half of it with a small W; us of those and of this: 22,016 x 2,048 at 256 rows 34.8 and 37.3; 10,496 x 3,584 at 300 34.4 and 38.2, 9,088 x 2,880 27.1 and 30.8; 5,888 x 1,536 at 300 12.7
+    and 16.1, 9,728 x 896 at 225 10.0 and 12.4, 7,936 x 768 at 384 9.6 and 11.9; the other way 27,648 x 5,120 at 150 78.7 and 66.4, 17,920 x 1,536
+    at 256 26.6 and 23.8, 12,288 x 2,560 at 225 32.2 and 28.6, 3,712 x 2,048 at 150 14.8 and 10.9.  Over 325 products of 42 sizes what is chosen
+    is 0.4 % behind the better of the two (with the line at 0.92 of the rows without padding, drawn before those tiles had eight wavefronts, 2.2 %)."""
+    best = spread_dealing(rows, out_features, in_features)
+    if best is None or rows <= 128:
+        return best and best[1]
+    number = gated_wide_tiling(rows, out_features, in_features)
+    of_w, of_a = GATED_WIDE_TILINGS[number] if number else GATED_TILINGS[gated_tiling(rows, out_features)]
+    tiles = -(-rows // of_a) * -(-out_features // of_w)
+    if tiles <= 256:
+        if of_w == of_a == 128 and ((tiles >= 110 and out_features * in_features <= 10500000) or (tiles >= 200 and best[1][1] > 2)):
+            return None
+        if best[0] > of_w + of_a:
+            return None
+    return best[1]
+
+
+@functools.lru_cache(maxsize=4096)
+def spread_dealing(rows, out_features, in_features):
+    """(rows that a compute unit reads, the plan) of the even dealing by itself, or None where no shape holds it."""
     if not 17 <= rows <= 512:
         return None
     units, best = out_features // 8, None
@@ -538,14 +557,7 @@ def spread_plan(rows, out_features, in_features):
         fits = [(tm * tw, n) for n, (tm, tw, bk) in enumerate(SPREAD_SHAPES) if tm >= tile_rows and tw >= of_w and in_features % bk == 0]
         if fits and (best is None or tile_rows + of_w <= best[0]):
             best = (tile_rows + of_w, (min(fits)[1], m_tiles, groups))
-    if best is None or rows <= 128:
-        return best and best[1]
-    number = gated_wide_tiling(rows, out_features, in_features)
-    of_w, of_a = GATED_WIDE_TILINGS[number] if number else GATED_TILINGS[gated_tiling(rows, out_features)]
-    tiles = -(-rows // of_a)
-    if -(-out_features // of_w) * tiles <= 256 and best[0] > 0.92 * (of_w + rows / tiles):
-        return None
-    return best[1]
+    return best
 
 
 SPREAD_NARROW_SHAPES = ((64, 16, 128), (64, 32, 128), (128, 32, 128), (64, 48, 128), (128, 48, 128))     # beside the others, for few columns

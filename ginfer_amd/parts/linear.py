@@ -404,10 +404,10 @@ def gated_linear(x, weight_gate_up, bounds=None):
 
 
 def spread_is_faster(plan, rows, out_features, in_features):
-    """Whether the product over tiles that are dealt evenly to the chip stands in for `plan`, the other rules' (by sizes alone; the
-    measurements stand beside the thresholds and ops.spread_plan)."""
+    """Whether the product over tiles that are dealt evenly to the chip, or over the others where ops.spread_plan has them as the faster still,
+    stands in for `plan`, the other rules' (by sizes alone; the measurements stand beside the thresholds and there)."""
     T = TUNING
-    if plan == ("tiles",) or ops.spread_plan(rows, out_features, in_features) is None:
+    if plan == ("tiles",) or ops.spread_dealing(rows, out_features, in_features) is None:
         return False
     if plan == ("skinny",):
         return (out_features >= T.spread_few_rows_min_out_features

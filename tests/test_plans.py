@@ -183,11 +183,13 @@ def test_gated_products_dealt_evenly():
             assert tile_rows <= tm and (m_tiles - 1) * tile_rows < rows and k % bk == 0 and 1 <= groups <= n // 8
             assert -(-(n // 8) // groups) * 8 <= tw and m_tiles * groups <= (512 if rows <= 64 else 256)
     plan = ops.spread_plan
+    faster = lambda plan, rows, n, k: L.spread_is_faster((plan,), rows, n, k)
     assert plan(64, 17920, 1536) == (0, 1, 256) and plan(128, 17920, 1536) == (1, 1, 256) and plan(161, 17920, 1536) == plan(256, 17920, 1536) == (3, 2, 128)
     assert plan(384, 17920, 1536) == (4, 2, 128) and plan(64, 37888, 3584) == (2, 1, 256) and plan(64, 59136, 8192) == (6, 1, 512)
     assert plan(16, 17920, 1536) is None and plan(513, 17920, 1536) is None and plan(65, 59136, 8192) is None
-    assert plan(253, 21120, 1792) is None and plan(264, 10496, 3584) is None and plan(256, 9088, 2880) == (7, 2, 128)
-    faster = lambda plan, rows, n, k: L.spread_is_faster((plan,), rows, n, k)
+    assert plan(256, 22016, 2048) is None and plan(300, 10496, 3584) is None and plan(225, 9728, 896) is None and plan(256, 9088, 2880) == (7, 2, 128)
+    assert faster("library", 225, 9728, 896) and faster("library", 300, 10496, 3584)      # by the other tiles
+    assert plan(150, 27648, 5120) == (8, 1, 256) and plan(225, 12288, 2560) and plan(150, 3712, 2048)
     assert faster("skinny", 17, 17920, 1536) and not faster("skinny", 17, 9728, 896) and faster("skinny", 33, 3072, 2048) and not faster("skinny", 34, 2688, 512)
     assert faster("library", 400, 17920, 1536) and faster("transposed", 512, 17920, 1536) and not faster("library", 92, 2048, 6144)
     assert faster("library", 384, 11136, 8192) and not faster("library", 508, 11136, 8192) and not faster("tiles", 64, 17920, 1536)
