@@ -748,7 +748,7 @@ def qkv_rope_skinny(x, w, bias, positions, cos, sin, slot_mapping, k_pages, v_pa
 def qkv_spread_plan(x, w, head_dim, rotary_dim):
     """The plan by which the q|k|v projection of 17 to 512 rows with its rotation and cache write is one kernel (csrc/gemm_tiles.hip), or None
     where its operands are not of the kind."""
-    if (isinstance(x, ScaledRows) or not gemm_tiles_supported(x, w) or not 17 <= x.shape[0] <= 512 or head_dim % 8 or rotary_dim != head_dim):
+    if (not 17 <= x.shape[0] <= 512 or isinstance(x, ScaledRows) or head_dim % 8 or rotary_dim != head_dim or not gemm_tiles_supported(x, w)):
         return None
     best = spread_few_columns(x.shape[0], w.shape[0], w.shape[1])
     return best and best[1]

@@ -29,7 +29,8 @@ def linear(x, weight, bias=None, out_dtype=None, parts_ok=False):
     wide = float32_out and bias is None and head_is_wide(x.shape[0], weight.shape[0], x.shape[1])
     tiles_ok = ((wide or (parts_ok and bias is None and not float32_out and TUNING.library_from_rows < x.shape[0] <= TUNING.tiles_parts_most_rows))
                 and ops.gemm_tiles_supported(x, weight))
-    spread_ok = parts_ok and bias is None and not float32_out and ops.gemm_tiles_supported(x, weight)
+    spread_ok = (parts_ok and bias is None and not float32_out and TUNING.library_from_rows < x.shape[0] <= TUNING.spread_parts_most_rows
+                 and (tiles_ok or ops.gemm_tiles_supported(x, weight)))      # the rows first: steps launched kernel by kernel wait for the host
     plan = None
     if autotune.active():
         key = ("linear", autotune.rows_class(x.shape[0]), weight.shape[0], x.shape[1], bias is not None, float32_out,
