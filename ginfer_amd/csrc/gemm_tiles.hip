@@ -31,22 +31,27 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 
 // act.kind 0: SiLU(v) * u; 1: g * sigmoid(alpha g) * (u + shift), g = min(v, limit), u = clamp(u, -limit, limit); 2: the same
-// with the sigmoid's limit, a step.  exp2 and the reciprocal are the hardware's: against 64 bits SiLU is off by at most 3 units of
+// with the sigmoid's limit, a step.  Without EXPF, exp2 and the reciprocal are the hardware's: against 64 bits SiLU is off by at most 3 units of
 // the 32-bit result's last place for v > -0.5, 6 down to -4, 18 down to -20 and 65 (4e-6 of it) down to -87, below which it is 0;
-// with expf and a division, as the kernel for up to 16 rows has it, by at most 3.4 everywhere.  The one rounding that follows is
+// with expf and a division (EXPF), as the kernel that streams the weights has it, by at most 3.4 everywhere.  The one rounding that follows is
 // 2^-9 of the result.  expf and the division cost 1 us of 27 at 64 rows and 41 of 464 at 2,048 (one tile's 128 results a thread
 // are straight code that no one else has fetched yet), a correction of exp2's argument and one step on the reciprocal 21.
 struct GateAct {
   int kind;
   float limit, alpha, shift;
 };
-__device__ __forceinline__ float gt_sigmoid(float z) { return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(z * -1.4426950408889634f)); }
+template <bool EXPF>
+__device__ __forceinline__ float gt_sigmoid(float z) {
+  if (EXPF) return 1.0f / (1.0f + expf(-z));
+  return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(z * -1.4426950408889634f));
+}
+template <bool EXPF = false>
 __device__ __forceinline__ float gt_act(float v, float u, const GateAct act) {
-  if (act.kind == 0) return (v * gt_sigmoid(v)) * u;
+  if (act.kind == 0) return (v * gt_sigmoid<EXPF>(v)) * u;
   v = fminf(v, act.limit);
   u = fminf(fmaxf(u, -act.limit), act.limit);
   if (act.kind == 2) return (v > 0.f ? v : 0.f) * (u + act.shift);
-  return (v * gt_sigmoid(act.alpha * v)) * (u + act.shift);
+  return (v * gt_sigmoid<EXPF>(act.alpha * v)) * (u + act.shift);
 }
 __device__ __forceinline__ uint2 gt_round4(const float (&y)[4]) {
   bf16x4 r;
@@ -437,14 +442,21 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 1) void gemm_spread_gated_kernel
   const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave % WM, wn = wave / WM % WN, wk = wave / (WM * WN);
   bf16_t* tile = reinterpret_cast<bf16_t*>(lds);       // through LDS, so that a row's columns leave side by side
+  auto results = [&](auto with_expf) {
+    constexpr bool EXPF = decltype(with_expf)::value;
 #pragma unroll
-  for (int t = 0; t < NI * MJ; ++t)
-    if (WK == 1 || t % 2 == wk) {
-      const int i = t / MJ, j = t % MJ;
-      const SpreadPairs v(acc[i][j]);
-      *reinterpret_cast<uint32_t*>(tile + ((wm * MJ + j) * 16 + c) * S::PITCH + (wn * NI + i) * 8 + 2 * g) =
-          gt_round2(gt_act(v.first[0], v.second[0], act), gt_act(v.first[1], v.second[1], act));
-    }
+    for (int t = 0; t < NI * MJ; ++t)
+      if (WK == 1 || t % 2 == wk) {
+        const int i = t / MJ, j = t % MJ;
+        const SpreadPairs v(acc[i][j]);
+        *reinterpret_cast<uint32_t*>(tile + ((wm * MJ + j) * 16 + c) * S::PITCH + (wn * NI + i) * 8 + 2 * g) =
+            gt_round2(gt_act<EXPF>(v.first[0], v.second[0], act), gt_act<EXPF>(v.first[1], v.second[1], act));
+      }
+  };
+  // Products that the kernel streaming the weights would take otherwise (up to 32 rows, or 64 of fewer than 4,096 rows of W) keep its
+  // activation: 0.3 to 0.4 us of 6 to 16 there; with more rows, whose other tiles have the hardware's too, it would be 0.4 to 2.7.
+  if (S::TM == 64 && (M <= 32 || cols < 2048)) results(std::true_type());
+  else results(std::false_type());
   __syncthreads();
   for (int idx = threadIdx.x; idx < S::TM * 2 * S::NB; idx += 64 * S::WAVES) {
     const int m = idx / (2 * S::NB), q = idx % (2 * S::NB);

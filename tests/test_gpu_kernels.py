@@ -1249,6 +1249,35 @@ def test_gated_product_dealt_evenly(shape, fill, m_tiles, K):
             ops.gemm_tiles_gated(a, w, tiling=plan)
 
 
+@pytest.mark.parametrize("rows,cols", [(17, 5632), (32, 5632), (33, 2040), (64, 2040), (64, 1024)])
+@pytest.mark.parametrize("alpha", [None, 2.0])                              # alpha times a gate is exact
+def test_gated_product_dealt_evenly_rounds_the_streaming_kernels_activation(rows, cols, alpha):
+    """Products that the weight-streaming kernel takes where they are not dealt evenly: gates and ups are exact (a row of A has one element),
+    gates over all that the sigmoid bends, so that the result is one rounding (2^-9) of what expf and a division make of them: off by at
+    most 4 units of the 32-bit result before it.  Gates whose result is no normal number are left out."""
+    from ginfer_amd.kernels import ops
+    K, n = 128, 2 * cols
+    a = torch.zeros((rows, K), dtype=torch.bfloat16)
+    a[torch.arange(rows), torch.arange(rows)] = 1.0
+    gen = torch.Generator().manual_seed(rows + cols)
+    w = torch.empty((n, K))
+    w[:cols] = torch.rand((cols, K), generator=gen) * 95.0 - 85.0            # gates from -85 to 10
+    w[cols:] = torch.rand((cols, K), generator=gen) + 1.0
+    w = w.bfloat16()
+    bounds = None if alpha is None else (10.0, alpha, 0.0)
+    if alpha is not None:
+        w[:cols] = (w[:cols].float() / alpha).bfloat16()
+    plan = ops.spread_dealing(rows, n, K)[1]
+    got = ops.gemm_tiles_gated(a.to(dev()), w.to(dev()), bounds=bounds, tiling=plan).cpu()
+    g, u = w.t()[:rows, :cols].double(), w.t()[:rows, cols:].double()
+    ref = g / (1.0 + torch.exp(-(1.0 if alpha is None else alpha) * g)) * u
+    ok = ref.abs() > 2.0 ** -120
+    spacing = 2.0 ** (torch.floor(torch.log2(torch.where(ok, ref.abs(), torch.ones_like(ref)))) - 7)     # of bfloat16 around the result
+    over = ((got.double() - ref).abs() - spacing / 2) / (spacing / 65536)      # in units of the 32-bit result's last place
+    assert ok.float().mean() > 0.9 and float(over[ok].max()) <= 4.0, float(over[ok].max())
+    close(got, ops.gemm_skinny(a.to(dev()), w.to(dev()), gated=True, gate_bounds=bounds), 0.0)
+
+
 @pytest.mark.parametrize("shape", range(15))
 @pytest.mark.parametrize("fill,m_tiles,K,parts", [(0.3, 1, 128, 1), (1.0, 1, 1280, 2), (0.99, 2, 2304, 6), (0.6, 3, 384, 3)])
 def test_product_of_few_columns_dealt_evenly(shape, fill, m_tiles, K, parts):
