@@ -27,10 +27,9 @@ def linear(x, weight, bias=None, out_dtype=None, parts_ok=False):
     float32_out = out_dtype == torch.float32
     skinny_ok = ops.gemm_skinny_supported(x, weight)
     wide = float32_out and bias is None and head_is_wide(x.shape[0], weight.shape[0], x.shape[1])
-    tiles_ok = ((wide or (parts_ok and bias is None and not float32_out and TUNING.library_from_rows < x.shape[0] <= TUNING.tiles_parts_most_rows))
-                and ops.gemm_tiles_supported(x, weight))
-    spread_ok = (parts_ok and bias is None and not float32_out and TUNING.library_from_rows < x.shape[0] <= TUNING.spread_parts_most_rows
-                 and (tiles_ok or ops.gemm_tiles_supported(x, weight)))      # the rows first: steps launched kernel by kernel wait for the host
+    tiles_ok = ((wide or (parts_ok and bias is None and not float32_out and TUNING.library_from_rows < x.shape[0]
+                          <= max(TUNING.tiles_parts_most_rows, TUNING.spread_parts_most_rows)))
+                and ops.gemm_tiles_supported(x, weight))      # the rows first: steps launched kernel by kernel wait for the host
     plan = None
     if autotune.active():
         key = ("linear", autotune.rows_class(x.shape[0]), weight.shape[0], x.shape[1], bias is not None, float32_out,
@@ -40,7 +39,7 @@ def linear(x, weight, bias=None, out_dtype=None, parts_ok=False):
         plan = linear_plan(x.shape[0], weight.shape[0], x.shape[1], bias is not None, float32_out, parts_ok, skinny_ok, tiles_ok)
         if wide and tiles_ok:
             plan = wide_plan(x.shape[0], weight.shape[0])
-        elif spread_ok:
+        elif tiles_ok:
             plan = spread_parts(plan, x.shape[0], weight.shape[0], x.shape[1]) or plan
     y = run_linear_plan(plan, x, weight, bias, out_dtype)
     return y[0] if float32_out and plan[0] == "tiles" else y

@@ -1,4 +1,7 @@
 """Decisions that are taken on the host from sizes alone: how a product is split over workgroups."""
+import pytest
+import torch
+
 from ginfer_amd.parts import linear as L
 
 
@@ -87,6 +90,29 @@ def test_products_over_tiles_in_parts_of_k():
     assert plan(64, 3584, 18944, f32=True)[0] == "skinny"
     assert L._parts_without_gaps(140, 10) == 10 and L._parts_without_gaps(9, 4) == 3 and L._parts_without_gaps(12, 5) == 4
     assert L._parts_without_gaps(1, 1) == 1
+
+
+def _plan_and_key(monkeypatch, product, operands, **kwargs):
+    """(the plan that the product of these operands runs, the key by which the tuner knows it), without running it."""
+    from ginfer_amd.kernels import autotune
+    ran = []
+    for name in ("run_linear_plan", "run_gated_plan"):
+        monkeypatch.setattr(L, name, lambda plan, x, *rest: ran.append(plan) or x)
+    with autotune.collecting() as keys:
+        product(*operands, **kwargs)
+    (plan,), (key,) = ran, keys
+    return plan, key
+
+
+@pytest.mark.parametrize("rows", [257, 272, 320, 384, 385])
+@pytest.mark.parametrize("n,k", [(1536, 8960), (3584, 18944), (2304, 1536)])
+def test_the_plan_that_runs_is_a_candidate(rows, n, k, monkeypatch):
+    """The rows between those that the fixed tiles take and the most that are dealt evenly: what runs by the rules, the tuner can keep."""
+    x, w = torch.empty((rows, k), dtype=torch.bfloat16), torch.empty((n, k), dtype=torch.bfloat16)
+    plan, key = _plan_and_key(monkeypatch, L.linear, (x, w), parts_ok=True)
+    assert (plan[0] == "tiles") == (rows <= 384 and k > 2048)
+    if rows % 16 == 0:                                 # the class's own count
+        assert plan in L.linear_candidates(key)
 
 
 def test_measured_plans_stand_before_all_rules(monkeypatch):
