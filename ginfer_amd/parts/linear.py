@@ -36,13 +36,19 @@ def linear(x, weight, bias=None, out_dtype=None, parts_ok=False):
                bool(parts_ok), skinny_ok, tiles_ok)
         plan = autotune.choose(key, (weight, bias))
     if plan is None:
-        plan = linear_plan(x.shape[0], weight.shape[0], x.shape[1], bias is not None, float32_out, parts_ok, skinny_ok, tiles_ok)
-        if wide and tiles_ok:
-            plan = wide_plan(x.shape[0], weight.shape[0])
-        elif tiles_ok:
-            plan = spread_parts(plan, x.shape[0], weight.shape[0], x.shape[1]) or plan
+        plan = linear_choice(x.shape[0], weight.shape[0], x.shape[1], bias is not None, float32_out, parts_ok, skinny_ok, tiles_ok)
     y = run_linear_plan(plan, x, weight, bias, out_dtype)
     return y[0] if float32_out and plan[0] == "tiles" else y
+
+
+def linear_choice(rows, out_features, in_features, has_bias, float32_out, parts_ok, skinny_ok, tiles_ok=False):
+    """The plan that runs by the rules: linear_plan's, or over tiles dealt evenly to the chip where those are the faster."""
+    plan = linear_plan(rows, out_features, in_features, has_bias, float32_out, parts_ok, skinny_ok, tiles_ok)
+    if not tiles_ok or has_bias:
+        return plan
+    if float32_out:
+        return wide_plan(rows, out_features) if head_is_wide(rows, out_features, in_features) else plan
+    return (parts_ok and spread_parts(plan, rows, out_features, in_features)) or plan
 
 
 def _dealing_number(shape, m_tiles, groups):
@@ -218,17 +224,16 @@ def run_linear_plan(plan, x, weight, bias, out_dtype):
 
 
 def linear_candidates(key):
-    """Every plan that does the product of an autotune key; the plan by the rules first."""
+    """Every plan that does the product of an autotune key; the plan that runs by the rules first, then the one it stands in for."""
     _, rows, out_features, in_features, has_bias, float32_out, parts_ok, skinny_ok, tiles_ok = key if len(key) > 8 else key + (False,)
-    plans = [linear_plan(rows, out_features, in_features, has_bias, float32_out, parts_ok, skinny_ok, tiles_ok)]
+    plans = [linear_choice(rows, out_features, in_features, has_bias, float32_out, parts_ok, skinny_ok, tiles_ok)]
 
     def add(plan):
         if plan not in plans:
             plans.append(plan)
 
     may_split = parts_ok and not float32_out
-    if tiles_ok and float32_out and not has_bias and head_is_wide(rows, out_features, in_features):
-        add(wide_plan(rows, out_features))
+    add(linear_plan(rows, out_features, in_features, has_bias, float32_out, parts_ok, skinny_ok, tiles_ok))
     if skinny_ok:
         tiles = (1, 4) if rows > 16 else (1,)
         for nt in tiles:
@@ -244,9 +249,6 @@ def linear_candidates(key):
         parts = tiles_parts(rows, out_features, in_features) if tiles_ok else 0
         if parts:
             add(("tiles", 1, parts))
-        spread = spread_parts(plans[0], rows, out_features, in_features) if tiles_ok else None
-        if spread:
-            add(spread)
         for parts in (2, 3, 4, 5, 7, 8, 10, 14, 16):
             if in_features % parts == 0 and (in_features // parts) % 8 == 0 and in_features // parts >= 512:
                 add(("library", parts))
@@ -397,10 +399,14 @@ def gated_linear(x, weight_gate_up, bounds=None):
         key = ("gated", autotune.rows_class(rows), out_features, in_features, skinny_ok, transposable, tiles_ok, bounds)
         plan = autotune.choose(key, (weight_gate_up,))
     if plan is None:
-        plan = gated_plan(rows, out_features, skinny_ok, transposable, in_features, tiles_ok)
-        if tiles_ok and spread_is_faster(plan, rows, out_features, in_features):
-            plan = ("tiles",)
+        plan = gated_choice(rows, out_features, skinny_ok, transposable, in_features, tiles_ok)
     return run_gated_plan(plan, x, weight_gate_up, bounds)
+
+
+def gated_choice(rows, out_features, skinny_ok, transposable, in_features, tiles_ok):
+    """The plan that runs by the rules: gated_plan's, or over tiles dealt evenly to the chip where those are the faster."""
+    plan = gated_plan(rows, out_features, skinny_ok, transposable, in_features, tiles_ok)
+    return ("tiles",) if tiles_ok and spread_is_faster(plan, rows, out_features, in_features) else plan
 
 
 def spread_is_faster(plan, rows, out_features, in_features):
@@ -452,7 +458,7 @@ def _gated_key(key):
 
 def gated_candidates(key):
     rows, out_features, in_features, skinny_ok, transposable, tiles_ok, _ = _gated_key(key)
-    plans = [gated_plan(rows, out_features, skinny_ok, transposable, in_features, tiles_ok)]
+    plans = [gated_choice(rows, out_features, skinny_ok, transposable, in_features, tiles_ok)]
     for plan, ok in ((("skinny",), skinny_ok), (("library",), True), (("transposed",), transposable), (("tiles",), tiles_ok)):
         if ok and plan not in plans:
             plans.append(plan)

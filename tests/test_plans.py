@@ -115,6 +115,22 @@ def test_the_plan_that_runs_is_a_candidate(rows, n, k, monkeypatch):
         assert plan in L.linear_candidates(key)
 
 
+@pytest.mark.parametrize("rows", [1, 16, 32, 48, 64, 96, 128, 224, 256, 272, 384, 400, 512, 528, 2048])
+def test_the_tuner_starts_from_the_plan_that_linear_and_gated_linear_run(rows, monkeypatch):
+    """Whatever another plan must beat by a margin is what runs without the tuner: products whose parts are added, heads, gated products."""
+    bf16 = lambda *shape: torch.empty(shape, dtype=torch.bfloat16)
+    for n, k in ((1536, 8960), (3584, 18944), (1536, 1536), (896, 4864), (2304, 1528)):
+        plan, key = _plan_and_key(monkeypatch, L.linear, (bf16(rows, k), bf16(n, k)), parts_ok=True)
+        assert L.linear_candidates(key)[0] == plan, key
+    for n, k in ((151936, 1536), (152064, 3584), (32768, 1536)):
+        plan, key = _plan_and_key(monkeypatch, L.linear, (bf16(rows, k), bf16(n, k)), out_dtype=torch.float32)
+        assert L.linear_candidates(key)[0] == plan, key
+    for n, k in ((17920, 1536), (37888, 3584), (9728, 896), (2048, 6144), (3072, 2048), (11136, 8192)):
+        for bounds in (None, (7.0, 1.702, 1.0)):
+            plan, key = _plan_and_key(monkeypatch, L.gated_linear, (bf16(rows, k), bf16(n, k)), bounds=bounds)
+            assert L.gated_candidates(key)[0] == plan, key
+
+
 def test_measured_plans_stand_before_all_rules(monkeypatch):
     monkeypatch.setattr(L.TUNING, "measured_plans", {"64,3584,18944": ("library", 2), "64,1536,8960": ("tiles", 1, 7)})
     plan = lambda rows, n, k, tiles_ok=True: L.linear_plan(rows, n, k, False, False, True, rows <= 64, tiles_ok)
@@ -129,11 +145,12 @@ def test_the_tuner_starts_from_the_plan_that_runs():
         for n, k in ((1536, 8960), (3584, 3584), (3072, 8192), (896, 4864), (3584, 18944)):
             for tiles_ok in (False, True):
                 plans = L.linear_candidates(("linear", rows, n, k, False, False, True, rows <= 64, tiles_ok))
-                assert plans[0] == L.linear_plan(rows, n, k, False, False, True, rows <= 64, tiles_ok)
+                assert plans[0] == L.linear_choice(rows, n, k, False, False, True, rows <= 64, tiles_ok)
+                assert L.linear_plan(rows, n, k, False, False, True, rows <= 64, tiles_ok) in plans[:2]
                 assert tiles_ok or not any(p[0] == "tiles" for p in plans)
                 assert len(set(plans)) == len(plans) and ("library", 1) in plans
     # parts that do not divide K are candidates like any other
-    assert L.linear_candidates(("linear", 64, 3072, 8192, False, False, True, True, True))[0] == ("tiles", 1, 5)
+    assert ("tiles", 1, 5) in L.linear_candidates(("linear", 64, 3072, 8192, False, False, True, True, True))
 
 
 def test_tiles_of_the_gated_product():
@@ -245,7 +262,7 @@ def test_few_columns_dealt_evenly():
     assert not any(parts(rows, n, k) for rows, n, k in ((16, 1536, 8960), (48, 1536, 1536), (64, 2048, 11008), (91, 3584, 3584), (250, 4096, 14336),
                                                          (300, 2304, 1536), (385, 1536, 8960), (128, 1536, 960), (64, 1528, 8960)))
     key = ("linear", 128, 1536, 8960, False, False, True, False, True)
-    assert L.linear_candidates(key)[0] == L.linear_plan(*key[1:]) and ("tiles", L._dealing_number(14, 1, 32), 8) in L.linear_candidates(key)
+    assert L.linear_candidates(key)[:2] == [("tiles", L._dealing_number(14, 1, 32), 8), L.linear_plan(*key[1:])]
 
 
 def test_heads_of_many_columns():
@@ -258,7 +275,7 @@ def test_heads_of_many_columns():
         shape, m_tiles, groups = ops.spread_many_columns(64, n)
         assert shape == 2 and m_tiles == 1 and groups % 256 == 0 and -(-(n // 8) // groups) * 8 <= ops.SPREAD_SHAPES[shape][1]
     key = ("linear", 64, 151936, 1536, False, True, False, True, True)
-    assert L.linear_candidates(key)[:2] == [("library", 1), L.wide_plan(64, 151936)]
+    assert L.linear_candidates(key)[:2] == [L.wide_plan(64, 151936), ("library", 1)]
 
 
 def test_steps_of_a_trip():
@@ -321,7 +338,7 @@ def test_the_gated_product_is_one_plan_of_several():
     """The tuner starts from the plan that runs, can leave it, and tries tiles where the rule does not take them."""
     key = lambda rows, n, k, tiles_ok=True, bounds=None: ("gated", rows, n, k, rows <= 64, bounds is None and rows % 8 == 0, tiles_ok, bounds)
     assert L.gated_candidates(key(64, 17920, 1536)) == [("tiles",), ("skinny",), ("library",), ("transposed",)]
-    assert L.gated_candidates(key(512, 17920, 1536)) == [("transposed",), ("library",), ("tiles",)]
+    assert L.gated_candidates(key(512, 17920, 1536)) == [("tiles",), ("library",), ("transposed",)]
     assert L.gated_candidates(key(300, 17920, 1536, False)) == [("library",)]
     assert L.gated_candidates(key(100, 17920, 1536, True, (7.0, 1.702, 1.0))) == [("tiles",), ("library",)]
     assert L.gated_plan(64, 17920, True, True, 1536, True) == ("tiles",) and L.gated_plan(64, 17920, True, True, 1536, False) == ("library",)
