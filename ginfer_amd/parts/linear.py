@@ -48,7 +48,9 @@ def linear_choice(rows, out_features, in_features, has_bias, float32_out, parts_
         return plan
     if float32_out:
         return wide_plan(rows, out_features) if head_is_wide(rows, out_features, in_features) else plan
-    return (parts_ok and spread_parts(plan, rows, out_features, in_features)) or plan
+    if not parts_ok or _measured_plan(rows, out_features, in_features, skinny_ok, tiles_ok):
+        return plan
+    return spread_parts(plan, rows, out_features, in_features) or plan
 
 
 def _dealing_number(shape, m_tiles, groups):
@@ -74,7 +76,7 @@ def spread_parts(plan, rows, out_features, in_features):
     the other rules' (by sizes alone; the measurements stand beside the thresholds); else None."""
     T = TUNING
     if (not T.library_from_rows < rows <= T.spread_parts_most_rows or out_features % 16 or in_features % 64
-            or in_features < T.spread_parts_min_in_features or T.measured_plans):
+            or in_features < T.spread_parts_min_in_features):
         return None
     if plan[0] == "skinny" and rows <= T.spread_parts_beyond_rows:
         return None
@@ -171,9 +173,9 @@ def linear_plan(rows, out_features, in_features, has_bias, float32_out, parts_ok
     float32 partial sums [parts, M, N] for the consumer to add."""
     may_split = parts_ok and not float32_out
     if may_split and not has_bias:
-        measured = TUNING.measured_plans.get("%d,%d,%d" % (autotune.rows_class(rows), out_features, in_features))
-        if measured is not None and {"skinny": skinny_ok, "tiles": tiles_ok}.get(measured[0], True):
-            return tuple(measured)
+        measured = _measured_plan(rows, out_features, in_features, skinny_ok, tiles_ok)
+        if measured:
+            return measured
         parts = tiles_parts(rows, out_features, in_features) if tiles_ok else 0
         if parts:
             return ("tiles", 1, parts)
@@ -194,6 +196,15 @@ def linear_plan(rows, out_features, in_features, has_bias, float32_out, parts_ok
         if parts > 1:
             return ("library", parts)
     return ("library", 1)
+
+
+def _measured_plan(rows, out_features, in_features, skinny_ok, tiles_ok):
+    """The plan that the tuning table holds for this very product whose parts are added, or None: none, or its kernel does not take the
+    operands."""
+    if not TUNING.measured_plans:
+        return None
+    plan = TUNING.measured_plans.get("%d,%d,%d" % (autotune.rows_class(rows), out_features, in_features))
+    return tuple(plan) if plan is not None and {"skinny": skinny_ok, "tiles": tiles_ok}.get(plan[0], True) else None
 
 
 def run_linear_plan(plan, x, weight, bias, out_dtype):

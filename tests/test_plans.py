@@ -140,6 +140,17 @@ def test_measured_plans_stand_before_all_rules(monkeypatch):
     assert L.linear_plan(64, 3584, 18944, True, False, True, True, True)[0] == "skinny"             # a bias: no parts
 
 
+def test_a_measured_plan_is_of_its_own_size_alone(monkeypatch):
+    """It stands before the even dealing too, and leaves the products of other sizes, and operands that it is not for, to the rules."""
+    choice = lambda rows, n, k, skinny_ok: L.linear_choice(rows, n, k, False, False, True, skinny_ok, True)
+    sizes = [(64, 1536, 8960, True), (128, 3584, 18944, False), (384, 1536, 8960, False)]
+    by_rules = [choice(*size) for size in sizes]
+    assert all(plan[0] == "tiles" and plan[1] != 1 for plan in by_rules)
+    monkeypatch.setattr(L.TUNING, "measured_plans", {"64,1024,8192": ("library", 4), "384,1536,8960": ("library", 5), "64,1536,8960": ("skinny", 4, 10)})
+    assert [choice(*size) for size in sizes] == [("skinny", 4, 10), by_rules[1], ("library", 5)]
+    assert choice(64, 1536, 8960, False) == by_rules[0]
+
+
 def test_the_tuner_starts_from_the_plan_that_runs():
     for rows in (16, 17, 64, 128, 256):
         for n, k in ((1536, 8960), (3584, 3584), (3072, 8192), (896, 4864), (3584, 18944)):
