@@ -3,7 +3,7 @@ import math
 
 import torch
 
-from ..kernels import ops
+from ..kernels import autotune, ops
 from ..kernels.tuning import TUNING
 from ..weights.loader import WeightSpec
 from .base import Part, KVCacheSpec
@@ -34,15 +34,75 @@ def _projection_in_parts(rows, in_features, out_features):
 
 def _projection_way(x, w_qkv, head_dim, rotary_dim):
     """("fused",), ("parts", n) or ("library",): how rows x become q, k and v where their product is not dealt evenly to the chip."""
-    rows, K = x.shape
-    if ops.qkv_rope_skinny_supported(x, w_qkv, head_dim, rotary_dim):
-        return ("library",) if _library_then_rotation_is_faster(rows, K, w_qkv.shape[0]) else ("fused",)
-    if (not isinstance(x, ops.ScaledRows) and ops.gemm_skinny_supported(x, w_qkv) and (rotary_dim // 2) % 4 == 0
-            and (head_dim - rotary_dim) % 4 == 0 and head_dim % 4 == 0):
-        parts = _projection_in_parts(rows, K, w_qkv.shape[0])
-        if parts:
-            return ("parts", parts)
-    return ("library",)
+    fused_ok = ops.qkv_rope_skinny_supported(x, w_qkv, head_dim, rotary_dim)
+    return _other_way(x.shape[0], x.shape[1], w_qkv.shape[0], fused_ok, not fused_ok and _parts_supported(x, w_qkv, head_dim, rotary_dim))
+
+
+def _parts_supported(x, w_qkv, head_dim, rotary_dim):
+    return (not isinstance(x, ops.ScaledRows) and ops.gemm_skinny_supported(x, w_qkv) and (rotary_dim // 2) % 4 == 0
+            and (head_dim - rotary_dim) % 4 == 0 and head_dim % 4 == 0)
+
+
+def _other_way(rows, in_features, out_features, fused_ok, parts_ok):
+    if fused_ok:
+        return ("library",) if _library_then_rotation_is_faster(rows, in_features, out_features) else ("fused",)
+    parts = _projection_in_parts(rows, in_features, out_features) if parts_ok else 0
+    return ("parts", parts) if parts else ("library",)
+
+
+def projection_choice(x, w_qkv, has_bias, num_heads, num_kv_heads, head_dim, rotary_dim):
+    """(the way that rows x become q, k and v, the tuner's key for it or None): ("spread", plan) over tiles dealt evenly to the chip, where
+    they hold the product, or one of _projection_way's."""
+    plan = ops.qkv_spread_plan(x, w_qkv, head_dim, rotary_dim)
+    key = None
+    if plan and autotune.active():
+        fused_ok = ops.qkv_rope_skinny_supported(x, w_qkv, head_dim, rotary_dim)
+        key = ("qkv", autotune.rows_class(x.shape[0]), w_qkv.shape[0], x.shape[1], has_bias, num_heads, num_kv_heads, head_dim, rotary_dim,
+               fused_ok, not fused_ok and _parts_supported(x, w_qkv, head_dim, rotary_dim))
+    return ("spread", plan) if plan else _projection_way(x, w_qkv, head_dim, rotary_dim), key
+
+
+def project(way, x, w, bias, positions, cos, sin, slot_mapping, k_pages, v_pages, num_heads, num_kv_heads, head_dim, write_kv):
+    """q|k|v of rows x: q rotated (the columns behind it are the kernel's own), k and v in their pages."""
+    place = (positions, cos, sin, slot_mapping, k_pages, v_pages, num_heads, num_kv_heads, head_dim)
+    if way[0] == "fused":
+        # few rows (decode): projection, rotation and cache write in one kernel
+        return ops.qkv_rope_skinny(x, w, bias, *place, write_kv=write_kv)
+    if way[0] == "spread":
+        # more rows: the same, over tiles that are dealt evenly to the chip (by the rows that come, where a plan stands for a class of them)
+        return ops.qkv_spread(x, w, bias, *place, write_kv=write_kv, plan=way[1] if len(way) > 1 else None)
+    if way[0] == "parts":
+        # the product with K split over workgroups (every workgroup then reads a share of the rows only), its 32-bit
+        # parts added up by the kernel that rotates and writes the cache
+        sums = ops.gemm_skinny(x, w, None, out_dtype=torch.float32, nt=2, grid_splits=way[1])
+        return ops.rope_kv_from_parts(sums, bias, *place, write_kv=write_kv)
+    qkv = linear(x, w, bias)
+    ops.rope_kv_write(qkv, *place, write_kv=write_kv)
+    return qkv
+
+
+def projection_candidates(key):
+    """Every way to do the projection of an autotune key; the one that runs by the rules first."""
+    _, rows, out_features, in_features, _, _, _, _, _, fused_ok, parts_ok = key
+    ways = [("spread",)]
+    for way in (_other_way(rows, in_features, out_features, fused_ok, parts_ok), ("fused",) if fused_ok else None, ("library",)):
+        if way and way not in ways:
+            ways.append(way)
+    return ways
+
+
+def _projection_timing(key, operands, device):
+    """For the tuner: random rows, tokens of one request side by side in pages of 16."""
+    _, rows, _, in_features, _, nh, nkv, hd, rotary_dim = key[:9]
+    x = (torch.randn((rows, in_features), device=device) * 0.5).to(torch.bfloat16)
+    positions, slots = torch.zeros(rows, dtype=torch.int32, device=device), torch.arange(rows, device=device)
+    cos, sin = torch.ones((1, rotary_dim // 2), device=device), torch.zeros((1, rotary_dim // 2), device=device)
+    k_pages = torch.zeros((-(-rows // 16), nkv, 16, hd), dtype=torch.bfloat16, device=device)
+    v_pages = torch.zeros((-(-rows // 16), nkv, hd, 16), dtype=torch.bfloat16, device=device)
+    return lambda way, i: project(way, x, *operands[i], positions, cos, sin, slots, k_pages, v_pages, nh, nkv, hd, True)
+
+
+autotune.register_kind("qkv", projection_candidates, _projection_timing)
 
 
 @register_mixer("attention")
@@ -104,26 +164,11 @@ class Attention(Part):
         """into_norm = (residual, norm): where the output projection's kernel can, the result is added to the
         residual here and the rows of `norm` come back as ops.ScaledRows; else the result comes back as ever."""
         cos, sin = self.position.tables()
-        spread = ops.qkv_spread_plan(x, self.w_qkv, self.hd, self.position.rotary_dim)
-        way = ("spread",) if spread else _projection_way(x, self.w_qkv, self.hd, self.position.rotary_dim)
-        if way[0] == "fused":
-            # few rows (decode): projection, rotation and cache write in one kernel
-            qkv = ops.qkv_rope_skinny(x, self.w_qkv, self.b_qkv, step.positions, cos, sin, cache.slot_mapping,
-                                      cache.k_pages, cache.v_pages, self.nh, self.nkv, self.hd, write_kv=cache.owner)
-        elif way[0] == "spread":
-            # more rows: the same, over tiles that are dealt evenly to the chip
-            qkv = ops.qkv_spread(x, self.w_qkv, self.b_qkv, step.positions, cos, sin, cache.slot_mapping, cache.k_pages, cache.v_pages,
-                                 self.nh, self.nkv, self.hd, write_kv=cache.owner, plan=spread)
-        elif way[0] == "parts":
-            # the product with K split over workgroups (every workgroup then reads a share of the rows only), its 32-bit
-            # parts added up by the kernel that rotates and writes the cache
-            sums = ops.gemm_skinny(x, self.w_qkv, None, out_dtype=torch.float32, nt=2, grid_splits=way[1])
-            qkv = ops.rope_kv_from_parts(sums, self.b_qkv, step.positions, cos, sin, cache.slot_mapping, cache.k_pages,
-                                         cache.v_pages, self.nh, self.nkv, self.hd, write_kv=cache.owner)
-        else:
-            qkv = linear(x, self.w_qkv, self.b_qkv)
-            ops.rope_kv_write(qkv, step.positions, cos, sin, cache.slot_mapping, cache.k_pages, cache.v_pages,
-                              self.nh, self.nkv, self.hd, write_kv=cache.owner)
+        way, key = projection_choice(x, self.w_qkv, self.b_qkv is not None, self.nh, self.nkv, self.hd, self.position.rotary_dim)
+        if key is not None:
+            way = autotune.choose(key, (self.w_qkv, self.b_qkv)) or way
+        qkv = project(way, x, self.w_qkv, self.b_qkv, step.positions, cos, sin, cache.slot_mapping, cache.k_pages, cache.v_pages,
+                      self.nh, self.nkv, self.hd, cache.owner)
         a = ops.paged_attention(qkv, cache.k_pages, cache.v_pages, cache.block_table, step, self.nh, self.nkv,
                                 self.hd, self.scale, self.window)
         if into_norm is not None:

@@ -74,6 +74,38 @@ def test_every_candidate_plan_of_the_gated_product(rows, n, k):
             assert err <= 1.2e-2, "plan %s: %.3g" % (plan, err)
 
 
+@pytest.mark.parametrize("rows,nh,nkv,hd,K", [(17, 4, 2, 64, 1536), (64, 4, 2, 48, 1152), (100, 3, 1, 128, 640)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_every_way_of_the_projection(rows, nh, nkv, hd, K, bias):
+    """Rotated q and the pages of k and v by every way that the tuner may keep, and that it times them all."""
+    from ginfer_amd.kernels import autotune, ops
+    from ginfer_amd.parts import attention
+    x, w, b, xd, wd, bd = _operands(rows, (nh + 2 * nkv) * hd, K, rows + K, bias)
+    with autotune.collecting() as keys:
+        way, key = attention.projection_choice(x, w, bias, nh, nkv, hd, hd)
+        assert way[0] == "spread" and autotune.choose(key, (w, b)) is None
+    ways = attention.projection_candidates(key)
+    assert [way[0] for way in ways] == {17: ["spread", "fused", "library"], 64: ["spread", "parts", "library"], 100: ["spread", "library"]}[rows]
+    table = autotune.Table()
+    assert autotune.tune(keys, x.device, table) == 1 and table[key] in ways and set(table.report[0][2]) == set(ways)
+    positions = torch.arange(rows, dtype=torch.int32, device=x.device)
+    angle = torch.arange(rows)[:, None] * (1e4 ** (-2.0 * torch.arange(hd // 2) / hd))[None]
+    cos, sin = torch.cos(angle).float(), torch.sin(angle).float()
+    full = (xd @ wd.T + (bd if bias else 0.0)).view(rows, nh + 2 * nkv, hd)
+    lo, hi, c, s = full[..., :hd // 2], full[..., hd // 2:], cos.double()[:, None], sin.double()[:, None]
+    turned = torch.cat([lo * c - hi * s, lo * s + hi * c], dim=-1)
+    for way in ways:
+        kp = torch.zeros((-(-rows // 8), nkv, 8, hd), dtype=torch.bfloat16, device=x.device)
+        vp = torch.zeros((-(-rows // 8), nkv, hd, 8), dtype=torch.bfloat16, device=x.device)
+        qkv = attention.project(way, x, w, b, positions, cos.to(x.device), sin.to(x.device), torch.arange(rows, device=x.device), kp, vp,
+                                nh, nkv, hd, True)
+        got = dict(q=qkv[:, :nh * hd].reshape(rows, nh, hd), k=kp.permute(0, 2, 1, 3).reshape(-1, nkv, hd)[:rows],
+                   v=vp.permute(0, 3, 1, 2).reshape(-1, nkv, hd)[:rows])
+        for name, want in (("q", turned[:, :nh]), ("k", turned[:, nh:nh + nkv]), ("v", full[:, nh + nkv:])):
+            err = float((got[name].double().cpu() - want).abs().max() / want.abs().max())
+            assert err <= 1e-2, "%s by %s: %.3g" % (name, way, err)       # the library's rows are rounded before the rotation and after it
+
+
 def test_a_runner_that_times_its_plans(tmp_path):
     """Two layers of a 7B shape, 40 requests decoding side by side: the runner times the plans of its products when it
     records the step (the rules' plan for this down projection is not the fastest one), and logits stay the plain

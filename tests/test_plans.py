@@ -131,6 +131,43 @@ def test_the_tuner_starts_from_the_plan_that_linear_and_gated_linear_run(rows, m
             assert L.gated_candidates(key)[0] == plan, key
 
 
+@pytest.mark.parametrize("rows", [16, 17, 48, 64, 65, 272, 512, 513])
+@pytest.mark.parametrize("K,hd,rd", [(1536, 128, 128), (1152, 48, 48), (1152, 64, 32), (1096, 64, 64)])
+def test_the_projection_is_one_plan_of_several(rows, K, hd, rd, monkeypatch):
+    """What an attention part runs for q|k|v by the rules is what the tuner starts from, and another way that it keeps is taken."""
+    from types import SimpleNamespace
+    from ginfer_amd.kernels import autotune
+    from ginfer_amd.parts import attention, lookup
+    ran = []
+
+    class Ran(Exception):
+        pass
+
+    def project(way, *rest):
+        ran.append(way)
+        raise Ran
+    monkeypatch.setattr(attention, "project", project)
+    position = lookup("position", "rope_neox")(theta=1e4, rotary_dim=rd, max_positions=16, device="cpu")
+    part = lookup("mixer", "attention")(hidden_size=K, num_heads=4, num_kv_heads=2, head_dim=hd, qkv_bias=True, out_bias=False, window=None,
+                                        position=position, scale=None, dtype=torch.bfloat16, device="cpu")
+    part.bind_weights({n: torch.empty(s.shape, dtype=torch.bfloat16) for n, s in part.weight_specs().items()})
+    step = SimpleNamespace(positions=None)
+    cache = SimpleNamespace(slot_mapping=None, k_pages=None, v_pages=None, owner=True)
+    x = torch.empty((rows, K), dtype=torch.bfloat16)
+    with autotune.collecting() as keys, pytest.raises(Ran):
+        part.forward(x, step, cache)
+    assert (ran[0][0] == "spread") == (17 <= rows <= 512 and rd == hd and K % 64 == 0) == bool(keys)
+    for key in keys:
+        ways = attention.projection_candidates(key)
+        assert ways[0][0] == ran[0][0] and ("library",) in ways and len(set(ways)) == len(ways) >= 2
+        for way in ways:
+            table = autotune.Table()
+            table[key] = way
+            with autotune.using(table), pytest.raises(Ran):
+                part.forward(x, step, cache)
+            assert ran[-1] == way
+
+
 def test_measured_plans_stand_before_all_rules(monkeypatch):
     monkeypatch.setattr(L.TUNING, "measured_plans", {"64,3584,18944": ("library", 2), "64,1536,8960": ("tiles", 1, 7)})
     plan = lambda rows, n, k, tiles_ok=True: L.linear_plan(rows, n, k, False, False, True, rows <= 64, tiles_ok)
