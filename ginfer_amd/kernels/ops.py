@@ -591,6 +591,12 @@ def spread_few_columns(rows, out_features, in_features, parts=1):
     return best
 
 
+def spread_share(plan, rows, out_features):
+    """(rows of A and rows of W that the largest share of a plan has, what its tile has room for of each, elements of a slab)."""
+    (room_a, room_w, slab), m_tiles, groups = (SPREAD_SHAPES + SPREAD_NARROW_SHAPES)[plan[0]], plan[1], plan[2]
+    return -(-(-(-rows // m_tiles)) // 16) * 16, -(-(out_features // 8) // groups) * 8, room_a, room_w, slab
+
+
 def spread_many_columns(rows, out_features):
     """(number in SPREAD_SHAPES, row tiles, groups of columns) of a product of up to 64 rows by more columns than one round of the chip holds, dealt evenly to
     as many rounds as tiles of 160 rows of W make (151,936 x 1,536 at 33 rows 92.8 us, over tiles of 128 rows 94.4, of 32 101)."""

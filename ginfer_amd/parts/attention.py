@@ -50,16 +50,37 @@ def _other_way(rows, in_features, out_features, fused_ok, parts_ok):
     return ("parts", parts) if parts else ("library",)
 
 
+def _dealing_is_slower(plan, rows, in_features, out_features):
+    """Whether the other ways are faster than q|k|v over tiles dealt evenly to the chip by `plan`, by sizes alone (the measurements stand
+    beside the thresholds)."""
+    T = TUNING
+    if rows <= T.qkv_spread_up_to_rows:
+        return False
+    _, m_tiles, groups = plan
+    _, _, room_a, room_w, _ = ops.spread_share(plan, rows, out_features)
+    padded = room_a * room_w * m_tiles * groups / (rows * out_features)
+    if room_a >= T.qkv_spread_tall_tile:
+        return m_tiles > 2 or padded > T.qkv_spread_tall_padded
+    if (in_features % 128 or room_w < T.qkv_spread_wide_tile or in_features < T.qkv_spread_long_k
+            or out_features * in_features <= T.qkv_spread_many_weights):
+        return False
+    if m_tiles == 3:
+        return in_features >= T.qkv_spread_longer_k and rows > T.qkv_spread_longer_k_up_to_rows
+    return m_tiles > 3 and padded > T.qkv_spread_wide_padded
+
+
 def projection_choice(x, w_qkv, has_bias, num_heads, num_kv_heads, head_dim, rotary_dim):
     """(the way that rows x become q, k and v, the tuner's key for it or None): ("spread", plan) over tiles dealt evenly to the chip, where
-    they hold the product, or one of _projection_way's."""
+    they hold the product and are the faster, or one of _projection_way's."""
     plan = ops.qkv_spread_plan(x, w_qkv, head_dim, rotary_dim)
     key = None
     if plan and autotune.active():
         fused_ok = ops.qkv_rope_skinny_supported(x, w_qkv, head_dim, rotary_dim)
         key = ("qkv", autotune.rows_class(x.shape[0]), w_qkv.shape[0], x.shape[1], has_bias, num_heads, num_kv_heads, head_dim, rotary_dim,
                fused_ok, not fused_ok and _parts_supported(x, w_qkv, head_dim, rotary_dim))
-    return ("spread", plan) if plan else _projection_way(x, w_qkv, head_dim, rotary_dim), key
+    if plan and not _dealing_is_slower(plan, *x.shape, w_qkv.shape[0]):
+        return ("spread", plan), key
+    return _projection_way(x, w_qkv, head_dim, rotary_dim), key
 
 
 def project(way, x, w, bias, positions, cos, sin, slot_mapping, k_pages, v_pages, num_heads, num_kv_heads, head_dim, write_kv):
@@ -84,8 +105,10 @@ def project(way, x, w, bias, positions, cos, sin, slot_mapping, k_pages, v_pages
 def projection_candidates(key):
     """Every way to do the projection of an autotune key; the one that runs by the rules first."""
     _, rows, out_features, in_features, _, _, _, _, _, fused_ok, parts_ok = key
-    ways = [("spread",)]
-    for way in (_other_way(rows, in_features, out_features, fused_ok, parts_ok), ("fused",) if fused_ok else None, ("library",)):
+    spread, other = ("spread",), _other_way(rows, in_features, out_features, fused_ok, parts_ok)
+    slower = _dealing_is_slower(ops.spread_few_columns(rows, out_features, in_features)[1], rows, in_features, out_features)
+    ways = [other, spread] if slower else [spread, other]
+    for way in (("fused",) if fused_ok else None, ("library",)):
         if way and way not in ways:
             ways.append(way)
     return ways

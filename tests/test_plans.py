@@ -168,6 +168,23 @@ def test_the_projection_is_one_plan_of_several(rows, K, hd, rd, monkeypatch):
             assert ran[-1] == way
 
 
+def test_the_projection_is_dealt_evenly_where_that_is_faster():
+    """Sizes on both sides of the lines, as measured; the tuner starts from what runs there too."""
+    from ginfer_amd.kernels import autotune
+    from ginfer_amd.parts import attention
+    def way(rows, n, k):
+        x, w = torch.empty((rows, k), dtype=torch.bfloat16), torch.empty((n, k), dtype=torch.bfloat16)
+        with autotune.collecting():
+            way, key = attention.projection_choice(x, w, True, n // 128 - 4, 2, 128, 128)
+        assert attention.projection_candidates((key[0], rows) + key[2:])[0][0] == way[0] and ("spread",) in attention.projection_candidates(key)
+        return way[0]
+    spread = [(17, 2048, 1536), (512, 2048, 1536), (384, 4608, 3584), (512, 4608, 3584), (256, 10240, 8192), (300, 6144, 4096), (512, 6144, 4096),
+              (448, 7168, 5120), (300, 8192, 6144), (320, 8192, 3584)]
+    library = [(257, 10240, 7680), (281, 10240, 4160), (403, 7168, 4096), (418, 8192, 6912), (384, 8192, 6144), (462, 6144, 7936), (430, 6144, 4096),
+               (512, 10240, 5760), (442, 12288, 8128), (500, 12288, 6720)]
+    assert [way(*size) for size in spread] == ["spread"] * len(spread) and [way(*size) for size in library] == ["library"] * len(library)
+
+
 def test_measured_plans_stand_before_all_rules(monkeypatch):
     monkeypatch.setattr(L.TUNING, "measured_plans", {"64,3584,18944": ("library", 2), "64,1536,8960": ("tiles", 1, 7)})
     plan = lambda rows, n, k, tiles_ok=True: L.linear_plan(rows, n, k, False, False, True, rows <= 64, tiles_ok)
