@@ -426,9 +426,18 @@ def spread_is_faster(plan, rows, out_features, in_features):
     T = TUNING
     if plan == ("tiles",) or ops.spread_dealing(rows, out_features, in_features) is None:
         return False
+    weights, whole = out_features * in_features, in_features % 128 == 0
     if plan == ("skinny",):
-        return (out_features >= T.spread_few_rows_min_out_features
-                or rows > T.spread_beyond_rows and out_features * in_features >= T.spread_min_weights)
+        if out_features >= T.spread_few_rows_min_out_features:
+            return weights >= (T.spread_few_rows_min_weights if whole else T.spread_few_rows_min_weights_half)
+        return whole and rows > T.spread_beyond_rows and weights >= T.spread_min_weights
+    dealing = ops.spread_plan(rows, out_features, in_features) if in_features >= T.spread_full_from_in_features else None
+    if dealing:
+        tile_rows, own, room_a, room_w, slab = ops.spread_share(dealing, rows, out_features)
+        full = tile_rows * own / (room_a * room_w)
+        if slab == 64 and (full <= T.spread_least_full or (dealing[1] > 2 and room_a == 128 and full <= T.spread_least_full_long_k
+                                                           and in_features >= T.spread_full_long_k)):
+            return False
     if rows > SKINNY_MAX_ROWS and in_features > T.spread_most_k_of_columns * out_features:
         return False
     return rows <= T.spread_long_k_up_to_rows or in_features <= T.spread_most_in_features

@@ -298,9 +298,20 @@ def test_gated_products_dealt_evenly():
     assert plan(256, 22016, 2048) is None and plan(300, 10496, 3584) is None and plan(225, 9728, 896) is None and plan(256, 9088, 2880) == (7, 2, 128)
     assert faster("library", 225, 9728, 896) and faster("library", 300, 10496, 3584)      # by the other tiles
     assert plan(150, 27648, 5120) == (8, 1, 256) and plan(225, 12288, 2560) and plan(150, 3712, 2048)
-    assert faster("skinny", 17, 17920, 1536) and not faster("skinny", 17, 9728, 896) and faster("skinny", 33, 3072, 2048) and not faster("skinny", 34, 2688, 512)
+    assert faster("skinny", 17, 17920, 1536) and not faster("skinny", 17, 9728, 896) and faster("skinny", 49, 3072, 2048) and not faster("skinny", 49, 2688, 512)
     assert faster("library", 400, 17920, 1536) and faster("transposed", 512, 17920, 1536) and not faster("library", 92, 2048, 6144)
     assert faster("library", 384, 11136, 8192) and not faster("library", 508, 11136, 8192) and not faster("tiles", 64, 17920, 1536)
+
+
+def test_gated_products_leave_the_even_dealing_where_it_is_slower():
+    """Drawn sizes on both sides of the lines: few rows of a W that the streaming kernel takes, a K that is no multiple of 128, tiles that are
+    mostly room."""
+    faster = lambda plan, rows, n, k: L.spread_is_faster((plan,), rows, n, k)
+    assert all(faster("skinny", *size) for size in ((17, 17920, 1536), (32, 14720, 1024), (49, 2048, 6144), (64, 3072, 2048), (24, 11392, 1088)))
+    assert not any(faster("skinny", *size) for size in ((34, 1792, 7488), (64, 1280, 4032), (57, 3968, 7232), (36, 1536, 4096), (48, 3072, 2048),
+                                                        (20, 11264, 832), (20, 11264, 1024 - 64), (17, 11264, 768)))
+    assert all(faster("library", *size) for size in ((64, 8192, 8000), (289, 5248, 4096), (197, 6912, 3584), (64, 5120, 3392), (128, 17920, 8192)))
+    assert not any(faster("library", *size) for size in ((32, 4096, 8000), (17, 4224, 4544), (289, 5248, 6528), (296, 5376, 6144), (197, 6912, 7552)))
 
 
 def test_few_columns_dealt_evenly():
