@@ -515,25 +515,27 @@ SPREAD_SHAPES = ((64, 80, 128), (128, 80, 128), (64, 160, 64), (128, 160, 64), (
                  (64, 128, 64), (128, 128, 64), (192, 128, 64), (256, 128, 64))     # room for rows of A and of W, elements of a slab
 
 
-@functools.lru_cache(maxsize=4096)
 def spread_plan(rows, out_features, in_features):
     """(number in SPREAD_SHAPES, row tiles, groups of columns) of the gated product of 17 to 512 rows by `out_features` rows of W
-    dealt evenly to the chip (csrc/gemm_tiles.hip), or None where the tiles of gated_tiling and gated_wide_tiling are the faster or
-    no shape holds it.  One workgroup to each of the 256 compute units, in the split that has them read the fewest rows, and up to
-    64 rows two, one after the other, where one cannot hold its share of W.  Beyond 128 rows the other tiles are better where they
-    fit one round and read fewer rows with their padding, or are of 128 x 128 and fill most of it, against three row tiles here, or
-    half of it with a small W; us of those and of this: 22,016 x 2,048 at 256 rows 34.8 and 37.3; 10,496 x 3,584 at 300 34.4 and 38.2, 9,088 x 2,880 27.1 and 30.8; 5,888 x 1,536 at 300 12.7
-    and 16.1, 9,728 x 896 at 225 10.0 and 12.4, 7,936 x 768 at 384 9.6 and 11.9; the other way 27,648 x 5,120 at 150 78.7 and 66.4, 17,920 x 1,536
-    at 256 26.6 and 23.8, 12,288 x 2,560 at 225 32.2 and 28.6, 3,712 x 2,048 at 150 14.8 and 10.9.  Over 325 products of 42 sizes what is chosen
-    is 0.4 % behind the better of the two (with the line at 0.92 of the rows without padding, drawn before those tiles had eight wavefronts, 2.2 %)."""
+    dealt evenly to the chip (csrc/gemm_tiles.hip), or None where the tiles of gated_tiling and gated_wide_tiling are the faster (the lines
+    and what they were measured on stand in kernels/tuning.py) or no shape holds it.  One workgroup to each of the 256 compute units, in
+    the split that has them read the fewest rows, and up to 64 rows two, one after the other, where one cannot hold its share of W."""
+    T = TUNING
+    return _spread_plan(rows, out_features, in_features, T.spread_up_to_rows, T.spread_square_tiles, T.spread_square_tiles_few_weights,
+                        T.spread_square_few_weights)
+
+
+@functools.lru_cache(maxsize=4096)
+def _spread_plan(rows, out_features, in_features, up_to_rows, square_tiles, square_tiles_few_weights, square_few_weights):
     best = spread_dealing(rows, out_features, in_features)
-    if best is None or rows <= 128:
+    if best is None or rows <= up_to_rows:
         return best and best[1]
     number = gated_wide_tiling(rows, out_features, in_features)
     of_w, of_a = GATED_WIDE_TILINGS[number] if number else GATED_TILINGS[gated_tiling(rows, out_features)]
     tiles = -(-rows // of_a) * -(-out_features // of_w)
     if tiles <= 256:
-        if of_w == of_a == 128 and ((tiles >= 110 and out_features * in_features <= 10500000) or (tiles >= 200 and best[1][1] > 2)):
+        if of_w == of_a == 128 and ((tiles >= square_tiles_few_weights and out_features * in_features <= square_few_weights)
+                                    or (tiles >= square_tiles and best[1][1] > 2)):
             return None
         if best[0] > of_w + of_a:
             return None

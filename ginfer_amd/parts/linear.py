@@ -64,11 +64,12 @@ def _dealing(number):
 
 
 def _parts_estimate(rows, out_features, in_features, read, parts):
-    """us that a product in parts of K and the norm that adds them are taken to differ by: a compute unit's rows of W and A at the 50 GB/s it
-    takes in and all of W at 5.2 TB/s, which hide each other in part, the parts' way to memory and back, and what the norm's loop over
+    """us that a product in parts of K and the norm that adds them are taken to differ by: a compute unit's rows of W and A and all of W at
+    the rates that they come in at, which hide each other in part, the parts' way to memory and back, and what the norm's loop over
     a number of parts it was not compiled for costs."""
-    streams = math.hypot(read * 2 * in_features / parts / 50e3, out_features * in_features * 2 / 5.2e6)
-    return streams + parts * rows * out_features * 8 / 3e6 + (0 if parts in (1, 2, 4, 8) else 3)
+    T = TUNING
+    streams = math.hypot(read * 2 * in_features / parts / T.parts_estimate_unit_rate, out_features * in_features * 2 / T.parts_estimate_chip_rate)
+    return streams + parts * rows * out_features * 8 / T.parts_estimate_parts_rate + (0 if parts in (1, 2, 4, 8) else T.parts_estimate_odd_parts)
 
 
 def spread_parts(plan, rows, out_features, in_features):
@@ -80,10 +81,10 @@ def spread_parts(plan, rows, out_features, in_features):
         return None
     if plan[0] == "skinny" and rows <= T.spread_parts_beyond_rows:
         return None
-    if rows > 256 and in_features <= T.spread_parts_short_k:
+    if rows > T.spread_parts_many_rows and in_features <= T.spread_parts_short_k:
         return None
     if (plan[0] == "library" and out_features * in_features > T.spread_parts_library_weights
-            and T.spread_parts_library_from_rows < rows <= 256):
+            and T.spread_parts_library_from_rows < rows <= T.spread_parts_many_rows):
         return None
     best = None
     for parts in (1, 2, 4, 8):
@@ -97,7 +98,7 @@ def spread_parts(plan, rows, out_features, in_features):
     if plan[0] == "tiles":
         tile = 64 if rows <= SKINNY_MAX_ROWS else 128
         other = _parts_estimate(rows, out_features, in_features, 64 + tile, plan[2])
-        if best[0] > T.spread_parts_share_of_tiles * other or (rows <= 128 and best[1][2] == plan[2]):
+        if best[0] > T.spread_parts_share_of_tiles * other or (rows <= T.spread_parts_few_rows and best[1][2] == plan[2]):
             return None
     return best[1]
 

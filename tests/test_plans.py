@@ -314,6 +314,18 @@ def test_gated_products_leave_the_even_dealing_where_it_is_slower():
     assert not any(faster("library", *size) for size in ((32, 4096, 8000), (17, 4224, 4544), (289, 5248, 6528), (296, 5376, 6144), (197, 6912, 7552)))
 
 
+def test_the_tables_lines_hold_after_a_size_was_seen(monkeypatch):
+    """Plans by size are remembered, the lines that a user sets are not passed over for that."""
+    from ginfer_amd.kernels import ops
+    seen = ops.spread_plan(256, 17920, 1536), ops.spread_plan(300, 10496, 3584)
+    assert seen[0] and seen[1] is None
+    for name, value in (("spread_up_to_rows", 512), ("spread_square_tiles", 257)):
+        with monkeypatch.context() as m:
+            m.setattr(L.TUNING, name, value)
+            assert ops.spread_plan(300, 10496, 3584)
+    assert (ops.spread_plan(256, 17920, 1536), ops.spread_plan(300, 10496, 3584)) == seen
+
+
 def test_few_columns_dealt_evenly():
     """A plan's tiles hold what it deals out, its parts of K are whole slabs, and it stands where it was measured the faster."""
     from ginfer_amd.kernels import ops
