@@ -522,11 +522,12 @@ def spread_plan(rows, out_features, in_features):
     the split that has them read the fewest rows, and up to 64 rows two, one after the other, where one cannot hold its share of W."""
     T = TUNING
     return _spread_plan(rows, out_features, in_features, T.spread_up_to_rows, T.spread_square_tiles, T.spread_square_tiles_few_weights,
-                        T.spread_square_few_weights)
+                        T.spread_square_few_weights, T.spread_tall_tiles_up_to_rows, T.spread_wide_tiles_read)
 
 
 @functools.lru_cache(maxsize=4096)
-def _spread_plan(rows, out_features, in_features, up_to_rows, square_tiles, square_tiles_few_weights, square_few_weights):
+def _spread_plan(rows, out_features, in_features, up_to_rows, square_tiles, square_tiles_few_weights, square_few_weights, tall_up_to_rows,
+                 wide_read):
     best = spread_dealing(rows, out_features, in_features)
     if best is None or rows <= up_to_rows:
         return best and best[1]
@@ -537,7 +538,9 @@ def _spread_plan(rows, out_features, in_features, up_to_rows, square_tiles, squa
         if of_w == of_a == 128 and ((tiles >= square_tiles_few_weights and out_features * in_features <= square_few_weights)
                                     or (tiles >= square_tiles and best[1][1] > 2)):
             return None
-        if best[0] > of_w + of_a:
+        if (of_w, of_a) == (256, 128) and rows > tall_up_to_rows:
+            return None
+        if best[0] > (of_w + of_a) * (wide_read if number == 7 else 1.0):
             return None
     return best[1]
 

@@ -296,6 +296,8 @@ def test_gated_products_dealt_evenly():
     assert plan(384, 17920, 1536) == (4, 2, 128) and plan(64, 37888, 3584) == (2, 1, 256) and plan(64, 59136, 8192) == (6, 1, 512)
     assert plan(16, 17920, 1536) is None and plan(513, 17920, 1536) is None and plan(65, 59136, 8192) is None
     assert plan(256, 22016, 2048) is None and plan(300, 10496, 3584) is None and plan(225, 9728, 896) is None and plan(256, 9088, 2880) == (7, 2, 128)
+    assert plan(218, 22912, 1152) is None and plan(220, 24576, 7360) is None and plan(200, 18944, 1152) and plan(301, 8448, 2240) is None
+    assert plan(385, 14336, 2048) is None and plan(512, 16384, 2048) is None and plan(384, 14336, 2048) and plan(512, 17920, 1536)
     assert faster("library", 225, 9728, 896) and faster("library", 300, 10496, 3584)      # by the other tiles
     assert plan(150, 27648, 5120) == (8, 1, 256) and plan(225, 12288, 2560) and plan(150, 3712, 2048)
     assert faster("skinny", 17, 17920, 1536) and not faster("skinny", 17, 9728, 896) and faster("skinny", 49, 3072, 2048) and not faster("skinny", 49, 2688, 512)
