@@ -79,7 +79,8 @@ def spread_parts(plan, rows, out_features, in_features):
     if (not T.library_from_rows < rows <= T.spread_parts_most_rows or out_features % 16 or in_features % 64
             or in_features < T.spread_parts_min_in_features):
         return None
-    if plan[0] == "skinny" and rows <= T.spread_parts_beyond_rows:
+    if plan[0] == "skinny" and (rows <= T.spread_parts_beyond_rows or (in_features % 128 and out_features < T.spread_parts_half_min_out_features
+                                                                       and in_features < T.spread_parts_half_min_in_features)):
         return None
     if rows > T.spread_parts_many_rows and in_features <= T.spread_parts_short_k:
         return None
@@ -99,6 +100,14 @@ def spread_parts(plan, rows, out_features, in_features):
         tile = 64 if rows <= SKINNY_MAX_ROWS else 128
         other = _parts_estimate(rows, out_features, in_features, 64 + tile, plan[2])
         if best[0] > T.spread_parts_share_of_tiles * other or (rows <= T.spread_parts_few_rows and best[1][2] == plan[2]):
+            return None
+        dealing, parts = _dealing(best[1][1]), best[1][2]
+        tile_rows, own, room_a, room_w, slab = ops.spread_share(dealing, rows, out_features)
+        if slab == 64 and rows <= SKINNY_MAX_ROWS and parts <= 4 and tile_rows * own <= T.spread_parts_least_full * room_a * room_w:
+            return None
+        if slab == 64 and rows > T.spread_parts_few_rows and room_a == 128 and (
+                own <= T.spread_parts_least_columns * room_w and parts <= 4
+                or own <= T.spread_parts_least_columns_row_tiles * room_w and dealing[1] > 2):
             return None
     return best[1]
 

@@ -351,6 +351,10 @@ def test_few_columns_dealt_evenly():
     assert parts(96, 1536, 1536)[2] == 2 and parts(64, 2048, 2048) and parts(17, 5120, 13824)
     assert not any(parts(rows, n, k) for rows, n, k in ((16, 1536, 8960), (48, 1536, 1536), (64, 2048, 11008), (91, 3584, 3584), (250, 4096, 14336),
                                                          (300, 2304, 1536), (385, 1536, 8960), (128, 1536, 960), (64, 1528, 8960)))
+    # tiles of 128 columns that own few of them, where slabs of 128 do not divide a part
+    assert not any(parts(rows, n, k) for rows, n, k in ((64, 1664, 1984), (50, 640, 1856), (31, 1152, 3904), (63, 512, 3904), (170, 1984, 5760), (203, 704, 16512),
+                                                         (227, 1280, 5056), (149, 2048, 5312)))
+    assert all(parts(rows, n, k) for rows, n, k in ((64, 1664, 2112), (64, 2048, 1984), (64, 1664, 1920), (31, 3072, 6208), (170, 1984, 12224), (207, 3136, 9024), (24, 2688, 4096)))
     key = ("linear", 128, 1536, 8960, False, False, True, False, True)
     assert L.linear_candidates(key)[:2] == [("tiles", L._dealing_number(14, 1, 32), 8), L.linear_plan(*key[1:])]
 
