@@ -426,7 +426,9 @@ __device__ __forceinline__ uint32_t gt_round2(float a, float b) {
   return __builtin_bit_cast(uint32_t, r);
 }
 
-template <int NI, int MJ, int WN, int WM, int WK, int NBUF>
+// EXPF: products that the kernel streaming the weights would take otherwise (up to 32 rows, or 64 of fewer than 4,096 rows of W) keep its
+// activation: 0.3 to 0.4 us of 6 to 16 there; with more rows, whose other tiles have the hardware's too, it would be 0.4 to 2.7.
+template <bool EXPF, int NI, int MJ, int WN, int WM, int WK, int NBUF>
 __global__ __launch_bounds__(64 * WN * WM * WK, 1) void gemm_spread_gated_kernel(
     bf16_t* __restrict__ C, int64_t ldc, const bf16_t* __restrict__ A, int64_t lda, const bf16_t* __restrict__ W, int M, int cols,
     int K, int m_tiles, int tile_rows, int groups, GateAct act) {
@@ -442,21 +444,14 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 1) void gemm_spread_gated_kernel
   const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave % WM, wn = wave / WM % WN, wk = wave / (WM * WN);
   bf16_t* tile = reinterpret_cast<bf16_t*>(lds);       // through LDS, so that a row's columns leave side by side
-  auto results = [&](auto with_expf) {
-    constexpr bool EXPF = decltype(with_expf)::value;
 #pragma unroll
-    for (int t = 0; t < NI * MJ; ++t)
-      if (WK == 1 || t % 2 == wk) {
-        const int i = t / MJ, j = t % MJ;
-        const SpreadPairs v(acc[i][j]);
-        *reinterpret_cast<uint32_t*>(tile + ((wm * MJ + j) * 16 + c) * S::PITCH + (wn * NI + i) * 8 + 2 * g) =
-            gt_round2(gt_act<EXPF>(v.first[0], v.second[0], act), gt_act<EXPF>(v.first[1], v.second[1], act));
-      }
-  };
-  // Products that the kernel streaming the weights would take otherwise (up to 32 rows, or 64 of fewer than 4,096 rows of W) keep its
-  // activation: 0.3 to 0.4 us of 6 to 16 there; with more rows, whose other tiles have the hardware's too, it would be 0.4 to 2.7.
-  if (S::TM == 64 && (M <= 32 || cols < 2048)) results(std::true_type());
-  else results(std::false_type());
+  for (int t = 0; t < NI * MJ; ++t)
+    if (WK == 1 || t % 2 == wk) {
+      const int i = t / MJ, j = t % MJ;
+      const SpreadPairs v(acc[i][j]);
+      *reinterpret_cast<uint32_t*>(tile + ((wm * MJ + j) * 16 + c) * S::PITCH + (wn * NI + i) * 8 + 2 * g) =
+          gt_round2(gt_act<EXPF>(v.first[0], v.second[0], act), gt_act<EXPF>(v.first[1], v.second[1], act));
+    }
   __syncthreads();
   for (int idx = threadIdx.x; idx < S::TM * 2 * S::NB; idx += 64 * S::WAVES) {
     const int m = idx / (2 * S::NB), q = idx % (2 * S::NB);
@@ -635,9 +630,12 @@ extern "C" int ga_gemm_spread_gated(void* C, int64_t ldc, const void* A, int64_t
   case n: {                                                                                                                              \
     if (!spread_fits<__VA_ARGS__>(M, cols / 4, K / 64, m_tiles, groups, tile_rows)) return -7;                                           \
     constexpr int bytes = SpreadTile<__VA_ARGS__>::LDS;                                                                                  \
-    if (const int raised = spread_room(gemm_spread_gated_kernel<__VA_ARGS__>, bytes)) return raised;                                     \
-    hipLaunchKernelGGL((gemm_spread_gated_kernel<__VA_ARGS__>), GA_SPREAD_GRID(1), dim3(64 * SpreadTile<__VA_ARGS__>::WAVES), bytes,     \
-                       stream, (bf16_t*)C, ldc, (const bf16_t*)A, lda, (const bf16_t*)W, M, cols, K, m_tiles, tile_rows, groups, act);   \
+    constexpr bool few = SpreadTile<__VA_ARGS__>::TM == 64;                                                                              \
+    const auto kernel = few && (M <= 32 || cols < 2048) ? gemm_spread_gated_kernel<few, __VA_ARGS__>                                     \
+                                                        : gemm_spread_gated_kernel<false, __VA_ARGS__>;                                  \
+    if (const int raised = spread_room(kernel, bytes)) return raised;                                                                    \
+    hipLaunchKernelGGL(kernel, GA_SPREAD_GRID(1), dim3(64 * SpreadTile<__VA_ARGS__>::WAVES), bytes, stream, (bf16_t*)C, ldc,             \
+                       (const bf16_t*)A, lda, (const bf16_t*)W, M, cols, K, m_tiles, tile_rows, groups, act);                            \
     return GA_CHECK_LAUNCH();                                                                                                            \
   }
     GA_SPREAD_GATED(CASE)
