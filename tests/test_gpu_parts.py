@@ -143,9 +143,11 @@ def test_attention_part_in_portions(dtype, tol, window):
 
 @pytest.mark.parametrize("T", [47, 48, 64, 65])
 @pytest.mark.parametrize("hd,rd", [(32, 16), (48, 48)])
-def test_attention_part_whose_rotation_the_fused_kernel_does_not_take(T, hd, rd):
-    """One prompt of the rows that take the projection in parts of K (48 to 64), and of a row fewer and more, against the plain block."""
-    from ginfer_amd.parts import lookup, KVView, StepContext
+def test_attention_part_whose_rotation_the_fused_kernel_does_not_take(T, hd, rd, monkeypatch):
+    """One prompt of the rows that take the projection in parts of K (48 to 64), and of a row fewer and more, against the plain block: by
+    the way that forward takes, and by the other ways where heads that are rotated whole would be dealt evenly."""
+    from ginfer_amd.kernels import ops
+    from ginfer_amd.parts import attention, lookup, KVView, StepContext
     from ginfer_amd.parts.attention import _projection_way
     Hd, nh, nkv, ps, dtype = 1152, 4, 2, 8, torch.bfloat16
     pos = lookup("position", "rope_neox")(theta=1e4, rotary_dim=rd, max_positions=96, device=dev())
@@ -154,17 +156,25 @@ def test_attention_part_whose_rotation_the_fused_kernel_does_not_take(T, hd, rd)
     w = {n: rnd(s.shape, i, 0.05).to(dtype) for i, (n, s) in enumerate(part.weight_specs().items())}
     part.bind_weights({n: t.to(dev()) for n, t in w.items()})
     x = rnd((T, Hd), 20).to(dtype)
-    assert _projection_way(x.to(dev()), part.w_qkv, hd, rd) == (("parts", 3) if 48 <= T <= 64 else ("library",))
+    other = ("parts", 3) if 48 <= T <= 64 else ("library",)
+    assert _projection_way(x.to(dev()), part.w_qkv, hd, rd) == other
     sin, cos = pm.rope_tables(1e4, rd, 96)
     ref, _ = pm.attention_block(x.double(), {"p." + n: t.double() for n, t in w.items()}, "p",
                                 dict(num_attention_heads=nh, num_key_value_heads=nkv, head_dim=hd), list(range(T)), sin, cos, None)
-    kp = torch.full((9, nkv, ps, hd), float("nan"), dtype=dtype, device=dev())
-    vp = torch.full((9, nkv, hd, ps), float("nan"), dtype=dtype, device=dev())
     i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev())
-    view = KVView(kp, vp, i32([list(range(9))]), torch.arange(T, device=dev()), ps, True)
-    step = StepContext(token_ids=None, positions=torch.arange(T, dtype=torch.int32, device=dev()), token_entry=i32([0] * T), cu_tokens=i32([0, T]),
-                       q_start=i32([0]), logit_rows=None, num_tokens=T, num_entries=1, host_q_start=[0], host_q_len=[T], caches=[view], extra={})
-    close(part.forward(x.to(dev()), step, view), ref, dict(PART_DTYPES)[dtype])
+    ran, project = [], attention.project
+    monkeypatch.setattr(attention, "project", lambda way, *rest: ran.append(way) or project(way, *rest))
+    for dealt in (True, False):
+        if not dealt:
+            monkeypatch.setattr(ops, "qkv_spread_plan", lambda *operands: None)
+        kp = torch.full((9, nkv, ps, hd), float("nan"), dtype=dtype, device=dev())
+        vp = torch.full((9, nkv, hd, ps), float("nan"), dtype=dtype, device=dev())
+        view = KVView(kp, vp, i32([list(range(9))]), torch.arange(T, device=dev()), ps, True)
+        step = StepContext(token_ids=None, positions=torch.arange(T, dtype=torch.int32, device=dev()), token_entry=i32([0] * T),
+                           cu_tokens=i32([0, T]), q_start=i32([0]), logit_rows=None, num_tokens=T, num_entries=1, host_q_start=[0],
+                           host_q_len=[T], caches=[view], extra={})
+        close(part.forward(x.to(dev()), step, view), ref, dict(PART_DTYPES)[dtype])
+    assert ran[0][0] == ("spread" if rd == hd else other[0]) and ran[1] == other
 
 
 @pytest.mark.parametrize("T", [1, 5, 16, 17])
