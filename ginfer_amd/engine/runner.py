@@ -599,9 +599,12 @@ def padded_rows(rows):
     """Token rows of the recorded step that `rows` of them are laid into: 64, 128, 256, 384, 512 and on by doubling, few sizes, so that
     few recorded steps serve many.  384 stands between because a step of 512 takes 8 to 16 % longer for the rows it does not have:
     290 rows beside each other's arrivals 3,919 -> 3,602 us (1.5B shape), one prompt of 300 3,341 -> 2,988, in 32-bit 14,560 -> 12,280.
-    192 gains nothing (161 rows 2,571 and 2,599 us).  320 is not among them: the 1.5B shape's bfloat16 steps lose by it (290 rows 3,602 ->
-    3,925, one prompt of 300 2,988 -> 3,371, for the library's products), though others would gain (300 rows in 32-bit 12,280 -> 10,297, the
-    puguzen shape 1,090 -> 1,019); 448 was timed at no number of rows that it holds."""
+    These lines were drawn when bfloat16 products of 129 to 512 rows were the library's, whose time hardly fell with the rows.  The package's
+    now fall with them, so that sizes between would gain: a step of us now -> as one of 192, 163 rows in ten prompts of the
+    1.5B shape 2,381 -> 2,234, in 32-bit 8,072 -> 7,682, puguzen 759 -> 677, titozen 780 -> 730; as one of 320, 290 rows beside each other's
+    arrivals 3,427 -> 3,365, one prompt of 290 2,804 -> 2,803, in 32-bit 12,590 -> 10,603, puguzen 1,017 -> 985, titozen 1,006 -> 953; as one of
+    448, one prompt of 446 3,194 -> 3,157, in 32-bit 14,750 -> 13,900, puguzen 1,228 -> 1,216.  But the 7B shape, whose steps of 129 to 196 rows run
+    unrecorded at the rows that they have, would be laid into 192: 140 rows 4,690 -> 4,985, 163 4,853 -> 5,000, 190 4,957 -> 4,989."""
     size = 64
     while size < rows:
         size = {256: 384, 384: 512}.get(size, 2 * size)
