@@ -442,7 +442,8 @@ GATED_TILINGS = ((128, 64), (128, 256), (256, 128), (256, 256), (128, 128))     
 
 
 def gated_tiling(rows, out_features):
-    """The tiles of the gated product of `rows` rows by `out_features` rows of W: its number in GATED_TILINGS.  Few rows: the
+    """The tiles of the gated product of `rows` rows by `out_features` rows of W, where it is not dealt evenly (spread_plan: nearly all
+    up to 512 rows, and all of 17 to 64 of up to 81,920 rows of W): its number in GATED_TILINGS.  Few rows: the
     smallest that hold them and keep to one round of the chip's 256 compute units; more: the fastest of what was measured."""
     columns = -(-out_features // 128)
     if rows <= 64 and columns <= 256:
@@ -461,17 +462,19 @@ GATED_WIDE_TILINGS = {6: (192, 64), 7: (192, 128), 8: (192, 256)}
 
 def gated_wide_tiling(rows, out_features, in_features):
     """The tiles of 192 rows of W that the gated product takes in place of gated_tiling's, or None: where they fill one round of the
-    chip's 256 compute units, or few, better.  us beside the tiles that they replace, or beside the library where those are not
-    taken, as replays of a graph over several layers' weights: 37,888 rows of W, K 3,584: 64 rows 62.2 -> 54.6 (198 workgroups for 148),
-    128 rows 67.8 -> 61.1; 28,672 rows, K 4,096 the other way, 53.0 -> 59.6 (150 for 224).  17,920 rows, K 1,536: 161 rows 27.4 -> 24.4
-    (188 workgroups for 140), 256 rows 29.1 -> 26.5; 22,016 rows, K 2,048: 256 rows 36.9 -> 35.6 (230 for 172).  A round of 192 x 256 takes
-    0.82 (K 3,584) to 0.89 (K 1,536) of one of 256 x 256: beyond 1,024 rows it stands where it makes that up in rounds, nearly full:
-    17,920 rows of W: 1,025 rows 79.8 -> 77.2, 1,280 86.9 -> 82.0, 2,048 129 -> 119 (752 tiles in 3 rounds; 560 of 256 x 256 in 3), but 4,096 rows
-    226 -> 238 (6 rounds for 5); 22,016: 1,536 rows 152 -> 144, but 2,048 175 -> 188 (4 for 3).  With a longer K the library
-    has most of that many rows: 28,672, K 4,096 1,025 rows 227 -> 251; 12,288, K 3,072 2,048 rows 138 -> 137.  385 to 512 rows in one nearly full
-    round: up to a K of 4,096 (22,016 rows of W at 400 rows: K 1,024 42.4 -> 30.4, 2,048 61.5 -> 51.9, 3,072 79.9 -> 74.2 (24,576 rows of W),
-    4,096 94.6 -> 91.0; the other way 21,504, K 5,120 103.9 -> 107.6, 24,576, K 8,192 172 -> 179, at 500 rows 178 -> 201), and at 512, where the
-    library's transposed product fits the rows, to 2,560 (65.7 -> 65.0; 24,576, K 3,072 75.6 -> 77.0, K 4,096 94.5 -> 98.6)."""
+    chip's 256 compute units, or few, better; up to 512 rows what is dealt evenly stands before both (spread_plan), so that up to 64 rows
+    only a product of up to 16 runs in tiles of 64 rows of A.  The lines up to 1,024 rows of A were drawn with four wavefronts to a tile of
+    192 x 128 or 192 x 256, which have eight now.  us beside the tiles that they replace, as replays of a graph over several layers'
+    weights, drawn with four: 17,920 rows of W, K 1,536: 161 rows 27.4 -> 24.4 (188 workgroups for 140), 256 rows 29.1 -> 26.5; 22,016 rows, K 2,048:
+    256 rows 36.9 -> 35.6 (230 for 172).  With eight, against those of 256 x 256: a round of 192 x 256 takes 0.86 (17,920 rows of W, K 1,536 at 1,025
+    rows) of one of theirs, so beyond 1,024 rows it stands where it makes that up in rounds, nearly full: 17,920 rows of W: 1,025 rows 83.4 -> 72.0, 1,280
+    89.1 -> 79.1, 2,048 127 -> 115 (752 tiles in 3 rounds; 560 of 256 x 256 in 3), but 4,096 rows 223 -> 232 (6 rounds for 5); 22,016: 1,536 rows
+    160 -> 143, but 2,048 176 -> 190 (4 for 3).  Against the library: 12,288, K 3,072 2,048 rows 153 -> 141; the longer K that is left to it
+    was behind with four (28,672, K 4,096 1,025 rows 227 -> 251) and is ahead with eight (275 -> 261).  385 to 512 rows in one nearly
+    full round, against the library: up to a K of 4,096 (22,016 rows of W at 400 rows: K 1,024 44.6 -> 28.4, 2,048 60.6 -> 49.5; 24,576 rows: 3,072
+    80.9 -> 74.1, 4,096 98.7 -> 96.7; the other way 21,504, K 5,120 104.5 -> 107.9, 24,576, K 8,192 175 -> 181, at 500 rows 185 -> 186), and at 512, where
+    the library's transposed product fits the rows, to 2,560 (68.5 -> 63.1; beyond it was behind with four wavefronts, 24,576, K 3,072 75.6 -> 77.0, and
+    is ahead with eight, 79.6 -> 76.2, K 4,096 102.3 -> 98.5)."""
     wide, rounds = -(-out_features // 192), lambda of_w, of_a: -(-(-(-out_features // of_w) * -(-rows // of_a)) // 256)
     if rows <= 128:
         return (6 if rows <= 64 else 7) if rounds(128, 128) > 1 and wide <= 256 else None
