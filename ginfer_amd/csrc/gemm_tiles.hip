@@ -239,8 +239,9 @@ static int gt_check(const void* C, const void* A, int64_t lda, const void* W, in
 // takes in the same bytes, whatever the sizes; a tile has room for NB blocks of 16 rows of W and TM rows of A, and what of that
 // it does not own is not loaded.  Eight wavefronts, WN x WM of the tile's blocks of v_mfma_f32_16x16x32_bf16 and WK of a slab's K.
 //
-// What bounds it: loads return in order, so a compute unit's stream of lines, some from its L2 and some from memory, goes at the
-// pace of the latter: 45 to 50 GB/s a compute unit in every mixture, 110 from L2 alone.  So the bytes a compute unit takes in
+// What bounds it: few rows, the weights' way from memory (64 rows by 17,920 rows of W, K 1,536: 55 MB in 10.6 us, 5.2 TB/s, where a
+// compute unit takes in 39 GB/s).  From about 128 rows on, where most of what a unit takes in comes from its L2: loads return in order, so its stream
+// of lines goes at the pace of those from memory, 45 to 50 GB/s a unit (110 with none from memory).  Either way the bytes a compute unit takes in
 // are what counts: all 256 at work with a few rows fewer each, not the 188 of tiles of 192 x 128 (256 rows by 17,920 rows of W, K 1,536:
 // the loads alone 20.8 us there, 18.0 here, of 26.0 and 22.9 whole).  W is asked for as memory that is read once (nt), so that A
 // stays in the L2s: 18.1 -> 17.4 us with a line of W wanted twice, 11.5 -> 10.6 with it wanted once (64 rows).  Slabs of 128 elements
@@ -590,7 +591,8 @@ static int spread_check(int M, int m_tiles, int groups) {
 // 291, 2,048 rows 552 -> 464; 19,456 rows, K 2,560: 128 rows 46.0 -> 44.0 (128 x 256 tiles 49.1), 384 rows 64.0 -> 57.8 (all with four
 // wavefronts to a tile; what eight give stands above).
 // Tiles of 192 rows of W stand beside the others (6 to 8) where those leave the chip's rounds emptier (gated_wide_tiling in
-// kernels/ops.py has the rule and the figures).
+// kernels/ops.py has the rule and the figures).  17 to 64 rows of up to 81,920 rows of W are dealt evenly (below), so that 0 and 6 are left to calls of up
+// to 16 rows, which a step's products make with the kernel that streams the weights.
 extern "C" int ga_gemm_tiles_gated(void* C, int64_t ldc, const void* A, int64_t lda, const void* W, int M, int cols, int K, int kind,
                                    float limit, float alpha, float shift, int tiling, hipStream_t stream) {
   if (M <= 0) return 0;
