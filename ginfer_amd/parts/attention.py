@@ -34,6 +34,8 @@ def _projection_in_parts(rows, in_features, out_features):
 
 def _projection_way(x, w_qkv, head_dim, rotary_dim):
     """("fused",), ("parts", n) or ("library",): how rows x become q, k and v where their product is not dealt evenly to the chip."""
+    if x.shape[0] > ops.SKINNY_MAX_ROWS:        # neither of the others takes them; such steps are launched kernel by kernel
+        return ("library",)
     fused_ok = ops.qkv_rope_skinny_supported(x, w_qkv, head_dim, rotary_dim)
     return _other_way(x.shape[0], x.shape[1], w_qkv.shape[0], fused_ok, not fused_ok and _parts_supported(x, w_qkv, head_dim, rotary_dim))
 

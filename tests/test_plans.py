@@ -168,6 +168,24 @@ def test_the_projection_is_one_plan_of_several(rows, K, hd, rd, monkeypatch):
             assert ran[-1] == way
 
 
+@pytest.mark.parametrize("rows", [65, 512, 513, 2048])
+@pytest.mark.parametrize("K,hd,rd", [(1536, 128, 128), (1152, 48, 48), (1152, 64, 32), (1096, 64, 64)])
+def test_projections_of_more_rows_than_the_streaming_kernels_take(rows, K, hd, rd, monkeypatch):
+    """Steps launched kernel by kernel wait for the host: such rows go to the library without a look at the other kernels' operands, which
+    would not take them whatever they are."""
+    from ginfer_amd.kernels import ops
+    from ginfer_amd.parts import attention
+    x, w = torch.empty((rows, K + 16), dtype=torch.bfloat16), torch.empty((8 * hd, K), dtype=torch.bfloat16)
+    operands = [(x[:, :K], w), (x[:, 8:K + 8], w), (x[:, 1:K + 1], w), (x[:, :K].float(), w.float()), (x[:, :K], w[:, ::1].t().contiguous().t())]
+    for a, b in operands:
+        assert not ops.gemm_skinny_supported(a, b) and not ops.qkv_rope_skinny_supported(a, b, hd, rd)
+        assert not attention._parts_supported(a, b, hd, rd)
+    asked = []
+    for name in ("gemm_skinny_supported", "qkv_rope_skinny_supported"):
+        monkeypatch.setattr(ops, name, lambda *args: asked.append(args))
+    assert all(attention._projection_way(a, b, hd, rd) == ("library",) for a, b in operands) and not asked
+
+
 def test_the_projection_is_dealt_evenly_where_that_is_faster():
     """Sizes on both sides of the lines, as measured; the tuner starts from what runs there too."""
     from ginfer_amd.kernels import autotune
