@@ -12,64 +12,11 @@
 //   exp(-softplus(-z) / tau), all in 32-bit.
 // head_norm_gate (times out_scale; weight: shared by the heads, or every head its own): out[t, h, :] = o[t, h, :] / sqrt(mean(o[t, h, :]^2) + eps) (* weight[:]) (* silu(gate[t, h, :]), or * sigmoid of it).
 // silu_inputs: the recurrence reads silu(q), silu(k), silu(v) in place of the projection's numbers.
+#include "decay_rows.h"
 #include "decay_walk.h"
 #include "ginfer_amd.h"
 
 #define DS_THREADS 256
-
-// q, k and v as the recurrence reads them: the projection's numbers or their silu, turned by position, scaled
-template <bool ROT>
-struct DecayRows {
-  static constexpr bool K_OF_A = false;
-  struct Fixed {};
-  __device__ __forceinline__ Fixed fixed(int) const { return {}; }
-  struct Plain { float q, k, a; };
-  struct Turned { float q, k, a, q2, k2, c, s; };
-  typedef typename std::conditional<ROT, Turned, Plain>::type Raw;
-  const float *q, *k, *v;              // the entry's first token, the head's first channel or column
-  const float* decay;                  // the same of [tokens, heads * dim]; or one number, and both steps are 0
-  const float *cos_t, *sin_t;          // the first token's position
-  int64_t stride;
-  int decay_token, decay_channel, half;
-  float q_scale, k_scale;
-  bool acts;                           // whether finish and finish_v apply the silu: asked once a tile, not per element
-  template <bool ACT>
-  __device__ __forceinline__ float act(float z) const { return ACT ? z / (1.0f + expf(-z)) : z; }
-  __device__ __forceinline__ void load(Raw& x, int start, int t, int i) const {
-    const float *qp = q + start * stride, *kp = k + start * stride;
-    const uint32_t row = (uint32_t)t * (uint32_t)stride;
-    x.q = qp[row + i];
-    x.k = kp[row + i];
-    x.a = (decay + (int64_t)start * decay_token)[(uint32_t)(t * decay_token + i * decay_channel)];
-    if constexpr (ROT) {               // (a channel that is not turned reads what channel 0 reads, and drops it)
-      const int at = i < 2 * half ? i : 0, f = at < half ? at : at - half, other = at < half ? at + half : at - half;
-      x.c = (cos_t + (int64_t)start * half)[(uint32_t)(t * half + f)];
-      x.s = (sin_t + (int64_t)start * half)[(uint32_t)(t * half + f)];
-      x.q2 = qp[row + other];
-      x.k2 = kp[row + other];
-    }
-  }
-  template <bool ACT>
-  __device__ __forceinline__ void finish(const Raw& x, const Fixed&, int i, float& qv, float& kv, float& a) const {
-    qv = act<ACT>(x.q);
-    kv = act<ACT>(x.k);
-    if constexpr (ROT) {
-      if (i < 2 * half) {              // the pair (lo, hi) becomes (lo c - hi s, hi c + lo s)
-        const float qo = act<ACT>(x.q2), ko = act<ACT>(x.k2);
-        qv = i < half ? qv * x.c - qo * x.s : qv * x.c + qo * x.s;
-        kv = i < half ? kv * x.c - ko * x.s : kv * x.c + ko * x.s;
-      }
-    }
-    qv *= q_scale;
-    kv *= k_scale;
-    a = x.a;
-  }
-  __device__ __forceinline__ float load_v(int start, int t, int c) const {
-    return (v + start * stride)[(uint32_t)t * (uint32_t)stride + c];
-  }
-  template <bool ACT>
-  __device__ __forceinline__ float finish_v(float x) const { return act<ACT>(x); }
-};
 
 // Measured on MI355X, the projection just written, us, before (16 columns a workgroup whose every wavefront brings, walks and adds
 // up, operands in single reads, three barriers a tile) -> now, a decay per channel and a constant one with rotation.  12 heads of
@@ -86,10 +33,10 @@ __global__ __launch_bounds__(dw_threads(COLS)) void decay_scan_kernel(
     int64_t stride, const float* __restrict__ decay, const float* __restrict__ head_decay, const float* __restrict__ cos_t,
     const float* __restrict__ sin_t, int rot_dims, float q_scale, float k_scale, float* __restrict__ state,
     const int64_t* __restrict__ slots, const int32_t* __restrict__ cu, const int32_t* __restrict__ q_start, int heads,
-    int dim, int vdim, int silu_inputs) {
+    int dim, int vdim, int silu_inputs, int most) {
   const int e = blockIdx.x, h = blockIdx.y;
   const int first = cu[e], n = cu[e + 1] - first;
-  if (n <= 0) return;
+  if (n <= 0 || n > most) return;
   const int start = q_start[e];
   DecayRows<ROT> rows;
   rows.q = q + first * stride + h * dim;
@@ -325,7 +272,7 @@ __global__ __launch_bounds__(DS_THREADS) void wide_norm_gate_rows_kernel(T* __re
 
 extern "C" int ga_decay_scan(void* out, const void* q, const void* k, const void* v, int64_t stride, const void* decay,
                              const void* head_decay, const void* cos_t, const void* sin_t, int rot_dims, float q_scale,
-                             float k_scale, void* state, const void* slots, const void* cu, const void* q_start, int way, int entries,
+                             float k_scale, void* state, const void* slots, const void* cu, const void* q_start, int way, int most, int entries,
                              int heads, int dim, int vdim, int silu_inputs, hipStream_t stream) {
   if (entries <= 0) return 0;
   if (heads <= 0 || dim <= 0 || vdim <= 0 || dim > 16 * DW_SLICES || (way != 1 && way != 8 && way != 16)) return -1;
@@ -337,7 +284,7 @@ extern "C" int ga_decay_scan(void* out, const void* q, const void* k, const void
                                  stream, (float*)out, (const float*)q, (const float*)k, (const float*)v, stride, (const float*)decay,   \
                                  (const float*)head_decay, (const float*)cos_t, (const float*)sin_t, rot_dims, q_scale, k_scale,        \
                                  (float*)state, (const int64_t*)slots, (const int32_t*)cu, (const int32_t*)q_start, heads, dim, vdim,   \
-                                 silu_inputs)
+                                 silu_inputs, most)
 #define GR(R, C, T) do { if (rot_dims > 0) GO(R, C, T, true); else GO(R, C, T, false); } while (0)
   DW_WAY(way, rows, dw_many(entries, heads, vdim), GR);
 #undef GR

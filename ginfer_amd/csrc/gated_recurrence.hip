@@ -7,40 +7,11 @@
 // order (decay_walk.h): a token's result does not depend on how the request's tokens were cut into steps, nor on what else
 // is in the batch.
 // A second kernel norms each head's output over its value columns (RMS, with a weight per column).
+#include "decay_rows.h"
 #include "decay_walk.h"
 #include "ginfer_amd.h"
 
 #define GR_THREADS 256
-
-__device__ __forceinline__ float gr_sigmoid(float z) { return 1.0f / (1.0f + expf(-z)); }
-
-struct ForgetRows {
-  struct Raw { float q, f; };
-  struct Fixed { float bias, lower; };
-  const float *proj, *v;               // the entry's first token, the head's first channel or column
-  const float *bias, *lower;           // the head's
-  int64_t stride;
-  int hd;
-  static constexpr bool acts = false, K_OF_A = true;
-  __device__ __forceinline__ Fixed fixed(int i) const { return {bias[i], lower[i]}; }
-  __device__ __forceinline__ void load(Raw& x, int start, int t, int i) const {
-    const float* p = proj + start * stride;
-    const uint32_t at = (uint32_t)t * (uint32_t)stride + i;
-    x.q = p[at];
-    x.f = p[at + hd];
-  }
-  template <bool>
-  __device__ __forceinline__ void finish(const Raw& x, const Fixed& c, int i, float& q, float& k, float& f) const {
-    q = x.q * gr_sigmoid(x.q);
-    f = c.lower + (1.0f - c.lower) * gr_sigmoid(x.f + c.bias);
-    k = 1.0f - f;
-  }
-  __device__ __forceinline__ float load_v(int start, int t, int c) const {
-    return (v + start * stride)[(uint32_t)t * (uint32_t)stride + c];
-  }
-  template <bool>
-  __device__ __forceinline__ float finish_v(float x) const { return x; }
-};
 
 // Measured on MI355X, the caches emptied before, us, before the walk of decay_walk.h -> now.  12 heads of 64 x 128: 2,048 tokens of
 // one request 534 -> 181; five entries of 918 262 -> 183; 495 tokens beside 16 single ones 136 -> 64; 64 entries of 33 79 -> 65,
@@ -54,10 +25,11 @@ __global__ __launch_bounds__(dw_threads(COLS)) void hgrn2_scan_kernel(float* __r
                                                                        int64_t proj_stride, const float* __restrict__ f_bias,
                                                                        const float* __restrict__ lower, float* __restrict__ state,
                                                                        const int64_t* __restrict__ slots, const int32_t* __restrict__ cu,
-                                                                       const int32_t* __restrict__ q_start, int heads, int dim, int vdim) {
+                                                                       const int32_t* __restrict__ q_start, int heads, int dim, int vdim,
+                                                                       int most) {
   const int e = blockIdx.x, h = blockIdx.y;
   const int first = cu[e], n = cu[e + 1] - first;
-  if (n <= 0) return;
+  if (n <= 0 || n > most) return;
   ForgetRows rows;
   rows.proj = proj + first * proj_stride + h * dim;
   rows.v = proj + first * proj_stride + 2 * heads * dim + h * vdim;
@@ -86,7 +58,7 @@ __global__ __launch_bounds__(GR_THREADS) void headwise_rmsnorm_kernel(T* __restr
 }
 
 extern "C" int ga_hgrn2_scan(void* out, const void* proj, int64_t proj_stride, const void* f_bias, const void* lower,
-                             void* state, const void* slots, const void* cu, const void* q_start, int way, int entries,
+                             void* state, const void* slots, const void* cu, const void* q_start, int way, int most, int entries,
                              int heads, int dim, int vdim, hipStream_t stream) {
   if (entries <= 0) return 0;
   if (heads <= 0 || dim <= 0 || vdim <= 0 || dim > 16 * DW_SLICES || (way != 1 && way != 8 && way != 16)) return -1;
@@ -94,7 +66,7 @@ extern "C" int ga_hgrn2_scan(void* out, const void* proj, int64_t proj_stride, c
   const int rows = (dim + DW_SLICES - 1) / DW_SLICES;
 #define GO(R, C, T) hipLaunchKernelGGL((hgrn2_scan_kernel<R, C, T>), dim3(entries, heads, (vdim + C - 1) / C), dim3(dw_threads(C)), 0, stream, \
                                        (float*)out, (const float*)proj, proj_stride, (const float*)f_bias, (const float*)lower,            \
-                                       (float*)state, (const int64_t*)slots, (const int32_t*)cu, (const int32_t*)q_start, heads, dim, vdim)
+                                       (float*)state, (const int64_t*)slots, (const int32_t*)cu, (const int32_t*)q_start, heads, dim, vdim, most)
   DW_WAY(way, rows, dw_many(entries, heads, vdim), GO);
 #undef GO
   return GA_CHECK_LAUNCH();

@@ -131,9 +131,9 @@ int ga_short_conv_update(void* state, const void* x, const void* slots, const vo
                          int width, int taps, int64_t x_stride, hipStream_t stream);
 
 // ---- gated_recurrence.hip: the HGRN2 recurrence.  proj float [tokens, 2 heads dim + heads vdim] (row stride given) holds
-// (q before its SiLU | forget-gate logits | v); way: how the tokens are walked (decay_walk.h), 1, 8 or 16; state float [slots, heads, dim, vdim]; out float [tokens, heads, vdim]
+// (q before its SiLU | forget-gate logits | v); way: how the tokens are walked (decay_walk.h), 1, 8 or 16; most: longer entries are left alone; state float [slots, heads, dim, vdim]; out float [tokens, heads, vdim]
 int ga_hgrn2_scan(void* out, const void* proj, int64_t proj_stride, const void* f_bias, const void* lower, void* state,
-                  const void* slots, const void* cu, const void* q_start, int way, int entries,
+                  const void* slots, const void* cu, const void* q_start, int way, int most, int entries,
                   int heads, int dim, int vdim, hipStream_t stream);
 // out [rows, vdim] (compute dtype) = x / sqrt(mean(x^2) + eps) * weight, x float [rows, vdim], weight float [vdim]
 int ga_headwise_rmsnorm(void* out, const void* x, const void* weight, int64_t rows, int vdim, float eps, int out_bf16,
@@ -318,11 +318,22 @@ int ga_layer_norm_add(void* residual, int num_tokens, const void* y1, int y1_f32
 // head.  q, k, v: 32-bit rows with a common stride; a from `decay` float [tokens, heads dim] or from `head_decay` float
 // [heads] (exactly one of them); q and k turned on their first rot_dims coordinates (pairs i, i + rot_dims / 2; tables float
 // [positions, rot_dims / 2]) and multiplied by q_scale, k_scale; state float [slots, heads, dim, vdim], zeros for a request
-// whose q_start is 0; way: how the tokens are walked (decay_walk.h), 1, 8 or 16; out float [tokens, heads, vdim]
+// whose q_start is 0; way: how the tokens are walked (decay_walk.h), 1, 8 or 16; most: longer entries are left alone; out float [tokens, heads, vdim]
 int ga_decay_scan(void* out, const void* q, const void* k, const void* v, int64_t stride, const void* decay,
                   const void* head_decay, const void* cos_t, const void* sin_t, int rot_dims, float q_scale, float k_scale,
-                  void* state, const void* slots, const void* cu, const void* q_start, int way, int entries,
+                  void* state, const void* slots, const void* cu, const void* q_start, int way, int most, int entries,
                   int heads, int dim, int vdim, int silu_inputs, hipStream_t stream);
+// ---- decay_chunk.hip: the same recurrence, and ga_hgrn2_scan's, in chunks of 64 tokens on the matrix cores (32-bit products), for up to 128 rows
+// of state; work: 8-byte aligned, of ga_decay_chunk_floats floats; entries of fewer than `least` tokens are left to the walk (whose `most` leaves
+// it longer ones); silu_inputs without a rotation only; the rest as ga_decay_scan and ga_hgrn2_scan have it
+int64_t ga_decay_chunk_floats(int tokens, int entries, int heads, int dim, int vdim);
+int ga_decay_chunk(void* out, void* work, const void* q, const void* k, const void* v, int64_t stride, const void* decay,
+                   const void* head_decay, const void* cos_t, const void* sin_t, int rot_dims, float q_scale, float k_scale,
+                   void* state, const void* slots, const void* cu, const void* q_start, int tokens, int entries, int heads,
+                   int dim, int vdim, int silu_inputs, int least, hipStream_t stream);
+int ga_hgrn2_chunk(void* out, void* work, const void* proj, int64_t stride, const void* f_bias, const void* lower, void* state,
+                   const void* slots, const void* cu, const void* q_start, int tokens, int entries, int heads, int dim,
+                   int vdim, int least, hipStream_t stream);
 // decay float [tokens, channels] = sigmoid(a2 low + bias)^(1 / tau); low: 32-bit rows of `rank` numbers with a stride; a2t:
 // a2 transposed, float [rank, channels]
 int ga_gla_decay(void* decay, const void* low, int64_t low_stride, const void* a2t, const void* bias, int tokens,

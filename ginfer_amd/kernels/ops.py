@@ -1292,9 +1292,50 @@ def _walk_of(step, tokens, entries, heads, dim, vdim, turned=False):
     return decay_walk_way(tokens, entries, max(lens, default=0) if known else 0, heads, dim, vdim, turned)
 
 
-def hgrn2_scan(proj, f_bias, lower, state, slots, step, heads, dim, vdim, update=True):
+DECAY_CHUNK_MAX_DIM = 128
+_ALL = 2 ** 31 - 1
+
+
+def decay_in_chunks(lens, dim):
+    """From how many tokens on the entries of a step go in chunks of 64 over the matrix cores (csrc/decay_chunk.hip), shorter ones being
+    walked; None: all are walked.  The walk's time is its longest entry's chain, the chunks' three launches and then the work, so the
+    longest entry decides, and with few rows of state, whose chunks are filled up to 64, how many more tokens there are.  us walked -> in
+    chunks, HGRN2 and retention: 12 heads of 64 x 128: one entry of 384 28 -> 28, 448 32 -> 29, 2,048 152 -> 45, 145 -> 45; 500 beside
+    32 single tokens 76 -> 43 (the walk of the single ones in it), ten of 450 134 -> 86; 16 of 64 x 64: one of 448 31 -> 26, twenty of
+    450 171 -> 147; 28 of 128 x 128: one of 320 89 -> 51, 2,048 526 -> 149, ten of 450 474 -> 387, but ten of 200 218 -> 255; 16 of 32 x
+    64: one of 700 34 -> 28, 2,048 113 -> 50, five of 918 113 -> 78, but one of 512 26 -> 29, ten of 450 74 -> 78, twenty 117 -> 141."""
+    T, longest = TUNING, max(lens, default=0)
+    few = dim <= T.decay_chunk_few_rows
+    since = T.decay_chunk_from_few_rows if few else T.decay_chunk_from if dim <= 64 else T.decay_chunk_from_many_rows
+    if dim > DECAY_CHUNK_MAX_DIM or longest < since or (few and sum(lens) > T.decay_chunk_few_rows_entries * longest):
+        return None
+    return T.decay_chunk_least
+
+
+def _decay_split(step, tokens, entries, heads, dim, vdim, chunked, turned=False):
+    """(way of the walk or None, its longest entry, tokens from which on an entry goes in chunks or None)"""
+    lens = getattr(step, "host_q_len", None)
+    known = lens is not None and len(lens) == entries and "static_plan" not in (getattr(step, "extra", None) or {})
+    least = decay_in_chunks(lens, dim) if chunked and known else None
+    if least is None:
+        return _walk_of(step, tokens, entries, heads, dim, vdim, turned), _ALL, None
+    short = [n for n in lens if 0 < n < least]
+    if not short:
+        return None, 0, least
+    return decay_walk_way(sum(short), len(short), max(short), heads, dim, vdim, turned), least - 1, least
+
+
+def _decay_chunk_work(tokens, entries, heads, dim, vdim, device):
+    lib = build.load("decay_chunk")
+    lib.ga_decay_chunk_floats.restype = ctypes.c_int64
+    floats = lib.ga_decay_chunk_floats(_i(tokens), _i(entries), _i(heads), _i(dim), _i(vdim))
+    return lib, torch.empty((floats,), dtype=torch.float32, device=device)
+
+
+def hgrn2_scan(proj, f_bias, lower, state, slots, step, heads, dim, vdim, update=True, chunked=False):
     """proj float32 [T, 2 heads dim + heads vdim]: (q before its SiLU | forget-gate logits | v); f_bias, lower float32
-    [heads dim]; state float32 [slots, heads, dim, vdim], advanced in place.  Returns float32 [T, heads, vdim]."""
+    [heads dim]; state float32 [slots, heads, dim, vdim], advanced in place.  Returns float32 [T, heads, vdim].
+    chunked: as decay_scan's."""
     _dev(proj, f_bias, lower, state, slots)
     T = proj.shape[0]
     _need(proj.dtype == torch.float32 and proj.dim() == 2 and proj.stride(1) == 1 and proj.shape[1] == 2 * heads * dim + heads * vdim,
@@ -1309,10 +1350,17 @@ def hgrn2_scan(proj, f_bias, lower, state, slots, step, heads, dim, vdim, update
     _need(update, "the recurrence always advances its state")
     proj = _near_rows(proj)
     out = torch.empty((T, heads, vdim), dtype=torch.float32, device=proj.device)
-    lib = build.load("gated_recurrence")
-    _check(lib.ga_hgrn2_scan(_ptr(out), _ptr(proj), _i64(proj.stride(0)), _ptr(f_bias), _ptr(lower), _ptr(state), _ptr(slots),
-                             _ptr(step.cu_tokens), _ptr(step.q_start), _i(_walk_of(step, T, E, heads, dim, vdim)), _i(E), _i(heads),
-                             _i(dim), _i(vdim), _stream()), "hgrn2_scan")
+    way, most, least = _decay_split(step, T, E, heads, dim, vdim, chunked)
+    if least is not None:
+        lib, work = _decay_chunk_work(T, E, heads, dim, vdim, proj.device)
+        _check(lib.ga_hgrn2_chunk(_ptr(out), _ptr(work), _ptr(proj), _i64(proj.stride(0)), _ptr(f_bias), _ptr(lower), _ptr(state),
+                                  _ptr(slots), _ptr(step.cu_tokens), _ptr(step.q_start), _i(T), _i(E), _i(heads), _i(dim), _i(vdim),
+                                  _i(least), _stream()), "hgrn2_chunk")
+    if way is not None:
+        lib = build.load("gated_recurrence")
+        _check(lib.ga_hgrn2_scan(_ptr(out), _ptr(proj), _i64(proj.stride(0)), _ptr(f_bias), _ptr(lower), _ptr(state), _ptr(slots),
+                                 _ptr(step.cu_tokens), _ptr(step.q_start), _i(way), _i(most), _i(E), _i(heads), _i(dim), _i(vdim),
+                                 _stream()), "hgrn2_scan")
     return out
 
 
@@ -1956,13 +2004,16 @@ def gla_decay(proj, low_start, a2t, bias, tau):
 
 
 def decay_scan(proj, q_start, k_start, v_start, state, slots, step, heads, dim, vdim, decay=None, head_decay=None, cos=None,
-               sin=None, q_scale=1.0, k_scale=1.0, silu_inputs=False):
+               sin=None, q_scale=1.0, k_scale=1.0, silu_inputs=False, chunked=False):
     """Linear attention with a decay as a recurrence over per-request state: S_t = diag(a_t) S_(t-1) + k_t v_t^T, o_t = S_t^T
     q_t per head.  q, k, v are column blocks of the float32 projection `proj` (starting at q_start, k_start, v_start; heads *
     dim, heads * dim, heads * vdim wide).  a: `decay` float32 [T, heads * dim], or `head_decay` float32 [heads].  cos, sin
     float32 [positions, r / 2]: q and k are turned on their first r coordinates (pairs i, i + r / 2) by the tokens' positions,
     then multiplied by q_scale and k_scale.  state float32 [slots, heads, dim, vdim] is advanced in place (zeros where an
-    entry's q_start is 0).  silu_inputs: the recurrence reads silu(q), silu(k) and silu(v).  Returns float32 [T, heads, vdim]."""
+    entry's q_start is 0).  silu_inputs: the recurrence reads silu(q), silu(k) and silu(v).  Returns float32 [T, heads, vdim].
+    Without `chunked` every token's sums are taken in an order of their own, so the bits do not depend on how the tokens were cut
+    into steps; chunked: long prompt portions may go in chunks of 64 tokens over the matrix cores (csrc/decay_chunk.hip; 32-bit operands
+    and sums; decay_in_chunks says which), and results differ by rounding with the cut."""
     _dev(proj, state, slots, decay, head_decay, cos, sin)
     T = proj.shape[0]
     if proj.dim() == 2 and proj.stride(1) == 1:
@@ -1987,11 +2038,19 @@ def decay_scan(proj, q_start, k_start, v_start, state, slots, step, heads, dim, 
           "state must be contiguous float32 [slots, %d, %d, %d]", heads, dim, vdim)
     E = _step_entries(step, slots)
     out = torch.empty((T, heads, vdim), dtype=torch.float32, device=proj.device)
-    lib = build.load("decay_scan")
-    _check(lib.ga_decay_scan(_ptr(out), _ptr(q), _ptr(k), _ptr(v), _i64(proj.stride(0)), _ptr(decay), _ptr(head_decay),
-                             _ptr(cos), _ptr(sin), _i(rot), _f(q_scale), _f(k_scale), _ptr(state), _ptr(slots),
-                             _ptr(step.cu_tokens), _ptr(step.q_start), _i(_walk_of(step, T, E, heads, dim, vdim, rot > 0)), _i(E), _i(heads),
-                             _i(dim), _i(vdim), _i(1 if silu_inputs else 0), _stream()), "decay_scan")
+    way, most, least = _decay_split(step, T, E, heads, dim, vdim, chunked and not (silu_inputs and rot), rot > 0)
+    if least is not None:
+        lib, work = _decay_chunk_work(T, E, heads, dim, vdim, proj.device)
+        _check(lib.ga_decay_chunk(_ptr(out), _ptr(work), _ptr(q), _ptr(k), _ptr(v), _i64(proj.stride(0)), _ptr(decay), _ptr(head_decay),
+                                  _ptr(cos), _ptr(sin), _i(rot), _f(q_scale), _f(k_scale), _ptr(state), _ptr(slots), _ptr(step.cu_tokens),
+                                  _ptr(step.q_start), _i(T), _i(E), _i(heads), _i(dim), _i(vdim), _i(1 if silu_inputs else 0), _i(least),
+                                  _stream()), "decay_chunk")
+    if way is not None:
+        lib = build.load("decay_scan")
+        _check(lib.ga_decay_scan(_ptr(out), _ptr(q), _ptr(k), _ptr(v), _i64(proj.stride(0)), _ptr(decay), _ptr(head_decay),
+                                 _ptr(cos), _ptr(sin), _i(rot), _f(q_scale), _f(k_scale), _ptr(state), _ptr(slots), _ptr(step.cu_tokens),
+                                 _ptr(step.q_start), _i(way), _i(most), _i(E), _i(heads), _i(dim), _i(vdim), _i(1 if silu_inputs else 0),
+                                 _stream()), "decay_scan")
     return out
 
 

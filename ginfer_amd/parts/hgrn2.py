@@ -43,11 +43,11 @@ class HGRN2(Part):
         self.w_o = t["o"]
 
     def kernel_modules(self):
-        return ["gated_recurrence", "gemm"] + (["gemm_skinny"] if self.dtype == torch.bfloat16 else [])
+        return ["gated_recurrence", "gemm"] + (["gemm_skinny", "decay_chunk"] if self.dtype == torch.bfloat16 else [])
 
     def forward(self, x, step, cache):
         proj = linear(x, self.w_qfv, None, out_dtype=torch.float32)
         o = ops.hgrn2_scan(proj, self.f_bias, self.lower, cache.state, cache.slots, step, self.nh, self.dk, self.dv,
-                           update=cache.owner)
+                           update=cache.owner, chunked=self.dtype == torch.bfloat16)
         o = ops.headwise_rmsnorm(o, self.norm_weight, self.eps, self.dtype)
         return linear(o.view(x.shape[0], self.nh * self.dv), self.w_o)

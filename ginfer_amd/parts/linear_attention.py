@@ -49,7 +49,7 @@ class _DecayedLinearAttention(Part):
                 "o": WeightSpec((H, v))}
 
     def kernel_modules(self):
-        return ["decay_scan", "gemm"] + (["gemm_skinny", "gemm_tiles"] if self.dtype == torch.bfloat16 else [])
+        return ["decay_scan", "gemm"] + (["gemm_skinny", "gemm_tiles", "decay_chunk"] if self.dtype == torch.bfloat16 else [])
 
     # column blocks of the stacked projection
     @property
@@ -100,7 +100,8 @@ class GatedLinearAttention(_DecayedLinearAttention):
         proj = self._project(x)
         decay = ops.gla_decay(proj, self._rest0, self.w_a2, self.b_a2, self.tau)
         o = ops.decay_scan(proj, 0, self._k0, self._v0, cache.state, cache.slots, step, self.nh, self.dk, self.dv,
-                           decay=decay, q_scale=self.dk ** -0.5)
+                           decay=decay, q_scale=self.dk ** -0.5,
+                           chunked=self.dtype == torch.bfloat16)
         o = ops.head_norm_gate(o, self.norm_weight, self.eps, self.dtype, proj=proj, gate_start=self._g0)
         return linear(o, self.w_o)
 
@@ -133,7 +134,8 @@ class Retention(_DecayedLinearAttention):
         proj = self._project(x)
         cos, sin = self.position.tables() if self.position is not None else (None, None)
         o = ops.decay_scan(proj, 0, self._k0, self._v0, cache.state, cache.slots, step, self.nh, self.dk, self.dv,
-                           head_decay=self.head_decay, cos=cos, sin=sin, k_scale=self.dk ** -0.5)
+                           head_decay=self.head_decay, cos=cos, sin=sin, k_scale=self.dk ** -0.5,
+                           chunked=self.dtype == torch.bfloat16)
         o = ops.head_norm_gate(o, None, self.eps, self.dtype, proj=proj, gate_start=self._g0)
         return linear(o, self.w_o)
 
@@ -165,7 +167,8 @@ class LightningAttention(_DecayedLinearAttention):
     def forward(self, x, step, cache):
         proj = self._project(x)
         o = ops.decay_scan(proj, 0, self._k0, self._v0, cache.state, cache.slots, step, self.nh, self.dk, self.dv,
-                           head_decay=self.head_decay, silu_inputs=True)
+                           head_decay=self.head_decay, silu_inputs=True,
+                           chunked=self.dtype == torch.bfloat16)
         # the norm runs over the heads together: one "head" as wide as all of them
         o = ops.head_norm_gate(o.view(o.shape[0], 1, self.nh * self.dv), self.norm_weight, self.eps, self.dtype, proj=proj,
                                gate_start=self._g0, sigmoid_gate=True)
