@@ -10,6 +10,7 @@
 // D[n = (l/16)*4+i][m = l%16].  Both operands come from global memory in 16-byte loads, 8 lanes to a row, and turn into
 // that layout in the wavefront's own piece of LDS (SkinnyTrip).
 #include "common.h"
+#include <type_traits>
 #include "ginfer_amd.h"   // the entry points below are checked against their declarations
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
@@ -17,6 +18,7 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 
 #define SK_WAVES 8
+#define GA_FOLD_TARGET 256       // the chip's compute units
 #define SK_THREADS (SK_WAVES * 64)
 
 
@@ -48,12 +50,15 @@ struct NormOut {
 // further ones are fetched at the end.
 struct NormInLoads {
   float v[4];
-  __device__ __forceinline__ void load(const NormIn& in, int M, int wave, int lane) {
+  // (no branch stands around a load: what does not exist reads a number of `anything`, or another part, and drops it)
+  __device__ __forceinline__ void load(const NormIn& in, const void* anything, int M, int wave, int lane) {
+    const float* from = in.sumsq ? in.sumsq : reinterpret_cast<const float*>(anything);
+    const int parts = in.sumsq ? in.parts : 1;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int m = M <= 8 ? wave : wave * 2 + (j >> 1);
       const int p = M <= 8 ? lane + 64 * j : lane + 64 * (j & 1);
-      v[j] = (in.sumsq && m < M && p < in.parts) ? in.sumsq[(int64_t)m * in.parts + p] : 0.f;
+      v[j] = from[(in.sumsq && m < M ? m * parts : 0) + min(p, parts - 1)];
     }
   }
   // the rows' factors; rstd: 16 floats of LDS, a barrier before they are read.  Lane l adds parts l, l + 64, ...
@@ -63,7 +68,10 @@ struct NormInLoads {
     const int rows = M <= 8 ? 1 : 2, early = M <= 8 ? 4 : 2;
     for (int i = 0; i < rows; ++i) {
       const int m = M <= 8 ? wave : wave * 2 + i;
-      float t = M <= 8 ? (v[0] + v[1]) + (v[2] + v[3]) : (i == 0 ? v[0] + v[1] : v[2] + v[3]);
+      float x[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[j] = m < M && lane + 64 * (M <= 8 ? j : j & 1) < in.parts ? v[j] : 0.f;
+      float t = M <= 8 ? (x[0] + x[1]) + (x[2] + x[3]) : (i == 0 ? x[0] + x[1] : x[2] + x[3]);
       if (m < M)
         for (int p = lane + 64 * early; p < in.parts; p += 64) t += in.sumsq[(int64_t)m * in.parts + p];
       t = wave_sum(t);
@@ -90,11 +98,16 @@ struct NormInLoads {
 // UNROLL is 1 wherever several workgroups share a compute unit: their wavefronts cover each other's trips, and longer trips were up
 // to three times slower, spread over fewer of them.  A workgroup alone on its unit asks for more at once (ga_skinny_trip); two trips
 // under way at once were slower than one everywhere.
-template <int NT, int MB>
+// Loads go through buffer descriptors (a base for all lanes, 32-bit offsets of each): a lane without a row, or past its end of K, names an
+// offset beyond the buffer and gets zeros without touching memory, so that no load stands behind a branch and none waits for another.
+#define SK_NOTHING 0x80000000u
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t sk_buffer(const bf16_t* base) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(base), 0, 0x7fffffff, 0x00027000);
+}
+template <int NT, int MB, int MATS = 1>    // MATS: bases of W, each with NT / MATS tiles
 struct SkinnySource {
-  const bf16_t* wp[NT][2];                 // the lane's rows of each tile: l / 8 and 8 more
-  const bf16_t* ap[MB][2];
-  bool wok[NT][2], aok[MB][2];
+  __amdgpu_buffer_rsrc_t w[MATS], a[MB];
+  uint32_t wat[NT][2], aat[MB][2];         // bytes to the lane's piece of its rows of each tile, l / 8 and 8 more
   int ke[2], kend;
 };
 // 16 rows of 8 pieces of 16 bytes; piece p of row r lies at p ^ (r / 2): 16 lanes that read one piece of 16 rows meet all banks once
@@ -102,18 +115,20 @@ struct SkinnySource {
 template <int NT, int MB, int UNROLL>
 struct SkinnyTrip {
   u32x4 a[UNROLL][NT][2], b[UNROLL][MB][2];
-  __device__ __forceinline__ void load(const SkinnySource<NT, MB>& src, int k, int lane) {
-    const u32x4 zero = {0u, 0u, 0u, 0u};
+  template <int MATS>
+  __device__ __forceinline__ void load(const SkinnySource<NT, MB, MATS>& src, int k, int lane) {
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u)
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        const int kk = k + u * 64 + (lane & 7) * 8;
-        const bool ok = kk < src.ke[j];
+        const int from = (k + u * 64) * 2;
+        const bool ok = k + u * 64 + (lane & 7) * 8 < src.ke[j];
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) a[u][nt][j] = (ok && src.wok[nt][j]) ? *reinterpret_cast<const u32x4*>(src.wp[nt][j] + kk) : zero;
+        for (int nt = 0; nt < NT; ++nt)
+          a[u][nt][j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(src.w[nt / (NT / MATS)], ok ? src.wat[nt][j] : SK_NOTHING, from, 0));
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) b[u][mb][j] = (ok && src.aok[mb][j]) ? *reinterpret_cast<const u32x4*>(src.ap[mb][j] + kk) : zero;
+        for (int mb = 0; mb < MB; ++mb)
+          b[u][mb][j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(src.a[mb], ok ? src.aat[mb][j] : SK_NOTHING, from, 0));
       }
   }
   __device__ __forceinline__ void multiply(f32x4 (&acc)[NT][MB], u32x4* area, int lane) const {
@@ -146,12 +161,28 @@ struct SkinnyTrip {
   }
 };
 
-template <int NT, int MB, int UNROLL>
-__device__ __forceinline__ void skinny_accumulate(f32x4 (&acc)[NT][MB], const SkinnySource<NT, MB>& src, u32x4* area, int lane) {
-  for (int k = 0; k < src.kend; k += 64 * UNROLL) {
+// beside(): asks for what the epilogue needs from memory, behind the first trip's loads: nothing may come between a kernel's
+// start and those.  (Nothing in it may use what it loads unless that has to be; conversions belong to the epilogue.)  us as replays of a
+// graph over weights beyond the 256 MB cache at 1, 8 and 16 rows, before (the norm's and the epilogue's operands first and converted, loads
+// behind branches, K dealt out in 64-bit divisions, arguments from memory) -> after: with the folded norm 1,536 columns of 1,536 4.8, 5.0, 5.6 ->
+// 4.0, 4.2, 4.7; of 8,960 9.7, 11.1, 14.0 -> 8.4, 10.0, 12.5; 3,584 of 3,584 8.7, 8.7, 9.9 -> 8.4, 8.3, 9.3; of 18,944 28.8, 29.0, 33.3 -> 27.7, 28.3,
+// 32.7; gated 17,920 x 1,536 13.9, 13.7, 15.3 -> 12.7, 13.1, 14.9; 37,888 x 3,584 51.1, 51.7, 54.1 -> 50.7, 50.8, 53.6; q|k|v of 2,048 columns of
+// 1,536 5.3, 5.5, 6.1 -> 4.9, 5.0, 5.8; the head, 151,936 x 1,536 80.5, 88.6 -> 79.9, 89.0 (figures below that name the same sizes are from before).
+template <int NT, int MB, int UNROLL, int MATS, typename Beside>
+__device__ __forceinline__ void skinny_accumulate(f32x4 (&acc)[NT][MB], const SkinnySource<NT, MB, MATS>& src, u32x4* area, int lane,
+                                                  Beside beside) {
+  {
+    SkinnyTrip<NT, MB, UNROLL> trip;
+    trip.load(src, 0, lane);
+    __builtin_amdgcn_sched_barrier(0);
+    beside();
+    __builtin_amdgcn_sched_barrier(0);         // no load moves behind a product
+    trip.multiply(acc, area, lane);
+  }
+  for (int k = 64 * UNROLL; k < src.kend; k += 64 * UNROLL) {
     SkinnyTrip<NT, MB, UNROLL> trip;
     trip.load(src, k, lane);
-    __builtin_amdgcn_sched_barrier(0);         // no load moves behind a product
+    __builtin_amdgcn_sched_barrier(0);
     trip.multiply(acc, area, lane);
   }
 }
@@ -183,12 +214,20 @@ struct Packed {
 template <int PACK>
 struct KRange {
   int shift[2], ke[2], kend;               // of tile rows 0 to 7 and 8 to 15
-  __device__ __forceinline__ KRange(int first_unit, int steps, int units, int K) {
+  // units: PER_PART (a power of two) times `parts`; in 32 bits, which the launchers see to (in 64 the divisions were some 400
+  // instructions in front of the first load)
+  template <int PER_PART>
+  static __device__ __forceinline__ int first_step(int unit, int steps, int parts) {
+    const uint32_t x = (uint32_t)(unit * steps) / PER_PART;
+    return (int)(parts == 1 ? x : x / (uint32_t)parts);
+  }
+  template <int PER_PART>
+  __device__ __forceinline__ KRange(int first_unit, int steps, int parts, int K, std::integral_constant<int, PER_PART>) {
     int longest = 0;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int q = PACK == 2 ? j : 0;
-      const int b = (int)(((int64_t)(first_unit + q) * steps) / units), e = (int)(((int64_t)(first_unit + q + 1) * steps) / units);
+      const int b = first_step<PER_PART>(first_unit + q, steps, parts), e = first_step<PER_PART>(first_unit + q + 1, steps, parts);
       longest = e - b > longest ? e - b : longest;
       shift[j] = b * 64;
       ke[j] = (e * 64 < K ? e * 64 : K) - b * 64;
@@ -220,12 +259,10 @@ __device__ __forceinline__ float gate_act(float v, float u, const GateAct act) {
 }
 
 template <int NT, int MB, int KS, typename TC, bool GATED, int PACK, int UNROLL = 1>
-__global__ __launch_bounds__(SK_THREADS) void gemm_skinny_kernel(TC* __restrict__ C, int64_t ldc,
-                                                                 const bf16_t* __restrict__ A, int64_t lda,
-                                                                 const bf16_t* __restrict__ W,
-                                                                 const bf16_t* __restrict__ bias, int M, int N,
-                                                                 int K, int ksteps, NormIn norm_in,
-                                                                 NormOut norm_out, int fold_cols, GateAct act) {
+__global__ __launch_bounds__(SK_THREADS) void gemm_skinny_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
+                                                                 int64_t lda, int M, int N, int K, int parts, int fold_cols,
+                                                                 TC* __restrict__ C, int64_t ldc, const bf16_t* __restrict__ bias,
+                                                                 NormIn norm_in, NormOut norm_out, GateAct act) {
   static_assert(PACK == 1 || MB == 1, "a packed tile holds at most 8 rows of A");
   using Area = SkinnyArea<NT, MB>;
   __shared__ __attribute__((aligned(16))) unsigned char area[SK_WAVES][Area::BYTES];
@@ -233,55 +270,57 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_skinny_kernel(TC* __restrict_
   using P = Packed<PACK>;
   constexpr int CP = P::CP;
   constexpr int GROUPS = SK_WAVES / KS;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
   auto red = [&](int w, int n, int m) -> float& { return reinterpret_cast<float*>(area[w])[n * (MB * 16 + 1) + m]; };
   const int grp = wave / KS, ks = wave % KS;
   constexpr int NCOL = GATED ? CP : NT * CP;       // output columns of a group
   // A product that folds the norm after it owns `fold_cols` (<= CP) columns per workgroup: as many as spread the
   // columns over all compute units (every workgroup reads all rows of A, so fewer, larger workgroups cost more
   // than the empty tile rows of more, smaller ones).
-  const bool fuse_out = !GATED && NT == 1 && KS == SK_WAVES && MB == 1 && norm_out.residual != nullptr;
+  constexpr bool MAY_FUSE = !GATED && NT == 1 && KS == SK_WAVES && MB == 1;
+  const bool fuse_out = MAY_FUSE && fold_cols > 0;
   const int my_cols = fuse_out ? fold_cols : NCOL;
   const int n0 = fuse_out ? blockIdx.x * fold_cols : (blockIdx.x * GROUPS + grp) * NCOL;
-  const KRange<PACK> kr((blockIdx.y * KS + ks) * PACK, ksteps, gridDim.y * KS * PACK, K);
-  SkinnySource<NT, MB> src;
+  const KRange<PACK> kr((blockIdx.y * KS + ks) * PACK, (K + 63) / 64, parts, K, std::integral_constant<int, KS * PACK>());
+  SkinnySource<NT, MB, GATED ? 2 : 1> src;
   src.kend = kr.kend;
+  src.w[0] = sk_buffer(W + (int64_t)n0 * K);
+  if constexpr (GATED) src.w[1] = sk_buffer(W + ((int64_t)N + n0) * K);
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) src.a[mb] = sk_buffer(A + mb * 16 * lda);
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     const int tr = (lane >> 3) + 8 * j;            // the row of a tile that the lane brings a piece of
+    const uint32_t from = (kr.shift[j] + (lane & 7) * 8) * 2;
     src.ke[j] = kr.ke[j];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
-      const int n = GATED ? n0 + P::col(tr) : n0 + nt * CP + P::col(tr);
-      src.wok[nt][j] = n < N && (!fuse_out || P::col(tr) < my_cols);
-      src.wp[nt][j] = W + ((int64_t)(src.wok[nt][j] ? n : 0) + (GATED ? (int64_t)nt * N : 0)) * K + kr.shift[j];
+      const int n = P::col(tr) + (GATED ? 0 : nt * CP);
+      src.wat[nt][j] = n0 + n < N && (!fuse_out || n < my_cols) ? (uint32_t)n * (uint32_t)K * 2 + from : SK_NOTHING;
     }
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-      const int m = mb * 16 + P::col(tr);
-      src.aok[mb][j] = m < M;
-      src.ap[mb][j] = A + (int64_t)(src.aok[mb][j] ? m : 0) * lda + kr.shift[j];
-    }
+    for (int mb = 0; mb < MB; ++mb)
+      src.aat[mb][j] = mb * 16 + P::col(tr) < M ? (uint32_t)P::col(tr) * (uint32_t)lda * 2 + from : SK_NOTHING;
   }
   f32x4 acc[NT][MB];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) acc[nt][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // what the epilogue needs from memory is asked for now, so that it arrives while the weights stream
   NormInLoads in_loads;
-  if (MB == 1) in_loads.load(norm_in, M, wave, lane);
-  float out_res = 0.f, out_gain = 0.f;       // NormOut: thread t holds row t / CP, column t % CP of the workgroup
-  if (fuse_out) {
-    const int m = threadIdx.x / CP, n = n0 + threadIdx.x % CP;
-    if (threadIdx.x < CP * CP && m < M && n < N && threadIdx.x % CP < my_cols) {
-      out_res = norm_out.residual[(int64_t)m * norm_out.ldr + n];
-      out_gain = norm_out.gain_f32 ? reinterpret_cast<const float*>(norm_out.gain)[n]
-                                   : bf16_to_f32(reinterpret_cast<const bf16_t*>(norm_out.gain)[n]);
+  float out_res = 0.f;                       // NormOut: thread t holds row t / CP, column t % CP of the workgroup
+  uint32_t out_gain[2] = {0, 0};             // its two halves, or a bfloat16 twice
+  skinny_accumulate<NT, MB, UNROLL>(acc, src, reinterpret_cast<u32x4*>(area[wave]), lane, [&]() {
+    if constexpr (MB == 1) in_loads.load(norm_in, A, M, wave, lane);
+    if constexpr (MAY_FUSE) {                // (threads without a column, and products without a norm, read something else)
+      const int m = min((int)threadIdx.x / CP, M - 1), n = min(n0 + (int)threadIdx.x % CP, N - 1), wide = norm_out.gain_f32 ? 2 : 1;
+      const float* res = fuse_out ? norm_out.residual : reinterpret_cast<const float*>(A);
+      const bf16_t* gain = fuse_out ? reinterpret_cast<const bf16_t*>(norm_out.gain) : A;
+      out_res = res[fuse_out ? (int64_t)m * norm_out.ldr + n : 0];
+      out_gain[0] = gain[fuse_out ? n * wide : 0];
+      out_gain[1] = gain[fuse_out ? n * wide + wide - 1 : 0];
     }
-  }
-
-  skinny_accumulate<NT, MB, UNROLL>(acc, src, reinterpret_cast<u32x4*>(area[wave]), lane);
+  });
   if (MB == 1) in_loads.finish(norm_in, rstd, M, wave, lane);
   // the KS parts of a group meet in LDS and are added in wavefront order, the halves of a packed tile in theirs
 #pragma unroll
@@ -313,7 +352,7 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_skinny_kernel(TC* __restrict_
       if (bias) v += bf16_to_f32(bias[n]);
       h = out_res + v;
       norm_out.residual[(int64_t)m * norm_out.ldr + n] = h;
-      norm_out.scaled[(int64_t)m * norm_out.lds + n] = f32_to_bf16(h * out_gain);
+      norm_out.scaled[(int64_t)m * norm_out.lds + n] = f32_to_bf16(h * __uint_as_float(out_gain[1] << 16 | (norm_out.gain_f32 ? out_gain[0] : 0)));
     }
     float sq = h * h;
 #pragma unroll
@@ -321,7 +360,7 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_skinny_kernel(TC* __restrict_
     if (nl == 0 && m < M) norm_out.sumsq[(int64_t)m * gridDim.x + blockIdx.x] = sq;
     return;
   }
-  const bool partial = gridDim.y > 1;
+  const bool partial = parts > 1;
   float* Pp = reinterpret_cast<float*>(C) + (int64_t)blockIdx.y * M * N;      // parts are [y][M][N], dense
   constexpr int MROWS = PACK == 1 ? MB * 16 : CP;
   for (int idx = threadIdx.x; idx < GROUPS * NCOL * MROWS; idx += SK_THREADS) {
@@ -353,42 +392,46 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_skinny_kernel(TC* __restrict_
 // The same dealing serves a plain product of many columns (the head): TILES tiles of 16 columns of W a workgroup, the
 // bias added to the sums.  GATED: the first half of the tiles is the gate's, the second the up matrix's.
 template <int TILES, typename TC, bool GATED>
-__global__ __launch_bounds__(SK_THREADS) void gemm_even_kernel(TC* __restrict__ C, int64_t ldc,
-                                                               const bf16_t* __restrict__ A, int64_t lda,
-                                                               const bf16_t* __restrict__ W,
-                                                               const bf16_t* __restrict__ bias, int M, int N, int K,
-                                                               int ksteps, NormIn norm_in, GateAct act) {
+__global__ __launch_bounds__(SK_THREADS) void gemm_even_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
+                                                               int64_t lda, int M, int N, int K, int each, int rest,
+                                                               int rounds, TC* __restrict__ C, int64_t ldc, const bf16_t* __restrict__ bias,
+                                                               NormIn norm_in, GateAct act) {
   static_assert(!GATED || TILES % 2 == 0, "as many tiles of the gate as of the up matrix");
   constexpr int PER = GATED ? TILES / 2 : TILES;             // tiles of one matrix
   using Area = SkinnyArea<TILES, 1>;
   __shared__ __attribute__((aligned(16))) unsigned char area[SK_WAVES][Area::BYTES];
   __shared__ float rstd[16];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
   auto red = [&](int w, int n, int m) -> float& { return reinterpret_cast<float*>(area[w])[n * 17 + m]; };
-  const int c0 = (int)(((int64_t)blockIdx.x * N) / gridDim.x), c1 = (int)(((int64_t)(blockIdx.x + 1) * N) / gridDim.x);
-  const int cols = c1 - c0;                                  // <= PER * 16 by the launcher's choice of the grid
-  const KRange<1> kr(wave, ksteps, SK_WAVES, K);
-  SkinnySource<TILES, 1> src;
+  // b N / G = b each + b rest / G, G = GA_FOLD_TARGET rounds: in 32 bits
+  auto first = [&](uint32_t b) {
+    const uint32_t x = b * (uint32_t)rest / GA_FOLD_TARGET;
+    return (int)(b * (uint32_t)each + (rounds == 1 ? x : x / (uint32_t)rounds));
+  };
+  const int c0 = first(blockIdx.x), cols = first(blockIdx.x + 1) - c0;      // cols <= PER * 16 by the launcher's choice of the grid
+  const KRange<1> kr(wave, (K + 63) / 64, 1, K, std::integral_constant<int, SK_WAVES>());
+  SkinnySource<TILES, 1, GATED ? 2 : 1> src;
   src.kend = kr.kend;
+  src.w[0] = sk_buffer(W + (int64_t)c0 * K);
+  if constexpr (GATED) src.w[1] = sk_buffer(W + ((int64_t)N + c0) * K);
+  src.a[0] = sk_buffer(A);
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     const int tr = (lane >> 3) + 8 * j;                      // the row of a tile that the lane brings a piece of
+    const uint32_t from = (kr.shift[j] + (lane & 7) * 8) * 2;
     src.ke[j] = kr.ke[j];
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
       const int cl = (t % PER) * 16 + tr;                    // its column within the workgroup's range
-      src.wok[t][j] = cl < cols;
-      src.wp[t][j] = W + ((int64_t)(src.wok[t][j] ? c0 + cl : 0) + (GATED && t >= PER ? (int64_t)N : 0)) * K + kr.shift[j];
+      src.wat[t][j] = cl < cols ? (uint32_t)cl * (uint32_t)K * 2 + from : SK_NOTHING;
     }
-    src.aok[0][j] = tr < M;
-    src.ap[0][j] = A + (int64_t)(src.aok[0][j] ? tr : 0) * lda + kr.shift[j];
+    src.aat[0][j] = tr < M ? (uint32_t)tr * (uint32_t)lda * 2 + from : SK_NOTHING;
   }
   f32x4 acc[TILES][1];
 #pragma unroll
   for (int t = 0; t < TILES; ++t) acc[t][0] = f32x4{0.f, 0.f, 0.f, 0.f};
   NormInLoads in_loads;
-  in_loads.load(norm_in, M, wave, lane);
-  skinny_accumulate<TILES, 1, 1>(acc, src, reinterpret_cast<u32x4*>(area[wave]), lane);
+  skinny_accumulate<TILES, 1, 1>(acc, src, reinterpret_cast<u32x4*>(area[wave]), lane, [&]() { in_loads.load(norm_in, A, M, wave, lane); });
   in_loads.finish(norm_in, rstd, M, wave, lane);
 #pragma unroll
   for (int t = 0; t < TILES; ++t)
@@ -431,7 +474,6 @@ static int auto_pack(int M, int workgroups_of_full_tiles) {
 // above, us with a tile's columns -> as few as make 256 workgroups, at 1, 8 and 16 rows: 1,536 columns of 8,960 9.1 -> 9.1, 10.2 -> 9.8, 15.6 ->
 // 13.5; 896 of 4,864 (112 of 8 -> 224 of 4) 6.7 -> 6.7, 7.4 -> 7.0, 11.2 -> 9.8; 2,048 of 11,008 at 16 rows 19.6 -> 17.3; 1,536 of 1,536 level,
 // level, 6.3 -> 6.1.  Never more workgroups than GA_FOLD_TARGET.
-#define GA_FOLD_TARGET 256
 // The gated product of up to 16 rows goes to the kernel that deals its columns evenly from this many (activation)
 // columns on: a workgroup then has at least 8 of them.
 #define GA_GATED_EVEN_MIN_COLUMNS 2048
@@ -489,6 +531,11 @@ extern "C" int ga_skinny_norm_parts(int M, int N) {
 // 10.4, 9.8, 10.7, 9.9; 37 (3,584 of 18,944) 39.6, 29.2, 28.8, 28.6, 28.6 and 35.8, 28.0, 27.5, 27.9, 28.3.
 extern "C" int ga_skinny_trip(int steps) { return steps <= 5 ? steps : steps <= 8 ? (steps + 1) / 2 : 3; }
 
+// offsets inside a tile's 96 rows, and steps of K times their consumers, are 32-bit
+static bool sk_too_far(int64_t K, int64_t lda, int64_t parts = 1) {
+  return K >= 1 << 23 || lda >= 1 << 26 || lda < 0 || parts * 16 * ((K + 63) / 64) >= 1ll << 31;
+}
+
 // A [M, K] (row stride lda), W [N, K] contiguous, bias [N] or null.  grid_splits == 1: C [M, N] (row
 // stride ldc) in bfloat16 or float.  grid_splits > 1: C is float [grid_splits][M][N], parts to be added
 // by the consumer.  gated: W is [2N, K] (gate over up), C [M, N] = silu(A.gate^T) * (A.up^T), no bias, no
@@ -498,7 +545,8 @@ static int gemm_skinny_launch(void* C, int64_t ldc, const void* A, int64_t lda, 
                               int M, int N, int K, int out_f32, int nt, int ks, int grid_splits, int gated, int pack,
                               const GaSkinnyNorm* norm, GateAct act, hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
-  if (M > 64 || K <= 0 || K % 8 || lda % 8 || grid_splits < 1) return -1;
+  if (M > 64 || K <= 0 || K % 8 || lda % 8 || grid_splits < 1 || sk_too_far(K, M > 1 ? lda : 0, grid_splits)) return -1;
+  if (M == 1) lda = K;                           // one row has no next one, whatever its stride says
   const int mb = (M + 15) / 16;
   NormIn norm_in = {nullptr, 0, 0.f, 0.f};
   NormOut norm_out = {nullptr, 0, nullptr, 0, nullptr, 0, nullptr};
@@ -526,13 +574,12 @@ static int gemm_skinny_launch(void* C, int64_t ldc, const void* A, int64_t lda, 
   if (pack != 1 && (pack != 2 || M > 8)) return -2;
   const bool may_be_even = gated || (grid_splits == 1 && !norm_out.residual && ks == SK_WAVES);
   const int workgroups = mb == 1 && pack == 1 && may_be_even ? ga_skinny_even_workgroups(M, N, gated) : 0;
-  if (workgroups > 0) {
+  if (workgroups > 0 && workgroups < 1 << 16) {       // (its columns are counted in 32 bits)
     const int most = (N + workgroups - 1) / workgroups, per = (most + 15) / 16;      // tiles of one matrix
-    const int ksteps = (K + 63) / 64;
     dim3 grid(workgroups), block(SK_THREADS);
 #define LAUNCH_EVEN(TILES, TC, G)                                                                              \
-  hipLaunchKernelGGL((gemm_even_kernel<TILES, TC, G>), grid, block, 0, stream, (TC*)C, ldc, (const bf16_t*)A, \
-                     lda, (const bf16_t*)W, (const bf16_t*)bias, M, N, K, ksteps, norm_in, act)
+  hipLaunchKernelGGL((gemm_even_kernel<TILES, TC, G>), grid, block, 0, stream, (const bf16_t*)A,  \
+                     (const bf16_t*)W, lda, M, N, K, N / workgroups, N % workgroups, workgroups / GA_FOLD_TARGET, (TC*)C, ldc, (const bf16_t*)bias, norm_in, act)
 #define PICK_EVEN(TC)                                                                                          \
   if (gated) {                                                                                                 \
     if (per == 1) LAUNCH_EVEN(2, TC, true); else if (per == 2) LAUNCH_EVEN(4, TC, true); else LAUNCH_EVEN(6, TC, true); \
@@ -560,8 +607,8 @@ static int gemm_skinny_launch(void* C, int64_t ldc, const void* A, int64_t lda, 
   const int trip = alone ? ga_skinny_trip(steps) : head ? 3 : 1;
   if (trip > 1 && mb == 1 && nt == 1 && ks == SK_WAVES && !gated) {
 #define LAUNCH_TRIP(TC, PK, UNROLL)                                                                                     \
-  hipLaunchKernelGGL((gemm_skinny_kernel<1, 1, SK_WAVES, TC, false, PK, UNROLL>), grid, block, 0, stream, (TC*)C, ldc, \
-                     (const bf16_t*)A, lda, (const bf16_t*)W, (const bf16_t*)bias, M, N, K, ksteps, norm_in, norm_out, fcols, act)
+  hipLaunchKernelGGL((gemm_skinny_kernel<1, 1, SK_WAVES, TC, false, PK, UNROLL>), grid, block, 0, stream, (const bf16_t*)A, \
+                     (const bf16_t*)W, lda, M, N, K, grid_splits, fcols, (TC*)C, ldc, (const bf16_t*)bias, norm_in, norm_out, act)
 #define PICK_TRIP(TC, PK)                        \
   switch (trip) {                                \
     case 2: LAUNCH_TRIP(TC, PK, 2); break;       \
@@ -579,9 +626,9 @@ static int gemm_skinny_launch(void* C, int64_t ldc, const void* A, int64_t lda, 
     return GA_CHECK_LAUNCH();
   }
 #define LAUNCH(NT, MB, KS, TC, G, PK)                                                                     \
-  hipLaunchKernelGGL((gemm_skinny_kernel<NT, MB, KS, TC, G, PK>), grid, block, 0, stream, (TC*)C, ldc,   \
-                     (const bf16_t*)A, lda, (const bf16_t*)W, (const bf16_t*)bias, M, N, K, ksteps,      \
-                     norm_in, norm_out, fcols, act)
+  hipLaunchKernelGGL((gemm_skinny_kernel<NT, MB, KS, TC, G, PK>), grid, block, 0, stream, (const bf16_t*)A, \
+                     (const bf16_t*)W, lda, M, N, K, grid_splits, fcols, (TC*)C, ldc, (const bf16_t*)bias,     \
+                     norm_in, norm_out, act)
 #define PICK_KS(NT, MB, TC, G, PK)                                                                        \
   switch (ks) {                                                                                           \
     case 1: LAUNCH(NT, MB, 1, TC, G, PK); break;                                                          \
@@ -646,11 +693,10 @@ extern "C" int ga_gemm_skinny_bounded_gate(void* C, int64_t ldc, const void* A, 
 // columns to fill the chip otherwise, and its K cannot be split over workgroups (the epilogue needs whole sums).
 template <int MB, int KS, int PACK, bool HALF, int UNROLL = 1>
 __global__ __launch_bounds__(SK_THREADS) void qkv_rope_skinny_kernel(
-    bf16_t* __restrict__ q_out, const bf16_t* __restrict__ A, int64_t lda, const bf16_t* __restrict__ W,
-    const bf16_t* __restrict__ bias, const int32_t* __restrict__ positions, const float* __restrict__ cos_t,
+    const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, int64_t lda, const int32_t* __restrict__ positions, int M, int K, int nh,
+    int nkv, int hd, int ucols, bf16_t* __restrict__ q_out, const bf16_t* __restrict__ bias, const float* __restrict__ cos_t,
     const float* __restrict__ sin_t, const int64_t* __restrict__ slot_mapping, bf16_t* __restrict__ k_pages,
-    bf16_t* __restrict__ v_pages, int M, int K, int nh, int nkv, int hd, int page_size, int write_kv,
-    int ksteps, NormIn norm_in, int ucols) {
+    bf16_t* __restrict__ v_pages, int page_size, int write_kv, NormIn norm_in) {
   static_assert(PACK == 1 || MB == 1, "a packed tile holds at most 8 rows of A");
   static_assert(PACK == 1 || !HALF, "a tile is packed or half empty, not both");
   using Area = SkinnyArea<2, MB>;
@@ -660,7 +706,7 @@ __global__ __launch_bounds__(SK_THREADS) void qkv_rope_skinny_kernel(
   using P = Packed<PACK>;
   constexpr int CP = HALF ? 8 : P::CP;
   constexpr int GROUPS = SK_WAVES / KS;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
   const int grp = wave / KS, ks = wave % KS;
   // a unit's two tiles hold `ucols` (<= CP) columns each: fewer than a tile's where that spreads the product over more
   // compute units (the lanes of the other columns load nothing)
@@ -681,66 +727,72 @@ __global__ __launch_bounds__(SK_THREADS) void qkv_rope_skinny_kernel(
       row1 = row0 + ucols;
     }
   }
-  const KRange<PACK> kr(ks * PACK, ksteps, KS * PACK, K);
-  SkinnySource<2, MB> src;
+  const KRange<PACK> kr(ks * PACK, (K + 63) / 64, 1, K, std::integral_constant<int, KS * PACK>());
+  SkinnySource<2, MB, 2> src;
   src.kend = kr.kend;
+  src.w[0] = sk_buffer(W + (int64_t)row0 * K);
+  src.w[1] = sk_buffer(W + (int64_t)row1 * K);
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb) src.a[mb] = sk_buffer(A + mb * 16 * lda);
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     const int tr = (lane >> 3) + 8 * j;            // the row of a tile that the lane brings a piece of
+    const uint32_t from = (kr.shift[j] + (lane & 7) * 8) * 2;
     src.ke[j] = kr.ke[j];
     const int wrow = HALF ? (tr & 7) : P::col(tr);
-    src.wok[0][j] = src.wok[1][j] = unit_ok && (!HALF || tr < 8) && wrow < ucols;
-    src.wp[0][j] = W + (int64_t)(row0 + wrow) * K + kr.shift[j];
-    src.wp[1][j] = W + (int64_t)(row1 + wrow) * K + kr.shift[j];
+    src.wat[0][j] = src.wat[1][j] = unit_ok && (!HALF || tr < 8) && wrow < ucols ? (uint32_t)wrow * (uint32_t)K * 2 + from : SK_NOTHING;
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-      const int m = mb * 16 + P::col(tr);
-      src.aok[mb][j] = m < M;
-      src.ap[mb][j] = A + (int64_t)(src.aok[mb][j] ? m : 0) * lda + kr.shift[j];
-    }
+    for (int mb = 0; mb < MB; ++mb)
+      src.aat[mb][j] = mb * 16 + P::col(tr) < M ? (uint32_t)P::col(tr) * (uint32_t)lda * 2 + from : SK_NOTHING;
   }
-  // What the epilogue needs from memory (position, slot, cosine and sine, bias) is asked for now, so that
-  // it arrives while the weights stream: an epilogue item is (unit of the workgroup, column, row of A).
+  // What the epilogue needs from memory is asked for while the weights stream: an epilogue item is (unit of the workgroup, column, row of
+  // A).  Positions first, before the weights; slots, biases and, where the positions are in by then, cosines and sines beside them.
   constexpr int MROWS = PACK == 1 ? MB * 16 : CP;
   constexpr int ITEMS = (GROUPS * CP * MROWS + SK_THREADS - 1) / SK_THREADS;
+  int e_pos[ITEMS];
   int64_t e_slot[ITEMS];
-  float e_cos[ITEMS], e_sin[ITEMS], e_blo[ITEMS], e_bhi[ITEMS];
+  float e_cos[ITEMS], e_sin[ITEMS];
+  uint32_t e_blo[ITEMS], e_bhi[ITEMS];           // biases as they lie in memory
+  const bf16_t* biases = bias ? bias : W;        // (a load that stands behind no branch is not waited for at the branch's end)
+  const int64_t* slots = write_kv ? slot_mapping : reinterpret_cast<const int64_t*>(W);
+  auto item = [&](int it, int& nl, int& m, int& u) {
+    const int idx = threadIdx.x + it * SK_THREADS, rest = idx / ucols;
+    nl = idx % ucols;
+    m = rest / GROUPS;
+    u = blockIdx.x * GROUPS + rest % GROUPS;
+  };
 #pragma unroll
   for (int it = 0; it < ITEMS; ++it) {
-    const int idx = threadIdx.x + it * SK_THREADS;
-    const int nl = idx % ucols, rest = idx / ucols;
-    const int gi = rest % GROUPS, m = rest / GROUPS;
-    const int u = blockIdx.x * GROUPS + gi;
-    e_slot[it] = -1;
-    e_cos[it] = 1.f;
-    e_sin[it] = e_blo[it] = e_bhi[it] = 0.f;
-    if (m < M && u < units) {
-      if (write_kv) e_slot[it] = slot_mapping[m];
-      if (u < qk_units) {
-        const int head = u / upq, j = (u % upq) * ucols + nl;
-        const int p = positions[m];
-        e_cos[it] = cos_t[(int64_t)p * half + j];
-        e_sin[it] = sin_t[(int64_t)p * half + j];
-        if (bias) {
-          e_blo[it] = bf16_to_f32(bias[head * hd + j]);
-          e_bhi[it] = bf16_to_f32(bias[head * hd + j + half]);
-        }
-      } else if (bias) {
-        const int v = u - qk_units;
-        const int at = (nh + nkv + v / upv) * hd + (v % upv) * 2 * ucols + nl;
-        e_blo[it] = bf16_to_f32(bias[at]);
-        e_bhi[it] = bf16_to_f32(bias[at + ucols]);
-      }
-    }
+    int nl, m, u;
+    item(it, nl, m, u);
+    e_pos[it] = positions[min(m, M - 1)];
   }
+  auto beside = [&]() {
+#pragma unroll
+    for (int it = 0; it < ITEMS; ++it) {
+      int nl, m, u;
+      item(it, nl, m, u);
+      m = min(m, M - 1);
+      u = min(u, units - 1);
+      const int v = u - qk_units, head = v < 0 ? u / upq : nh + nkv + v / upv, j = v < 0 ? (u % upq) * ucols + nl : (v % upv) * 2 * ucols + nl;
+      e_slot[it] = slots[m];
+      e_blo[it] = biases[head * hd + j];
+      e_bhi[it] = biases[head * hd + j + (v < 0 ? half : ucols)];
+      const int64_t at = v < 0 ? (int64_t)e_pos[it] * half + j : 0;
+      e_cos[it] = cos_t[at];
+      e_sin[it] = sin_t[at];
+    }
+  };
   f32x4 acc[2][MB];
 #pragma unroll
   for (int nt = 0; nt < 2; ++nt)
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) acc[nt][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
   NormInLoads in_loads;
-  if (MB == 1) in_loads.load(norm_in, M, wave, lane);
-  skinny_accumulate<2, MB, UNROLL>(acc, src, reinterpret_cast<u32x4*>(area[wave]), lane);
+  skinny_accumulate<2, MB, UNROLL>(acc, src, reinterpret_cast<u32x4*>(area[wave]), lane, [&]() {
+    if (MB == 1) in_loads.load(norm_in, A, M, wave, lane);
+    beside();
+  });
   if (MB == 1) in_loads.finish(norm_in, rstd, M, wave, lane);
   const bool scale_rows = MB == 1 && norm_in.sumsq != nullptr;
 #pragma unroll
@@ -752,10 +804,9 @@ __global__ __launch_bounds__(SK_THREADS) void qkv_rope_skinny_kernel(
   __syncthreads();
 #pragma unroll
   for (int it = 0; it < ITEMS; ++it) {
-    const int idx = threadIdx.x + it * SK_THREADS;
-    const int nl = idx % ucols, rest = idx / ucols;
-    const int gi = rest % GROUPS, m = rest / GROUPS;
-    const int u = blockIdx.x * GROUPS + gi;
+    int nl, m, u;
+    item(it, nl, m, u);
+    const int gi = u % GROUPS;
     if (m >= M || u >= units) continue;
     float lo = 0.f, hi = 0.f;
 #pragma unroll
@@ -770,9 +821,9 @@ __global__ __launch_bounds__(SK_THREADS) void qkv_rope_skinny_kernel(
       lo *= rstd[m];
       hi *= rstd[m];
     }
-    lo += e_blo[it];
-    hi += e_bhi[it];
-    const int64_t slot = e_slot[it];
+    lo += bias ? __uint_as_float(e_blo[it] << 16) : 0.f;
+    hi += bias ? __uint_as_float(e_bhi[it] << 16) : 0.f;
+    const int64_t slot = write_kv ? e_slot[it] : -1;
     int64_t page = 0, off = 0;
     if (slot >= 0) slot_page(slot, page_size, page, off);
     if (u < qk_units) {
@@ -817,7 +868,8 @@ extern "C" int ga_qkv_rope_skinny(void* q_out, const void* A, int64_t lda, const
                                   int nkv, int hd, int page_size, int write_kv, int pack, const GaSkinnyNorm* norm,
                                   hipStream_t stream) {
   if (M <= 0) return 0;
-  if (M > 64 || K <= 0 || K % 8 || lda % 8 || hd % 32 || nh <= 0 || nkv <= 0) return -1;
+  if (M > 64 || K <= 0 || K % 8 || lda % 8 || hd % 32 || nh <= 0 || nkv <= 0 || sk_too_far(K, M > 1 ? lda : 0)) return -1;
+  if (M == 1) lda = K;
   const int mb = (M + 15) / 16;
   NormIn norm_in = {nullptr, 0, 0.f, 0.f};
   if (norm && norm->residual) return -6;
@@ -841,10 +893,10 @@ extern "C" int ga_qkv_rope_skinny(void* q_out, const void* A, int64_t lda, const
   // columns of 3,584) 11.4 -> 11.6 at 1 row, 12.4 -> 11.9 at 8
   const bool both = pack == 2 && (ksteps + 2 * ks - 1) / (2 * ks) == 2;
 #define LAUNCH(MB, PK, HF, ...)                                                                           \
-  hipLaunchKernelGGL((qkv_rope_skinny_kernel<MB, 8, PK, HF, ##__VA_ARGS__>), grid, block, 0, stream, (bf16_t*)q_out,    \
-                     (const bf16_t*)A, lda, (const bf16_t*)W, (const bf16_t*)bias, (const int32_t*)positions, \
+  hipLaunchKernelGGL((qkv_rope_skinny_kernel<MB, 8, PK, HF, ##__VA_ARGS__>), grid, block, 0, stream, (const bf16_t*)A,  \
+                     (const bf16_t*)W, lda, (const int32_t*)positions, M, K, nh, nkv, hd, ucols, (bf16_t*)q_out, (const bf16_t*)bias, \
                      (const float*)cos_t, (const float*)sin_t, (const int64_t*)slot_mapping, (bf16_t*)k_pages, \
-                     (bf16_t*)v_pages, M, K, nh, nkv, hd, page_size, write_kv, ksteps, norm_in, ucols)
+                     (bf16_t*)v_pages, page_size, write_kv, norm_in)
   switch (mb) {
     case 1:
       if (both) LAUNCH(1, 2, false, 2); else if (pack == 2) LAUNCH(1, 2, false); else if (half_tiles) LAUNCH(1, 1, true); else LAUNCH(1, 1, false);
