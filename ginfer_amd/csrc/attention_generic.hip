@@ -565,8 +565,8 @@ __global__ __launch_bounds__(64 * (MA_MAX_COMPUTE + MA_LOADERS)) void paged_atte
             s[b][r] = s[b][r] * mul;
             mx = fmaxf(mx, s[b][r]);
           }
-        mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
-        mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
+        mx = max_across_32(mx);
+        mx = max_across_16(mx);
         m_new = fmaxf(m, mx);
         alpha = expf(m - m_new);                   // exp(-inf) = 0 on a token's first tile
 #pragma unroll
@@ -583,8 +583,8 @@ __global__ __launch_bounds__(64 * (MA_MAX_COMPUTE + MA_LOADERS)) void paged_atte
             s[b][r] = (active && c >= lo && c <= pos) ? s[b][r] * mul : -INFINITY;
             mx = fmaxf(mx, s[b][r]);
           }
-        mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
-        mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
+        mx = max_across_32(mx);
+        mx = max_across_16(mx);
         m_new = fmaxf(m, mx);                      // finite for a token that sees the tile: it holds one of its keys
         alpha = active ? expf(m - m_new) : 1.f;
 #pragma unroll
@@ -600,9 +600,9 @@ __global__ __launch_bounds__(64 * (MA_MAX_COMPUTE + MA_LOADERS)) void paged_atte
 #pragma unroll
       for (int r = 0; r < 4; ++r) u[r] = (s[0][r] + s[2][r]) + (s[1][r] + s[3][r]);     // key bits 5, then 4
 #pragma unroll
-      for (int r = 0; r < 4; ++r) u[r] = u[r] + __shfl_xor(u[r], 32, WAVE);             // key bit 3
+      for (int r = 0; r < 4; ++r) u[r] = add_across_32(u[r]);             // key bit 3
 #pragma unroll
-      for (int r = 0; r < 4; ++r) u[r] = u[r] + __shfl_xor(u[r], 16, WAVE);             // key bit 2
+      for (int r = 0; r < 4; ++r) u[r] = add_across_16(u[r]);             // key bit 2
       const float sum = (u[0] + u[2]) + (u[1] + u[3]);                                  // key bits 1 and 0
       l = __builtin_fmaf(l, alpha, sum);
       m = m_new;
@@ -747,8 +747,8 @@ __global__ __launch_bounds__(64 * (HA_COMPUTE + HA_LOADERS)) void paged_attentio
       s[r] = valid[r] ? s[r] : -INFINITY;
       mx = fmaxf(mx, s[r]);
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
-    mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
+    mx = max_across_32(mx);
+    mx = max_across_16(mx);
     if (kq == 0) mx_s[wave * 16 + col] = mx;
     __syncthreads();
     const float m_new = fmaxf(fmaxf(m, fmaxf(mx_s[col], mx_s[16 + col])), fmaxf(mx_s[32 + col], mx_s[48 + col]));
@@ -763,9 +763,9 @@ __global__ __launch_bounds__(64 * (HA_COMPUTE + HA_LOADERS)) void paged_attentio
       u[r] = (pr[0] + pr[32 * 16]) + (pr[16 * 16] + pr[48 * 16]);                     // key bits 5, then 4
     }
 #pragma unroll
-    for (int r = 0; r < 4; ++r) u[r] = u[r] + __shfl_xor(u[r], 32, WAVE);             // key bit 3
+    for (int r = 0; r < 4; ++r) u[r] = add_across_32(u[r]);             // key bit 3
 #pragma unroll
-    for (int r = 0; r < 4; ++r) u[r] = u[r] + __shfl_xor(u[r], 16, WAVE);             // key bit 2
+    for (int r = 0; r < 4; ++r) u[r] = add_across_16(u[r]);             // key bit 2
     const float sum = (u[0] + u[2]) + (u[1] + u[3]);                                  // key bits 1 and 0
     l = __builtin_fmaf(l, alpha, sum);
     m = live ? m_new : m;

@@ -241,8 +241,8 @@ __device__ __forceinline__ void tile_softmax(bf16x8 (&pb)[NB], f32x4 (&s)[NB][2]
     // 2^LAZY_MAX, harmless in 32-bit sums, and the tile costs no exchange between lanes: the four lanes
     // of a column keep partial sums of their own keys (added up once, by finish_sums, after the loop).
     if (__any(mx * scale > m[nb] + LAZY_MAX)) {
-      mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
+      mx = max_across_16(mx);
+      mx = max_across_32(mx);
       const float m_new = fmaxf(m[nb], mx * scale);
       if (m_new != -INFINITY) {
         const float alpha = fast_exp2(m[nb] - m_new);      // exp2(-inf) = 0 the first time
@@ -383,8 +383,8 @@ template <int NB>
 __device__ __forceinline__ void finish_sums(float (&l)[NB]) {
 #pragma unroll
   for (int nb = 0; nb < NB; ++nb) {
-    l[nb] += __shfl_xor(l[nb], 16, WAVE);
-    l[nb] += __shfl_xor(l[nb], 32, WAVE);
+    l[nb] = add_across_16(l[nb]);
+    l[nb] = add_across_32(l[nb]);
   }
 }
 
@@ -405,6 +405,18 @@ __device__ __forceinline__ void load_q(bf16x8 (&q)[KB], const bf16_t* row /* nul
   for (int kb = 0; kb < KB; ++kb) {
     q[kb] = zero8();
     if (row && kb * 32 + g * 8 < HD) q[kb] = load8(row + kb * 32 + g * 8);
+  }
+}
+
+// The same for columns that are heads side by side from `first` (the same for the whole wavefront) on.  A column without a head
+// names an offset beyond the buffer and gets zeros: a load behind a branch would be waited for at the branch's end, a way to memory before the keys are
+// asked for.
+__device__ __forceinline__ void load_q_columns(bf16x8 (&q)[KB], const bf16_t* first, bool live, int c, int g) {
+  const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(first), 0, 16 * HD * 2, 0x00027000);
+#pragma unroll
+  for (int kb = 0; kb < KB; ++kb) {
+    const uint32_t at = live && kb * 32 + g * 8 < HD ? (uint32_t)(c * HD + kb * 32 + g * 8) * 2u : 0x80000000u;
+    q[kb] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rows, at, 0, 0));
   }
 }
 
@@ -437,23 +449,20 @@ __device__ __forceinline__ int longest_span(int longest, int window) {
 // at 100 to 250, 28 heads in 4 groups, took 8.25 us for 7.9)
 template <bool ONE>
 __global__ __launch_bounds__(64 * DEC_WAVES) void attn_decode_split_kernel(
-    bf16_t* __restrict__ out, int64_t out_stride, float* __restrict__ part_o, float* __restrict__ part_ml,
-    const bf16_t* __restrict__ q, int64_t q_stride, const bf16_t* __restrict__ k_pages,
-    const bf16_t* __restrict__ v_pages, const int32_t* __restrict__ block_table, int table_width,
-    const int4* __restrict__ decode_info, int nh, int nkv, int head_blocks, int ps_shift, int window,
-    float scale, const Splits splits, const HeadExtras ex) {
+    const int4* __restrict__ decode_info, const int32_t* __restrict__ block_table, const bf16_t* __restrict__ q, int64_t q_stride,
+    int table_width, int ps_shift, int nkv, int group, int head_blocks, int window, const bf16_t* __restrict__ k_pages,
+    const bf16_t* __restrict__ v_pages, float scale, const Splits splits, bf16_t* __restrict__ out, int64_t out_stride,
+    float* __restrict__ part_o, float* __restrict__ part_ml, const HeadExtras ex) {
   __shared__ float o_s[DEC_WAVES][HD][17];
   __shared__ float m_s[DEC_WAVES][16], l_s[DEC_WAVES][16], mx_s[16], lsum_s[16];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;
   const int ti = blockIdx.x, split = ONE ? 0 : blockIdx.z;
   const int kvh = blockIdx.y / head_blocks, hb = blockIdx.y % head_blocks;
-  const int group = nh / nkv;
+  const int nh = nkv * group;
   const int4 info = decode_info[ti];       // (row of the step, position, entry of the block table, longest context or 0): one load
-  const int t = info.x, pos = __builtin_amdgcn_readfirstlane(info.y), num_splits = ONE ? 1 : splits.count;
+  const int t = __builtin_amdgcn_readfirstlane(info.x), pos = __builtin_amdgcn_readfirstlane(info.y), num_splits = ONE ? 1 : splits.count;
   const int lo = first_visible_key(pos, window);
   const bool col_ok = hb * 16 + c < group;
-  const int head = kvh * group + hb * 16 + c;
-
   f32x4 o[1][DB];
   float m[1], l[1];
   init_state<1>(o, m, l);
@@ -464,7 +473,7 @@ __global__ __launch_bounds__(64 * DEC_WAVES) void attn_decode_split_kernel(
     int end = ((pos + 32) / 32) * 32;
     if (!ONE && begin + length < end) end = begin + length;
     bf16x8 qr[1][KB];
-    load_q(qr[0], col_ok ? q + (int64_t)t * q_stride + (int64_t)head * HD : nullptr, g);
+    load_q_columns(qr[0], q + (int64_t)t * q_stride + (int64_t)(kvh * group + hb * 16) * HD, col_ok, c, g);
     const int cpos[1] = {col_ok ? pos : -1}, clo[1] = {lo};
     const int32_t* bt = block_table + (int64_t)__builtin_amdgcn_readfirstlane(info.z) * table_width;
     // every live column of a decode wavefront sees the same keys: lo..pos
@@ -481,27 +490,22 @@ __global__ __launch_bounds__(64 * DEC_WAVES) void attn_decode_split_kernel(
   float mx = -INFINITY;
 #pragma unroll
   for (int w = 0; w < DEC_WAVES; ++w) mx = fmaxf(mx, m_s[w][c]);
+  // per column: the common max and the sum of the rescaled sums, once
+  if (threadIdx.x < 16) {
+    float lsum = 0.f;
+#pragma unroll
+    for (int w = 0; w < DEC_WAVES; ++w) {
+      const float mw = m_s[w][c];
+      if (mw != -INFINITY) lsum += l_s[w][c] * fast_exp2(mw - mx);
+    }
+    mx_s[c] = mx;
+    lsum_s[c] = lsum;
+  }
   const float f = (m[0] == -INFINITY) ? 0.f : fast_exp2(m[0] - mx);
 #pragma unroll
   for (int db = 0; db < DB; ++db)
 #pragma unroll
     for (int i = 0; i < 4; ++i) o_s[wave][db * 16 + g * 4 + i][c] = o[0][db][i] * f;
-  __syncthreads();
-  // per column: the common max and the sum of the rescaled sums, once (the outputs in o_s are rescaled already)
-  if (threadIdx.x < 16) {
-    const int cc = threadIdx.x;
-    float mcc = -INFINITY;
-#pragma unroll
-    for (int w = 0; w < DEC_WAVES; ++w) mcc = fmaxf(mcc, m_s[w][cc]);
-    float lsum = 0.f;
-#pragma unroll
-    for (int w = 0; w < DEC_WAVES; ++w) {
-      const float mw = m_s[w][cc];
-      if (mw != -INFINITY) lsum += l_s[w][cc] * fast_exp2(mw - mcc);
-    }
-    mx_s[cc] = mcc;
-    lsum_s[cc] = lsum;
-  }
   __syncthreads();
   const int64_t slot_base = ((int64_t)ti * nh + kvh * group + hb * 16) * num_splits + split;
   for (int idx = threadIdx.x; idx < 16 * HD; idx += 64 * DEC_WAVES) {
@@ -532,9 +536,8 @@ __global__ __launch_bounds__(64 * DEC_WAVES) void attn_decode_split_kernel(
 #define MAX_SPLITS 256
 template <int EARLY, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void attn_decode_combine_kernel(
-    bf16_t* __restrict__ out, int64_t out_stride, const float* __restrict__ part_o,
-    const float* __restrict__ part_ml, const int4* __restrict__ decode_info, int nh, int num_splits,
-    const HeadExtras ex) {
+    const float* __restrict__ part_o, const float* __restrict__ part_ml, const int4* __restrict__ decode_info, int nh, int num_splits,
+    bf16_t* __restrict__ out, int64_t out_stride, int special, const HeadExtras ex) {
   static_assert(WAVES == 1 || EARLY == 32, "a wavefront's splits");
   constexpr int DPL = (HD + 63) / 64, SLOTS = WAVES * EARLY;
   __shared__ float w_s[SLOTS];
@@ -542,22 +545,27 @@ __global__ __launch_bounds__(64 * WAVES) void attn_decode_combine_kernel(
   const int ti = blockIdx.x, head = blockIdx.y, lane = threadIdx.x & 63;
   const int s0 = WAVES == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * EARLY;      // a scalar: 64 addresses hang on it
   const int64_t base = ((int64_t)ti * nh + head) * num_splits;
+  // (a buffer as long as the splits: what lies behind them comes as zeros, without an address worked out for it)
+  const __amdgpu_buffer_rsrc_t outputs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(part_o + base * HD), 0, num_splits * HD * 4, 0x00027000);
+  const __amdgpu_buffer_rsrc_t sums = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(part_ml + base * 2), 0, num_splits * 8, 0x00027000);
   float o[DPL][EARLY];
-  const int row = decode_info[ti].x;
 #pragma unroll
   for (int i = 0; i < DPL; ++i) {
     const int d = lane + 64 * i < HD ? lane + 64 * i : 0;
 #pragma unroll
-    for (int s = 0; s < EARLY; ++s) o[i][s] = part_o[(base + (s0 + s < num_splits ? s0 + s : 0)) * HD + d];
+    for (int s = 0; s < EARLY; ++s)
+      o[i][s] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(outputs, ((s0 + s) * HD + d) * 4, 0, 0));
   }
   constexpr int MINE = (SLOTS + 63) / 64;
   float ms[MINE], ls[MINE];
 #pragma unroll
   for (int j = 0; j < MINE; ++j) {
-    const int s = lane + 64 * j < num_splits ? lane + 64 * j : 0;
-    ms[j] = part_ml[(base + s) * 2];
-    ls[j] = part_ml[(base + s) * 2 + 1];
+    const auto v = __builtin_amdgcn_raw_buffer_load_b64(sums, (lane + 64 * j) * 8, 0, 0);
+    ms[j] = __uint_as_float(v[0]);
+    ls[j] = __uint_as_float(v[1]);
   }
+  // the row is asked for with them, by every lane: as a scalar load it would come a way to memory after everything else
+  int row = (int)__builtin_amdgcn_raw_buffer_load_b32(__builtin_amdgcn_make_buffer_rsrc(const_cast<int4*>(decode_info + ti), 0, 16, 0x00027000), 0, 0, 0);
   float mx = -INFINITY;
 #pragma unroll
   for (int j = 0; j < MINE; ++j) mx = lane + 64 * j < num_splits ? fmaxf(mx, ms[j]) : mx;
@@ -572,7 +580,10 @@ __global__ __launch_bounds__(64 * WAVES) void attn_decode_combine_kernel(
     }
   total = wave_sum(total);
   __syncthreads();
-  const float inv = 1.f / sink_sum(total, mx, ex.sinks, head) * head_gate(ex, row, head);
+  row = __builtin_amdgcn_readfirstlane(row);
+  float inv = 1.f;                           // (special: there are sinks or gates; without them `ex` is not asked for)
+  if (special) inv = 1.f / sink_sum(total, mx, ex.sinks, head) * head_gate(ex, row, head);
+  else inv = 1.f / total;
   bf16_t* op = out + (int64_t)row * out_stride + (int64_t)head * HD;
 #pragma unroll
   for (int i = 0; i < DPL; ++i) {
@@ -1037,18 +1048,18 @@ extern "C" int ga_attn_decode(void* out, int64_t out_stride, const void* q, int6
                          num_splits > 1 ? 0xffffffffu / (uint32_t)num_splits + 1u : 0u};
   dim3 grid(n_tokens, nkv * head_blocks, num_splits);
 #define SPLIT(ONE)                                                                                           \
-  hipLaunchKernelGGL(attn_decode_split_kernel<ONE>, grid, dim3(64 * DEC_WAVES), 0, stream, (bf16_t*)out, out_stride, \
-                     (float*)workspace_o, (float*)workspace_ml, (const bf16_t*)q, q_stride,                   \
-                     (const bf16_t*)k_pages, (const bf16_t*)v_pages, (const int32_t*)block_table, table_width, \
-                     (const int4*)decode_info, nh, nkv, head_blocks, ps_shift, window, scale * LOG2E, splits, ex)
+  hipLaunchKernelGGL(attn_decode_split_kernel<ONE>, grid, dim3(64 * DEC_WAVES), 0, stream, (const int4*)decode_info, \
+                     (const int32_t*)block_table, (const bf16_t*)q, q_stride, table_width, ps_shift, nkv, group, head_blocks, window, \
+                     (const bf16_t*)k_pages, (const bf16_t*)v_pages, scale * LOG2E, splits, (bf16_t*)out, out_stride,  \
+                     (float*)workspace_o, (float*)workspace_ml, ex)
   if (num_splits == 1) SPLIT(true); else SPLIT(false);
 #undef SPLIT
   int rc = GA_CHECK_LAUNCH();
   if (rc || num_splits == 1) return rc;
 #define COMBINE(EARLY, WAVES)                                                                                \
-  hipLaunchKernelGGL((attn_decode_combine_kernel<EARLY, WAVES>), dim3(n_tokens, nh), dim3(64 * WAVES), 0, stream, (bf16_t*)out, \
-                     out_stride, (const float*)workspace_o, (const float*)workspace_ml,                        \
-                     (const int4*)decode_info, nh, num_splits, ex)
+  hipLaunchKernelGGL((attn_decode_combine_kernel<EARLY, WAVES>), dim3(n_tokens, nh), dim3(64 * WAVES), 0, stream, \
+                     (const float*)workspace_o, (const float*)workspace_ml, (const int4*)decode_info, nh, num_splits,        \
+                     (bf16_t*)out, out_stride, ex.sinks || ex.gate, ex)
   if (num_splits <= 8) COMBINE(8, 1);
   else if (num_splits <= 16) COMBINE(16, 1);
   else if (num_splits <= 32) COMBINE(32, 1);
@@ -1086,8 +1097,8 @@ extern "C" int ga_attn_prefill(void* out, int64_t out_stride, const void* q, int
                               tile_rows, nh, nkv, page_size, window, scale, fill_workgroups, prefer_workgroups, parts, part_o,
                               part_ml, ex, stream);
   if (rc || n_part_rows == 0) return rc;
-  hipLaunchKernelGGL((attn_decode_combine_kernel<8, 1>), dim3(n_part_rows, nh), dim3(64), 0, stream, (bf16_t*)out, out_stride,
-                     (const float*)part_o, (const float*)part_ml, (const int4*)part_rows, nh, num_parts, ex);
+  hipLaunchKernelGGL((attn_decode_combine_kernel<8, 1>), dim3(n_part_rows, nh), dim3(64), 0, stream, (const float*)part_o,
+                     (const float*)part_ml, (const int4*)part_rows, nh, num_parts, (bf16_t*)out, out_stride, ex.sinks || ex.gate, ex);
   return GA_CHECK_LAUNCH();
 }
 

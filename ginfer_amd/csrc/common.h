@@ -30,16 +30,50 @@ template <> struct Num<bf16_t> {
   static __device__ __forceinline__ void st(bf16_t* p, float v) { *p = f32_to_bf16(v); }
 };
 
+// What the lanes l and l ^ 32, or l ^ 16, hold, in one order for both: by swaps of registers between rows of lanes, where a shuffle goes
+// through the LDS pipe and is waited for.
+struct LanePair {
+  float a, b;
+};
+__device__ __forceinline__ LanePair lanes_across_32(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return {__uint_as_float(r[0]), __uint_as_float(r[1])};
+}
+__device__ __forceinline__ LanePair lanes_across_16(float v) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return {__uint_as_float(r[0]), __uint_as_float(r[1])};
+}
+__device__ __forceinline__ float add_across_32(float v) { const LanePair p = lanes_across_32(v); return p.a + p.b; }
+__device__ __forceinline__ float add_across_16(float v) { const LanePair p = lanes_across_16(v); return p.a + p.b; }
+__device__ __forceinline__ float max_across_32(float v) { const LanePair p = lanes_across_32(v); return fmaxf(p.a, p.b); }
+__device__ __forceinline__ float max_across_16(float v) { const LanePair p = lanes_across_16(v); return fmaxf(p.a, p.b); }
+// lane l's from lane l - N of its row of 16 (around), or by a permutation of four neighbours
+template <int CTRL>
+__device__ __forceinline__ float lane_moved(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+#define LANES_ROR_8 0x128
+#define LANES_ROR_4 0x124
+#define LANES_XOR_2 0x4e
+#define LANES_XOR_1 0xb1
+
 // butterfly reductions over the 64 lanes of a wavefront: every lane ends with the same value, and
-// the order of the additions is the same whatever the data
+// the order of the additions is the same whatever the data: lanes 32 apart, 16, 8, 4, 2, 1.  (Once lanes 8 apart hold the same, turning
+// a row by 4 brings what lies 4 across.)
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
+  v = add_across_16(add_across_32(v));
+  v += lane_moved<LANES_ROR_8>(v);
+  v += lane_moved<LANES_ROR_4>(v);
+  v += lane_moved<LANES_XOR_2>(v);
+  v += lane_moved<LANES_XOR_1>(v);
   return v;
 }
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, WAVE));
+  v = max_across_16(max_across_32(v));
+  v = fmaxf(v, lane_moved<LANES_ROR_8>(v));
+  v = fmaxf(v, lane_moved<LANES_ROR_4>(v));
+  v = fmaxf(v, lane_moved<LANES_XOR_2>(v));
+  v = fmaxf(v, lane_moved<LANES_XOR_1>(v));
   return v;
 }
 

@@ -302,8 +302,8 @@ __device__ __forceinline__ void decay_chunk_out(const DecayChunkArgs& x, const C
   }
 #pragma unroll
   for (int t = 0; t < DK_RUN; ++t) {
-    m[t] += __shfl_xor(m[t], 16, WAVE);
-    m[t] += __shfl_xor(m[t], 32, WAVE);
+    m[t] = add_across_16(m[t]);
+    m[t] = add_across_32(m[t]);
   }
   __syncthreads();
   // q times what decayed since the run began, k times what decays to its end

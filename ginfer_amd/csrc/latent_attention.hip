@@ -454,8 +454,8 @@ __device__ __forceinline__ void lt_walk(f32x4 (&acc)[NS][RP / 16], float (&m_run
         sc[j] = (kp <= pos_c[k] && kp >= pos_c[k] - back) ? s[k][j >> 2][j & 3] * scale2 : -INFINITY;
         mt = fmaxf(mt, sc[j]);
       }
-      mt = fmaxf(mt, __shfl_xor(mt, 16, WAVE));
-      mt = fmaxf(mt, __shfl_xor(mt, 32, WAVE));
+      mt = max_across_16(mt);
+      mt = max_across_32(mt);
       const bool raise = mt > m_run[k] + LT_SLACK;                          // also where the column has seen no key yet
       const float m_new = raise ? mt : m_run[k];
       alpha[k] = raise ? __builtin_amdgcn_exp2f(m_run[k] - m_new) : 1.f;
@@ -596,8 +596,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void latent_attention_rows_kernel(
 #pragma unroll
       for (int k = 0; k < NS; ++k) {
         float l = l_run[k];
-        l += __shfl_xor(l, 16, WAVE);
-        l += __shfl_xor(l, 32, WAVE);
+        l = add_across_16(l);
+        l = add_across_32(l);
         int h;
         const int tc = token_of(k, h);
         if (tc >= t && tc <= last)
@@ -639,8 +639,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void latent_attention_heads_kernel(
   lt_walk<RP, KP, 1, WAVES>(acc, m_run, l_run, qb, tiles_lds, c_pages, block_table + (int64_t)e * table_width, row, ps_shift,
                             pos_c, back, lo, pos, first, last, scale2, wave, c, g);
   float l = l_run[0];
-  l += __shfl_xor(l, 16, WAVE);
-  l += __shfl_xor(l, 32, WAVE);
+  l = add_across_16(l);
+  l = add_across_32(l);
   if (!head_ok) return;
   if (splits == 1) {
     lt_store<RP>(out + (int64_t)h * out_h + (int64_t)t * out_t, acc[0], lt_finish(m_run[0], l, sink, gate, t, h, heads), rank, g);

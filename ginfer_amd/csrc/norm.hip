@@ -57,23 +57,28 @@ __global__ void add_rmsnorm_kernel(T* __restrict__ out, float* __restrict__ resi
 // too depends on H alone.
 #define VEC_CHUNKS 4
 
+// eight numbers as they lie in memory
 template <typename D>
-__device__ __forceinline__ void load8f(float (&v)[8], const D* p);
+struct Eight;
 template <>
-__device__ __forceinline__ void load8f<float>(float (&v)[8], const float* p) {
-  const float4 a = *reinterpret_cast<const float4*>(p), b = *reinterpret_cast<const float4*>(p + 4);
-  v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-}
+struct Eight<float> {
+  float4 a, b;
+  __device__ __forceinline__ void load(const float* p) { a = *reinterpret_cast<const float4*>(p); b = *reinterpret_cast<const float4*>(p + 4); }
+  __device__ __forceinline__ void get(float (&v)[8]) const { v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w; }
+};
 template <>
-__device__ __forceinline__ void load8f<bf16_t>(float (&v)[8], const bf16_t* p) {
-  const uint4 u = *reinterpret_cast<const uint4*>(p);
-  const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+struct Eight<bf16_t> {
+  uint4 u;
+  __device__ __forceinline__ void load(const bf16_t* p) { u = *reinterpret_cast<const uint4*>(p); }
+  __device__ __forceinline__ void get(float (&v)[8]) const {
+    const uint32_t w[4] = {u.x, u.y, u.z, u.w};
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    v[2 * i] = __uint_as_float(w[i] << 16);
-    v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+    for (int i = 0; i < 4; ++i) {
+      v[2 * i] = __uint_as_float(w[i] << 16);
+      v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+    }
   }
-}
+};
 template <typename T>
 __device__ __forceinline__ void store8f(T* p, const float (&v)[8]);
 template <>
@@ -91,36 +96,63 @@ __device__ __forceinline__ void store8f<bf16_t>(bf16_t* p, const float (&v)[8]) 
   *reinterpret_cast<uint4*>(p) = u;
 }
 
-template <typename T, typename G, typename D, int PARTS /* 0: runtime */>
+// All that a row needs is asked for at once, the gain too: after the meeting it would be a way to memory of its own (and the arguments
+// that the loads need come first, in registers).  CHUNKS: of 8 * NORM_THREADS elements, as many as hold a row.
+template <typename T, typename G, typename D, int PARTS /* 0: runtime */, int CHUNKS>
 __global__ __launch_bounds__(NORM_THREADS) void add_rmsnorm_vec_kernel(
-    T* __restrict__ out, float* __restrict__ residual, const D* __restrict__ delta, int parts_rt,
-    int64_t part_stride, const G* __restrict__ gain, const int32_t* __restrict__ rows, int hidden, float eps) {
+    float* __restrict__ residual, const D* __restrict__ delta, const G* __restrict__ gain, const int32_t* __restrict__ rows,
+    int64_t part_stride, int hidden, int parts_rt, float eps, T* __restrict__ out) {
   __shared__ float scratch[NORM_THREADS / WAVE];
-  const int parts = PARTS ? PARTS : parts_rt;
+  constexpr int AT_ONCE = PARTS * CHUNKS <= 16 ? PARTS : 0;      // parts in registers beside each other
   const int64_t r = blockIdx.x;
   const int64_t t = rows ? (int64_t)rows[r] : r;
   float* res = residual + t * hidden;
   const D* d = delta ? delta + t * hidden : nullptr;
   const bool write_back = (rows == nullptr) && (d != nullptr);
-  float h[VEC_CHUNKS][8];
-  float ss = 0.f;
+  Eight<float> from[CHUNKS];
+  Eight<G> gains[CHUNKS];
+  Eight<D> all[CHUNKS][AT_ONCE > 0 ? AT_ONCE : 1];
 #pragma unroll
-  for (int c = 0; c < VEC_CHUNKS; ++c) {
+  for (int c = 0; c < CHUNKS; ++c) {
     const int i = (c * NORM_THREADS + threadIdx.x) * 8;
     if (i < hidden) {
-      load8f<float>(h[c], res + i);
+      from[c].load(res + i);
+      gains[c].load(gain + i);
       if (d) {
-        float add[8];
-        load8f<D>(add, d + i);
-        for (int p = 1; p < parts; ++p) {
-          float more[8];
-          load8f<D>(more, d + p * part_stride + i);
 #pragma unroll
-          for (int j = 0; j < 8; ++j) add[j] += more[j];
+        for (int p = 0; p < (AT_ONCE > 0 ? AT_ONCE : 1); ++p) all[c][p].load(d + p * part_stride + i);
+      }
+    }
+  }
+  float h[CHUNKS][8];
+  float ss = 0.f;
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c) {
+    const int i = (c * NORM_THREADS + threadIdx.x) * 8;
+    if (i < hidden) {
+      from[c].get(h[c]);
+      if (d) {
+        float add[8], more[8];
+        all[c][0].get(add);
+        if constexpr (AT_ONCE > 0) {
+#pragma unroll
+          for (int p = 1; p < AT_ONCE; ++p) {
+            all[c][p].get(more);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) add[j] += more[j];
+          }
+        } else {
+          const int parts = PARTS ? PARTS : parts_rt;
+          for (int p = 1; p < parts; ++p) {
+            Eight<D> one;
+            one.load(d + p * part_stride + i);
+            one.get(more);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) add[j] += more[j];
+          }
         }
 #pragma unroll
         for (int j = 0; j < 8; ++j) h[c][j] += add[j];
-        if (write_back) store8f<float>(res + i, h[c]);
       }
 #pragma unroll
       for (int j = 0; j < 8; ++j) ss += h[c][j] * h[c][j];
@@ -130,14 +162,15 @@ __global__ __launch_bounds__(NORM_THREADS) void add_rmsnorm_vec_kernel(
   const float rms = sqrtf(ss / (float)hidden + eps);
   T* o = out + r * hidden;
 #pragma unroll
-  for (int c = 0; c < VEC_CHUNKS; ++c) {
+  for (int c = 0; c < CHUNKS; ++c) {
     const int i = (c * NORM_THREADS + threadIdx.x) * 8;
     if (i < hidden) {
       float g[8], y[8];
-      load8f<G>(g, gain + i);
+      gains[c].get(g);
 #pragma unroll
       for (int j = 0; j < 8; ++j) y[j] = (h[c][j] * g[j]) / rms;
       store8f<T>(o + i, y);
+      if (write_back) store8f<float>(res + i, h[c]);      // (earlier, and what the gain waits for would be the store too)
     }
   }
 }
@@ -152,13 +185,20 @@ extern "C" int ga_add_rmsnorm(void* out, void* residual, const void* delta, int 
   dim3 grid(num_rows), block(NORM_THREADS);
   const int64_t stride = (int64_t)num_tokens * hidden;
   if (hidden % 8 == 0 && hidden <= 8 * NORM_THREADS * VEC_CHUNKS) {
+#define CLAUNCH(T, G, D, P, C)                                                                       \
+  hipLaunchKernelGGL((add_rmsnorm_vec_kernel<T, G, D, P, C>), grid, block, 0, stream, (float*)residual, (const D*)delta, \
+                     (const G*)gain, (const int32_t*)rows, stride, hidden, delta_parts, eps, (T*)out)
 #define VLAUNCH(T, G, D, P)                                                                          \
-  hipLaunchKernelGGL((add_rmsnorm_vec_kernel<T, G, D, P>), grid, block, 0, stream, (T*)out,         \
-                     (float*)residual, (const D*)delta, delta_parts, stride, (const G*)gain,         \
-                     (const int32_t*)rows, hidden, eps)
+  do {                                                                                               \
+    if (hidden <= 8 * NORM_THREADS) CLAUNCH(T, G, D, P, 1);                                          \
+    else if (hidden <= 16 * NORM_THREADS) CLAUNCH(T, G, D, P, 2);                                    \
+    else CLAUNCH(T, G, D, P, VEC_CHUNKS);                                                            \
+  } while (0)
 #define VPARTS(T, G)                                                                                 \
-  if (delta_parts == 4) VLAUNCH(T, G, float, 4); else if (delta_parts == 2) VLAUNCH(T, G, float, 2); \
-  else if (delta_parts == 8) VLAUNCH(T, G, float, 8); else VLAUNCH(T, G, float, 0)
+  do {                                                                                               \
+    if (delta_parts == 4) VLAUNCH(T, G, float, 4); else if (delta_parts == 2) VLAUNCH(T, G, float, 2); \
+    else if (delta_parts == 8) VLAUNCH(T, G, float, 8); else VLAUNCH(T, G, float, 0);                 \
+  } while (0)
     if (delta_parts > 0) {
       if (is_bf16) {
         if (gain_is_f32) { VPARTS(bf16_t, float); } else { VPARTS(bf16_t, bf16_t); }
@@ -172,6 +212,7 @@ extern "C" int ga_add_rmsnorm(void* out, void* residual, const void* delta, int 
     }
 #undef VPARTS
 #undef VLAUNCH
+#undef CLAUNCH
     return GA_CHECK_LAUNCH();
   }
 #define LAUNCH(T, G, D, PARTS)                                                                    \
