@@ -62,8 +62,8 @@ __device__ __forceinline__ uint2 gt_round4(const float (&y)[4]) {
 
 template <int NI, int MJ, int WN, int WM, int NBUF, bool GATED>
 __global__ __launch_bounds__(64 * WN * WM, 1) void gemm_tiles_kernel(
-    void* __restrict__ C, int64_t ldc, const bf16_t* __restrict__ A, int64_t lda, const bf16_t* __restrict__ W, int M, int cols,
-    int K, int m_tiles, int n_tiles, int slabs_per_part, GateAct act) {
+    const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, int64_t lda, int M, int cols, int K, int m_tiles, int n_tiles,
+    int slabs_per_part, void* __restrict__ C, int64_t ldc, GateAct act) {
   constexpr int WAVES = WN * WM, TN = 32 * NI * WN, TM = 32 * MJ * WM, COLS = GATED ? TN / 2 : TN;
   constexpr int BK = 64, ROW = 2 * BK, RPL = 1024 / ROW;             // bytes a row of a slab, rows a load brings
   constexpr int LW = TN / RPL / WAVES, LA = TM / RPL / WAVES, LOADS = LW + LA, SLAB = (TN + TM) * ROW;
@@ -162,12 +162,20 @@ __global__ __launch_bounds__(64 * WN * WM, 1) void gemm_tiles_kernel(
     half_slab(1, std::true_type());
     brought();
   }
-  for (; s < slabs; ++s) {
+  // the last slabs: each waits for the next one only
+  auto last = [&](auto left) {
+    if (s >= slabs) return;
     half_slab(0, std::false_type());
-    lds_wait_and_meet<0>();
+    lds_wait_and_meet<decltype(left)::value * LOADS>();
     cur = cur == lds + (NBUF - 1) * SLAB ? lds : cur + SLAB;
     half_slab(1, std::false_type());
-  }
+    ++s;
+  };
+  if constexpr (NBUF >= 4) last(std::integral_constant<int, 2>());
+  if constexpr (NBUF >= 3) last(std::integral_constant<int, 1>());
+  last(std::integral_constant<int, 0>());
+  last(std::integral_constant<int, 0>());
+  static_assert(NBUF <= 4, "the last slabs");
   if constexpr (!GATED) {
     float* P = reinterpret_cast<float*>(C) + (int64_t)blockIdx.y * M * cols;
 #pragma unroll
@@ -222,7 +230,7 @@ static int gt_launch(void* C, int64_t ldc, const void* A, int64_t lda, const voi
   const int per_part = (K / 64 + parts - 1) / parts;
   if ((parts - 1) * per_part >= K / 64) return -4;       // a part without a slab
   hipLaunchKernelGGL((gemm_tiles_kernel<NI, MJ, WN, WM, NBUF, GATED>), dim3((unsigned)groups, parts), dim3(64 * WN * WM), bytes, stream,
-                     C, ldc, (const bf16_t*)A, lda, (const bf16_t*)W, M, cols, K, (int)m_tiles, (int)n_tiles, per_part, act);
+                     (const bf16_t*)A, (const bf16_t*)W, lda, M, cols, K, (int)m_tiles, (int)n_tiles, per_part, C, ldc, act);
   return GA_CHECK_LAUNCH();
 }
 
@@ -368,12 +376,23 @@ __device__ __forceinline__ void spread_sums(f32x4 (&acc)[NI][MJ], unsigned char*
     step(1, std::true_type());
     brought();
   }
-  for (; s < slabs; ++s) {
+  // the last NBUF slabs (or all, where K has fewer: then all are in): each waits for the next one only
+  auto last = [&](auto left) {
+    if (s >= slabs) return;
     step(0, std::false_type());
-    lds_wait_and_meet<0>();
+    wait_for(left);
     turn();
     step(1, std::false_type());
-  }
+    ++s;
+  };
+  if constexpr (NBUF >= 7) last(std::integral_constant<int, 5>());
+  if constexpr (NBUF >= 6) last(std::integral_constant<int, 4>());
+  if constexpr (NBUF >= 5) last(std::integral_constant<int, 3>());
+  if constexpr (NBUF >= 4) last(std::integral_constant<int, 2>());
+  if constexpr (NBUF >= 3) last(std::integral_constant<int, 1>());
+  last(std::integral_constant<int, 0>());
+  last(std::integral_constant<int, 0>());
+  static_assert(NBUF >= 2 && NBUF <= 7, "the last slabs");
   __syncthreads();
   constexpr int T = NI * MJ;
   if constexpr (WK == 2) {                        // the parts of K meet: block t's sums are the wavefront's with wk = t % 2
@@ -398,14 +417,18 @@ __device__ __forceinline__ void spread_sums(f32x4 (&acc)[NI][MJ], unsigned char*
 // that share rows of W are neighbours on one XCD.
 struct SpreadShare {
   int m0, live, u0, own;
-  __device__ __forceinline__ bool take(int M, int units, int m_tiles, int tile_rows, int groups) {
+  // units of W are each * groups + rest; in 32 bits (in 64 the divisions stood in front of the first load for half a microsecond)
+  __device__ __forceinline__ bool take(int M, int each, int rest, int m_tiles, int tile_rows, int groups) {
     const int total = m_tiles * groups, run = (total + 7) / 8, at8 = blockIdx.x / 8, id = (blockIdx.x % 8) * run + at8;
     if (at8 >= run || id >= total) return false;
     const int b = id / m_tiles;
     m0 = id % m_tiles * tile_rows;
     live = min(tile_rows, M - m0);
-    u0 = __builtin_amdgcn_readfirstlane((int)((int64_t)b * units / groups));
-    own = __builtin_amdgcn_readfirstlane((int)((int64_t)(b + 1) * units / groups)) - u0;
+    auto first = [&](int x) {                     // x * units / groups
+      return x * each + (groups <= 1 << 16 ? (int)((uint32_t)x * (uint32_t)rest / (uint32_t)groups) : (int)((int64_t)x * rest / groups));
+    };
+    u0 = __builtin_amdgcn_readfirstlane(first(b));
+    own = __builtin_amdgcn_readfirstlane(first(b + 1)) - u0;
     return true;
   }
 };
@@ -431,12 +454,12 @@ __device__ __forceinline__ uint32_t gt_round2(float a, float b) {
 // activation: 0.3 to 0.4 us of 6 to 16 there; with more rows, whose other tiles have the hardware's too, it would be 0.4 to 2.7.
 template <bool EXPF, int NI, int MJ, int WN, int WM, int WK, int NBUF>
 __global__ __launch_bounds__(64 * WN * WM * WK, 1) void gemm_spread_gated_kernel(
-    bf16_t* __restrict__ C, int64_t ldc, const bf16_t* __restrict__ A, int64_t lda, const bf16_t* __restrict__ W, int M, int cols,
-    int K, int m_tiles, int tile_rows, int groups, GateAct act) {
+    const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, int64_t lda, int M, int cols, int K, int m_tiles, int tile_rows,
+    int groups, int each, int rest, bf16_t* __restrict__ C, int64_t ldc, GateAct act) {
   using S = SpreadTile<NI, MJ, WN, WM, WK, NBUF>;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   SpreadShare mine;
-  if (!mine.take(M, cols / 4, m_tiles, tile_rows, groups)) return;
+  if (!mine.take(M, each, rest, m_tiles, tile_rows, groups)) return;
   const int c0 = 4 * mine.u0;
   f32x4 acc[NI][MJ];
   // rows 0 to 3 of a unit are gates, 4 to 7 the same columns' ups
@@ -464,12 +487,12 @@ __global__ __launch_bounds__(64 * WN * WM * WK, 1) void gemm_spread_gated_kernel
 // The same for partial sums [parts][M][cols]: the grid's y is the part of K, a unit eight neighbouring columns.
 template <int NI, int MJ, int WN, int WM, int WK, int NBUF>
 __global__ __launch_bounds__(64 * WN * WM * WK, 1) void gemm_spread_parts_kernel(
-    float* __restrict__ C, const bf16_t* __restrict__ A, int64_t lda, const bf16_t* __restrict__ W, int M, int cols, int K, int m_tiles,
-    int tile_rows, int groups, int slabs_per_part) {
+    const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, int lda, int M, int cols, int K, int m_tiles, int tile_rows, int groups,
+    int each, int rest, int slabs_per_part, float* __restrict__ C) {
   using S = SpreadTile<NI, MJ, WN, WM, WK, NBUF>;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   SpreadShare mine;
-  if (!mine.take(M, cols / 8, m_tiles, tile_rows, groups)) return;
+  if (!mine.take(M, each, rest, m_tiles, tile_rows, groups)) return;
   const int c0 = 8 * mine.u0, slab0 = blockIdx.y * slabs_per_part;
   f32x4 acc[NI][MJ];
   spread_sums<NI, MJ, WN, WM, WK, NBUF>(acc, lds, A, lda, W, K, slab0, min(slabs_per_part, K / S::BK - slab0), mine.m0, mine.live, mine.own,
@@ -495,68 +518,110 @@ struct SpreadQkv {
   const float *cos_t, *sin_t;
   const int64_t* slots;
   bf16_t *k_pages, *v_pages;
-  int nh, nkv, hd, page_size, write_kv;
+  int nh, nkv, page_size, write_kv;
 };
 template <int NI, int MJ, int WN, int WM, int WK, int NBUF>
 __global__ __launch_bounds__(64 * WN * WM * WK, 1) void gemm_spread_qkv_kernel(
-    bf16_t* __restrict__ q_out, const bf16_t* __restrict__ A, int64_t lda, const bf16_t* __restrict__ W, int M, int K, int m_tiles,
-    int tile_rows, int groups, const SpreadQkv x) {
+    const bf16_t* __restrict__ A, const bf16_t* __restrict__ W, int lda, int K, int M, int m_tiles, int tile_rows, int groups, int each,
+    int rest, int hd, int turned_heads, bf16_t* __restrict__ q_out, const SpreadQkv x) {
   using S = SpreadTile<NI, MJ, WN, WM, WK, NBUF>;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   SpreadShare mine;
-  if (!mine.take(M, (x.nh + 2 * x.nkv) * x.hd / 8, m_tiles, tile_rows, groups)) return;
-  const int half = x.hd / 2, per_head = x.hd / 8, turned = (x.nh + x.nkv) * per_head;      // units of a head; of q and k
-  // the first row of W of a unit, and how far on its second four rows lie
-  auto unit_row = [&](int u) { return u < turned ? u / per_head * x.hd + u % per_head * 4 : u * 8; };
+  if (!mine.take(M, each, rest, m_tiles, tile_rows, groups)) return;
+  const int half = hd / 2, per_head = hd / 8, turned = turned_heads * per_head;      // units of a head; of q and k
+  const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave % WM, wn = wave / WM % WN, wk = wave / (WM * WN);
+  // What the epilogue needs from memory: positions and slots of the lane's rows, asked for now (through buffer descriptors: plain loads
+  // would be moved down to their use); then, a few blocks at a time, cosines, sines and biases, and the stores.  Block by block each would wait for two
+  // ways to memory.
+  int pos[MJ];
+  int64_t slots[MJ];
+  {
+    const __amdgpu_buffer_rsrc_t at_pos = __builtin_amdgcn_make_buffer_rsrc(const_cast<int32_t*>(x.positions + mine.m0), 0, mine.live * 4, 0x00027000);
+    const __amdgpu_buffer_rsrc_t at_slot = __builtin_amdgcn_make_buffer_rsrc(const_cast<int64_t*>(x.slots + mine.m0), 0, x.write_kv ? mine.live * 8 : 0, 0x00027000);
+#pragma unroll
+    for (int j = 0; j < MJ; ++j) {
+      const int row = min((wm * MJ + j) * 16 + c, mine.live - 1);
+      pos[j] = (int)__builtin_amdgcn_raw_buffer_load_b32(at_pos, row * 4, 0, 0);
+      slots[j] = __builtin_bit_cast(int64_t, __builtin_amdgcn_raw_buffer_load_b64(at_slot, row * 8, 0, 0));
+    }
+  }
+  // the first row of W of a unit, and how far on its second four rows lie (heads of a power of two: by shifts, a division is some 20 instructions)
+  const int shift = (per_head & (per_head - 1)) == 0 ? __builtin_ctz(per_head) : -1;
+  auto unit_row = [&](int u) {
+    const int head = shift >= 0 ? u >> shift : u / per_head;
+    return u < turned ? head * hd + (u - head * per_head) * 4 : u * 8;
+  };
   auto unit_step = [&](int u) { return u < turned ? half : 4; };
   f32x4 acc[NI][MJ];
   spread_sums<NI, MJ, WN, WM, WK, NBUF>(acc, lds, A, lda, W, K, 0, K / S::BK, mine.m0, mine.live, mine.own, [&](int r) {
     const int u = mine.u0 + r / 8;
     return unit_row(u) + (r & 3) + ((r & 4) ? unit_step(u) : 0);
   });
-  const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave % WM, wn = wave / WM % WN, wk = wave / (WM * WN);
+  constexpr int BLOCKS = NI * MJ / WK + NI * MJ % WK, TOGETHER = BLOCKS < 4 ? BLOCKS : 4;      // of a wavefront; whose operands are asked for at once
+  const bf16_t* biases = x.bias ? x.bias : W;
 #pragma unroll
-  for (int t = 0; t < NI * MJ; ++t)
-    if (WK == 1 || t % 2 == wk) {
-      const int i = t / MJ, row = (wm * MJ + t % MJ) * 16 + c, m = mine.m0 + row;
-      const int lu = (wn * NI + i) * 2 + (g >> 1), u = mine.u0 + lu;
-      const SpreadPairs v(acc[i][t % MJ]);
-      if (row >= mine.live || lu >= mine.own) continue;
-      const int n = unit_row(u) + 2 * (g & 1), step = unit_step(u);          // columns n, n + 1 and their partners
-      float lo[2] = {v.first[0], v.first[1]}, hi[2] = {v.second[0], v.second[1]};
-      if (x.bias) {
+  for (int b0 = 0; b0 < BLOCKS; b0 += TOGETHER) {
+    float2 cs[TOGETHER], sn[TOGETHER];
+    uint32_t blo[TOGETHER], bhi[TOGETHER];           // two columns' biases as they lie in memory
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          lo[e] += bf16_to_f32(x.bias[n + e]);
-          hi[e] += bf16_to_f32(x.bias[n + step + e]);
-        }
-      }
-      const int64_t slot = x.write_kv && u >= x.nh * per_head ? x.slots[m] : -1;
-      int64_t page = 0, off = 0;
-      if (slot >= 0) slot_page(slot, x.page_size, page, off);
-      if (u < turned) {
-        const int j = n % x.hd, head = n / x.hd;
-        const int64_t at = (int64_t)x.positions[m] * half + j;
-        const float c0 = x.cos_t[at], c1 = x.cos_t[at + 1], s0 = x.sin_t[at], s1 = x.sin_t[at + 1];
-        const uint32_t a = gt_round2(lo[0] * c0 - hi[0] * s0, lo[1] * c1 - hi[1] * s1), b = gt_round2(lo[0] * s0 + hi[0] * c0, lo[1] * s1 + hi[1] * c1);
-        bf16_t* o = nullptr;
-        if (head < x.nh) o = q_out + ((int64_t)m * x.nh + head) * x.hd + j;
-        else if (slot >= 0) o = x.k_pages + ((page * x.nkv + (head - x.nh)) * x.page_size + off) * x.hd + j;
-        if (o) {
-          *reinterpret_cast<uint32_t*>(o) = a;
-          *reinterpret_cast<uint32_t*>(o + half) = b;
-        }
-      } else if (slot >= 0) {
-        const int d = n - (x.nh + x.nkv) * x.hd;                     // column of the v heads
-        bf16_t* o = x.v_pages + (page * x.nkv * x.hd + d) * (int64_t)x.page_size + off;
+    for (int y = 0; y < TOGETHER; ++y) {
+      const int t = min(WK * (b0 + y) + (WK == 2 ? wk : 0), NI * MJ - 1), i = t / MJ;     // (where none is left: dropped below)
+      const int u = min(mine.u0 + (wn * NI + i) * 2 + (g >> 1), mine.u0 + mine.own - 1);
+      const int n = unit_row(u) + 2 * (g & 1), step = unit_step(u);
+      int p = pos[0];
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          o[(int64_t)e * x.page_size] = f32_to_bf16(lo[e]);
-          o[(int64_t)(step + e) * x.page_size] = f32_to_bf16(hi[e]);
-        }
-      }
+      for (int j = 1; j < MJ; ++j) p = t % MJ == j ? pos[j] : p;
+      const int64_t at = u < turned ? (int64_t)p * half + (shift >= 0 ? n & (hd - 1) : n % hd) : 0;
+      cs[y] = *reinterpret_cast<const float2*>(x.cos_t + at);
+      sn[y] = *reinterpret_cast<const float2*>(x.sin_t + at);
+      blo[y] = *reinterpret_cast<const uint32_t*>(biases + n);
+      bhi[y] = *reinterpret_cast<const uint32_t*>(biases + n + step);
     }
+#pragma unroll
+    for (int y = 0; y < TOGETHER; ++y)
+#pragma unroll
+      for (int k = 0; k < WK; ++k) {                 // block t of the two that y stands for is the wavefront's with wk = k
+        const int t = WK * (b0 + y) + k;
+        if (t >= NI * MJ || (WK == 2 && k != wk)) continue;
+        const int i = t / MJ, row = (wm * MJ + t % MJ) * 16 + c, m = mine.m0 + row;
+        const int lu = (wn * NI + i) * 2 + (g >> 1), u = mine.u0 + lu;
+        const SpreadPairs v(acc[i][t % MJ]);
+        if (row >= mine.live || lu >= mine.own) continue;
+        const int n = unit_row(u) + 2 * (g & 1), step = unit_step(u);          // columns n, n + 1 and their partners
+        float lo[2] = {v.first[0], v.first[1]}, hi[2] = {v.second[0], v.second[1]};
+        if (x.bias) {
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            lo[e] += __uint_as_float(e ? blo[y] & 0xffff0000u : blo[y] << 16);
+            hi[e] += __uint_as_float(e ? bhi[y] & 0xffff0000u : bhi[y] << 16);
+          }
+        }
+        const int64_t slot = x.write_kv && u >= x.nh * per_head ? slots[t % MJ] : -1;
+        int64_t page = 0, off = 0;
+        if (slot >= 0) slot_page(slot, x.page_size, page, off);
+        if (u < turned) {
+          const int j = shift >= 0 ? n & (hd - 1) : n % hd, head = shift >= 0 ? n >> (shift + 3) : n / hd;
+          const float c0 = cs[y].x, c1 = cs[y].y, s0 = sn[y].x, s1 = sn[y].y;
+          const uint32_t a = gt_round2(lo[0] * c0 - hi[0] * s0, lo[1] * c1 - hi[1] * s1), b = gt_round2(lo[0] * s0 + hi[0] * c0, lo[1] * s1 + hi[1] * c1);
+          bf16_t* o = nullptr;
+          if (head < x.nh) o = q_out + ((int64_t)m * x.nh + head) * hd + j;
+          else if (slot >= 0) o = x.k_pages + ((page * x.nkv + (head - x.nh)) * x.page_size + off) * hd + j;
+          if (o) {
+            *reinterpret_cast<uint32_t*>(o) = a;
+            *reinterpret_cast<uint32_t*>(o + half) = b;
+          }
+        } else if (slot >= 0) {
+          const int d = n - turned_heads * hd;                         // column of the v heads
+          bf16_t* o = x.v_pages + (page * x.nkv * hd + d) * (int64_t)x.page_size + off;
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            o[(int64_t)e * x.page_size] = f32_to_bf16(lo[e]);
+            o[(int64_t)(step + e) * x.page_size] = f32_to_bf16(hi[e]);
+          }
+        }
+      }
+  }
 }
 
 // The tiles: NI, MJ, WN, WM, WK, buffers; room for 16 MJ WM rows of A and 16 NI WN of W.  The first ten serve the gated product, all of
@@ -636,8 +701,8 @@ extern "C" int ga_gemm_spread_gated(void* C, int64_t ldc, const void* A, int64_t
     const auto kernel = few && (M <= 32 || cols < 2048) ? gemm_spread_gated_kernel<few, __VA_ARGS__>                                     \
                                                         : gemm_spread_gated_kernel<false, __VA_ARGS__>;                                  \
     if (const int raised = spread_room(kernel, bytes)) return raised;                                                                    \
-    hipLaunchKernelGGL(kernel, GA_SPREAD_GRID(1), dim3(64 * SpreadTile<__VA_ARGS__>::WAVES), bytes, stream, (bf16_t*)C, ldc,             \
-                       (const bf16_t*)A, lda, (const bf16_t*)W, M, cols, K, m_tiles, tile_rows, groups, act);                            \
+    hipLaunchKernelGGL(kernel, GA_SPREAD_GRID(1), dim3(64 * SpreadTile<__VA_ARGS__>::WAVES), bytes, stream, (const bf16_t*)A,            \
+                       (const bf16_t*)W, lda, M, cols, K, m_tiles, tile_rows, groups, cols / 4 / groups, cols / 4 % groups, (bf16_t*)C, ldc, act); \
     return GA_CHECK_LAUNCH();                                                                                                            \
   }
     GA_SPREAD_GATED(CASE)
@@ -665,8 +730,8 @@ extern "C" int ga_gemm_spread_parts(void* C, const void* A, int64_t lda, const v
     if (!spread_fits<__VA_ARGS__>(M, cols / 8, K / 64, m_tiles, groups, tile_rows) || (parts > 1 && per_part % slab)) return -7;         \
     if (const int raised = spread_room(gemm_spread_parts_kernel<__VA_ARGS__>, bytes)) return raised;                                     \
     hipLaunchKernelGGL((gemm_spread_parts_kernel<__VA_ARGS__>), GA_SPREAD_GRID(parts), dim3(64 * SpreadTile<__VA_ARGS__>::WAVES), bytes, \
-                       stream, (float*)C, (const bf16_t*)A, lda, (const bf16_t*)W, M, cols, K, m_tiles, tile_rows, groups,               \
-                       per_part / slab);                                                                                                 \
+                       stream, (const bf16_t*)A, (const bf16_t*)W, (int)lda, M, cols, K, m_tiles, tile_rows, groups, cols / 8 / groups,  \
+                       cols / 8 % groups, per_part / slab, (float*)C);                                                                   \
     return GA_CHECK_LAUNCH();                                                                                                            \
   }
     GA_SPREAD_GATED(CASE) GA_SPREAD_NARROW(CASE)
@@ -691,7 +756,7 @@ extern "C" int ga_qkv_spread(void* q_out, const void* A, int64_t lda, const void
   if (rc) return rc;
   if (spread_check(M, m_tiles, groups)) return -1;
   const SpreadQkv x = {(const bf16_t*)bias, (const int32_t*)positions, (const float*)cos_t, (const float*)sin_t, (const int64_t*)slot_mapping,
-                       (bf16_t*)k_pages, (bf16_t*)v_pages, nh, nkv, hd, page_size, write_kv};
+                       (bf16_t*)k_pages, (bf16_t*)v_pages, nh, nkv, page_size, write_kv};
   int tile_rows;
   switch (shape) {
 #define CASE(n, ...)                                                                                                                     \
@@ -700,7 +765,8 @@ extern "C" int ga_qkv_spread(void* q_out, const void* A, int64_t lda, const void
     constexpr int bytes = SpreadTile<__VA_ARGS__>::LDS;                                                                                  \
     if (const int raised = spread_room(gemm_spread_qkv_kernel<__VA_ARGS__>, bytes)) return raised;                                       \
     hipLaunchKernelGGL((gemm_spread_qkv_kernel<__VA_ARGS__>), GA_SPREAD_GRID(1), dim3(64 * SpreadTile<__VA_ARGS__>::WAVES), bytes,       \
-                       stream, (bf16_t*)q_out, (const bf16_t*)A, lda, (const bf16_t*)W, M, K, m_tiles, tile_rows, groups, x);            \
+                       stream, (const bf16_t*)A, (const bf16_t*)W, (int)lda, K, M, m_tiles, tile_rows, groups, (int)(cols / 8) / groups, \
+                       (int)(cols / 8) % groups, hd, nh + nkv, (bf16_t*)q_out, x);                                                       \
     return GA_CHECK_LAUNCH();                                                                                                            \
   }
     GA_SPREAD_GATED(CASE) GA_SPREAD_NARROW(CASE)
