@@ -12,36 +12,17 @@
 // 151,936 of 1,536 175, 245, 369, 488 -> 165, 189, 220, 265.)
 // It is templated on storage, so that it also serves bfloat16 operands (the kernel tests' oracle and the
 // fallback for shapes the bfloat16 kernels refuse).
-//
 #include "common.h"
 #include <type_traits>
 #include "ginfer_amd.h"   // the entry points below are checked against their declarations
 
 #define GEMM_THREADS 256
 
-// four consecutive elements as floats; `wide`: one load (the address is a multiple of four elements)
+// the first `valid` of four consecutive elements as floats, zeros behind them
 template <typename T>
-__device__ __forceinline__ void load4(float (&v)[4], const T* p, int valid, bool wide);
-template <>
-__device__ __forceinline__ void load4<float>(float (&v)[4], const float* p, int valid, bool wide) {
-  if (wide && valid == 4) {
-    const float4 x = *reinterpret_cast<const float4*>(p);
-    v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
-  } else {
+__device__ __forceinline__ void load4(float (&v)[4], const T* p, int valid) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = i < valid ? p[i] : 0.f;
-  }
-}
-template <>
-__device__ __forceinline__ void load4<bf16_t>(float (&v)[4], const bf16_t* p, int valid, bool wide) {
-  if (wide && valid == 4) {
-    const uint2 x = *reinterpret_cast<const uint2*>(p);
-    v[0] = bf16_to_f32((bf16_t)(x.x & 0xffffu)); v[1] = bf16_to_f32((bf16_t)(x.x >> 16));
-    v[2] = bf16_to_f32((bf16_t)(x.y & 0xffffu)); v[3] = bf16_to_f32((bf16_t)(x.y >> 16));
-  } else {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = i < valid ? bf16_to_f32(p[i]) : 0.f;
-  }
+  for (int i = 0; i < 4; ++i) v[i] = i < valid ? Num<T>::ld(p + i) : 0.f;
 }
 
 // four consecutive elements at any address that an element may have, in one load all the same: the device takes vector loads
@@ -136,9 +117,9 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_nt_matrix_kernel(const TA* 
   auto fetch_carefully = [&](float (&xa)[GA][4], float (&xw)[GW][4], int k0) {
     const int k = k0 + (tid % (TK / 4)) * 4, valid = k < K ? (K - k < 4 ? K - k : 4) : 0;
 #pragma unroll
-    for (int i = 0; i < GA; ++i) load4<TA>(xa[i], pa[i] + k0, valid, false);
+    for (int i = 0; i < GA; ++i) load4<TA>(xa[i], pa[i] + k0, valid);
 #pragma unroll
-    for (int i = 0; i < GW; ++i) load4<TW>(xw[i], pw[i] + k0, valid, false);
+    for (int i = 0; i < GW; ++i) load4<TW>(xw[i], pw[i] + k0, valid);
   };
   auto stage = [&](int b, float (&xa)[GA][4], float (&xw)[GW][4]) {
 #pragma unroll

@@ -40,9 +40,8 @@ int ga_rope_kv_from_parts(void* q_out, const void* parts, int n_parts, const voi
                           int tokens, int nh, int nkv, int hd, int rotary_dim, int page_size, int write_kv,
                           hipStream_t stream);
 
-// ---- gemm.hip: C [M, N] = A [M, K] . W [N, K]^T + bias in true 32-bit: the matrix cores' 32-bit instructions (and plain FMA
-// for 33 to 64 rows of very wide products), every element one accumulator over ascending k: the same bits whichever
-// kernel runs (the 32-bit path; also bfloat16 in)
+// ---- gemm.hip: C [M, N] = A [M, K] . W [N, K]^T + bias in true 32-bit on the matrix cores' 32-bit instructions, every
+// element one accumulator over ascending k: the same bits whichever tile runs (the 32-bit path; also bfloat16 in)
 int ga_gemm_nt(void* C, int64_t ldc, const void* A, int64_t lda, const void* W, const void* bias, int M, int N, int K,
                int in_bf16, int out_bf16, hipStream_t stream);
 

@@ -305,7 +305,7 @@ def paged_attention_generic(q, k_pages, v_pages, block_table, token_entry, posit
 
 
 def gemm_nt(a, w, bias=None, out=None, out_dtype=None):
-    """a [M, K] . w [N, K]^T (+ bias [N]) -> [M, N]; 32-bit accumulation, plain FMA.  a and w share a
+    """a [M, K] . w [N, K]^T (+ bias [N]) -> [M, N]; 32-bit accumulation over ascending k.  a and w share a
     dtype (float32 or bfloat16); out is that dtype or float32."""
     _dev(a, w, bias, out)
     _need(a.dim() == 2 and w.dim() == 2 and a.shape[1] == w.shape[1],
@@ -427,8 +427,8 @@ def gemm_skinny_supported(a, w):
     """Whether the matrix-core kernel for few rows takes these operands (the rows first: every product of a longer step, launched kernel
     by kernel, asks)."""
     return (a.dim() == 2 and 0 < a.shape[0] <= SKINNY_MAX_ROWS and a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
-            and a.shape[1] % 8 == 0 and a.shape[1] < 1 << 23 and a.stride(1) == 1 and a.stride(0) % 8 == 0 and a.stride(0) < 1 << 26
-            and a.data_ptr() % 16 == 0 and w.is_contiguous() and w.data_ptr() % 16 == 0)
+            and a.shape[1] % 8 == 0 and a.shape[1] < 1 << 23 and a.stride(1) == 1 and a.stride(0) % 8 == 0
+            and (a.shape[0] == 1 or a.stride(0) < 1 << 26) and a.data_ptr() % 16 == 0 and w.is_contiguous() and w.data_ptr() % 16 == 0)
 
 
 def gemm_tiles_supported(a, w):
