@@ -392,7 +392,7 @@ class ModelRunner:
     # ---- recorded steps that hold prompt portions
     def _run_padded(self, host, borrow):
         """A step with prompt portions, short enough that the host's launches would take longer than the device's
-        work: it is laid into a recorded step of fixed sizes (token rows by `padded_rows`, entries powers of two, the context
+        work: it is laid into a recorded step of fixed sizes (token rows by `recorded_rows`, entries powers of two, the context
         bucket), recorded the second time such sizes are seen.  Rows and entries beyond the step's own
         are padding: tokens of an extra entry whose one page is page 0, which write nothing to the cache; the tiles
         and single-token records that fill the plan point at the first padding row.  Rows do not mix in any kernel,
@@ -400,8 +400,8 @@ class ModelRunner:
         T, E, R = host["T"], host["E"], len(host["rows"])
         if T + 1 > self._padded_max_rows or E > TUNING.graph_max_rows:
             return None
-        t_pad = padded_rows(T + 1)
-        if t_pad > self._padded_max_rows:
+        t_pad = recorded_rows(T + 1, self._padded_max_rows)
+        if t_pad is None:
             return None
         e_pad = 8                        # entries 8, 16, ... 256
         while e_pad < E:
@@ -596,19 +596,25 @@ def pad_step(host, t_pad, e_pad, width, pad_slot, n_single=None):
 
 
 def padded_rows(rows):
-    """Token rows of the recorded step that `rows` of them are laid into: 64, 128, 256, 384, 512 and on by doubling, few sizes, so that
-    few recorded steps serve many.  384 stands between because a step of 512 takes 8 to 16 % longer for the rows it does not have:
-    290 rows beside each other's arrivals 3,919 -> 3,602 us (1.5B shape), one prompt of 300 3,341 -> 2,988, in 32-bit 14,560 -> 12,280.
-    These lines were drawn when bfloat16 products of 129 to 512 rows were the library's, whose time hardly fell with the rows.  The package's
-    now fall with them, so that sizes between would gain: a step of us now -> as one of 192, 163 rows in ten prompts of the
-    1.5B shape 2,381 -> 2,234, in 32-bit 8,072 -> 7,682, puguzen 759 -> 677, titozen 780 -> 730; as one of 320, 290 rows beside each other's
-    arrivals 3,427 -> 3,365, one prompt of 290 2,804 -> 2,803, in 32-bit 12,590 -> 10,603, puguzen 1,017 -> 985, titozen 1,006 -> 953; as one of
-    448, one prompt of 446 3,194 -> 3,157, in 32-bit 14,750 -> 13,900, puguzen 1,228 -> 1,216.  But the 7B shape, whose steps of 129 to 196 rows run
-    unrecorded at the rows that they have, would be laid into 192: 140 rows 4,690 -> 4,985, 163 4,853 -> 5,000, 190 4,957 -> 4,989."""
+    """64, 128, 256, 384, 512 and on by doubling: which steps are recorded at all goes by these sizes (recorded_rows)."""
     size = 64
     while size < rows:
         size = {256: 384, 384: 512}.get(size, 2 * size)
     return size
+
+
+def recorded_rows(rows, most):
+    """Token rows of the recorded step that `rows` of them are laid into, or None: multiples of 64 up to 512, a size more or two to
+    every one of `padded_rows`, where that one is no larger than `most` (the 7B shape, whose steps of 129 to 196 rows run unrecorded at the rows that
+    they have, would be slower in 192: 140 rows 4,690 -> 4,985 us, 190 4,957 -> 4,989).  The package's products take time by the rows, so that what
+    is padded costs: a step of the 1.5B shape, us, in the sizes of `padded_rows` -> in these: 161 rows in ten prompts 2,146 -> 2,038 (256 -> 192), 290
+    beside each other's arrivals 3,093 -> 3,002 (384 -> 320); when last measured, before later gains of either, 163 rows in 32-bit 8,072 -> 7,682, puguzen
+    759 -> 677, titozen 780 -> 730, 290 in 32-bit 12,590 -> 10,603, puguzen 1,017 -> 985, titozen 1,006 -> 953, one prompt of 446 3,194 -> 3,157, in 32-bit
+    14,750 -> 13,900, puguzen 1,228 -> 1,216.  What it costs: nine sizes to record at the start instead of six."""
+    size = padded_rows(rows)
+    if size > most:
+        return None
+    return -(-rows // 64) * 64 if size <= 512 else size
 
 
 def _context_bucket(max_kv):

@@ -124,3 +124,11 @@ def test_one_length_of_splits_for_contexts_far_apart():
     assert p["decode_info"][:3].tolist() == host["decode_info"].tolist() and host_arrays([40], [0])["decode_info"].shape == (0, 4)
     assert ops.single_tokens_length([99, 59]) == 0 and ops.single_tokens_length([99, 58]) == 100 and ops.single_tokens_length([7]) == 0
     assert host_arrays([1, 1], [99, 59])["decode_info"].tolist() == [[0, 99, 0, 0], [1, 59, 1, 0]]
+
+
+def test_rows_that_a_step_is_laid_into():
+    """Multiples of 64, where the next of the sizes by which steps are recorded is no larger than what a model's steps may have."""
+    from ginfer_amd.engine.runner import recorded_rows
+    assert [recorded_rows(n, 512) for n in (1, 64, 65, 129, 193, 257, 321, 385, 449, 512, 513)] == [64, 64, 128, 192, 256, 320, 384, 448, 512, 512, None]
+    assert [recorded_rows(n, 214) for n in (65, 128, 129, 192)] == [128, 128, None, None]
+    assert [recorded_rows(n, 500) for n in (257, 384, 385)] == [320, 384, None] and recorded_rows(513, 1024) == 1024 and recorded_rows(1, 50) is None
