@@ -446,18 +446,19 @@ __device__ __forceinline__ int longest_span(int longest, int window) {
   return window ? min(longest, ((window < 0 ? -window : window) + 62) / 32 * 32) : longest;
 }
 // ONE: the launch has one split, which is all of a token's keys (its own instantiation: with the length worked out as for several, 64 tokens
-// at 100 to 250, 28 heads in 4 groups, took 8.25 us for 7.9)
-template <bool ONE>
-__global__ __launch_bounds__(64 * DEC_WAVES) void attn_decode_split_kernel(
-    const int4* __restrict__ decode_info, const int32_t* __restrict__ block_table, const bf16_t* __restrict__ q, int64_t q_stride,
-    int table_width, int ps_shift, int nkv, int group, int head_blocks, int window, const bf16_t* __restrict__ k_pages,
-    const bf16_t* __restrict__ v_pages, float scale, const Splits splits, bf16_t* __restrict__ out, int64_t out_stride,
-    float* __restrict__ part_o, float* __restrict__ part_ml, const HeadExtras ex) {
-  __shared__ float o_s[DEC_WAVES][HD][17];
-  __shared__ float m_s[DEC_WAVES][16], l_s[DEC_WAVES][16], mx_s[16], lsum_s[16];
+// at 100 to 250, 28 heads in 4 groups, took 8.25 us for 7.9).  WAVES: of the workgroup, 0: as many as it has, up to PREFILL_WAVES.
+constexpr int dec_lds_floats(int waves) { return waves * (HD * 17 + 32) + 32; }
+template <int WAVES, bool ONE>
+__device__ __forceinline__ void decode_split(
+    float* lds, int ti, int y, int split, const int4* __restrict__ decode_info, const int32_t* __restrict__ block_table,
+    const bf16_t* __restrict__ q, int64_t q_stride, int table_width, int ps_shift, int nkv, int group, int head_blocks, int window,
+    const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ v_pages, float scale, const Splits& splits, bf16_t* __restrict__ out,
+    int64_t out_stride, float* __restrict__ part_o, float* __restrict__ part_ml, const HeadExtras& ex) {
+  constexpr int MOST = WAVES ? WAVES : PREFILL_WAVES;
+  const int waves = WAVES ? WAVES : blockDim.x >> 6;
+  float *o_s = lds, *m_s = o_s + waves * HD * 17, *l_s = m_s + waves * 16, *mx_s = l_s + waves * 16, *lsum_s = mx_s + 16;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;
-  const int ti = blockIdx.x, split = ONE ? 0 : blockIdx.z;
-  const int kvh = blockIdx.y / head_blocks, hb = blockIdx.y % head_blocks;
+  const int kvh = y / head_blocks, hb = y % head_blocks;
   const int nh = nkv * group;
   const int4 info = decode_info[ti];       // (row of the step, position, entry of the block table, longest context or 0): one load
   const int t = __builtin_amdgcn_readfirstlane(info.x), pos = __builtin_amdgcn_readfirstlane(info.y), num_splits = ONE ? 1 : splits.count;
@@ -478,25 +479,27 @@ __global__ __launch_bounds__(64 * DEC_WAVES) void attn_decode_split_kernel(
     const int32_t* bt = block_table + (int64_t)__builtin_amdgcn_readfirstlane(info.z) * table_width;
     // every live column of a decode wavefront sees the same keys: lo..pos
     attend_tiles<1, DECODE_DEPTH>(o, m, l, qr, cpos, clo, k_pages, v_pages, bt, table_width, kvh, nkv, ps_shift, lo,
-                                  pos, lo, pos, begin + 32 * wave, end, 32 * DEC_WAVES, scale, ex.cap);
+                                  pos, lo, pos, begin + 32 * wave, end, 32 * waves, scale, ex.cap);
     finish_sums<1>(l);
   }
   // the wavefronts' states meet: common max, rescaled sums and outputs added in wavefront order
   if (g == 0) {
-    m_s[wave][c] = m[0];
-    l_s[wave][c] = l[0];
+    m_s[wave * 16 + c] = m[0];
+    l_s[wave * 16 + c] = l[0];
   }
   __syncthreads();
   float mx = -INFINITY;
 #pragma unroll
-  for (int w = 0; w < DEC_WAVES; ++w) mx = fmaxf(mx, m_s[w][c]);
+  for (int w = 0; w < MOST; ++w)
+    if (WAVES || w < waves) mx = fmaxf(mx, m_s[w * 16 + c]);
   // per column: the common max and the sum of the rescaled sums, once
   if (threadIdx.x < 16) {
     float lsum = 0.f;
 #pragma unroll
-    for (int w = 0; w < DEC_WAVES; ++w) {
-      const float mw = m_s[w][c];
-      if (mw != -INFINITY) lsum += l_s[w][c] * fast_exp2(mw - mx);
+    for (int w = 0; w < MOST; ++w) {
+      if (!WAVES && w >= waves) break;
+      const float mw = m_s[w * 16 + c];
+      if (mw != -INFINITY) lsum += l_s[w * 16 + c] * fast_exp2(mw - mx);
     }
     mx_s[c] = mx;
     lsum_s[c] = lsum;
@@ -505,15 +508,16 @@ __global__ __launch_bounds__(64 * DEC_WAVES) void attn_decode_split_kernel(
 #pragma unroll
   for (int db = 0; db < DB; ++db)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) o_s[wave][db * 16 + g * 4 + i][c] = o[0][db][i] * f;
+    for (int i = 0; i < 4; ++i) o_s[(wave * HD + db * 16 + g * 4 + i) * 17 + c] = o[0][db][i] * f;
   __syncthreads();
   const int64_t slot_base = ((int64_t)ti * nh + kvh * group + hb * 16) * num_splits + split;
-  for (int idx = threadIdx.x; idx < 16 * HD; idx += 64 * DEC_WAVES) {
+  for (int idx = threadIdx.x; idx < 16 * HD; idx += 64 * waves) {
     const int cc = idx / HD, d = idx % HD;
     if (hb * 16 + cc >= group) continue;
     float acc = 0.f;
 #pragma unroll
-    for (int w = 0; w < DEC_WAVES; ++w) acc += o_s[w][d][cc];
+    for (int w = 0; w < MOST; ++w)
+      if (WAVES || w < waves) acc += o_s[(w * HD + d) * 17 + cc];
     if (num_splits == 1) {
       const int hh = kvh * group + hb * 16 + cc;
       out[(int64_t)t * out_stride + (int64_t)hh * HD + d] = f32_to_bf16(acc / sink_sum(lsum_s[cc], mx_s[cc], ex.sinks, hh) * head_gate(ex, t, hh));
@@ -526,6 +530,17 @@ __global__ __launch_bounds__(64 * DEC_WAVES) void attn_decode_split_kernel(
       }
     }
   }
+}
+
+template <bool ONE>
+__global__ __launch_bounds__(64 * DEC_WAVES) void attn_decode_split_kernel(
+    const int4* __restrict__ decode_info, const int32_t* __restrict__ block_table, const bf16_t* __restrict__ q, int64_t q_stride,
+    int table_width, int ps_shift, int nkv, int group, int head_blocks, int window, const bf16_t* __restrict__ k_pages,
+    const bf16_t* __restrict__ v_pages, float scale, const Splits splits, bf16_t* __restrict__ out, int64_t out_stride,
+    float* __restrict__ part_o, float* __restrict__ part_ml, const HeadExtras ex) {
+  __shared__ float lds[dec_lds_floats(DEC_WAVES)];
+  decode_split<DEC_WAVES, ONE>(lds, blockIdx.x, blockIdx.y, ONE ? 0 : blockIdx.z, decode_info, block_table, q, q_stride, table_width, ps_shift, nkv,
+                               group, head_blocks, window, k_pages, v_pages, scale, splits, out, out_stride, part_o, part_ml, ex);
 }
 
 // grid (decode tokens, nh), WAVES wavefronts: merges the splits of one (token, head).  Wavefront w adds the splits [w EARLY, (w + 1) EARLY) in
@@ -665,33 +680,32 @@ __device__ __forceinline__ void write_rows(const f32x4 (&o)[NB][DB], const float
   }
 }
 
+// Workgroups are handed out in the order of their linear number and go to the 8 XCDs in turn, each with an L2 of its
+// own.  They are renumbered with the grid's y (kv head x head block) running fastest, linear = x * extent of y + y
+// (one to one for any extents): the heaviest tiles of every y go out first, so that in a step of more workgroups than
+// the chip holds the long walks do not start last; and where y's extent divides 8 an XCD sees one y only, its L2
+// holding the keys and values of one kv head instead of all of them.
+struct TilePlace {
+  int x, y;
+  __device__ __forceinline__ TilePlace(int linear, int extent) : x(linear / extent), y(linear % extent) {}
+};
+
 // grid (tiles, nkv * head_blocks); a workgroup holds hpw * splits wavefronts: hpw query heads of one kv
 // head, and for each head `splits` wavefronts that take the key tiles s, s + splits, ... of the same
 // 16*NB rows, so that the longest rows of a causal prompt are not one wavefront's serial work.  The
 // states of a head's wavefronts meet in LDS: wavefront 0 of the head merges and writes the rows.
 // tiles: int32 [n][4] = (entry, first token row of the step, rows (<= 16*NB), first position).
 template <int NB>
-__global__ __launch_bounds__(64 * PREFILL_WAVES) void attn_prefill_kernel(
+__device__ __forceinline__ void prefill_plain(
+    float* lds /* [hpw][splits-1][NB] x { o[HD][17], m[16], l[16] } */, int bx, int by,
     bf16_t* __restrict__ out, int64_t out_stride, const bf16_t* __restrict__ q, int64_t q_stride,
     const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ v_pages,
     const int32_t* __restrict__ block_table, int table_width, const int32_t* __restrict__ tiles, int nh,
     int nkv, int head_blocks, int hpw, int splits, int ps_shift, int window, float scale,
     const int32_t* __restrict__ parts, float* __restrict__ part_o, float* __restrict__ part_ml,
-    const HeadExtras ex) {
-  extern __shared__ float lds[];          // [hpw][splits-1][NB] x { o[HD][17], m[16], l[16] }
+    const HeadExtras& ex) {
   constexpr int STATE = HD * 17 + 32;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;
-  // Workgroups are handed out in the order of their linear number and go to the 8 XCDs in turn, each with an L2 of its
-  // own.  They are renumbered with the grid's y (kv head x head block) running fastest, linear = x * extent of y + y
-  // (one to one for any extents): the heaviest tiles of every y go out first, so that in a step of more workgroups than
-  // the chip holds the long walks do not start last; and where y's extent divides 8 an XCD sees one y only, its L2
-  // holding the keys and values of one kv head instead of all of them.
-  int by = blockIdx.y, bx = blockIdx.x;
-  if (gridDim.y > 1) {
-    const int linear = blockIdx.x + blockIdx.y * gridDim.x;
-    by = linear % gridDim.y;
-    bx = linear / gridDim.y;
-  }
   const int kvh = by / head_blocks, hb = by % head_blocks;
   const int group = nh / nkv;
   const int hl = wave / splits, split = wave % splits;
@@ -775,6 +789,20 @@ __global__ __launch_bounds__(64 * PREFILL_WAVES) void attn_prefill_kernel(
   write_rows<NB>(o, m, l, out, out_stride, part_o, part_ml, kp, row0, rows, head, nh, c, g, ex);
 }
 
+template <int NB>
+__global__ __launch_bounds__(64 * PREFILL_WAVES) void attn_prefill_kernel(
+    bf16_t* __restrict__ out, int64_t out_stride, const bf16_t* __restrict__ q, int64_t q_stride,
+    const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ v_pages,
+    const int32_t* __restrict__ block_table, int table_width, const int32_t* __restrict__ tiles, int nh,
+    int nkv, int head_blocks, int hpw, int splits, int ps_shift, int window, float scale,
+    const int32_t* __restrict__ parts, float* __restrict__ part_o, float* __restrict__ part_ml,
+    const HeadExtras ex) {
+  extern __shared__ float lds[];
+  const TilePlace at(blockIdx.x + blockIdx.y * gridDim.x, gridDim.y);
+  prefill_plain<NB>(lds, at.x, at.y, out, out_stride, q, q_stride, k_pages, v_pages, block_table, table_width, tiles, nh, nkv, head_blocks, hpw, splits, ps_shift, window, scale,
+                    parts, part_o, part_ml, ex);
+}
+
 // ----------------------------------------------------------------------------- prefill, operands through LDS
 // For head sizes of 64, 128 and 256.  The wavefronts of a workgroup that attend the same rows to the same key
 // tiles (the heads of a kv group, side by side) take their K and V operands from LDS, where ONE further
@@ -843,25 +871,19 @@ __device__ __forceinline__ void produce_tile(unsigned char* stage, const bf16_t*
 // grid (tiles, nkv * head_blocks); a workgroup holds hpw * splits consumers (hpw heads, each head's keys dealt
 // to `splits` wavefronts as in the kernel above) and after them `splits` producers, one per stream of tiles.
 template <int NB, int STAGES>
-__global__ __launch_bounds__(64 * PREFILL_WAVES) void attn_prefill_shared_kernel(
+__device__ __forceinline__ void prefill_shared(
+    unsigned char* ring, int bx, int by,
     bf16_t* __restrict__ out, int64_t out_stride, const bf16_t* __restrict__ q, int64_t q_stride,
     const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ v_pages,
     const int32_t* __restrict__ block_table, int table_width, const int32_t* __restrict__ tiles, int nh,
     int nkv, int head_blocks, int hpw, int splits, int ps_shift, int window, float scale,
     const int32_t* __restrict__ parts, float* __restrict__ part_o, float* __restrict__ part_ml,
-    const HeadExtras ex) {
+    const HeadExtras& ex) {
   static_assert(STAGES == 2 || STAGES == 3, "two or three stages");
-  extern __shared__ __attribute__((aligned(16))) unsigned char ring[];
   float* lds = reinterpret_cast<float*>(ring);      // after the loop: [hpw][splits-1][NB] x { o[HD][17], m[16], l[16] }
   constexpr int STATE = HD * 17 + 32;
   const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  int by = blockIdx.y, bx = blockIdx.x;             // renumbered as in the kernel above
-  if (gridDim.y > 1) {
-    const int linear = blockIdx.x + blockIdx.y * gridDim.x;
-    by = linear % gridDim.y;
-    bx = linear / gridDim.y;
-  }
   const int kvh = by / head_blocks, hb = by % head_blocks;
   const int group = nh / nkv;
   const int consumers = hpw * splits;
@@ -1005,7 +1027,70 @@ __global__ __launch_bounds__(64 * PREFILL_WAVES) void attn_prefill_shared_kernel
   }
   write_rows<NB>(o, m, l, out, out_stride, part_o, part_ml, kp, row0, rows, head, nh, c, g, ex);
 }
+
+template <int NB, int STAGES>
+__global__ __launch_bounds__(64 * PREFILL_WAVES) void attn_prefill_shared_kernel(
+    bf16_t* __restrict__ out, int64_t out_stride, const bf16_t* __restrict__ q, int64_t q_stride,
+    const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ v_pages,
+    const int32_t* __restrict__ block_table, int table_width, const int32_t* __restrict__ tiles, int nh,
+    int nkv, int head_blocks, int hpw, int splits, int ps_shift, int window, float scale,
+    const int32_t* __restrict__ parts, float* __restrict__ part_o, float* __restrict__ part_ml,
+    const HeadExtras ex) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char ring[];
+  const TilePlace at(blockIdx.x + blockIdx.y * gridDim.x, gridDim.y);
+  prefill_shared<NB, STAGES>(ring, at.x, at.y, out, out_stride, q, q_stride, k_pages, v_pages, block_table, table_width, tiles, nh, nkv, head_blocks, hpw, splits, ps_shift, window, scale,
+                             parts, part_o, part_ml, ex);
+}
 #endif
+
+// ----------------------------------------------------------------------------- both in one launch
+// A step that holds prompt portions and single tokens: their workgroups share nothing but the launch, which ends when the last of either
+// does, where one kernel behind the other waited twice for workgroups that leave most of the chip idle (and a third time for the merge of the splits:
+// a token's keys are walked by the eight wavefronts that a prompt's workgroup has, so that contexts of some thousand keys need
+// none).  The single tokens' workgroups go out first, then the tiles', each beginning at a multiple of the eight XCDs
+// (us: 12 heads in 2 groups, 32 tokens at 130 to 900 beside prompts of 101 and 157 in a recorded step 12.8 + 10.9 + 4.6 -> 18.0, with the tiles first
+// 25.6, in turn by eights 20.6; 28 heads in 4 groups, 48 tokens at 300 to 1,500 beside 2,000 behind 2,048 cached 129 + 28 -> 135, 135, 188.
+// On streams of their own in the recorded graph the two were slower than one behind the other: a step of the former 3,002 -> 3,070).
+struct SingleTokens {
+  const int4* info;
+  int n, head_blocks, workgroups, tile_workgroups;       // (the last: of the prompts' part)
+  Splits splits;
+  float *part_o, *part_ml;
+};
+template <int NB, int STAGES /* 0: operands straight from memory */>
+__global__ __launch_bounds__(64 * PREFILL_WAVES) void attn_step_kernel(
+    bf16_t* __restrict__ out, int64_t out_stride, const bf16_t* __restrict__ q, int64_t q_stride,
+    const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ v_pages,
+    const int32_t* __restrict__ block_table, int table_width, const int32_t* __restrict__ tiles, int nh,
+    int nkv, int head_blocks, int hpw, int splits, int ps_shift, int window, float scale,
+    int tile_extent, const SingleTokens single, const HeadExtras ex) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char step_lds[];
+  const int first_tile = (single.workgroups + 7) / 8 * 8;
+  const bool tokens = (int)blockIdx.x < first_tile;
+  const int at = tokens ? (int)blockIdx.x : (int)blockIdx.x - first_tile;
+  if (at >= (tokens ? single.workgroups : single.tile_workgroups)) return;
+  if (tokens) {
+    const int group = nh / nkv, ys = nkv * single.head_blocks, rest = at / single.n, ti = at - rest * single.n, split = rest / ys;
+    float* lds = reinterpret_cast<float*>(step_lds);
+#define TOKENS(ONE)                                                                                                                       \
+  decode_split<0, ONE>(lds, ti, rest - split * ys, ONE ? 0 : split, single.info, block_table, q, q_stride, table_width, ps_shift, nkv, group, \
+                       single.head_blocks, window, k_pages, v_pages, scale, single.splits, out, out_stride, single.part_o, single.part_ml, ex)
+    if (single.splits.count > 1) TOKENS(false);
+    else TOKENS(true);
+#undef TOKENS
+    return;
+  }
+  const TilePlace tile(at, tile_extent);
+#if HAVE_PREFILL_SHARED
+  if constexpr (STAGES > 0) {
+    prefill_shared<NB, STAGES>(step_lds, tile.x, tile.y, out, out_stride, q, q_stride, k_pages, v_pages, block_table, table_width, tiles, nh, nkv, head_blocks, hpw, splits, ps_shift, window, scale,
+                               nullptr, nullptr, nullptr, ex);
+    return;
+  }
+#endif
+  prefill_plain<NB>(reinterpret_cast<float*>(step_lds), tile.x, tile.y, out, out_stride, q, q_stride, k_pages, v_pages, block_table, table_width, tiles, nh, nkv, head_blocks, hpw, splits, ps_shift, window, scale,
+                    nullptr, nullptr, nullptr, ex);
+}
 
 // What the kernels take as scale and cap: with capped scores the bound is the scale of the softmax, and scale / bound goes
 // into the tanh.  false: this library was not built for such scores (or for none but such).
@@ -1022,6 +1107,27 @@ static bool bound_scores(float& scale, HeadExtras& ex) {
 extern "C" int ga_attn_head_dim() { return HD; }
 // rows of a prefill tile: 16 or (head sizes up to 128) 32
 extern "C" int ga_attn_prefill_max_tile_rows() { return 16 * PREFILL_NB; }
+
+// no split shorter than a tile for each of a workgroup's wavefronts, unless the caller's own are
+static Splits splits_of(int split_keys, int num_splits, int waves) {
+  return {num_splits, split_keys < 32 * waves ? split_keys : 32 * waves, num_splits > 1 ? 0xffffffffu / (uint32_t)num_splits + 1u : 0u};
+}
+
+static int merge_splits(void* out, int64_t out_stride, const float* workspace_o, const float* workspace_ml, const void* decode_info, int n_tokens,
+                        int nh, int num_splits, const HeadExtras& ex, hipStream_t stream) {
+#define COMBINE(EARLY, WAVES)                                                                                \
+  hipLaunchKernelGGL((attn_decode_combine_kernel<EARLY, WAVES>), dim3(n_tokens, nh), dim3(64 * WAVES), 0, stream, \
+                     workspace_o, workspace_ml, (const int4*)decode_info, nh, num_splits,        \
+                     (bf16_t*)out, out_stride, ex.sinks || ex.gate, ex)
+  if (num_splits <= 8) COMBINE(8, 1);
+  else if (num_splits <= 16) COMBINE(16, 1);
+  else if (num_splits <= 32) COMBINE(32, 1);
+  else if (num_splits <= 64) COMBINE(32, 2);
+  else if (num_splits <= 128) COMBINE(32, 4);
+  else COMBINE(32, 8);
+#undef COMBINE
+  return GA_CHECK_LAUNCH();
+}
 
 // Decode tokens: decode_info holds, for every single new token of the step, int32 x 4 = (its row in the
 // step, its position, its entry of the block table, the longest context that its splits' length is made for or 0: its own).  workspace_o must hold
@@ -1043,9 +1149,7 @@ extern "C" int ga_attn_decode(void* out, int64_t out_stride, const void* q, int6
   if (num_splits > MAX_SPLITS) return -5;
   HeadExtras ex = {(const float*)sinks, cap, (const float*)gate, gate_stride, gate_scale};
   if (!bound_scores(scale, ex)) return -20;
-  // no split shorter than a tile for each wavefront, unless the caller's own are
-  const Splits splits = {num_splits, split_keys < 32 * DEC_WAVES ? split_keys : 32 * DEC_WAVES,
-                         num_splits > 1 ? 0xffffffffu / (uint32_t)num_splits + 1u : 0u};
+  const Splits splits = splits_of(split_keys, num_splits, DEC_WAVES);
   dim3 grid(n_tokens, nkv * head_blocks, num_splits);
 #define SPLIT(ONE)                                                                                           \
   hipLaunchKernelGGL(attn_decode_split_kernel<ONE>, grid, dim3(64 * DEC_WAVES), 0, stream, (const int4*)decode_info, \
@@ -1054,27 +1158,16 @@ extern "C" int ga_attn_decode(void* out, int64_t out_stride, const void* q, int6
                      (float*)workspace_o, (float*)workspace_ml, ex)
   if (num_splits == 1) SPLIT(true); else SPLIT(false);
 #undef SPLIT
-  int rc = GA_CHECK_LAUNCH();
+  const int rc = GA_CHECK_LAUNCH();
   if (rc || num_splits == 1) return rc;
-#define COMBINE(EARLY, WAVES)                                                                                \
-  hipLaunchKernelGGL((attn_decode_combine_kernel<EARLY, WAVES>), dim3(n_tokens, nh), dim3(64 * WAVES), 0, stream, \
-                     (const float*)workspace_o, (const float*)workspace_ml, (const int4*)decode_info, nh, num_splits,        \
-                     (bf16_t*)out, out_stride, ex.sinks || ex.gate, ex)
-  if (num_splits <= 8) COMBINE(8, 1);
-  else if (num_splits <= 16) COMBINE(16, 1);
-  else if (num_splits <= 32) COMBINE(32, 1);
-  else if (num_splits <= 64) COMBINE(32, 2);
-  else if (num_splits <= 128) COMBINE(32, 4);
-  else COMBINE(32, 8);
-#undef COMBINE
-  return GA_CHECK_LAUNCH();
+  return merge_splits(out, out_stride, (const float*)workspace_o, (const float*)workspace_ml, decode_info, n_tokens, nh, num_splits, ex, stream);
 }
 
 static int attn_prefill_tiles(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k_pages,
                               const void* v_pages, const void* block_table, int table_width, const void* tiles,
                               int n_tiles, int tile_rows, int nh, int nkv, int page_size, int window, float scale,
                               int fill_workgroups, int prefer_workgroups, const void* parts, void* part_o,
-                              void* part_ml, const HeadExtras& ex, hipStream_t stream);
+                              void* part_ml, SingleTokens* single, const HeadExtras& ex, hipStream_t stream);
 
 // parts: null, or for every tile int32 x 4 = (first key, end of keys, index of the tile's first row among the rows that
 // come in parts, part + (number of parts << 16)); a tile whose keys are dealt to several workgroups stands in `tiles` once
@@ -1095,24 +1188,56 @@ extern "C" int ga_attn_prefill(void* out, int64_t out_stride, const void* q, int
   if (!parts) n_part_rows = 0;
   int rc = attn_prefill_tiles(out, out_stride, q, q_stride, k_pages, v_pages, block_table, table_width, tiles, n_tiles,
                               tile_rows, nh, nkv, page_size, window, scale, fill_workgroups, prefer_workgroups, parts, part_o,
-                              part_ml, ex, stream);
+                              part_ml, nullptr, ex, stream);
   if (rc || n_part_rows == 0) return rc;
   hipLaunchKernelGGL((attn_decode_combine_kernel<8, 1>), dim3(n_part_rows, nh), dim3(64), 0, stream, (const float*)part_o,
                      (const float*)part_ml, (const int4*)part_rows, nh, num_parts, (bf16_t*)out, out_stride, ex.sinks || ex.gate, ex);
   return GA_CHECK_LAUNCH();
 }
 
+// Single tokens and rows of prompt portions of one step: the two calls above in one launch (no tile in parts), whose workgroups have up to
+// PREFILL_WAVES wavefronts for either.
+extern "C" int ga_attn_step(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k_pages, const void* v_pages,
+                            const void* block_table, int table_width, const void* decode_info, int n_tokens, const void* tiles, int n_tiles,
+                            int tile_rows, int nh, int nkv, int page_size, int window, float scale, int split_keys, int num_splits,
+                            int fill_workgroups, int prefer_workgroups, void* workspace_o, void* workspace_ml, const void* sinks, float cap,
+                            const void* gate, int64_t gate_stride, float gate_scale, hipStream_t stream) {
+  if (n_tokens <= 0 || n_tiles <= 0) return -10;
+  if (nkv <= 0 || nh % nkv) return -1;
+  if (split_keys <= 0 || split_keys % 32 || num_splits <= 0) return -3;
+  if (num_splits > MAX_SPLITS) return -5;
+  HeadExtras ex = {(const float*)sinks, cap, (const float*)gate, gate_stride, gate_scale};
+  if (!bound_scores(scale, ex)) return -20;
+  const int head_blocks = (nh / nkv + 15) / 16;
+  const int64_t workgroups = (int64_t)n_tokens * nkv * head_blocks * num_splits;
+  if (workgroups > 1 << 21) return -9;
+  SingleTokens single = {(const int4*)decode_info, n_tokens, head_blocks, (int)workgroups, 0, splits_of(split_keys, num_splits, PREFILL_WAVES),
+                         (float*)workspace_o, (float*)workspace_ml};
+  const int rc = attn_prefill_tiles(out, out_stride, q, q_stride, k_pages, v_pages, block_table, table_width, tiles, n_tiles, tile_rows, nh, nkv,
+                                    page_size, window, scale, fill_workgroups, prefer_workgroups, nullptr, nullptr, nullptr, &single, ex, stream);
+  if (rc || num_splits == 1) return rc;
+  return merge_splits(out, out_stride, single.part_o, single.part_ml, decode_info, n_tokens, nh, num_splits, ex, stream);
+}
+
 static int attn_prefill_tiles(void* out, int64_t out_stride, const void* q, int64_t q_stride,
                               const void* k_pages, const void* v_pages, const void* block_table,
                               int table_width, const void* tiles, int n_tiles, int tile_rows, int nh, int nkv,
                               int page_size, int window, float scale, int fill_workgroups, int prefer_workgroups,
-                              const void* parts, void* part_o, void* part_ml, const HeadExtras& ex, hipStream_t stream) {
+                              const void* parts, void* part_o, void* part_ml, SingleTokens* single, const HeadExtras& ex,
+                              hipStream_t stream) {
   if (tile_rows != 16 && tile_rows != 16 * PREFILL_NB) return -6;
   int ps_shift = 0;
   while ((1 << ps_shift) < page_size) ++ps_shift;
   if ((1 << ps_shift) != page_size || page_size < 8) return -2;
   const int group = nh / nkv;
   const int nb = tile_rows / 16;
+  // the single tokens' part of a launch of both, whose workgroups have `waves` wavefronts: LDS, and the workgroups of the launch
+  auto beside = [&](int waves, int64_t tile_workgroups, size_t& lds) {
+    const size_t need = dec_lds_floats(waves) * sizeof(float);
+    if (need > lds) lds = need;
+    single->tile_workgroups = (int)tile_workgroups;
+    return (unsigned)(((int64_t)single->workgroups + 7) / 8 * 8 + (tile_workgroups + 7) / 8 * 8);
+  };
 #if defined(HAVE_PREFILL_SHARED) && !defined(PREFILL_SHARED_OFF)
   {
     // at least two heads of a group side by side, and tiles enough to fill the chip with such workgroups: the
@@ -1140,6 +1265,29 @@ static int attn_prefill_tiles(void* out, int64_t out_stride, const void* q, int6
       const size_t merge = (size_t)heads * (streams - 1) * nb * (HD * 17 + 32) * sizeof(float);
       if (merge > lds) lds = merge;
       dim3 grid(n_tiles, nkv * head_blocks), block(64 * (heads + 1) * streams);
+      if (single) {
+        const int64_t of_tiles = (int64_t)n_tiles * nkv * head_blocks;
+        if (of_tiles + single->workgroups > 1 << 22) return -9;
+        const unsigned both = beside((heads + 1) * streams, of_tiles, lds);
+#define LAUNCH_BOTH(NB, ST)                                                                                    \
+  do {                                                                                                         \
+    const void* fn = (const void*)attn_step_kernel<NB, ST>;                                                    \
+    if (lds > 48 * 1024 &&                                                                                     \
+        hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)           \
+      return -7;                                                                                               \
+    hipLaunchKernelGGL((attn_step_kernel<NB, ST>), dim3(both), block, lds, stream, (bf16_t*)out,               \
+                       out_stride, (const bf16_t*)q, q_stride, (const bf16_t*)k_pages, (const bf16_t*)v_pages, \
+                       (const int32_t*)block_table, table_width, (const int32_t*)tiles, nh, nkv, head_blocks,  \
+                       heads, streams, ps_shift, window, scale * LOG2E, nkv * head_blocks, *single, ex);       \
+  } while (0)
+        if (nb == 1) {
+          if (stages == 3) LAUNCH_BOTH(1, 3); else LAUNCH_BOTH(1, 2);
+        } else {
+          if (stages == 3) LAUNCH_BOTH(PREFILL_NB, 3); else LAUNCH_BOTH(PREFILL_NB, 2);
+        }
+#undef LAUNCH_BOTH
+        return GA_CHECK_LAUNCH();
+      }
 #define LAUNCH_SHARED(NB, ST)                                                                                  \
   do {                                                                                                         \
     const void* fn = (const void*)attn_prefill_shared_kernel<NB, ST>;                                          \
@@ -1174,8 +1322,23 @@ static int attn_prefill_tiles(void* out, int64_t out_stride, const void* q, int6
   if (hpw > 1 && splits > 4) splits = 4;
   const int head_blocks = group / hpw;
   if ((int64_t)nkv * head_blocks > 65535) return -4;
-  const size_t lds = (size_t)hpw * (splits - 1) * nb * (HD * 17 + 32) * sizeof(float);
+  size_t lds = (size_t)hpw * (splits - 1) * nb * (HD * 17 + 32) * sizeof(float);
   dim3 grid(n_tiles, nkv * head_blocks), block(64 * hpw * splits);
+  if (single) {
+    const int64_t of_tiles = (int64_t)n_tiles * nkv * head_blocks;
+    if (of_tiles + single->workgroups > 1 << 22) return -9;
+    const unsigned both = beside(hpw * splits, of_tiles, lds);
+    const void* fn = nb == 1 ? (const void*)attn_step_kernel<1, 0> : (const void*)attn_step_kernel<PREFILL_NB, 0>;
+    if (lds > 48 * 1024 && hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return -7;
+#define LAUNCH(NB)                                                                                        \
+  hipLaunchKernelGGL((attn_step_kernel<NB, 0>), dim3(both), block, lds, stream, (bf16_t*)out, out_stride, \
+                     (const bf16_t*)q, q_stride, (const bf16_t*)k_pages, (const bf16_t*)v_pages,          \
+                     (const int32_t*)block_table, table_width, (const int32_t*)tiles, nh, nkv, head_blocks, \
+                     hpw, splits, ps_shift, window, scale * LOG2E, nkv * head_blocks, *single, ex)
+    if (nb == 1) LAUNCH(1); else LAUNCH(PREFILL_NB);
+#undef LAUNCH
+    return GA_CHECK_LAUNCH();
+  }
 #define LAUNCH(NB)                                                                                        \
   hipLaunchKernelGGL(attn_prefill_kernel<NB>, grid, block, lds, stream, (bf16_t*)out, out_stride,         \
                      (const bf16_t*)q, q_stride, (const bf16_t*)k_pages, (const bf16_t*)v_pages,           \

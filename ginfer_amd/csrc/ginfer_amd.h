@@ -222,6 +222,12 @@ int ga_attn_prefill(void* out, int64_t out_stride, const void* q, int64_t q_stri
                     int tile_rows, int nh, int nkv, int page_size, int window, float scale, int fill_workgroups,
                     int prefer_workgroups, const void* parts, const void* part_rows, int n_part_rows, int num_parts, void* part_o,
                     void* part_ml, const void* sinks, float cap, const void* gate, int64_t gate_stride, float gate_scale, hipStream_t stream);
+// both in one launch, no tile in parts; workspaces as ga_attn_decode's
+int ga_attn_step(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k_pages, const void* v_pages,
+                 const void* block_table, int table_width, const void* decode_info, int n_tokens, const void* tiles, int n_tiles,
+                 int tile_rows, int nh, int nkv, int page_size, int window, float scale, int split_keys, int num_splits,
+                 int fill_workgroups, int prefer_workgroups, void* workspace_o, void* workspace_ml, const void* sinks, float cap,
+                 const void* gate, int64_t gate_stride, float gate_scale, hipStream_t stream);
 
 // ---- conv_rope_kv.hip: behind a fused q|k|v projection proj [tokens, (nh + nkv) hd + nkv vd] whose channels pass a
 // causal convolution of `taps` taps over time (w float [channels, taps], or null with taps 1: none; state float [slots,

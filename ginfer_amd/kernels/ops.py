@@ -955,7 +955,9 @@ def single_tokens_length(positions):
     return longest if total < TUNING.decode_own_splits_from_mean * longest * n else 0
 
 
-def _decode_splits(plan, window, nkv, head_blocks):
+def _decode_splits(plan, window, nkv, head_blocks, workgroups=None, least=None):
+    """(keys of a split, splits) of the step's single tokens; workgroups: how many the launch should make of them, least: keys of a
+    split that a launch would rather walk than merge (None: as alone in a launch)"""
     span = 0
     if plan.get("decode_span"):             # a recorded step: the split must fit every context of its bucket
         span = plan["decode_span"] if not window else min(plan["decode_span"], (abs(window) + 62) // 32 * 32)
@@ -964,7 +966,7 @@ def _decode_splits(plan, window, nkv, head_blocks):
             lo = first_visible_key(pos, window or 0)
             span = max(span, pos + 1 - (lo // 32) * 32)
     per_split = plan["n_decode"] * nkv * head_blocks
-    splits = max(1, min(TUNING.decode_target_workgroups // max(per_split, 1), -(-span // TUNING.decode_min_split_keys),
+    splits = max(1, min((workgroups or TUNING.decode_target_workgroups) // max(per_split, 1), -(-span // (least or TUNING.decode_min_split_keys)),
                         TUNING.decode_max_splits))
     split_keys = -(-(-(-span // splits)) // 32) * 32
     return split_keys, -(-span // split_keys)
@@ -973,7 +975,7 @@ def _decode_splits(plan, window, nkv, head_blocks):
 def paged_attention_mfma(q, k_pages, v_pages, block_table, step, num_heads, num_kv_heads, head_dim, scale,
                          window=None, out=None, sinks=None, soft_cap=None, gate=None, gate_scale=1.0):
     """bfloat16 attention of every token of the step on the matrix cores: single new tokens through the
-    split-key kernel, rows of prompt portions through the tiled kernel."""
+    split-key kernel, rows of prompt portions through the tiled kernel, both through one launch where a step holds both."""
     T = _check_attention_operands(q, k_pages, v_pages, block_table, step.token_entry, step.positions, num_heads,
                                   num_kv_heads, head_dim)
     page_size = k_pages.shape[2]
@@ -1002,12 +1004,24 @@ def paged_attention_mfma(q, k_pages, v_pages, block_table, step, num_heads, num_
     _need(out.dtype == q.dtype and out.shape == (T, num_heads * head_dim) and out.stride(1) == 1 and out.stride(0) % 4 == 0
           and out.data_ptr() % 8 == 0, "out must be [T, nh*hd] with rows at 8-byte addresses")
     w = int(window) if window else 0
+    # (the last: the workgroups of the one launch are counted in one dimension)
+    both = (plan["n_decode"] and plan["n_tiles"] and not plan["n_part_rows"]
+            and (plan["n_decode"] + plan["n_tiles"]) * num_heads < 1 << 20)
     if plan["n_decode"]:
         group = num_heads // num_kv_heads
-        split_keys, num_splits = _decode_splits(plan, w, num_kv_heads, -(-group // 16))
+        split_keys, num_splits = _decode_splits(plan, w, num_kv_heads, -(-group // 16),
+                                                *((TUNING.decode_beside_workgroups, TUNING.decode_beside_split_keys) if both else ()))
         n = plan["n_decode"] * num_heads * num_splits
         ws_o = torch.empty((n * head_dim,), dtype=torch.float32, device=q.device)
         ws_ml = torch.empty((n * 2,), dtype=torch.float32, device=q.device)
+    if both:
+        _check(lib.ga_attn_step(
+            _ptr(out), _i64(out.stride(0)), _ptr(q), _i64(q.stride(0)), _ptr(k_pages), _ptr(v_pages), _ptr(block_table),
+            _i(block_table.shape[1]), _ptr(plan["decode_info"]), _i(plan["n_decode"]), _ptr(plan["tiles"]), _i(plan["n_tiles"]), _i(tile_rows),
+            _i(num_heads), _i(num_kv_heads), _i(page_size), _i(w), _f(scale), _i(split_keys), _i(num_splits), _i(_prefill_fill(step, head_dim)),
+            _i(_prefill_prefer(step)), _ptr(ws_o), _ptr(ws_ml), _ptr(sinks), *extras, _stream()), "attn_step")
+        return out
+    if plan["n_decode"]:
         _check(lib.ga_attn_decode(
             _ptr(out), _i64(out.stride(0)), _ptr(q), _i64(q.stride(0)), _ptr(k_pages), _ptr(v_pages), _ptr(block_table),
             _i(block_table.shape[1]), _ptr(plan["decode_info"]), _i(plan["n_decode"]), _i(num_heads), _i(num_kv_heads), _i(page_size), _i(w), _f(scale), _i(split_keys),
