@@ -685,6 +685,13 @@ __device__ __forceinline__ void write_rows(const f32x4 (&o)[NB][DB], const float
 // (one to one for any extents): the heaviest tiles of every y go out first, so that in a step of more workgroups than
 // the chip holds the long walks do not start last; and where y's extent divides 8 an XCD sees one y only, its L2
 // holding the keys and values of one kv head instead of all of them.
+// Whether record i of four numbers is the same as the one in front of it: what fills a recorded step's plan is one record over and over, and
+// done once.  (us a layer: ten prompts of 13 to 19 tokens, 18 of 28 tiles of the plan are such, 8.2 -> 5.9; the step of
+// attn_step_kernel's figures 18.0 -> 16.2.)
+__device__ __forceinline__ bool stands_before(const int32_t* __restrict__ records, int i) {
+  const int32_t *a = records + (int64_t)i * 4, *b = records + (int64_t)max(i - 1, 0) * 4;
+  return i > 0 && a[0] == b[0] && a[1] == b[1] && a[2] == b[2] && a[3] == b[3];
+}
 struct TilePlace {
   int x, y;
   __device__ __forceinline__ TilePlace(int linear, int extent) : x(linear / extent), y(linear % extent) {}
@@ -712,6 +719,7 @@ __device__ __forceinline__ void prefill_plain(
   const bool head_ok = hb * hpw + hl < group;
   const int head = kvh * group + hb * hpw + hl;
   const int32_t* tile = tiles + (int64_t)bx * 4;
+  if (!parts && stands_before(tiles, bx)) return;
   const int entry = tile[0], row0 = tile[1], rows = tile[2], pos0 = tile[3];
   const int kv_min_t = first_visible_key(pos0, window);
   const KeyPart kp = key_part(parts, bx, (kv_min_t / 32) * 32, ((pos0 + rows - 1) / 32 + 1) * 32);
@@ -893,6 +901,7 @@ __device__ __forceinline__ void prefill_shared(
   const bool head_ok = !producer && hb * hpw + hl < group;
   const int head = kvh * group + hb * hpw + hl;
   const int32_t* tile = tiles + (int64_t)bx * 4;
+  if (!parts && stands_before(tiles, bx)) return;
   const int entry = __builtin_amdgcn_readfirstlane(tile[0]), row0 = __builtin_amdgcn_readfirstlane(tile[1]),
             rows = __builtin_amdgcn_readfirstlane(tile[2]), pos0 = __builtin_amdgcn_readfirstlane(tile[3]);
   const int kv_min = first_visible_key(pos0, window);
@@ -1076,7 +1085,7 @@ __global__ __launch_bounds__(64 * PREFILL_WAVES) void attn_step_kernel(
   decode_split<0, ONE>(lds, ti, rest - split * ys, ONE ? 0 : split, single.info, block_table, q, q_stride, table_width, ps_shift, nkv, group, \
                        single.head_blocks, window, k_pages, v_pages, scale, single.splits, out, out_stride, single.part_o, single.part_ml, ex)
     if (single.splits.count > 1) TOKENS(false);
-    else TOKENS(true);
+    else if (!stands_before(reinterpret_cast<const int32_t*>(single.info), ti)) TOKENS(true);
 #undef TOKENS
     return;
   }
