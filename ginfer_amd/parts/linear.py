@@ -28,7 +28,7 @@ def linear(x, weight, bias=None, out_dtype=None, parts_ok=False):
     skinny_ok = ops.gemm_skinny_supported(x, weight)
     wide = float32_out and bias is None and head_is_wide(x.shape[0], weight.shape[0], x.shape[1])
     tiles_ok = ((wide or (parts_ok and bias is None and not float32_out and TUNING.library_from_rows < x.shape[0]
-                          <= max(TUNING.tiles_parts_most_rows, TUNING.spread_parts_most_rows)))
+                          <= max(TUNING.tiles_parts_most_rows, TUNING.spread_parts_most_rows, TUNING.spread_parts_few_columns_most_rows)))
                 and ops.gemm_tiles_supported(x, weight))      # the rows first: steps launched kernel by kernel wait for the host
     plan = None
     if autotune.active():
@@ -76,13 +76,16 @@ def spread_parts(plan, rows, out_features, in_features):
     """The plan of a product whose parts of K the consumer adds, over tiles that are dealt evenly to the chip, where it is faster than `plan`,
     the other rules' (by sizes alone; the measurements stand beside the thresholds); else None."""
     T = TUNING
-    if (not T.library_from_rows < rows <= T.spread_parts_most_rows or out_features % 16 or in_features % 64
-            or in_features < T.spread_parts_min_in_features):
+    few_columns = out_features <= T.spread_parts_few_columns
+    if (not T.library_from_rows < rows <= (T.spread_parts_few_columns_most_rows if few_columns else T.spread_parts_most_rows)
+            or out_features % 16 or in_features % 64 or in_features < T.spread_parts_min_in_features):
         return None
     if plan[0] == "skinny" and (rows <= T.spread_parts_beyond_rows or (in_features % 128 and out_features < T.spread_parts_half_min_out_features
                                                                        and in_features < T.spread_parts_half_min_in_features)):
         return None
-    if rows > T.spread_parts_many_rows and in_features <= T.spread_parts_short_k:
+    if rows > T.spread_parts_many_rows and in_features <= T.spread_parts_short_k and not few_columns:
+        return None
+    if rows > T.spread_parts_most_rows and out_features * in_features >= T.spread_parts_few_columns_weights:
         return None
     if (plan[0] == "library" and out_features * in_features > T.spread_parts_library_weights
             and T.spread_parts_library_from_rows < rows <= T.spread_parts_many_rows):
