@@ -543,21 +543,32 @@ __global__ __launch_bounds__(64 * DEC_WAVES) void attn_decode_split_kernel(
                                group, head_blocks, window, k_pages, v_pages, scale, splits, out, out_stride, part_o, part_ml, ex);
 }
 
+// Whether record i of four numbers is the same as the one in front of it: what fills a recorded step's plan is one record over and over, and
+// done once.  (us a layer: ten prompts of 13 to 19 tokens, 18 of 28 tiles of the plan are such, 8.2 -> 5.9; the step of
+// attn_step_kernel's figures 18.0 -> 16.2.)
+__device__ __forceinline__ bool stands_before(const int32_t* __restrict__ records, int i) {
+  const int32_t *a = records + (int64_t)i * 4, *b = records + (int64_t)max(i - 1, 0) * 4;
+  return i > 0 && a[0] == b[0] && a[1] == b[1] && a[2] == b[2] && a[3] == b[3];
+}
+
 // grid (decode tokens, nh), WAVES wavefronts: merges the splits of one (token, head).  Wavefront w adds the splits [w EARLY, (w + 1) EARLY) in
 // ascending order, and the wavefronts' sums are added in theirs.  What bounds it is the way to memory: every partial output that a
 // lane will need is asked for at once, before the weights are worked out.  (More than 32 splits went through one wavefront, 8 at a
 // time; a decode step of one token at 16,000 with 128 of them 1,467 us, now 1,440.  Which splits have no keys is not asked either:
 // waiting for the token's position before the loads cost 0.7 us of a launch, and reading what nobody wrote 1.1.)
 #define MAX_SPLITS 256
+#define MERGE_EXTRAS 1               // there are sinks or gates
+#define MERGE_ONCE 2                 // a token that stands twice in a row is merged once (its splits were left out)
 template <int EARLY, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void attn_decode_combine_kernel(
     const float* __restrict__ part_o, const float* __restrict__ part_ml, const int4* __restrict__ decode_info, int nh, int num_splits,
-    bf16_t* __restrict__ out, int64_t out_stride, int special, const HeadExtras ex) {
+    bf16_t* __restrict__ out, int64_t out_stride, int how, const HeadExtras ex) {
   static_assert(WAVES == 1 || EARLY == 32, "a wavefront's splits");
   constexpr int DPL = (HD + 63) / 64, SLOTS = WAVES * EARLY;
   __shared__ float w_s[SLOTS];
   __shared__ float sums_s[WAVES > 1 ? WAVES : 1][WAVES > 1 ? DPL * 64 : 1];
   const int ti = blockIdx.x, head = blockIdx.y, lane = threadIdx.x & 63;
+  if ((how & MERGE_ONCE) && stands_before(reinterpret_cast<const int32_t*>(decode_info), ti)) return;
   const int s0 = WAVES == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * EARLY;      // a scalar: 64 addresses hang on it
   const int64_t base = ((int64_t)ti * nh + head) * num_splits;
   // (a buffer as long as the splits: what lies behind them comes as zeros, without an address worked out for it)
@@ -596,8 +607,8 @@ __global__ __launch_bounds__(64 * WAVES) void attn_decode_combine_kernel(
   total = wave_sum(total);
   __syncthreads();
   row = __builtin_amdgcn_readfirstlane(row);
-  float inv = 1.f;                           // (special: there are sinks or gates; without them `ex` is not asked for)
-  if (special) inv = 1.f / sink_sum(total, mx, ex.sinks, head) * head_gate(ex, row, head);
+  float inv = 1.f;                           // (without sinks and gates `ex` is not asked for)
+  if (how & MERGE_EXTRAS) inv = 1.f / sink_sum(total, mx, ex.sinks, head) * head_gate(ex, row, head);
   else inv = 1.f / total;
   bf16_t* op = out + (int64_t)row * out_stride + (int64_t)head * HD;
 #pragma unroll
@@ -685,13 +696,6 @@ __device__ __forceinline__ void write_rows(const f32x4 (&o)[NB][DB], const float
 // (one to one for any extents): the heaviest tiles of every y go out first, so that in a step of more workgroups than
 // the chip holds the long walks do not start last; and where y's extent divides 8 an XCD sees one y only, its L2
 // holding the keys and values of one kv head instead of all of them.
-// Whether record i of four numbers is the same as the one in front of it: what fills a recorded step's plan is one record over and over, and
-// done once.  (us a layer: ten prompts of 13 to 19 tokens, 18 of 28 tiles of the plan are such, 8.2 -> 5.9; the step of
-// attn_step_kernel's figures 18.0 -> 16.2.)
-__device__ __forceinline__ bool stands_before(const int32_t* __restrict__ records, int i) {
-  const int32_t *a = records + (int64_t)i * 4, *b = records + (int64_t)max(i - 1, 0) * 4;
-  return i > 0 && a[0] == b[0] && a[1] == b[1] && a[2] == b[2] && a[3] == b[3];
-}
 struct TilePlace {
   int x, y;
   __device__ __forceinline__ TilePlace(int linear, int extent) : x(linear / extent), y(linear % extent) {}
@@ -1084,8 +1088,9 @@ __global__ __launch_bounds__(64 * PREFILL_WAVES) void attn_step_kernel(
 #define TOKENS(ONE)                                                                                                                       \
   decode_split<0, ONE>(lds, ti, rest - split * ys, ONE ? 0 : split, single.info, block_table, q, q_stride, table_width, ps_shift, nkv, group, \
                        single.head_blocks, window, k_pages, v_pages, scale, single.splits, out, out_stride, single.part_o, single.part_ml, ex)
-    if (single.splits.count > 1) TOKENS(false);
-    else if (!stands_before(reinterpret_cast<const int32_t*>(single.info), ti)) TOKENS(true);
+    if (stands_before(reinterpret_cast<const int32_t*>(single.info), ti)) return;
+    if (single.splits.count == 1) TOKENS(true);
+    else TOKENS(false);
 #undef TOKENS
     return;
   }
@@ -1123,11 +1128,12 @@ static Splits splits_of(int split_keys, int num_splits, int waves) {
 }
 
 static int merge_splits(void* out, int64_t out_stride, const float* workspace_o, const float* workspace_ml, const void* decode_info, int n_tokens,
-                        int nh, int num_splits, const HeadExtras& ex, hipStream_t stream) {
+                        int nh, int num_splits, int once, const HeadExtras& ex, hipStream_t stream) {
+  const int how = (ex.sinks || ex.gate ? MERGE_EXTRAS : 0) | once;
 #define COMBINE(EARLY, WAVES)                                                                                \
   hipLaunchKernelGGL((attn_decode_combine_kernel<EARLY, WAVES>), dim3(n_tokens, nh), dim3(64 * WAVES), 0, stream, \
                      workspace_o, workspace_ml, (const int4*)decode_info, nh, num_splits,        \
-                     (bf16_t*)out, out_stride, ex.sinks || ex.gate, ex)
+                     (bf16_t*)out, out_stride, how, ex)
   if (num_splits <= 8) COMBINE(8, 1);
   else if (num_splits <= 16) COMBINE(16, 1);
   else if (num_splits <= 32) COMBINE(32, 1);
@@ -1169,7 +1175,7 @@ extern "C" int ga_attn_decode(void* out, int64_t out_stride, const void* q, int6
 #undef SPLIT
   const int rc = GA_CHECK_LAUNCH();
   if (rc || num_splits == 1) return rc;
-  return merge_splits(out, out_stride, (const float*)workspace_o, (const float*)workspace_ml, decode_info, n_tokens, nh, num_splits, ex, stream);
+  return merge_splits(out, out_stride, (const float*)workspace_o, (const float*)workspace_ml, decode_info, n_tokens, nh, num_splits, 0, ex, stream);
 }
 
 static int attn_prefill_tiles(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k_pages,
@@ -1200,7 +1206,7 @@ extern "C" int ga_attn_prefill(void* out, int64_t out_stride, const void* q, int
                               part_ml, nullptr, ex, stream);
   if (rc || n_part_rows == 0) return rc;
   hipLaunchKernelGGL((attn_decode_combine_kernel<8, 1>), dim3(n_part_rows, nh), dim3(64), 0, stream, (const float*)part_o,
-                     (const float*)part_ml, (const int4*)part_rows, nh, num_parts, (bf16_t*)out, out_stride, ex.sinks || ex.gate, ex);
+                     (const float*)part_ml, (const int4*)part_rows, nh, num_parts, (bf16_t*)out, out_stride, ex.sinks || ex.gate ? MERGE_EXTRAS : 0, ex);
   return GA_CHECK_LAUNCH();
 }
 
@@ -1225,7 +1231,7 @@ extern "C" int ga_attn_step(void* out, int64_t out_stride, const void* q, int64_
   const int rc = attn_prefill_tiles(out, out_stride, q, q_stride, k_pages, v_pages, block_table, table_width, tiles, n_tiles, tile_rows, nh, nkv,
                                     page_size, window, scale, fill_workgroups, prefer_workgroups, nullptr, nullptr, nullptr, &single, ex, stream);
   if (rc || num_splits == 1) return rc;
-  return merge_splits(out, out_stride, single.part_o, single.part_ml, decode_info, n_tokens, nh, num_splits, ex, stream);
+  return merge_splits(out, out_stride, single.part_o, single.part_ml, decode_info, n_tokens, nh, num_splits, MERGE_ONCE, ex, stream);
 }
 
 static int attn_prefill_tiles(void* out, int64_t out_stride, const void* q, int64_t q_stride,

@@ -955,9 +955,8 @@ def single_tokens_length(positions):
     return longest if total < TUNING.decode_own_splits_from_mean * longest * n else 0
 
 
-def _decode_splits(plan, window, nkv, head_blocks, workgroups=None, least=None):
-    """(keys of a split, splits) of the step's single tokens; workgroups: how many the launch should make of them, least: keys of a
-    split that a launch would rather walk than merge (None: as alone in a launch)"""
+def _decode_splits(plan, window, nkv, head_blocks, beside=False):
+    """(keys of a split, splits) of the step's single tokens; beside: in one launch with rows of prompt portions"""
     span = 0
     if plan.get("decode_span"):             # a recorded step: the split must fit every context of its bucket
         span = plan["decode_span"] if not window else min(plan["decode_span"], (abs(window) + 62) // 32 * 32)
@@ -966,8 +965,11 @@ def _decode_splits(plan, window, nkv, head_blocks, workgroups=None, least=None):
             lo = first_visible_key(pos, window or 0)
             span = max(span, pos + 1 - (lo // 32) * 32)
     per_split = plan["n_decode"] * nkv * head_blocks
-    splits = max(1, min((workgroups or TUNING.decode_target_workgroups) // max(per_split, 1), -(-span // (least or TUNING.decode_min_split_keys)),
-                        TUNING.decode_max_splits))
+    unsplit, least = 0, TUNING.decode_min_split_keys
+    if beside:
+        unsplit = TUNING.decode_beside_unsplit_keys
+        least = least if plan.get("decode_span") else max(least, unsplit)
+    splits = max(1, min(TUNING.decode_target_workgroups // max(per_split, 1), -(-span // least), TUNING.decode_max_splits)) if span > unsplit else 1
     split_keys = -(-(-(-span // splits)) // 32) * 32
     return split_keys, -(-span // split_keys)
 
@@ -1009,8 +1011,7 @@ def paged_attention_mfma(q, k_pages, v_pages, block_table, step, num_heads, num_
             and (plan["n_decode"] + plan["n_tiles"]) * num_heads < 1 << 20)
     if plan["n_decode"]:
         group = num_heads // num_kv_heads
-        split_keys, num_splits = _decode_splits(plan, w, num_kv_heads, -(-group // 16),
-                                                *((TUNING.decode_beside_workgroups, TUNING.decode_beside_split_keys) if both else ()))
+        split_keys, num_splits = _decode_splits(plan, w, num_kv_heads, -(-group // 16), both)
         n = plan["n_decode"] * num_heads * num_splits
         ws_o = torch.empty((n * head_dim,), dtype=torch.float32, device=q.device)
         ws_ml = torch.empty((n * 2,), dtype=torch.float32, device=q.device)
