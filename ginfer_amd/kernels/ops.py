@@ -955,8 +955,9 @@ def single_tokens_length(positions):
     return longest if total < TUNING.decode_own_splits_from_mean * longest * n else 0
 
 
-def _decode_splits(plan, window, nkv, head_blocks, beside=False):
-    """(keys of a split, splits) of the step's single tokens; beside: in one launch with rows of prompt portions"""
+def _decode_splits(plan, window, nkv, head_blocks, unsplit=0, least=0):
+    """(keys of a split, splits) of the step's single tokens; unsplit: the most keys that go in one split however few workgroups that makes;
+    least: keys of a split, where that is more than alone in a launch"""
     span = 0
     if plan.get("decode_span"):             # a recorded step: the split must fit every context of its bucket
         span = plan["decode_span"] if not window else min(plan["decode_span"], (abs(window) + 62) // 32 * 32)
@@ -965,11 +966,8 @@ def _decode_splits(plan, window, nkv, head_blocks, beside=False):
             lo = first_visible_key(pos, window or 0)
             span = max(span, pos + 1 - (lo // 32) * 32)
     per_split = plan["n_decode"] * nkv * head_blocks
-    unsplit, least = 0, TUNING.decode_min_split_keys
-    if beside:
-        unsplit = TUNING.decode_beside_unsplit_keys
-        least = least if plan.get("decode_span") else max(least, unsplit)
-    splits = max(1, min(TUNING.decode_target_workgroups // max(per_split, 1), -(-span // least), TUNING.decode_max_splits)) if span > unsplit else 1
+    splits = max(1, min(TUNING.decode_target_workgroups // max(per_split, 1), -(-span // max(TUNING.decode_min_split_keys, least)),
+                        TUNING.decode_max_splits)) if span > unsplit else 1
     split_keys = -(-(-(-span // splits)) // 32) * 32
     return split_keys, -(-span // split_keys)
 
@@ -1011,7 +1009,8 @@ def paged_attention_mfma(q, k_pages, v_pages, block_table, step, num_heads, num_
             and (plan["n_decode"] + plan["n_tiles"]) * num_heads < 1 << 20)
     if plan["n_decode"]:
         group = num_heads // num_kv_heads
-        split_keys, num_splits = _decode_splits(plan, w, num_kv_heads, -(-group // 16), both)
+        unsplit = TUNING.decode_beside_unsplit_keys if both else 0
+        split_keys, num_splits = _decode_splits(plan, w, num_kv_heads, -(-group // 16), unsplit, 0 if "static_plan" in (step.extra or {}) else unsplit)
         n = plan["n_decode"] * num_heads * num_splits
         ws_o = torch.empty((n * head_dim,), dtype=torch.float32, device=q.device)
         ws_ml = torch.empty((n * 2,), dtype=torch.float32, device=q.device)
@@ -1331,7 +1330,8 @@ def _decay_split(step, tokens, entries, heads, dim, vdim, chunked, turned=False)
     """(way of the walk or None, its longest entry, tokens from which on an entry goes in chunks or None)"""
     lens = getattr(step, "host_q_len", None)
     known = lens is not None and len(lens) == entries and "static_plan" not in (getattr(step, "extra", None) or {})
-    least = decay_in_chunks(lens, dim) if chunked and known else None
+    fits = heads <= 65535 and vdim <= 65536              # of the chunks' grids
+    least = decay_in_chunks(lens, dim) if chunked and known and fits else None
     if least is None:
         return _walk_of(step, tokens, entries, heads, dim, vdim, turned), _ALL, None
     short = [n for n in lens if 0 < n < least]

@@ -98,11 +98,11 @@ def test_which_entries_go_in_chunks():
     assert ops.decay_in_chunks([4096], ops.DECAY_CHUNK_MAX_DIM + 1) is None and ops.decay_in_chunks([], 64) is None
     assert ops.decay_in_chunks([700] * 7, 32) is None and ops.decay_in_chunks([700] * 7, 64) is not None
 
-    def split(lens, chunked=True, extra=None, dim=64):
+    def split(lens, chunked=True, extra=None, dim=64, vdim=128):
         step = _Step(lens, [0] * len(lens))
         step.extra = extra or {}
-        return ops._decay_split(step, sum(lens), len(lens), 12, dim, 128, chunked)
+        return ops._decay_split(step, sum(lens), len(lens), 12, dim, vdim, chunked)
     assert split([2048]) == (None, 0, T.decay_chunk_least)                 # nothing to walk
     assert split([2048, 1, 1]) == (1, T.decay_chunk_least - 1, T.decay_chunk_least)
-    for walked in (split([2048], chunked=False), split([2048], extra={"static_plan": {}}), split([100, 1])):
+    for walked in (split([2048], chunked=False), split([2048], extra={"static_plan": {}}), split([100, 1]), split([2048], vdim=65537)):
         assert walked[1:] == (ops._ALL, None)
